@@ -2,6 +2,7 @@
 // unpacked activations themselves.
 #pragma once
 #include "common.h"
+#include <type_traits>
 
 namespace bgemm {
 
@@ -36,6 +37,53 @@ __device__ __forceinline__ void bits8(const uint4 v, uint32_t& sg, uint32_t& nz)
         nz |= (z >> (8 + 2 * i)) | (z >> (25 + 2 * i));
     }
     sg &= 0xffu; nz &= 0xffu;
+}
+
+// Sign (and nonzero) bits of eight fp32 values as their fp16 roundings have them (`.to(torch.half)`): the rounding keeps
+// the sign, and gives zero up to and including 2^-25 (half the smallest fp16 number, a tie that goes to even).
+__device__ __forceinline__ void bits8(const float (&f)[8], uint32_t& sg, uint32_t& nz)
+{
+    sg = 0; nz = 0;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const uint32_t u = __float_as_uint(f[e]);
+        sg = (sg << 1) | (u >> 31);
+        nz = (nz << 1) | (uint32_t)((u & 0x7fffffffu) > 0x33000000u);
+    }
+}
+
+// Eight consecutive elements of a source row as loaded: one 16-byte load (fp16) or two (fp32), at element alignment
+// (the hardware takes vector loads at any address).
+template <bool F32> struct Raw8 { uint4 v[F32 ? 2 : 1]; };
+
+template <bool F32>
+__device__ __forceinline__ Raw8<F32> load_raw8(const void* row, const int64_t k)
+{
+    typedef typename std::conditional<F32, uint32_t, uint16_t>::type E;
+    Raw8<F32> r;
+    __builtin_memcpy(&r, reinterpret_cast<const E*>(row) + k, sizeof r);
+    return r;
+}
+
+// Their sign and nonzero bits, element e at bit 7 - e, after subtracting the zero point if there is one.
+template <bool F32>
+__device__ __forceinline__ void bits8(const Raw8<F32>& r, const bool centred, const float zf, uint32_t& sg, uint32_t& nz)
+{
+    if constexpr (F32) {
+        const uint32_t d[8] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w, r.v[1].x, r.v[1].y, r.v[1].z, r.v[1].w};
+        float f[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) f[e] = centred ? __fsub_rn(__uint_as_float(d[e]), zf) : __uint_as_float(d[e]);
+        bits8(f, sg, nz);
+    } else if (centred) {
+        const uint32_t d[4] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w};
+        float f[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            f[e] = __fsub_rn(__half2float(__ushort_as_half((uint16_t)(d[e >> 1] >> (16 * (e & 1))))), zf);
+        bits8(f, sg, nz);
+    } else
+        bits8(r.v[0], sg, nz);
 }
 
 // fp16 bit patterns of elements k0 .. k0 + 7 of one source row (fp16, or fp32 rounded to fp16 as
