@@ -12,7 +12,7 @@ namespace bgemm {
 
 // One operand to pack.  mode bit3: tiled output written by the row-segment waves (small operands:
 // sixteen times as many, shorter waves).  mode bit0: also write the (sign & nonzero) plane and make plane 0 the
-// nonzero plane.  mode bit1: write the logical layout instead of the tiled one.  mode bit2: the
+// nonzero plane; mode bit4: plane 0 = sign, plane 1 = nonzero.  mode bit1: write the logical layout instead of the tiled one.  mode bit2: the
 // source is fp32 (rounded to fp16 first, as the layers' `.to(torch.half)` does).
 // zp: device scalar of the source type subtracted before that rounding, or null.
 // A job may hold nmat = outer x inner matrices of `rows` rows each (tiled output only): matrix (o, i) starts
@@ -61,8 +61,8 @@ __device__ __forceinline__ void pack_wave(const PackJob& j, const int64_t gw, co
             bits8(h, sg, nz);
         }
     }
-    const bool ternary = j.mode & 1;
-    uint32_t p0 = ternary ? nz : sg, p1 = sg & nz;
+    const bool ternary = j.mode & (1 | 16);
+    uint32_t p0 = j.mode & 1 ? nz : sg, p1 = j.mode & 16 ? nz : sg & nz;
     const int sh = 8 * (3 - (lane & 3));
     p0 <<= sh; p1 <<= sh;
     p0 |= __shfl_xor(p0, 1); p0 |= __shfl_xor(p0, 2);
@@ -97,7 +97,8 @@ __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, co
         off0 = o * j.so + i * j.si + rtl * TILE_ROWS * j.ld;
         rows_left = j.rows - rtl * TILE_ROWS;
     }
-    const bool ternary = j.mode & 1, centred = j.zp != nullptr;
+    const bool ternary = j.mode & (1 | 16), centred = j.zp != nullptr;      // two planes are written
+    const bool nz_first = j.mode & 1, nz_second = j.mode & 16;
     float zf = 0.f;
     if (centred) zf = F32 ? *reinterpret_cast<const float*>(j.zp) : __half2float(*reinterpret_cast<const __half*>(j.zp));
     const int64_t left = j.K - kt * TILE_KBITS;
@@ -128,8 +129,8 @@ __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, co
                     bits8(raw[jj], centred, zf, sg, nz);
                     const uint32_t keep = r <= last_row ? 0xffu : 0u;
                     sg = (sg << shift) & keep; nz = (nz << shift) & keep;
-                    lds[b0 + r * 16] = (unsigned char)(ternary ? nz : sg);
-                    if (ternary) lds[1024 + b0 + r * 16] = (unsigned char)(sg & nz);
+                    lds[b0 + r * 16] = (unsigned char)(nz_first ? nz : sg);
+                    if (ternary) lds[1024 + b0 + r * 16] = (unsigned char)(nz_second ? nz : sg & nz);
                 }
             }
         };
@@ -145,8 +146,8 @@ __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, co
             uint32_t sg, nz;
             load8_as_half(src + (int64_t)(r < last_row ? r : last_row) * j.ld, F32, r <= last_row ? 8 * c : j.K, j.K, centred, zf, h);
             bits8(h, sg, nz);
-            lds[b0 + r * 16] = (unsigned char)(ternary ? nz : sg);
-            if (ternary) lds[1024 + b0 + r * 16] = (unsigned char)(sg & nz);
+            lds[b0 + r * 16] = (unsigned char)(nz_first ? nz : sg);
+            if (ternary) lds[1024 + b0 + r * 16] = (unsigned char)(nz_second ? nz : sg & nz);
         }
     }
     __builtin_amdgcn_wave_barrier();       // the tile was written by this wave alone: LDS keeps its order
@@ -195,7 +196,7 @@ static int make_job(PackJob* j, const void* src, int64_t rows, int64_t K, int64_
                     (long long)inner, (long long)so, (long long)si);
     memset(j, 0, sizeof *j);
     if (rows == 0 || K == 0 || outer * inner == 0) return BGEMM_OK;
-    if (!src || !d0 || ((mode & 1) && !d1)) return fail(BGEMM_ENULL, "%s: null pointer", who);
+    if (!src || !d0 || ((mode & (1 | 16)) && !d1)) return fail(BGEMM_ENULL, "%s: null pointer", who);
     if (((uintptr_t)d0 & 15) || ((uintptr_t)d1 & 15)) return fail(BGEMM_EALIGN, "%s: destination not 16-byte aligned", who);
     j->src = src; j->zp = zp; j->rows = rows; j->K = K; j->ld = ld;
     j->dst0 = (uint32_t*)d0; j->dst1 = (uint32_t*)d1; j->mode = mode;
@@ -287,6 +288,19 @@ extern "C" int bgemm_pack_batched(const void* src, int src_dtype, int ternary, c
     return pack_common(src, rows, K, ld, dst0_tiled, ternary ? dst1_tiled : nullptr,
                        (ternary ? 1 : 0) | (src_dtype == BGEMM_SRC_F32 ? 4 : 0), zero_point, (hipStream_t)stream,
                        "bgemm_pack_batched", batch_outer, batch_inner, stride_outer, stride_inner);
+}
+
+extern "C" int bgemm_pack_sign_nonzero_pair(const void* src_a, int64_t rows_a, int64_t ld_a, const void* zero_point_a, void* sign_a,
+                                            void* nonzero_a, const void* src_b, int64_t rows_b, int64_t ld_b, const void* zero_point_b,
+                                            void* sign_b, void* nonzero_b, int src_dtype, int64_t K, void* stream)
+{
+    const char* who = "bgemm_pack_sign_nonzero_pair";
+    if (src_dtype != BGEMM_SRC_F16 && src_dtype != BGEMM_SRC_F32) return fail(BGEMM_EINVAL, "%s: unknown source type %d", who, src_dtype);
+    const int mode = 16 | (src_dtype == BGEMM_SRC_F32 ? 4 : 0);
+    PackJob j0, j1;
+    int rc = make_job(&j0, src_a, rows_a, K, ld_a, sign_a, nonzero_a, mode, zero_point_a, who);
+    if (!rc) rc = make_job(&j1, src_b, rows_b, K, ld_b, sign_b, nonzero_b, mode, zero_point_b, who);
+    return rc ? rc : launch_jobs(j0, j1, (hipStream_t)stream, who);
 }
 
 namespace bgemm {

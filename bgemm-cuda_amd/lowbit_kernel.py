@@ -467,6 +467,57 @@ class DecodeChain:
             _b.check(_b.lib().bgemm_chain_status(self.workspace(N).data_ptr(), _stream()))
 
 
+# ---- training the binary Linear (bgemm_linear.py's layers call these) -----------------------------------------
+def pack_linear_operands(x, w, zpa, zpw):
+    """Sign and nonzero planes of ``(x - zpa).to(half)`` [N, K] and ``(w - zpw).to(half)`` [M, K], one launch for both
+    operands.  Returns two int32 tensors [2, words]: row 0 the sign plane, row 1 the nonzero plane."""
+    L = _b.lib()
+    xp = torch.empty((2, L.bgemm_tiled_words(x.shape[0], x.shape[1])), dtype=torch.int32, device=x.device)
+    wp = torch.empty((2, L.bgemm_tiled_words(w.shape[0], w.shape[1])), dtype=torch.int32, device=x.device)
+    with _on(x.device):
+        a, b = xp.data_ptr(), wp.data_ptr()
+        _b.check(L.bgemm_pack_sign_nonzero_pair(
+            x.data_ptr(), x.shape[0], x.stride(0), zpa.data_ptr(), a, a + 4 * xp.shape[1],
+            w.data_ptr(), w.shape[0], w.stride(0), zpw.data_ptr(), b, b + 4 * wp.shape[1],
+            SRC_F32 if x.dtype == torch.float32 else SRC_F16, x.shape[1], _stream()))
+    return xp, wp
+
+
+def unpack_signs(xp, N, wp, M, K, need_x=True, need_w=True):
+    """The fp16 matrices of -1, 0, +1 that the planes of ``pack_linear_operands`` stand for (None where not needed)."""
+    xs = torch.empty((N, K), dtype=torch.half, device=xp.device) if need_x else None
+    ws = torch.empty((M, K), dtype=torch.half, device=xp.device) if need_w else None
+    with _on(xp.device):
+        a, b = xp.data_ptr(), wp.data_ptr()
+        _b.check(_b.lib().bgemm_unpack_signs_pair(a, a + 4 * xp.shape[1], xs.data_ptr() if need_x else None, N,
+                                                  b, b + 4 * wp.shape[1], ws.data_ptr() if need_w else None, M, K, _stream()))
+    return xs, ws
+
+
+def linear_grad(wp, xp, g, K, sw, sa, bias_grad=True):
+    """One pass over the upstream gradient ``g`` [N, M]: ``(g16, grad_bias, grad_sw, grad_sa)`` of the scaled binary Linear."""
+    N, M = g.shape
+    L = _b.lib()
+    g16 = torch.empty((N, M), dtype=torch.half, device=g.device)
+    small = torch.empty(2 * M + 8, dtype=g.dtype, device=g.device)
+    gsw, gb, gsa = small[:M], small[M:2 * M] if bias_grad else None, small[2 * M:2 * M + 1]
+    ws = torch.empty(L.bgemm_linear_grad_workspace_bytes(N, M), dtype=torch.uint8, device=g.device)
+    with _on(g.device):
+        _b.check(L.bgemm_linear_grad(wp.data_ptr(), xp.data_ptr(), g.data_ptr(), SRC_F32 if g.dtype == torch.float32 else SRC_F16, N, M, K,
+                                     sw.data_ptr(), sa.data_ptr(), g16.data_ptr(), gb.data_ptr() if bias_grad else None, gsw.data_ptr(),
+                                     gsa.data_ptr(), ws.data_ptr(), ws.numel(), _stream()))
+    return g16, gb, gsw, gsa
+
+
+def bireal_grad(gx16, x, zpa):
+    """``gx16 * (2 - 2 * |(x - zpa).half()|.clamp(max=1))`` in x's type, one pass."""
+    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    with _on(x.device):
+        _b.check(_b.lib().bgemm_bireal_grad(gx16.data_ptr(), x.data_ptr(), SRC_F32 if x.dtype == torch.float32 else SRC_F16, x.stride(0),
+                                            zpa.data_ptr(), out.data_ptr(), x.shape[0], x.shape[1], _stream()))
+    return out
+
+
 # Opt-in cache of packed weights for the drop-in call.  The reference's interface takes fp16 weights
 # on every call, so every call packs them again: at decode shapes that is most of the time (reading
 # 90 MB of fp16 to produce 5.6 MB of bits).  With the cache on, a weight tensor that is the same object,

@@ -274,6 +274,31 @@ int bgemm_f16_forward(const void* W, const void* X, void* C, int64_t M, int64_t 
 int bgemm_f16_forward_static(const void* W, const void* X, void* C, int64_t M, int64_t N, int64_t K,
                              int splitK, int INSTR, void* stream);
 
+/* ---- training the binary Linear layer -------------------------------------------------------------
+ * y = half(acc) * sw * sa (+ bias), acc = MODE_XOR of (w - zpw, x - zpa) (tests/python/bgemm_linear.py:479-484), as
+ * autograd differentiates it: straight-through products of g16 = half((grad_out * sa) * sw) with the other operand's
+ * sign in {-1, 0, +1} (:149-165), and the scales' gradients.
+ *
+ * Two operands of one type and one K, packed in one launch: sign bits of half_rn(src - *zero_point) (-0.0 counts as
+ * negative) and the plane of its nonzero elements, tiled. */
+int bgemm_pack_sign_nonzero_pair(const void* src_a, int64_t rows_a, int64_t ld_a, const void* zero_point_a, void* sign_a,
+                                 void* nonzero_a, const void* src_b, int64_t rows_b, int64_t ld_b, const void* zero_point_b,
+                                 void* sign_b, void* nonzero_b, int src_dtype, int64_t K, void* stream);
+/* Those planes of up to two operands -> fp16 [rows][K] of -1, 0, +1 (16-byte aligned; dst NULL: that operand is left out). */
+int bgemm_unpack_signs_pair(const void* sign_a, const void* nonzero_a, void* dst_a, int64_t rows_a, const void* sign_b,
+                            const void* nonzero_b, void* dst_b, int64_t rows_b, int64_t K, void* stream);
+/* One pass over grad_out [N][M] (param_dtype, dense rows): g16 fp16 [N][M] as above, grad_bias [M] = column sums of
+ * grad_out, grad_sw [M], grad_sa (one value), each of param_dtype or NULL.  sums run in fp32, in an order that depends on
+ * the shape only.  M >= 2.  ws: bgemm_linear_grad_workspace_bytes(N, M) bytes, 256-byte aligned, no initialisation needed. */
+size_t bgemm_linear_grad_workspace_bytes(int64_t N, int64_t M);
+int bgemm_linear_grad(const void* W_sign, const void* X_sign, const void* grad_out, int param_dtype, int64_t N, int64_t M,
+                      int64_t K, const void* sw, const void* sa, void* g16, void* grad_bias, void* grad_sw, void* grad_sa,
+                      void* ws, size_t ws_bytes, void* stream);
+/* Bi-Real's input gradient: grad_x16 * (2 - 2 min(|half_rn(x - *zero_point)|, 1)), rounded to fp16 after every step
+ * (:186-219), stored as x_dtype [rows][K]; x has row stride ld. */
+int bgemm_bireal_grad(const void* grad_x16, const void* x, int x_dtype, int64_t ld, const void* zero_point, void* out,
+                      int64_t rows, int64_t K, void* stream);
+
 /* ---- a chain of dependent decode-shaped layers in one launch ------------------------------------
  * Layer l computes acc = MODE(W_l [M_l][K_l], x_l [N][K_l]) and hands layer l + 1 the bits of
  * half_rn(y - *next_zero_point), y = half(acc) * sw * sa (+ bias) evaluated as in bgemm_packed_forward_scaled
