@@ -1,5 +1,5 @@
 // fp16 / fp32 -> bit-plane packing and logical <-> tiled re-layout.  HBM-bound byte work.
-// Tiled output: a wave packs one 32-row x 256-bit tile, with all of its 16-byte loads in
+// Tiled output: a wave packs 8, 16 or 32 rows of one 32-row x 256-bit tile, with all of its 16-byte loads in
 // flight at once; each lane turns eight elements into a byte of sign (and nonzero) bits, the
 // bytes are put in tile order through LDS, and the tile leaves as one 16-byte store per lane.
 // Logical output (the reference's row-major words): a wave packs 512 elements of one row.
@@ -11,7 +11,7 @@
 namespace bgemm {
 
 // One operand to pack.  mode bit3: tiled output written by the row-segment waves (small operands:
-// sixteen times as many, shorter waves).  mode bit0: also write the (sign & nonzero) plane and make plane 0 the
+// many short waves); bit5 / bit6: by waves of 8 / 16 rows of a tile instead of all 32.  mode bit0: also write the (sign & nonzero) plane and make plane 0 the
 // nonzero plane; mode bit4: plane 0 = sign, plane 1 = nonzero.  mode bit1: write the logical layout instead of the tiled one.  mode bit2: the
 // source is fp32 (rounded to fp16 first, as the layers' `.to(torch.half)` does).
 // zp: device scalar of the source type subtracted before that rounding, or null.
@@ -78,17 +78,19 @@ __device__ __forceinline__ void pack_wave(const PackJob& j, const int64_t gw, co
     }
 }
 
-// One wave packs tile (rt, kt) = gw of the tiled layout.  The lanes are spread over as many 8-element chunks as the tile's
+// One wave packs RW of the 32 rows of tile (rt, kt) = gw / (32 / RW) of the tiled layout.  The lanes are spread over as many 8-element chunks as the tile's
 // rows have (8, 16 or 32), so that a short row does not leave most of the wave idle: CW lanes per row, 64 / CW rows per step.
-// lds: 2 KiB of this wave's own.
-// What bounds it is the read of the source: every load of a tile (of half a tile, fp32) is in flight before the first is
-// used.  Rows at any address and of any length take the same vector loads: rows and chunks past the end read the last ones
+// lds: RW * 64 bytes of this wave's own, the two K-halves' 16-byte slots of its rows (twice for two planes).
+// What bounds it is the read of the source: every load of the wave is in flight before the first is used.  Rows at any address and of any length take the same vector loads: rows and chunks past the end read the last ones
 // again (the last chunk as the row's last eight elements, its bits then shifted into place), so nothing branches.  With
 // element loads for such rows, as it was, fp16 [8195 + 2053, 4345] took 82.9 us; 19.3 us = 4.6 TB/s now (aligned rows: 5.1).
-template <bool F32>
+template <bool F32, int RW>
 __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, const int lane, unsigned char* lds)
 {
-    const int64_t rt = gw / j.KT, kt = gw - rt * j.KT;
+    constexpr int PARTS = TILE_ROWS / RW, PLANE = RW * 32;
+    const uint32_t tile = (uint32_t)gw / PARTS, kt32 = tile % (uint32_t)j.KT;
+    const int64_t rt = tile / (uint32_t)j.KT, kt = kt32;
+    const int row0 = (int)((uint32_t)gw % PARTS) * RW;               // the wave's first row in the tile
     if (rt * TILE_ROWS >= j.rows_out) return;              // whole wave leaves together
     // where the tile's first row lies in the source, and how many source rows there are from it on
     int64_t off0 = rt * TILE_ROWS * j.ld, rows_left = j.rows - rt * TILE_ROWS;
@@ -105,32 +107,32 @@ __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, co
     typedef typename std::conditional<F32, uint32_t, uint16_t>::type E;
     const E* const src = reinterpret_cast<const E*>(j.src) + off0;
     const int last_row = (int)(rows_left < TILE_ROWS ? rows_left : TILE_ROWS) - 1;
+    auto slot_byte = [](const int c, const int r) { return (c >> 4) * (RW * 16) + r * 16 + ((c >> 2) & 3) * 4 + (3 - (c & 3)); };
     if (j.K >= 8) {
         auto rows_by = [&](auto cw_tag) {
-            constexpr int CW = decltype(cw_tag)::value, RI = 64 / CW, STEPS = TILE_ROWS / RI, G = STEPS < (F32 ? 8 : 16) ? STEPS : (F32 ? 8 : 16);
+            constexpr int CW = decltype(cw_tag)::value, RI = 64 / CW, STEPS = RW / RI, G = STEPS < (F32 ? 8 : 16) ? STEPS : (F32 ? 8 : 16);
             const int c = lane & (CW - 1), rs = lane / CW;
-            const int b0 = tile_byte_of_chunk(c);
             const int64_t k0 = kt * TILE_KBITS + 8 * c, kc = k0 + 8 <= j.K ? k0 : j.K - 8;
             const int shift = k0 - kc < 8 ? (int)(k0 - kc) : 8;
             if (CW < 32)                           // the bytes of the chunks this tile does not have
-                for (int i = lane; i < (ternary ? 512 : 256); i += 64) reinterpret_cast<uint32_t*>(lds)[i] = 0u;
+                for (int i = lane; i < (ternary ? PLANE / 2 : PLANE / 4); i += 64) reinterpret_cast<uint32_t*>(lds)[i] = 0u;
 #pragma unroll
             for (int g = 0; g < STEPS; g += G) {
                 Raw8<F32> raw[G];
 #pragma unroll
                 for (int jj = 0; jj < G; jj++) {
-                    const int r = RI * (g + jj) + rs;
+                    const int r = row0 + RI * (g + jj) + rs;
                     raw[jj] = load_raw8<F32>(src + (int64_t)(r < last_row ? r : last_row) * j.ld, kc);
                 }
 #pragma unroll
                 for (int jj = 0; jj < G; jj++) {
-                    const int r = RI * (g + jj) + rs;
+                    const int r = RI * (g + jj) + rs, at = slot_byte(c, r);
                     uint32_t sg, nz;
                     bits8(raw[jj], centred, zf, sg, nz);
-                    const uint32_t keep = r <= last_row ? 0xffu : 0u;
+                    const uint32_t keep = row0 + r <= last_row ? 0xffu : 0u;
                     sg = (sg << shift) & keep; nz = (nz << shift) & keep;
-                    lds[b0 + r * 16] = (unsigned char)(nz_first ? nz : sg);
-                    if (ternary) lds[1024 + b0 + r * 16] = (unsigned char)(nz_second ? nz : sg & nz);
+                    lds[at] = (unsigned char)(nz_first ? nz : sg);
+                    if (ternary) lds[PLANE + at] = (unsigned char)(nz_second ? nz : sg & nz);
                 }
             }
         };
@@ -139,35 +141,45 @@ __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, co
         else rows_by(std::integral_constant<int, 32>{});
     } else {
         // rows of fewer than eight elements
-        const int c = lane & 31, b0 = tile_byte_of_chunk(c);
-        for (int jj = 0; jj < 16; jj++) {
-            const int r = 2 * jj + (lane >> 5);
+        const int c = lane & 31;
+        for (int jj = 0; jj < RW / 2; jj++) {
+            const int rl = 2 * jj + (lane >> 5), r = row0 + rl, at = slot_byte(c, rl);
             uint16_t h[8];
             uint32_t sg, nz;
             load8_as_half(src + (int64_t)(r < last_row ? r : last_row) * j.ld, F32, r <= last_row ? 8 * c : j.K, j.K, centred, zf, h);
             bits8(h, sg, nz);
-            lds[b0 + r * 16] = (unsigned char)(nz_first ? nz : sg);
-            if (ternary) lds[1024 + b0 + r * 16] = (unsigned char)(nz_second ? nz : sg & nz);
+            lds[at] = (unsigned char)(nz_first ? nz : sg);
+            if (ternary) lds[PLANE + at] = (unsigned char)(nz_second ? nz : sg & nz);
         }
     }
-    __builtin_amdgcn_wave_barrier();       // the tile was written by this wave alone: LDS keeps its order
-    reinterpret_cast<uint4*>(j.dst0)[gw * TILE_U4 + lane] = reinterpret_cast<const uint4*>(lds)[lane];
-    if (ternary) reinterpret_cast<uint4*>(j.dst1)[gw * TILE_U4 + lane] = reinterpret_cast<const uint4*>(lds + 1024)[lane];
+    __builtin_amdgcn_wave_barrier();       // the slots were written by this wave alone: LDS keeps its order
+    if (lane < 2 * RW) {
+        const int64_t at = (int64_t)tile * TILE_U4 + (lane / RW) * 32 + row0 + lane % RW;
+        reinterpret_cast<uint4*>(j.dst0)[at] = reinterpret_cast<const uint4*>(lds)[lane];
+        if (ternary) reinterpret_cast<uint4*>(j.dst1)[at] = reinterpret_cast<const uint4*>(lds + PLANE)[lane];
+    }
 }
 
 // Up to two operands per launch (the fp16 entry point packs weights and activations together).
 __global__ __launch_bounds__(256) void pack_f16_kernel(const PackJob j0, const PackJob j1)
 {
     __shared__ __align__(16) unsigned char s_tile[4][2048];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // the wave index as a scalar: the tile's coordinates and addresses stay on the scalar unit
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int64_t gw = (int64_t)blockIdx.x * 4 + wave;
     const bool first = gw < j0.waves;
     const PackJob& j = first ? j0 : j1;
     if (!first) gw -= j0.waves;
     if (gw >= j.waves) return;
     if (j.mode & (2 | 8)) pack_wave(j, gw, lane);
-    else if (j.mode & 4) pack_tile<true>(j, gw, lane, s_tile[wave]);
-    else pack_tile<false>(j, gw, lane, s_tile[wave]);
+    else if (j.mode & 64) {
+        if (j.mode & 4) pack_tile<true, 16>(j, gw, lane, s_tile[wave]);
+        else pack_tile<false, 16>(j, gw, lane, s_tile[wave]);
+    } else if (j.mode & 32) {
+        if (j.mode & 4) pack_tile<true, 8>(j, gw, lane, s_tile[wave]);
+        else pack_tile<false, 8>(j, gw, lane, s_tile[wave]);
+    } else if (j.mode & 4) pack_tile<true, 32>(j, gw, lane, s_tile[wave]);
+    else pack_tile<false, 32>(j, gw, lane, s_tile[wave]);
 }
 
 // dir 0: logical -> tiled (zero padding), dir 1: tiled -> logical.  One thread per tiled word.
@@ -204,10 +216,17 @@ static int make_job(PackJob* j, const void* src, int64_t rows, int64_t K, int64_
     j->nmat = outer * inner; j->inner = inner; j->so = so; j->si = si; j->mtiles = row_tiles(rows);
     j->rows_out = (mode & 2) ? rows : j->nmat * j->mtiles * TILE_ROWS;
     j->nseg = cdiv(j->KT * TILE_KBITS, 512);
-    // a wave per tile streams best, but an operand of a few hundred tiles would leave most SIMDs without one
-    // (measured crossover: 500 to 700 tiles)
-    if (!(mode & 2) && j->nmat * j->mtiles * j->KT < 640) j->mode |= 8;
-    j->waves = (j->mode & (2 | 8)) ? j->rows_out * j->nseg : j->nmat * j->mtiles * j->KT;
+    // Rows of a tile a wave takes.  A read of this kind wants many waves with a few loads each: four loads a lane (eight 16-byte
+    // ones, fp32) are 8 rows of a whole tile, 16 or 32 where K is so short that half or a quarter of the lanes' chunks hold any;
+    // on large fp16 operands 16 rows, where half as many waves to start weighs more (us, 32 / 16 / 8 rows a wave: fp32
+    // 8192^2 54.4 / 49.1 / 46.3, 8192 x 768 8.3 / 7.7 / 7.2; fp16 8192^2 28.8 / 26.5 / 28.2, 11008 x 4096 23.3 / 18.7 / 21.8,
+    // 8192 x 768 6.3 / 5.9 / 5.4, 98304 x 64 5.6 / 6.4 / 7.7, 8192 x 64 3.2 / 2.8 / 2.7).  Below 160 tiles single-row waves
+    // (128 x 4096 fp16 4.7 / 3.7 / 3.2 / 2.8 with one row).
+    const int64_t tiles = j->nmat * j->mtiles * j->KT;
+    int rows_per_wave = 8;
+    if (tiles >= 2048) rows_per_wave = K <= 64 ? 32 : K <= 128 || !(mode & 4) ? 16 : 8;
+    if (!(mode & 2)) j->mode |= tiles < 160 ? 8 : rows_per_wave == 8 ? 32 : rows_per_wave == 16 ? 64 : 0;
+    j->waves = (j->mode & (2 | 8)) ? j->rows_out * j->nseg : tiles * (TILE_ROWS / rows_per_wave);
     return BGEMM_OK;
 }
 
@@ -215,7 +234,7 @@ static int launch_jobs(const PackJob& j0, const PackJob& j1, hipStream_t st, con
 {
     const int64_t blocks = cdiv(j0.waves + j1.waves, 4);
     if (blocks == 0) return BGEMM_OK;
-    if (blocks > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
+    if (blocks > 0x3fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);      // (wave numbers are 32 bits wide)
     hipLaunchKernelGGL(pack_f16_kernel, dim3((unsigned)blocks), dim3(256), 0, st, j0, j1);
     return check_launch(who);
 }
