@@ -41,12 +41,12 @@ __device__ __forceinline__ float param(const void* p, const int64_t i)
 
 // A wave owns 64 columns (weight rows) and walks rt_per_chunk row tiles of 32: a lane holds the two neighbouring columns 2c
 // and 2c + 1 of sixteen rows, so G arrives as 8 (fp16: 4) bytes a lane and g16 leaves as 4, a half-wave a whole line; the
-// column sums stay in registers to the end.  The next row tile's G is requested before this one is multiplied.
+// column sums stay in registers to the end.  A row tile's G is requested before its bits are multiplied.
 // The operands are signed fp4 (+1 / -1), so the accumulator is the layer's output up to the padding bits of K, which are
-// +1 * +1 each: no popcounts, no row terms.  Bound by reading G and writing g16: [8192][3072] fp32, K = 768, see
-// launch_linear_grad.
+// +1 * +1 each: no popcounts, no row terms.  Bound by reading G and writing g16: [8192][3072] fp32
+// (150 MB), K = 768, 40.7 us = 3.7 TB/s on three waves a SIMD; with the next tile's G held in registers as well, on two, 54.2.
 template <bool F32>
-__global__ __launch_bounds__(256, 2) void linear_grad_kernel(const LinearGradArgs a)
+__global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArgs a)
 {
     typedef typename std::conditional<F32, float, __half>::type E;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -69,18 +69,16 @@ __global__ __launch_bounds__(256, 2) void linear_grad_kernel(const LinearGradArg
     const bool even = (a.M & 1) == 0;
 
     typedef typename std::conditional<F32, uint2, uint32_t>::type Pair;
-    Pair gr[2][16];
     const int t0 = chunk * a.rt_per_chunk, t1 = min(a.NT, t0 + a.rt_per_chunk);
-    auto request = [&](Pair (&to)[16], const int t) {
+    float s_b[2] = {0.f, 0.f}, s_w[2] = {0.f, 0.f}, s_a[2] = {0.f, 0.f};
+    const bool cols_in = ((int64_t)mg + 1) * 64 <= a.M;
+    for (int t = t0; t < t1; t++) {
+        Pair g[16];
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const int64_t n = (int64_t)t * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            __builtin_memcpy(&to[v], reinterpret_cast<const E*>(a.g) + (n < a.N ? n : a.N - 1) * a.M + mc, sizeof(Pair));
+            __builtin_memcpy(&g[v], reinterpret_cast<const E*>(a.g) + (n < a.N ? n : a.N - 1) * a.M + mc, sizeof(Pair));
         }
-    };
-    float s_b[2] = {0.f, 0.f}, s_w[2] = {0.f, 0.f}, s_a[2] = {0.f, 0.f};
-    auto tile = [&](const Pair (&g)[16], Pair (&next)[16], const int t) {
-        if (t + 1 < t1) request(next, t + 1);
         const uint4* xp = a.X + (int64_t)t * a.KT * TILE_U4 + lane;
         EngF4::Acc acc[2];
 #pragma unroll
@@ -97,47 +95,49 @@ __global__ __launch_bounds__(256, 2) void linear_grad_kernel(const LinearGradArg
                 acc[1] = EngF4::mma(EngF4::make(fx), EngF4::make(f1), acc[1]);
             }
         }
+        auto finish = [&](auto whole_c) {
+            constexpr bool WHOLE = decltype(whole_c)::value;      // every row and column of the wave's piece exists
+            __half* const to0 = a.g16 + ((int64_t)t * 32 + 4 * h) * a.M + m;
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int64_t n = (int64_t)t * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-            float u0, u1;
-            if constexpr (F32) { u0 = __uint_as_float(g[v].x); u1 = __uint_as_float(g[v].y); }
-            else { u0 = __half2float(__ushort_as_half((uint16_t)(g[v] & 0xffff))); u1 = __half2float(__ushort_as_half((uint16_t)(g[v] >> 16))); }
-            const bool row = n < a.N;
-            const float G0 = row && ok0 ? (moved ? u1 : u0) : 0.f, G1 = row && ok1 ? u1 : 0.f;
-            const float a0 = __half2float(__float2half_rn(acc[0][v])), a1 = __half2float(__float2half_rn(acc[1][v]));
-            float p0, p1;                         // (G * sa), then times sw, every step rounded to the parameters' type
-            __half h0, h1;
-            {
-#pragma clang fp contract(off)
-                if constexpr (F32) {
-                    p0 = G0 * sa; p1 = G1 * sa;
-                    h0 = __float2half_rn(p0 * sw0); h1 = __float2half_rn(p1 * sw1);
-                } else {
-                    const _Float16 q0 = (_Float16)G0 * (_Float16)sa, q1 = (_Float16)G1 * (_Float16)sa;
-                    const _Float16 r0 = q0 * (_Float16)sw0, r1 = q1 * (_Float16)sw1;
-                    p0 = (float)q0; p1 = (float)q1;
-                    __half_raw hr; hr.data = r0; h0 = __half(hr); hr.data = r1; h1 = __half(hr);
+            for (int v = 0; v < 16; v++) {
+                const int r = 8 * (v >> 2) + (v & 3);
+                float G0, G1;
+                if constexpr (F32) { G0 = __uint_as_float(g[v].x); G1 = __uint_as_float(g[v].y); }
+                else { G0 = __half2float(__ushort_as_half((uint16_t)(g[v] & 0xffff))); G1 = __half2float(__ushort_as_half((uint16_t)(g[v] >> 16))); }
+                const bool row = WHOLE || (int64_t)t * 32 + r + 4 * h < a.N;
+                if (!WHOLE) {
+                    G0 = row && ok0 ? (moved ? G1 : G0) : 0.f;
+                    G1 = row && ok1 ? G1 : 0.f;
                 }
-                s_b[0] += G0; s_b[1] += G1;
+                const float a0 = __half2float(__float2half_rn(acc[0][v])), a1 = __half2float(__float2half_rn(acc[1][v]));
+                float p0, p1;                         // (G * sa), then times sw, every step rounded to the parameters' type
+                __half h0, h1;
+                {
+#pragma clang fp contract(off)
+                    if constexpr (F32) {
+                        p0 = G0 * sa; p1 = G1 * sa;
+                        h0 = __float2half_rn(p0 * sw0); h1 = __float2half_rn(p1 * sw1);
+                    } else {
+                        const _Float16 q0 = (_Float16)G0 * (_Float16)sa, q1 = (_Float16)G1 * (_Float16)sa;
+                        const _Float16 r0 = q0 * (_Float16)sw0, r1 = q1 * (_Float16)sw1;
+                        p0 = (float)q0; p1 = (float)q1;
+                        __half_raw hr; hr.data = r0; h0 = __half(hr); hr.data = r1; h1 = __half(hr);
+                    }
+                    s_b[0] += G0; s_b[1] += G1;
+                }
                 s_w[0] += p0 * a0; s_w[1] += p1 * a1;
                 s_a[0] += G0 * (a0 * sw0); s_a[1] += G1 * (a1 * sw1);
-            }
-            if (row) {
-                __half* const to = a.g16 + n * a.M + m;
-                if (even) {
-                    if (ok0) *reinterpret_cast<uint32_t*>(to) = (uint32_t)__half_as_ushort(h0) | (uint32_t)__half_as_ushort(h1) << 16;
-                } else {
+                __half* const to = to0 + r * a.M;
+                if (WHOLE) {
+                    *reinterpret_cast<uint32_t*>(to) = (uint32_t)__half_as_ushort(h0) | (uint32_t)__half_as_ushort(h1) << 16;
+                } else if (row) {
                     if (ok0) to[0] = h0;
                     if (ok1) to[1] = h1;
                 }
             }
-        }
-    };
-    request(gr[0], t0);
-    for (int t = t0; t < t1; t += 2) {
-        tile(gr[0], gr[1], t);
-        if (t + 1 < t1) tile(gr[1], gr[0], t + 1);
+        };
+        if (even && cols_in && (t + 1) * 32 <= a.N) finish(std::true_type{});
+        else finish(std::false_type{});
     }
     float* const part = a.part + (int64_t)chunk * 3 * a.mpad + m;
 #pragma unroll
@@ -153,19 +153,19 @@ __global__ __launch_bounds__(256, 2) void linear_grad_kernel(const LinearGradArg
     }
 }
 
-// Adds the chunks up: a block of 256 threads takes 64 columns, four threads a column; the last block to finish adds the
+// Adds the chunks up: a block of 1024 threads takes 64 columns, sixteen threads a column; the last block to finish adds the
 // blocks' shares of the scalar.
 template <bool F32>
-__global__ __launch_bounds__(256) void linear_grad_sum_kernel(const float* __restrict__ part, float* __restrict__ block_sa,
+__global__ __launch_bounds__(1024) void linear_grad_sum_kernel(const float* __restrict__ part, float* __restrict__ block_sa,
                                                               uint32_t* ticket, const int chunks, const int64_t mpad, const int64_t M,
                                                               void* grad_bias, void* grad_sw, void* grad_sa)
 {
-    __shared__ float sum[3][4][64];
+    __shared__ float sum[3][16][64];
     __shared__ bool last;
     const int c = threadIdx.x & 63, q = threadIdx.x >> 6;
     const int64_t m = (int64_t)blockIdx.x * 64 + c;
     float s[3] = {0.f, 0.f, 0.f};
-    for (int k = q; k < chunks; k += 4)
+    for (int k = q; k < chunks; k += 16)
 #pragma unroll
         for (int i = 0; i < 3; i++) s[i] += part[((int64_t)k * 3 + i) * mpad + m];
 #pragma unroll
@@ -176,7 +176,9 @@ __global__ __launch_bounds__(256) void linear_grad_sum_kernel(const float* __res
         else reinterpret_cast<__half*>(to)[i] = __float2half_rn(v);
     };
     if (q < 3) {
-        float t = (sum[q][0][c] + sum[q][1][c]) + (sum[q][2][c] + sum[q][3][c]);
+        float t = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) t += sum[q][i][c];
         if (q < 2) {
             void* const to = q == 0 ? grad_bias : grad_sw;
             if (to && m < M) put(to, m, t);
@@ -307,11 +309,11 @@ extern "C" int bgemm_linear_grad(const void* W_sign, const void* X_sign, const v
     const dim3 grid((unsigned)cdiv(cols, 4), (unsigned)chunks);
     if (param_dtype == BGEMM_SRC_F32) {
         hipLaunchKernelGGL(linear_grad_kernel<true>, grid, dim3(256), 0, st, a);
-        hipLaunchKernelGGL(linear_grad_sum_kernel<true>, dim3((unsigned)cols), dim3(256), 0, st, a.part, block_sa, a.ticket, (int)chunks, a.mpad, M,
+        hipLaunchKernelGGL(linear_grad_sum_kernel<true>, dim3((unsigned)cols), dim3(1024), 0, st, a.part, block_sa, a.ticket, (int)chunks, a.mpad, M,
                            grad_bias, grad_sw, grad_sa);
     } else {
         hipLaunchKernelGGL(linear_grad_kernel<false>, grid, dim3(256), 0, st, a);
-        hipLaunchKernelGGL(linear_grad_sum_kernel<false>, dim3((unsigned)cols), dim3(256), 0, st, a.part, block_sa, a.ticket, (int)chunks, a.mpad, M,
+        hipLaunchKernelGGL(linear_grad_sum_kernel<false>, dim3((unsigned)cols), dim3(1024), 0, st, a.part, block_sa, a.ticket, (int)chunks, a.mpad, M,
                            grad_bias, grad_sw, grad_sa);
     }
     return check_launch(who);
