@@ -62,10 +62,8 @@ SIGNATURES = {
     "bgemm_f16_forward": (_int, [_p, _p, _p, _i64, _i64, _i64, _p, _sz, _int, _int, _p]),
     "bgemm_f16_forward_static": (_int, [_p, _p, _p, _i64, _i64, _i64, _int, _int, _p]),
     "bgemm_pack_sign_nonzero_pair": (_int, [_p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _p, _p, _p, _int, _i64, _p]),
-    "bgemm_unpack_signs_pair": (_int, [_p, _p, _p, _i64, _p, _p, _p, _i64, _i64, _p]),
-    "bgemm_linear_grad_workspace_bytes": (_sz, [_i64, _i64]),
-    "bgemm_linear_grad": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _sz, _p]),
-    "bgemm_bireal_grad": (_int, [_p, _p, _int, _i64, _p, _p, _i64, _i64, _p]),
+    "bgemm_linear_backward_workspace_bytes": (_sz, [_i64, _i64, _i64, _int, _int]),
+    "bgemm_linear_backward": (_int, [_p, _p, _p, _p, _p, _int, _i64, _i64, _i64, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "bgemm_chain_workspace_bytes": (_sz, [_int, _p, _int, _i64]),
     "bgemm_chain_forward": (_int, [_int, _p, _p, _int, _p, _p, _i64, _p, _int, _int, _p, _sz, _int, _p]),
     "bgemm_chain_status": (_int, [_p, _p]),

@@ -163,8 +163,7 @@ def _rows_2d(t):
 class _scaled_linear(torch.autograd.Function):
     """``fn(x - zpa, w - zpw) * sw * sa (+ bias)`` of the binary Linear modules (bgemm_linear.py:479-484) as one node, fn =
     bgemm_linear or bgemm_linear_bireal: the same values and gradients as the separate operations, in two launches
-    forward and two passes over the gradient backward besides the two dense products.  What is kept for the backward pass is
-    bits: sign and nonzero planes of both operands."""
+    forward and five backward.  What is kept for the backward pass is bits: sign and nonzero planes of both operands."""
 
     @staticmethod
     def forward(ctx, x, weight, sw, sa, bias, zpa, zpw, fn):
@@ -204,18 +203,13 @@ class _scaled_linear(torch.autograd.Function):
             raise RuntimeError("a scale of the binary layer was modified by an inplace operation between its forward and backward pass")
         need_x, need_w, need_sw, need_sa, need_b = ctx.needs_input_grad[:5]
         g = grad_out.reshape(N, M)
-        g16, gb, gsw, gsa = lowbit_kernel.linear_grad(wp[0], xp[0], g if g.is_contiguous() else g.contiguous(), K, sw, sa, ctx.has_bias and need_b)
-        xs, ws = lowbit_kernel.unpack_signs(xp, N, wp, M, K, need_w, need_x)
-        gx = gw = None
+        bireal = None
+        if ctx.fn is bgemm_linear_bireal and need_x:
+            bireal = (_rows_2d(ctx.saved_tensors[0]), ctx.saved_tensors[4])
+        gx, gw, gb, gsw, gsa = lowbit_kernel.linear_backward(xp, wp, g if g.is_contiguous() else g.contiguous(), K, sw, sa, need_x, need_w,
+                                                             ctx.has_bias and need_b, bireal)
         if need_x:
-            bireal = ctx.fn is bgemm_linear_bireal
-            gx = g16 @ ws
-            if bireal:
-                x, zpa = ctx.saved_tensors[0], ctx.saved_tensors[4]
-                gx = lowbit_kernel.bireal_grad(gx, _rows_2d(x), zpa)
-            gx = gx.to(g.dtype).reshape(*grad_out.shape[:-1], K)
-        if need_w:
-            gw = (g16.T @ xs).to(g.dtype)
+            gx = gx.reshape(*grad_out.shape[:-1], K)
         return gx, gw, gsw if need_sw else None, gsa.reshape(sa.shape) if need_sa else None, gb, None, None, None
 
 
@@ -412,7 +406,7 @@ class BGEMMLinear(_ScaledBinaryLinear):
         points that are no parameters, and sizes the kernels take."""
         w, dt = self.weight, self.weight.dtype
         if not (self.fuse_training and self._fn in (bgemm_linear, bgemm_linear_bireal) and torch.is_grad_enabled() and x.is_cuda
-                and dt in (torch.float32, torch.half) and 2 <= w.shape[0] < 2 ** 31 and 1 <= w.shape[1] < 2 ** 24
+                and dt in (torch.float32, torch.half) and 2 <= w.shape[0] <= 2 ** 20 and 1 <= w.shape[1] < 2 ** 24
                 and x.dim() >= 1 and x.shape[-1] == w.shape[1] and 0 < x.numel() // w.shape[1] <= 2 ** 20):
             return False
         scalars = (self.sa, self.zpa, self.zpw)

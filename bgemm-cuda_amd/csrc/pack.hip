@@ -329,17 +329,6 @@ namespace bgemm {
 // (four 16-byte loads when the source allows, all sixteen in flight), gathers their sign bits into a
 // word (bit r = row r), and the 32 x 32 bit matrix held by the 32 lanes of a wave half is transposed
 // in registers with five masked exchanges: lane r then holds the word of row r, bit k' = column k'.
-__device__ __forceinline__ unsigned transpose32(unsigned w, const int lane)
-{
-#pragma unroll
-    for (int j = 16; j >= 1; j >>= 1) {
-        const unsigned m = j == 16 ? 0x0000ffffu : j == 8 ? 0x00ff00ffu : j == 4 ? 0x0f0f0f0fu : j == 2 ? 0x33333333u : 0x55555555u;
-        const unsigned other = __shfl_xor(w, j);
-        w = (lane & j) ? (w & (m << j)) | ((other >> j) & m) : (w & m) | ((other & m) << j);
-    }
-    return w;
-}
-
 template <bool F32>
 __global__ __launch_bounds__(256) void pack_transposed_kernel(const void* __restrict__ src_, const int64_t rows,
                                                               const int64_t K, const int64_t ld, const int64_t inner,

@@ -124,6 +124,19 @@ __device__ __forceinline__ void load8_as_half(const void* row, const bool f32, c
     }
 }
 
+// The 32 x 32 bit matrix held by the 32 lanes of a wave half, transposed in registers with five masked exchanges: lane i's
+// bit j becomes lane j's bit i.
+__device__ __forceinline__ unsigned transpose32(unsigned w, const int lane)
+{
+#pragma unroll
+    for (int j = 16; j >= 1; j >>= 1) {
+        const unsigned m = j == 16 ? 0x0000ffffu : j == 8 ? 0x00ff00ffu : j == 4 ? 0x0f0f0f0fu : j == 2 ? 0x33333333u : 0x55555555u;
+        const unsigned other = __shfl_xor(w, j);
+        w = (lane & j) ? (w & (m << j)) | ((other >> j) & m) : (w & m) | ((other & m) << j);
+    }
+    return w;
+}
+
 // Byte of the tile that holds elements 8c .. 8c + 7 of tile row 0 (add 16 per row): word c >> 2 of the
 // row goes to slot h * 32 + r, position q; the row's first element is the word's most significant bit,
 // i.e. byte 3 of the little-endian word.

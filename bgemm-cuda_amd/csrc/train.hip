@@ -1,12 +1,14 @@
-// Training the binary Linear layer: what its backward pass needs besides the two dense products.
+// Training the binary Linear layer: its backward pass.
 //
 //   forward   y[n,m] = half(acc[n,m]) * sw[m] * sa (+ bias[m]),  acc = sum_k sign(x - zpa)[n,k] sign(w - zpw)[m,k]
-//   backward  g16 = half((G * sa) * sw[m])                     -> the upstream operand of both dense products
+//   backward  g16 = half((G * sa) * sw[m])
+//             grad_x[n,k] = sum_m g16[n,m] sign(w - zpw)[m,k]   grad_w[m,k] = sum_n g16[n,m] sign(x - zpa)[n,k]
 //             grad_sw[m] = sum_n (G * sa) * half(acc)           grad_sa = sum_n,m G * (half(acc) * sw[m])
 //             grad_bias[m] = sum_n G
 // (tests/python/bgemm_linear.py:479-484 as autograd differentiates it, :149-165).  As separate elementwise and reduction
 // kernels this is a dozen passes over [N][M] fp32 matrices.  Here it is one: acc is not kept from the forward pass but
-// multiplied again from the two operands' sign bits (a hundredth of the bytes), in the shadow of the read of G.
+// multiplied again from the two operands' sign bits (a hundredth of the bytes), in the shadow of the read of G; g16 leaves
+// in the order in which the matrix cores of the two products read it, and their other operand stays packed.
 #include "common.h"
 #include "mfma_engines.h"
 #include "pack_bits.h"
@@ -18,13 +20,25 @@ struct LinearGradArgs {
     const uint4* W; const uint4* X;      // sign bits, tiled
     const void* g;                        // upstream gradient [N][M], fp32 or fp16
     const void* sw; const void* sa;       // parameters, same type
-    __half* g16;                          // [N][M]
+    uint4* ga; uint4* gt;                 // g16 as fragments of rows n (contraction over m) and of rows m (over n), or null
     float* part;                          // [chunks][3][Mpad]: per row chunk sums of G, (G sa) acc, G (acc sw)
     uint32_t* ticket;
     int64_t N, M, K;
     int NT, KT, MT, rt_per_chunk;
     int64_t mpad;
 };
+
+// ---- operands of the two products -------------------------------------------------------------------------------------------
+// D[i,k] = sum_r A[i,r] S[r,k] with a dense 16-bit A and S in {-1, 0, +1}: v_mfma_f32_32x32x16 steps, 32 r a "contraction
+// tile" of two steps.  The order of r inside a tile is free as long as both operands keep it; the one taken here makes an
+// accumulator of another 32 x 32 product (a lane: one column, rows 8 g + 4 h + i) an operand as it stands:
+// lane half h, step s, element e  <->  r = 16 s + 4 h + (e & 3) + 8 (e >> 2).
+//   A: fragments, [row tile][contraction tile][step][lane] of 16 bytes (2 KiB a tile and plane).
+//   S: codes, [contraction tile][half][columns, padded to 256] words of sixteen 2-bit codes (sign, nonzero): register p of step s is
+//      (word << 2 (4 s + p)) & 0xc000c000, i.e. the two 16-bit floats +-2.0 (fp16 and bf16 alike) or 0: two vector instructions a
+//      register, zeros for free, and half the sum is the result.
+constexpr int FRAG_U4 = 128;            // 16-byte units of a fragment tile of one plane
+constexpr int GA_STRIDE = 136;          // LDS row of 64 halves, padded so that 8-byte reads down the rows meet no bank twice
 
 // One 32-bit word of signed fp4 operands at step s: +1.0, or -1.0 where the bit is set, in a nibble each.
 __device__ __forceinline__ unsigned pm1_nibbles(const unsigned w, const int s)
@@ -66,12 +80,14 @@ __global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArg
         wp[j] = a.W + rt * a.KT * TILE_U4 + (lane & 32) + (r & 31);
     }
     const float pad = (float)((int64_t)a.KT * TILE_KBITS - a.K);
-    const bool even = (a.M & 1) == 0;
 
     typedef typename std::conditional<F32, uint2, uint32_t>::type Pair;
     const int t0 = chunk * a.rt_per_chunk, t1 = min(a.NT, t0 + a.rt_per_chunk);
     float s_b[2] = {0.f, 0.f}, s_w[2] = {0.f, 0.f}, s_a[2] = {0.f, 0.f};
     const bool cols_in = ((int64_t)mg + 1) * 64 <= a.M;
+    const int CT = (int)(a.mpad / 32);                          // contraction tiles of the fragments of rows n
+    __shared__ __align__(16) unsigned char s_tile[4][32 * GA_STRIDE];
+    unsigned char* const st = s_tile[wave];
     for (int t = t0; t < t1; t++) {
         Pair g[16];
 #pragma unroll
@@ -95,17 +111,16 @@ __global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArg
                 acc[1] = EngF4::mma(EngF4::make(fx), EngF4::make(f1), acc[1]);
             }
         }
+        uint32_t hp[16];                       // the two columns' g16 of the lane's sixteen rows
         auto finish = [&](auto whole_c) {
             constexpr bool WHOLE = decltype(whole_c)::value;      // every row and column of the wave's piece exists
-            __half* const to0 = a.g16 + ((int64_t)t * 32 + 4 * h) * a.M + m;
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                const int r = 8 * (v >> 2) + (v & 3);
                 float G0, G1;
                 if constexpr (F32) { G0 = __uint_as_float(g[v].x); G1 = __uint_as_float(g[v].y); }
                 else { G0 = __half2float(__ushort_as_half((uint16_t)(g[v] & 0xffff))); G1 = __half2float(__ushort_as_half((uint16_t)(g[v] >> 16))); }
-                const bool row = WHOLE || (int64_t)t * 32 + r + 4 * h < a.N;
                 if (!WHOLE) {
+                    const bool row = (int64_t)t * 32 + 8 * (v >> 2) + (v & 3) + 4 * h < a.N;
                     G0 = row && ok0 ? (moved ? G1 : G0) : 0.f;
                     G1 = row && ok1 ? G1 : 0.f;
                 }
@@ -116,7 +131,10 @@ __global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArg
 #pragma clang fp contract(off)
                     if constexpr (F32) {
                         p0 = G0 * sa; p1 = G1 * sa;
-                        h0 = __float2half_rn(p0 * sw0); h1 = __float2half_rn(p1 * sw1);
+                        float q0 = p0 * sw0, q1 = p1 * sw1;
+                        // (kept in registers: product and conversion as one v_fma_mixlo_f16 would round once where torch rounds twice)
+                        asm("" : "+v"(q0), "+v"(q1));
+                        h0 = __float2half_rn(q0); h1 = __float2half_rn(q1);
                     } else {
                         const _Float16 q0 = (_Float16)G0 * (_Float16)sa, q1 = (_Float16)G1 * (_Float16)sa;
                         const _Float16 r0 = q0 * (_Float16)sw0, r1 = q1 * (_Float16)sw1;
@@ -127,17 +145,41 @@ __global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArg
                 }
                 s_w[0] += p0 * a0; s_w[1] += p1 * a1;
                 s_a[0] += G0 * (a0 * sw0); s_a[1] += G1 * (a1 * sw1);
-                __half* const to = to0 + r * a.M;
-                if (WHOLE) {
-                    *reinterpret_cast<uint32_t*>(to) = (uint32_t)__half_as_ushort(h0) | (uint32_t)__half_as_ushort(h1) << 16;
-                } else if (row) {
-                    if (ok0) to[0] = h0;
-                    if (ok1) to[1] = h1;
-                }
+                hp[v] = (uint32_t)__half_as_ushort(h0) | (uint32_t)__half_as_ushort(h1) << 16;
             }
         };
-        if (even && cols_in && (t + 1) * 32 <= a.N) finish(std::true_type{});
+        if (cols_in && (t + 1) * 32 <= a.N) finish(std::true_type{});
         else finish(std::false_type{});
+        if (a.gt) {
+            // rows m: a lane already holds what it holds in such a fragment, eight values of n a step (see frag_index)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    uint32_t w[4];
+#pragma unroll
+                    for (int p = 0; p < 4; p++)
+                        w[p] = __builtin_amdgcn_perm(hp[8 * s + 2 * p + 1], hp[8 * s + 2 * p], j ? 0x07060302u : 0x05040100u);
+                    a.gt[(((int64_t)mg * 2 + j) * a.NT + t) * FRAG_U4 + s * 64 + lane] = make_uint4(w[0], w[1], w[2], w[3]);
+                }
+        }
+        if (a.ga) {
+            // rows n: through the wave's own LDS area
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                *reinterpret_cast<uint32_t*>(st + (8 * (v >> 2) + 4 * h + (v & 3)) * GA_STRIDE + c * 4) = hp[v];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int i = 0; i < 4; i++) {              // contraction tile i >> 1 of the piece, step i & 1
+                const unsigned char* const from = st + c * GA_STRIDE + (16 * i + 4 * h) * 2;
+                const uint2 lo = *reinterpret_cast<const uint2*>(from), hi = *reinterpret_cast<const uint2*>(from + 16);
+                a.ga[((int64_t)t * CT + mg * 2 + (i >> 1)) * FRAG_U4 + (i & 1) * 64 + lane] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
     }
     float* const part = a.part + (int64_t)chunk * 3 * a.mpad + m;
 #pragma unroll
@@ -208,65 +250,189 @@ static int grad_rows_per_chunk(int64_t N, int64_t M)
     return (int)(want < 1 ? 1 : want > 16 ? 16 : want);
 }
 
-// Sign and nonzero planes of up to two operands -> fp16 matrices of -1, 0, +1.  A wave takes a tile: eight elements (a byte
-// of each plane) and one 16-byte store a lane.
-struct UnpackJob { const unsigned char* sg; const unsigned char* nz; __half* dst; int64_t rows, K, KT, waves; };
+// Sign and nonzero planes (tiled) of up to two operands -> codes.  A wave takes a tile of 32 rows x 256 columns: the rows are
+// the contraction, so the bit matrices are transposed in registers, 32 x 32 at a time.
+struct CodeJob { const uint4* sg; const uint4* nz; uint32_t* dst; int64_t KT, waves; };
 
-__global__ __launch_bounds__(256) void unpack_signs_kernel(const UnpackJob j0, const UnpackJob j1)
+__global__ __launch_bounds__(256) void sign_codes_kernel(const CodeJob j0, const CodeJob j1)
 {
     const int lane = threadIdx.x & 63;
-    int64_t gw = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    int64_t gw = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool first = gw < j0.waves;
-    const UnpackJob& j = first ? j0 : j1;
+    const CodeJob& j = first ? j0 : j1;
     if (!first) gw -= j0.waves;
     if (gw >= j.waves) return;
-    const int64_t rt = gw / j.KT, kt = gw - rt * j.KT;
-    const int c = lane & 31;
-    const int64_t k = kt * TILE_KBITS + 8 * c;
-    if (k >= j.K) return;
-    const bool whole = k + 8 <= j.K && (j.K & 7) == 0;
-    const unsigned char* const s = j.sg + gw * 1024 + tile_byte_of_chunk(c);
-    const unsigned char* const z = j.nz + gw * 1024 + tile_byte_of_chunk(c);
-    unsigned sb[16], zb[16];
+    const uint32_t rt = (uint32_t)gw / (uint32_t)j.KT, kt = (uint32_t)gw % (uint32_t)j.KT;
+    const uint4 s4 = j.sg[gw * TILE_U4 + lane], z4 = j.nz[gw * TILE_U4 + lane];
+    const unsigned sw[4] = {s4.x, s4.y, s4.z, s4.w}, zw[4] = {z4.x, z4.y, z4.z, z4.w};
+    const int64_t colpad = j.KT * TILE_KBITS;
+    uint32_t* const dst = j.dst + (int64_t)rt * 2 * colpad + kt * TILE_KBITS + (lane >> 5) * 128 + (lane & 31);
 #pragma unroll
-    for (int i = 0; i < 16; i++) { sb[i] = s[(2 * i + (lane >> 5)) * 16]; zb[i] = z[(2 * i + (lane >> 5)) * 16]; }
+    for (int q = 0; q < 4; q++) {
+        const unsigned ts = transpose32(__brev(sw[q]), lane), tz = transpose32(__brev(zw[q]), lane);      // bit r: row r of the lane's column
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int64_t row = rt * TILE_ROWS + 2 * i + (lane >> 5);
-        if (row >= j.rows) break;
-        union { uint32_t w[4]; uint16_t e[8]; uint4 u; } o;
+        for (int h = 0; h < 2; h++) {
+            unsigned v = 0;
 #pragma unroll
-        for (int p = 0; p < 4; p++) {
-            const uint32_t lo = (zb[i] >> (7 - 2 * p) & 1u) * (0x3c00u | (sb[i] >> (7 - 2 * p) & 1u) << 15);
-            const uint32_t hi = (zb[i] >> (6 - 2 * p) & 1u) * (0x3c00u | (sb[i] >> (6 - 2 * p) & 1u) << 15);
-            o.w[p] = lo | hi << 16;
+            for (int P = 0; P < 8; P++) {
+                const int s = P >> 2, p = P & 3, r = 16 * s + 4 * h + (p & 1) * 2 + 8 * (p >> 1);      // element 2 p; 2 p + 1 is r + 1
+                v |= ((ts >> r) & 1u) << (15 - 2 * P) | ((tz >> r) & 1u) << (14 - 2 * P);
+                v |= ((ts >> (r + 1)) & 1u) << (31 - 2 * P) | ((tz >> (r + 1)) & 1u) << (30 - 2 * P);
+            }
+            dst[h * colpad + q * 32] = v;
         }
-        uint16_t* const to = reinterpret_cast<uint16_t*>(j.dst) + row * j.K + k;
-        if (whole) *reinterpret_cast<uint4*>(to) = o.u;
-        else
-            for (int e = 0; e < 8 && k + e < j.K; e++) to[e] = o.e[e];
     }
 }
 
-// Bi-Real's surrogate on the input gradient: gx * (2 - 2 min(|x - zp|, 1)), every step rounded to fp16 as the separate
-// torch kernels round it (tests/python/bgemm_linear.py:186-219).
+// ---- the products -----------------------------------------------------------------------------------------------------------
+enum { PROD_F32 = 0, PROD_F16 = 1, PROD_BIREAL_F32 = 2, PROD_BIREAL_F16 = 3 };
+
+struct ProdArgs {
+    const uint4* A; const uint32_t* C;
+    int R, T, Ct;                         // row tiles, contraction tiles, column tiles
+    int64_t colpad, rows, cols;
+    int kind, paired;                     // paired: row tile 2 i + j holds rows 64 i + 2 * (row) + j
+    void* out;                            // [rows][cols]
+    const void* x; int64_t ldx; const void* zp;      // Bi-Real: the layer's input and its zero point
+};
+
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+typedef __bf16 b8v __attribute__((ext_vector_type(8)));
+
+// Bi-Real's surrogate 2 - 2 min(|half(x - zp)|, 1), rounded to fp16 as the separate torch kernels round it
+// (tests/python/bgemm_linear.py:186-219).
 template <bool F32>
-__global__ __launch_bounds__(256) void bireal_grad_kernel(const __half* __restrict__ gx, const void* __restrict__ x, const int64_t ld,
-                                                          const void* __restrict__ zp, void* __restrict__ out, const int64_t rows, const int64_t K)
+__device__ __forceinline__ _Float16 bireal_factor(const ProdArgs& a, const int64_t row, const int64_t col)
 {
-    const float z = param<F32>(zp, 0);
-    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x)
-    for (int64_t k = threadIdx.x; k < K; k += 256) {
-        const int64_t i = r * K + k;
-        const _Float16 xh = (_Float16)__fsub_rn(param<F32>(x, r * ld + k), z);
-        const _Float16 ax = (_Float16)fabsf((float)xh);
-        const _Float16 cl = ax > (_Float16)1.0f ? (_Float16)1.0f : ax;
-        const _Float16 d = (_Float16)2.0f - (_Float16)2.0f * cl;        // both steps exact or one fp16 rounding
-        __half_raw hr = __half_raw(gx[i]);
-        const _Float16 o = hr.data * d;
-        if constexpr (F32) reinterpret_cast<float*>(out)[i] = (float)o;
-        else reinterpret_cast<_Float16*>(out)[i] = o;
+    const _Float16 ax = (_Float16)fabsf(__fsub_rn(param<F32>(a.x, row * a.ldx + col), param<F32>(a.zp, 0)));
+    return (_Float16)2.0f - (_Float16)2.0f * (ax > (_Float16)1.0f ? (_Float16)1.0f : ax);
+}
+
+__device__ __forceinline__ void prod_store(const ProdArgs& a, const int64_t row, const int64_t col, const float v)
+{
+    const int64_t i = row * a.cols + col;
+    switch (a.kind) {
+    case PROD_F32: reinterpret_cast<float*>(a.out)[i] = v; break;
+    case PROD_F16: reinterpret_cast<_Float16*>(a.out)[i] = (_Float16)v; break;
+    case PROD_BIREAL_F32: reinterpret_cast<float*>(a.out)[i] = v * (float)bireal_factor<true>(a, row, col); break;
+    default: reinterpret_cast<_Float16*>(a.out)[i] = (_Float16)v * bireal_factor<false>(a, row, col); break;
     }
+}
+
+// A block of WC x KW = 8 waves owns one row tile and WC * RB column tiles; KW waves share a set of RB column tiles and split the
+// contraction, and their sums meet in LDS.  A wave reads its fragments straight from memory in the matrix cores' order, four
+// contraction tiles ahead, and makes the other operand's from one word per lane, 32 r and column tile.
+// NP = 3: A is fp32 split into three bf16 planes (all of its bits), multiplied one after the other into the same sums.
+template <int NP, int RB, int WC, int KW>
+__global__ __launch_bounds__(512, 2) void sign_product_kernel(const ProdArgs a)
+{
+    static_assert(WC * KW == 8, "eight waves a block");
+    constexpr int DEPTH = 4;
+    __shared__ float part[8][16][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = lane >> 5, wc = wave / KW, kw = wave % KW;
+    const int groups = (a.Ct + WC * RB - 1) / (WC * RB);
+    const int id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), rt = id / groups, ct0 = ((id % groups) * WC + wc) * RB;
+    int t0, t1;
+    split_range(a.T, KW, kw, &t0, &t1);
+    // (a fragment past the wave's range reads as zeros, a code past the operand's end too)
+    const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(a.A + (int64_t)rt * a.T * NP * FRAG_U4), 0,
+                                                                         t1 * NP * (FRAG_U4 * 16), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsC = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.C), 0, (int)(a.T * 2 * a.colpad * 4), 0x00020000);
+    const int voff_c = (int)(h * a.colpad * 4) + ct0 * 128 + (lane & 31) * 4, step_c = (int)(a.colpad * 8);
+
+    v16f acc[RB];
+#pragma unroll
+    for (int b = 0; b < RB; b++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[b][v] = 0.f;
+    v4i fa[DEPTH][NP][2];
+    unsigned fc[DEPTH][RB];
+    auto load = [&](v4i (&A)[NP][2], unsigned (&C)[RB], const int t) {
+#pragma unroll
+        for (int p = 0; p < NP; p++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) A[p][s] = __builtin_amdgcn_raw_buffer_load_b128(rsA, lane * 16 + (p * 2 + s) * 1024, t * NP * (FRAG_U4 * 16), 0);
+#pragma unroll
+        for (int b = 0; b < RB; b++) C[b] = __builtin_amdgcn_raw_buffer_load_b32(rsC, voff_c + b * 128, t * step_c, 0);
+    };
+    auto multiply = [&](const v4i (&A)[NP][2], const unsigned (&C)[RB]) {
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int b = 0; b < RB; b++) {
+                v4i f;
+#pragma unroll
+                for (int p = 0; p < 4; p++) f[p] = (int)((C[b] << (2 * (4 * s + p))) & 0xc000c000u);
+#pragma unroll
+                for (int p = 0; p < NP; p++) {
+                    if constexpr (NP == 1) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, A[p][s]), __builtin_bit_cast(h8v, f), acc[b], 0, 0, 0);
+                    else acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8v, A[p][s]), __builtin_bit_cast(b8v, f), acc[b], 0, 0, 0);
+                }
+            }
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) load(fa[d], fc[d], t0 + d);
+    for (int t = t0; t < t1; t += DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; d++) {
+            if (t + d >= t1) break;
+            multiply(fa[d], fc[d]);
+            load(fa[d], fc[d], t + d + DEPTH);
+        }
+    }
+
+    // the sums meet, one column tile of every set at a time, added in the order of the waves
+#pragma unroll
+    for (int b = 0; b < RB; b++) {
+        if (b) __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 16; v++) part[wave][v][lane] = acc[b][v];
+        __syncthreads();
+#pragma unroll
+        for (int o = 0; o < 2 * WC; o++) {
+            const int i = o * 512 + threadIdx.x, set = i >> 10, v = (i >> 6) & 15;
+            float sum = 0.f;
+#pragma unroll
+            for (int k = 0; k < KW; k++) sum += part[set * KW + k][v][lane];
+            const int r = 8 * (v >> 2) + 4 * h + (v & 3);
+            const int64_t row = a.paired ? (int64_t)(rt >> 1) * 64 + 2 * r + (rt & 1) : (int64_t)rt * 32 + r;
+            const int64_t col = ((int64_t)((id % groups) * WC + set) * RB + b) * 32 + (lane & 31);
+            if (row < a.rows && col < a.cols) prod_store(a, row, col, 0.5f * sum);
+        }
+    }
+}
+
+// Which split of a product: one block (eight waves, two a SIMD) a compute unit, so the cost of a choice is its rounds of blocks
+// times the matrix-core steps of one wave, plus the meetings of the sums.  Among equals the one whose blocks read the
+// fragments for more columns.
+template <int NP>
+static int launch_product(const ProdArgs& a, hipStream_t st, const char* who)
+{
+    if (a.T * 2 * a.colpad * 4 > 0x7fffffffLL || (int64_t)a.T * NP * FRAG_U4 * 16 > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
+    static const int RBS[3] = {6, 3, 1}, WCS[3] = {4, 2, 1};
+    int best = 0;
+    int64_t best_cost = -1, best_blocks = 0;
+    for (int i = 0; i < 9; i++) {
+        const int rb = RBS[i / 3], wc = WCS[i % 3], kw = 8 / wc;
+        const int64_t blocks = (int64_t)a.R * cdiv(a.Ct, wc * rb);
+        const int64_t cost = cdiv(blocks, 256) * (cdiv(a.T, kw) * 2 * NP * rb * 64 + 1500 + rb * 600);
+        if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = i; best_blocks = blocks; }
+    }
+    if (best_blocks > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: grid of %lld blocks", who, (long long)best_blocks);
+    const dim3 g((unsigned)best_blocks), b(512);
+    switch (best) {
+    case 0: hipLaunchKernelGGL((sign_product_kernel<NP, 6, 4, 2>), g, b, 0, st, a); break;
+    case 1: hipLaunchKernelGGL((sign_product_kernel<NP, 6, 2, 4>), g, b, 0, st, a); break;
+    case 2: hipLaunchKernelGGL((sign_product_kernel<NP, 6, 1, 8>), g, b, 0, st, a); break;
+    case 3: hipLaunchKernelGGL((sign_product_kernel<NP, 3, 4, 2>), g, b, 0, st, a); break;
+    case 4: hipLaunchKernelGGL((sign_product_kernel<NP, 3, 2, 4>), g, b, 0, st, a); break;
+    case 5: hipLaunchKernelGGL((sign_product_kernel<NP, 3, 1, 8>), g, b, 0, st, a); break;
+    case 6: hipLaunchKernelGGL((sign_product_kernel<NP, 1, 4, 2>), g, b, 0, st, a); break;
+    case 7: hipLaunchKernelGGL((sign_product_kernel<NP, 1, 2, 4>), g, b, 0, st, a); break;
+    default: hipLaunchKernelGGL((sign_product_kernel<NP, 1, 1, 8>), g, b, 0, st, a); break;
+    }
+    return check_launch(who);
 }
 
 }  // namespace bgemm
@@ -275,88 +441,98 @@ using namespace bgemm;
 
 static size_t grad_round(size_t b) { return (b + 255) / 256 * 256; }
 
-extern "C" size_t bgemm_linear_grad_workspace_bytes(int64_t N, int64_t M)
+// Workspace of a backward pass: [ticket] [blocks' shares of grad_sa] [chunk sums] [codes of w, fragments of rows n] (grad_x)
+// [codes of x, fragments of rows m] (grad_w), each rounded to 256 bytes.
+struct LinearWs { size_t block_sa, part, codes_w, ga, codes_x, gt, total; int64_t chunks, cols; };
+
+static LinearWs linear_ws(int64_t N, int64_t M, int64_t K, bool need_x, bool need_w)
 {
-    if (N <= 0 || M <= 0) return 0;
-    const int64_t chunks = cdiv(row_tiles(N), grad_rows_per_chunk(N, M)), cols = cdiv(M, 64);
-    return 256 + grad_round((size_t)cols * 4) + grad_round((size_t)chunks * 3 * cols * 64 * 4);
+    LinearWs w;
+    w.chunks = cdiv(row_tiles(N), grad_rows_per_chunk(N, M));
+    w.cols = cdiv(M, 64);
+    const size_t frags = (size_t)row_tiles(N) * w.cols * 2 * FRAG_U4 * 16, words = (size_t)k_tiles(K) * TILE_KBITS * 2 * 4;
+    w.block_sa = 256;
+    w.part = w.block_sa + grad_round((size_t)w.cols * 4);
+    w.codes_w = w.part + grad_round((size_t)w.chunks * 3 * w.cols * 64 * 4);
+    w.ga = w.codes_w + (need_x ? grad_round(w.cols * 2 * words) : 0);
+    w.codes_x = w.ga + (need_x ? frags : 0);
+    w.gt = w.codes_x + (need_w ? grad_round(row_tiles(N) * words) : 0);
+    w.total = w.gt + (need_w ? frags : 0);
+    return w;
 }
 
-extern "C" int bgemm_linear_grad(const void* W_sign, const void* X_sign, const void* grad_out, int param_dtype, int64_t N, int64_t M,
-                                 int64_t K, const void* sw, const void* sa, void* g16, void* grad_bias, void* grad_sw, void* grad_sa,
-                                 void* ws, size_t ws_bytes, void* stream)
+extern "C" size_t bgemm_linear_backward_workspace_bytes(int64_t N, int64_t M, int64_t K, int need_x, int need_w)
 {
-    const char* who = "bgemm_linear_grad";
+    return N <= 0 || M <= 0 || K <= 0 ? 0 : linear_ws(N, M, K, need_x, need_w).total;
+}
+
+extern "C" int bgemm_linear_backward(const void* W_sign, const void* W_nonzero, const void* X_sign, const void* X_nonzero,
+                                     const void* grad_out, int param_dtype, int64_t N, int64_t M, int64_t K, const void* sw, const void* sa,
+                                     const void* bireal_x, int64_t ldx, const void* zero_point, void* grad_x, void* grad_w,
+                                     void* grad_bias, void* grad_sw, void* grad_sa, void* ws, size_t ws_bytes, void* stream)
+{
+    const char* who = "bgemm_linear_backward";
     if (param_dtype != BGEMM_SRC_F16 && param_dtype != BGEMM_SRC_F32) return fail(BGEMM_EINVAL, "%s: unknown parameter type %d", who, param_dtype);
-    if (N < 1 || M < 2 || K < 1 || K >= (1LL << 24) || N > 0x7fffffff || M > 0x7fffffff)
-        return fail(BGEMM_EINVAL, "%s: bad shape N=%lld M=%lld K=%lld", who, (long long)N, (long long)M, (long long)K);
-    if (!W_sign || !X_sign || !grad_out || !sw || !sa || !g16 || !ws) return fail(BGEMM_ENULL, "%s: null pointer", who);
-    const unsigned esz = param_dtype == BGEMM_SRC_F32 ? 4 : 2;
-    if (((uintptr_t)W_sign & 15) || ((uintptr_t)X_sign & 15) || ((uintptr_t)g16 & 3) || ((uintptr_t)ws & 255) || ((uintptr_t)grad_out & (esz - 1)))
+    if (N < 1 || M < 2 || K < 1 || K >= (1LL << 24) || N > (1 << 20) || M > (1 << 20) || (bireal_x && ldx < K))
+        return fail(BGEMM_EINVAL, "%s: bad shape N=%lld M=%lld K=%lld ldx=%lld", who, (long long)N, (long long)M, (long long)K, (long long)ldx);
+    if (!W_sign || !X_sign || !grad_out || !sw || !sa || !ws || (grad_x && !W_nonzero) || (grad_w && !X_nonzero) || (bireal_x && !zero_point))
+        return fail(BGEMM_ENULL, "%s: null pointer", who);
+    const bool f32 = param_dtype == BGEMM_SRC_F32;
+    const unsigned esz = f32 ? 4 : 2;
+    if ((((uintptr_t)W_sign | (uintptr_t)W_nonzero | (uintptr_t)X_sign | (uintptr_t)X_nonzero) & 15) || ((uintptr_t)ws & 255) ||
+        (((uintptr_t)grad_out | (uintptr_t)grad_x | (uintptr_t)grad_w) & (esz - 1)))
         return fail(BGEMM_EALIGN, "%s: an operand is not aligned", who);
-    if (ws_bytes < bgemm_linear_grad_workspace_bytes(N, M)) return fail(BGEMM_EWORKSPACE, "%s: workspace of %zu bytes is too small", who, ws_bytes);
+    const LinearWs w = linear_ws(N, M, K, grad_x, grad_w);
+    if (ws_bytes < w.total) return fail(BGEMM_EWORKSPACE, "%s: workspace of %zu bytes, %zu needed", who, ws_bytes, w.total);
+    char* const base = (char*)ws;
+    const hipStream_t st = (hipStream_t)stream;
+
     LinearGradArgs a;
-    a.W = (const uint4*)W_sign; a.X = (const uint4*)X_sign; a.g = grad_out; a.sw = sw; a.sa = sa; a.g16 = (__half*)g16;
+    a.W = (const uint4*)W_sign; a.X = (const uint4*)X_sign; a.g = grad_out; a.sw = sw; a.sa = sa;
+    a.ga = grad_x ? (uint4*)(base + w.ga) : nullptr;
+    a.gt = grad_w ? (uint4*)(base + w.gt) : nullptr;
     a.N = N; a.M = M; a.K = K; a.NT = (int)row_tiles(N); a.KT = (int)k_tiles(K); a.MT = (int)row_tiles(M);
     a.rt_per_chunk = grad_rows_per_chunk(N, M);
-    const int64_t chunks = cdiv(a.NT, a.rt_per_chunk), cols = cdiv(M, 64);
-    if (chunks > 65535) return fail(BGEMM_EINVAL, "%s: too many rows", who);
-    a.mpad = cols * 64;
+    a.mpad = w.cols * 64;
     a.ticket = (uint32_t*)ws;
-    float* const block_sa = (float*)((char*)ws + 256);
-    a.part = (float*)((char*)ws + 256 + grad_round((size_t)cols * 4));
-    const hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((unsigned)cdiv(cols, 4), (unsigned)chunks);
-    if (param_dtype == BGEMM_SRC_F32) {
+    float* const block_sa = (float*)(base + w.block_sa);
+    a.part = (float*)(base + w.part);
+    if (w.chunks > 65535) return fail(BGEMM_EINVAL, "%s: too many rows", who);
+    const dim3 grid((unsigned)cdiv(w.cols, 4), (unsigned)w.chunks);
+    if (f32) {
         hipLaunchKernelGGL(linear_grad_kernel<true>, grid, dim3(256), 0, st, a);
-        hipLaunchKernelGGL(linear_grad_sum_kernel<true>, dim3((unsigned)cols), dim3(1024), 0, st, a.part, block_sa, a.ticket, (int)chunks, a.mpad, M,
+        hipLaunchKernelGGL(linear_grad_sum_kernel<true>, dim3((unsigned)w.cols), dim3(1024), 0, st, a.part, block_sa, a.ticket, (int)w.chunks, a.mpad, M,
                            grad_bias, grad_sw, grad_sa);
     } else {
         hipLaunchKernelGGL(linear_grad_kernel<false>, grid, dim3(256), 0, st, a);
-        hipLaunchKernelGGL(linear_grad_sum_kernel<false>, dim3((unsigned)cols), dim3(1024), 0, st, a.part, block_sa, a.ticket, (int)chunks, a.mpad, M,
+        hipLaunchKernelGGL(linear_grad_sum_kernel<false>, dim3((unsigned)w.cols), dim3(1024), 0, st, a.part, block_sa, a.ticket, (int)w.chunks, a.mpad, M,
                            grad_bias, grad_sw, grad_sa);
     }
-    return check_launch(who);
-}
+    int rc = check_launch(who);
+    if (rc || (!grad_x && !grad_w)) return rc;
 
-static int unpack_job(UnpackJob* j, const void* sg, const void* nz, void* dst, int64_t rows, int64_t K, const char* who)
-{
-    j->sg = (const unsigned char*)sg; j->nz = (const unsigned char*)nz; j->dst = (__half*)dst;
-    j->rows = rows; j->K = K; j->KT = k_tiles(K); j->waves = dst ? row_tiles(rows) * j->KT : 0;
-    if (!dst) return BGEMM_OK;
-    if (rows < 1 || K < 1) return fail(BGEMM_EINVAL, "%s: bad shape rows=%lld K=%lld", who, (long long)rows, (long long)K);
-    if (!sg || !nz) return fail(BGEMM_ENULL, "%s: null pointer", who);
-    if (((uintptr_t)dst & 15)) return fail(BGEMM_EALIGN, "%s: destination not 16-byte aligned", who);
-    return BGEMM_OK;
-}
+    // the codes of the weight cover as many contraction tiles as the fragments do (an even number): the last may be missing
+    const int64_t KT = a.KT;
+    CodeJob jw = {(const uint4*)W_sign, (const uint4*)W_nonzero, (uint32_t*)(base + w.codes_w), KT, grad_x ? (int64_t)a.MT * KT : 0};
+    CodeJob jx = {(const uint4*)X_sign, (const uint4*)X_nonzero, (uint32_t*)(base + w.codes_x), KT, grad_w ? (int64_t)a.NT * KT : 0};
+    const int64_t blocks = cdiv(jw.waves + jx.waves, 4);
+    if (blocks > 0x3fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
+    hipLaunchKernelGGL(sign_codes_kernel, dim3((unsigned)blocks), dim3(256), 0, st, jw, jx);
+    rc = check_launch(who);
 
-extern "C" int bgemm_unpack_signs_pair(const void* sign_a, const void* nonzero_a, void* dst_a, int64_t rows_a, const void* sign_b,
-                                       const void* nonzero_b, void* dst_b, int64_t rows_b, int64_t K, void* stream)
-{
-    const char* who = "bgemm_unpack_signs_pair";
-    UnpackJob j0, j1;
-    int rc = unpack_job(&j0, sign_a, nonzero_a, dst_a, rows_a, K, who);
-    if (!rc) rc = unpack_job(&j1, sign_b, nonzero_b, dst_b, rows_b, K, who);
-    if (rc) return rc;
-    const int64_t blocks = cdiv(j0.waves + j1.waves, 4);
-    if (blocks == 0) return BGEMM_OK;
-    if (blocks > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
-    hipLaunchKernelGGL(unpack_signs_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, j0, j1);
-    return check_launch(who);
-}
-
-extern "C" int bgemm_bireal_grad(const void* grad_x16, const void* x, int x_dtype, int64_t ld, const void* zero_point, void* out,
-                                 int64_t rows, int64_t K, void* stream)
-{
-    const char* who = "bgemm_bireal_grad";
-    if (x_dtype != BGEMM_SRC_F16 && x_dtype != BGEMM_SRC_F32) return fail(BGEMM_EINVAL, "%s: unknown type %d", who, x_dtype);
-    if (rows < 0 || K < 0 || ld < K) return fail(BGEMM_EINVAL, "%s: bad shape rows=%lld K=%lld ld=%lld", who, (long long)rows, (long long)K, (long long)ld);
-    if (rows == 0 || K == 0) return BGEMM_OK;
-    if (!grad_x16 || !x || !zero_point || !out) return fail(BGEMM_ENULL, "%s: null pointer", who);
-    const dim3 grid((unsigned)(rows < 16384 ? rows : 16384));
-    if (x_dtype == BGEMM_SRC_F32)
-        hipLaunchKernelGGL(bireal_grad_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, (const __half*)grad_x16, x, ld, zero_point, out, rows, K);
-    else
-        hipLaunchKernelGGL(bireal_grad_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, (const __half*)grad_x16, x, ld, zero_point, out, rows, K);
-    return check_launch(who);
+    ProdArgs p;
+    p.colpad = KT * TILE_KBITS; p.cols = K; p.Ct = (int)cdiv(K, 32);
+    p.x = nullptr; p.ldx = 0; p.zp = nullptr;
+    if (!rc && grad_x) {
+        p.A = a.ga; p.C = jw.dst; p.R = a.NT; p.T = (int)(w.cols * 2); p.rows = N; p.paired = 0; p.out = grad_x;
+        p.kind = f32 ? PROD_F32 : PROD_F16;
+        if (bireal_x) { p.kind = f32 ? PROD_BIREAL_F32 : PROD_BIREAL_F16; p.x = bireal_x; p.ldx = ldx; p.zp = zero_point; }
+        rc = launch_product<1>(p, st, who);
+    }
+    if (!rc && grad_w) {
+        p.A = a.gt; p.C = jx.dst; p.R = (int)(w.cols * 2); p.T = a.NT; p.rows = M; p.paired = 1; p.out = grad_w;
+        p.kind = f32 ? PROD_F32 : PROD_F16;
+        rc = launch_product<1>(p, st, who);
+    }
+    return rc;
 }

@@ -483,39 +483,28 @@ def pack_linear_operands(x, w, zpa, zpw):
     return xp, wp
 
 
-def unpack_signs(xp, N, wp, M, K, need_x=True, need_w=True):
-    """The fp16 matrices of -1, 0, +1 that the planes of ``pack_linear_operands`` stand for (None where not needed)."""
-    xs = torch.empty((N, K), dtype=torch.half, device=xp.device) if need_x else None
-    ws = torch.empty((M, K), dtype=torch.half, device=xp.device) if need_w else None
-    with _on(xp.device):
-        a, b = xp.data_ptr(), wp.data_ptr()
-        _b.check(_b.lib().bgemm_unpack_signs_pair(a, a + 4 * xp.shape[1], xs.data_ptr() if need_x else None, N,
-                                                  b, b + 4 * wp.shape[1], ws.data_ptr() if need_w else None, M, K, _stream()))
-    return xs, ws
-
-
-def linear_grad(wp, xp, g, K, sw, sa, bias_grad=True):
-    """One pass over the upstream gradient ``g`` [N, M]: ``(g16, grad_bias, grad_sw, grad_sa)`` of the scaled binary Linear."""
+def linear_backward(xp, wp, g, K, sw, sa, need_x=True, need_w=True, bias_grad=True, bireal=None):
+    """Gradients of the scaled binary Linear from the planes of ``pack_linear_operands`` and the upstream gradient ``g`` [N, M]:
+    ``(grad_x [N, K], grad_w [M, K], grad_bias, grad_sw, grad_sa)``, None where not needed.  ``bireal=(x, zpa)`` multiplies the
+    input gradient by Bi-Real's surrogate of ``(x - zpa).half()``."""
     N, M = g.shape
     L = _b.lib()
-    g16 = torch.empty((N, M), dtype=torch.half, device=g.device)
-    small = torch.empty(2 * M + 8, dtype=g.dtype, device=g.device)
-    gsw, gb, gsa = small[:M], small[M:2 * M] if bias_grad else None, small[2 * M:2 * M + 1]
-    ws = torch.empty(L.bgemm_linear_grad_workspace_bytes(N, M), dtype=torch.uint8, device=g.device)
-    with _on(g.device):
-        _b.check(L.bgemm_linear_grad(wp.data_ptr(), xp.data_ptr(), g.data_ptr(), SRC_F32 if g.dtype == torch.float32 else SRC_F16, N, M, K,
-                                     sw.data_ptr(), sa.data_ptr(), g16.data_ptr(), gb.data_ptr() if bias_grad else None, gsw.data_ptr(),
-                                     gsa.data_ptr(), ws.data_ptr(), ws.numel(), _stream()))
-    return g16, gb, gsw, gsa
-
-
-def bireal_grad(gx16, x, zpa):
-    """``gx16 * (2 - 2 * |(x - zpa).half()|.clamp(max=1))`` in x's type, one pass."""
-    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    with _on(x.device):
-        _b.check(_b.lib().bgemm_bireal_grad(gx16.data_ptr(), x.data_ptr(), SRC_F32 if x.dtype == torch.float32 else SRC_F16, x.stride(0),
-                                            zpa.data_ptr(), out.data_ptr(), x.shape[0], x.shape[1], _stream()))
-    return out
+    dt, dev = g.dtype, g.device
+    gx = torch.empty((N, K), dtype=dt, device=dev) if need_x else None
+    gw = torch.empty((M, K), dtype=dt, device=dev) if need_w else None
+    gsw = torch.empty(M, dtype=dt, device=dev)
+    gb = torch.empty(M, dtype=dt, device=dev) if bias_grad else None
+    gsa = torch.empty((), dtype=dt, device=dev)
+    x, zpa = bireal if bireal is not None else (None, None)
+    with _on(dev):
+        ws = torch.empty(L.bgemm_linear_backward_workspace_bytes(N, M, K, need_x, need_w), dtype=torch.uint8, device=dev)
+        w0, x0 = wp.data_ptr(), xp.data_ptr()
+        _b.check(L.bgemm_linear_backward(
+            w0, w0 + 4 * wp.shape[1], x0, x0 + 4 * xp.shape[1], g.data_ptr(), SRC_F32 if dt == torch.float32 else SRC_F16, N, M, K,
+            sw.data_ptr(), sa.data_ptr(), x.data_ptr() if x is not None else None, x.stride(0) if x is not None else 0,
+            zpa.data_ptr() if x is not None else None, gx.data_ptr() if need_x else None, gw.data_ptr() if need_w else None,
+            gb.data_ptr() if bias_grad else None, gsw.data_ptr(), gsa.data_ptr(), ws.data_ptr(), ws.numel(), _stream()))
+    return gx, gw, gb, gsw, gsa
 
 
 # Opt-in cache of packed weights for the drop-in call.  The reference's interface takes fp16 weights

@@ -284,20 +284,17 @@ int bgemm_f16_forward_static(const void* W, const void* X, void* C, int64_t M, i
 int bgemm_pack_sign_nonzero_pair(const void* src_a, int64_t rows_a, int64_t ld_a, const void* zero_point_a, void* sign_a,
                                  void* nonzero_a, const void* src_b, int64_t rows_b, int64_t ld_b, const void* zero_point_b,
                                  void* sign_b, void* nonzero_b, int src_dtype, int64_t K, void* stream);
-/* Those planes of up to two operands -> fp16 [rows][K] of -1, 0, +1 (16-byte aligned; dst NULL: that operand is left out). */
-int bgemm_unpack_signs_pair(const void* sign_a, const void* nonzero_a, void* dst_a, int64_t rows_a, const void* sign_b,
-                            const void* nonzero_b, void* dst_b, int64_t rows_b, int64_t K, void* stream);
-/* One pass over grad_out [N][M] (param_dtype, dense rows): g16 fp16 [N][M] as above, grad_bias [M] = column sums of
- * grad_out, grad_sw [M], grad_sa (one value), each of param_dtype or NULL.  sums run in fp32, in an order that depends on
- * the shape only.  M >= 2.  ws: bgemm_linear_grad_workspace_bytes(N, M) bytes, 256-byte aligned, no initialisation needed. */
-size_t bgemm_linear_grad_workspace_bytes(int64_t N, int64_t M);
-int bgemm_linear_grad(const void* W_sign, const void* X_sign, const void* grad_out, int param_dtype, int64_t N, int64_t M,
-                      int64_t K, const void* sw, const void* sa, void* g16, void* grad_bias, void* grad_sw, void* grad_sa,
-                      void* ws, size_t ws_bytes, void* stream);
-/* Bi-Real's input gradient: grad_x16 * (2 - 2 min(|half_rn(x - *zero_point)|, 1)), rounded to fp16 after every step
- * (:186-219), stored as x_dtype [rows][K]; x has row stride ld. */
-int bgemm_bireal_grad(const void* grad_x16, const void* x, int x_dtype, int64_t ld, const void* zero_point, void* out,
-                      int64_t rows, int64_t K, void* stream);
+/* The backward pass.  W_* / X_*: those planes of the weight [M][K] and the input [N][K]; grad_out [N][M] of param_dtype, dense
+ * rows.  Outputs, of param_dtype, dense, each NULL where it is not wanted: grad_x [N][K] = g16 sign(w), grad_w [M][K] =
+ * g16^T sign(x) (fp16 products, fp32 sums, rounded once), grad_bias [M] = column sums of grad_out, grad_sw [M], grad_sa (one
+ * value).  bireal_x (the input itself, row stride ldx, with its zero point): grad_x is multiplied by Bi-Real's
+ * 2 - 2 min(|half_rn(x - *zero_point)|, 1) (:186-219); NULL otherwise.  Every sum runs in an order that depends on the shape only.
+ * M >= 2; N, M <= 2^20.  ws: the number of bytes below, 256-byte aligned, no initialisation needed. */
+size_t bgemm_linear_backward_workspace_bytes(int64_t N, int64_t M, int64_t K, int need_x, int need_w);
+int bgemm_linear_backward(const void* W_sign, const void* W_nonzero, const void* X_sign, const void* X_nonzero,
+                          const void* grad_out, int param_dtype, int64_t N, int64_t M, int64_t K, const void* sw, const void* sa,
+                          const void* bireal_x, int64_t ldx, const void* zero_point, void* grad_x, void* grad_w,
+                          void* grad_bias, void* grad_sw, void* grad_sa, void* ws, size_t ws_bytes, void* stream);
 
 /* ---- a chain of dependent decode-shaped layers in one launch ------------------------------------
  * Layer l computes acc = MODE(W_l [M_l][K_l], x_l [N][K_l]) and hands layer l + 1 the bits of
