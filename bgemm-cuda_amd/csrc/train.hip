@@ -250,9 +250,10 @@ static int grad_rows_per_chunk(int64_t N, int64_t M)
     return (int)(want < 1 ? 1 : want > 16 ? 16 : want);
 }
 
-// Sign and nonzero planes (tiled) of up to two operands -> codes.  A wave takes a tile of 32 rows x 256 columns: the rows are
-// the contraction, so the bit matrices are transposed in registers, 32 x 32 at a time.
-struct CodeJob { const uint4* sg; const uint4* nz; uint32_t* dst; int64_t KT, waves; };
+// Sign and nonzero planes (tiled) of up to two operands -> codes.  A wave takes one word per row and half of a tile of 32 rows x
+// 256 columns (2 x 32 columns): the rows are the contraction, so the 32 x 32 bit matrices are transposed in registers.  A
+// launch of this size is latency: a wave a tile, four words a lane, took 12.8 us for [8192 + 3072, 768].
+struct CodeJob { const uint32_t* sg; const uint32_t* nz; uint32_t* dst; int64_t KT, waves; };
 
 __global__ __launch_bounds__(256) void sign_codes_kernel(const CodeJob j0, const CodeJob j1)
 {
@@ -262,25 +263,21 @@ __global__ __launch_bounds__(256) void sign_codes_kernel(const CodeJob j0, const
     const CodeJob& j = first ? j0 : j1;
     if (!first) gw -= j0.waves;
     if (gw >= j.waves) return;
-    const uint32_t rt = (uint32_t)gw / (uint32_t)j.KT, kt = (uint32_t)gw % (uint32_t)j.KT;
-    const uint4 s4 = j.sg[gw * TILE_U4 + lane], z4 = j.nz[gw * TILE_U4 + lane];
-    const unsigned sw[4] = {s4.x, s4.y, s4.z, s4.w}, zw[4] = {z4.x, z4.y, z4.z, z4.w};
+    const uint32_t tile = (uint32_t)gw >> 2, q = (uint32_t)gw & 3, rt = tile / (uint32_t)j.KT, kt = tile % (uint32_t)j.KT;
+    const int64_t at = (int64_t)tile * TILE_WORDS + lane * 4 + q;
+    const unsigned ts = transpose32(__brev(j.sg[at]), lane), tz = transpose32(__brev(j.nz[at]), lane);      // bit r: row r of the lane's column
     const int64_t colpad = j.KT * TILE_KBITS;
-    uint32_t* const dst = j.dst + (int64_t)rt * 2 * colpad + kt * TILE_KBITS + (lane >> 5) * 128 + (lane & 31);
+    uint32_t* const dst = j.dst + (int64_t)rt * 2 * colpad + kt * TILE_KBITS + (lane >> 5) * 128 + q * 32 + (lane & 31);
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const unsigned ts = transpose32(__brev(sw[q]), lane), tz = transpose32(__brev(zw[q]), lane);      // bit r: row r of the lane's column
+    for (int h = 0; h < 2; h++) {
+        unsigned v = 0;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            unsigned v = 0;
-#pragma unroll
-            for (int P = 0; P < 8; P++) {
-                const int s = P >> 2, p = P & 3, r = 16 * s + 4 * h + (p & 1) * 2 + 8 * (p >> 1);      // element 2 p; 2 p + 1 is r + 1
-                v |= ((ts >> r) & 1u) << (15 - 2 * P) | ((tz >> r) & 1u) << (14 - 2 * P);
-                v |= ((ts >> (r + 1)) & 1u) << (31 - 2 * P) | ((tz >> (r + 1)) & 1u) << (30 - 2 * P);
-            }
-            dst[h * colpad + q * 32] = v;
+        for (int P = 0; P < 8; P++) {
+            const int s = P >> 2, p = P & 3, r = 16 * s + 4 * h + (p & 1) * 2 + 8 * (p >> 1);      // element 2 p; 2 p + 1 is r + 1
+            v |= ((ts >> r) & 1u) << (15 - 2 * P) | ((tz >> r) & 1u) << (14 - 2 * P);
+            v |= ((ts >> (r + 1)) & 1u) << (31 - 2 * P) | ((tz >> (r + 1)) & 1u) << (30 - 2 * P);
         }
+        dst[h * colpad] = v;
     }
 }
 
@@ -319,44 +316,50 @@ __device__ __forceinline__ void prod_store(const ProdArgs& a, const int64_t row,
     }
 }
 
-// A block of WC x KW = 8 waves owns one row tile and WC * RB column tiles; KW waves share a set of RB column tiles and split the
-// contraction, and their sums meet in LDS.  A wave reads its fragments straight from memory in the matrix cores' order, four
-// contraction tiles ahead, and makes the other operand's from one word per lane, 32 r and column tile.
+// A block owns one row tile and RB column tiles, its KW waves split the contraction and their sums meet in LDS.  A wave multiplies
+// its fragments from the registers they were loaded into, three contraction tiles ahead, and makes the other operand's from one
+// word per lane, contraction tile and column tile: no barrier before the meeting, three blocks of four waves a compute unit.
 // NP = 3: A is fp32 split into three bf16 planes (all of its bits), multiplied one after the other into the same sums.
-template <int NP, int RB, int WC, int KW>
-__global__ __launch_bounds__(512, 2) void sign_product_kernel(const ProdArgs a)
+// What bounds it: the matrix cores at the power this card has for them.  They run a dense fp16 product of normal numbers at 1190
+// TFLOP/s, of normal numbers by +-1 at 1430 and of zeros at 1720 (8192^3, the library's kernel); [8192, 3072] x [3072, 768] takes
+// 42.2 us here, of which 30 are the loop (1290 TFLOP/s) and 12 launch, first loads, meeting and 25 MB of stores,
+// [3072, 8192] x [8192, 768] 38.7.  Fragments shared by the waves of a block through a double buffer in LDS (two row tiles a wave,
+// half the vector instructions, a barrier a stage): 42.1 and 46.5; two row tiles a wave without: 43.1 and 40.4; six column tiles a
+// wave, the vector cache read at 37 of its 64 bytes a cycle: 46.6 and 59.8; eight waves a block (one block a unit): 55.1 and 42.0.
+template <int NP, int RB, int KW>
+__global__ __launch_bounds__(KW * 64, 2) void sign_product_kernel(const ProdArgs a)
 {
-    static_assert(WC * KW == 8, "eight waves a block");
-    constexpr int DEPTH = 4;
-    __shared__ float part[8][16][64];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int h = lane >> 5, wc = wave / KW, kw = wave % KW;
-    const int groups = (a.Ct + WC * RB - 1) / (WC * RB);
-    const int id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), rt = id / groups, ct0 = ((id % groups) * WC + wc) * RB;
+    constexpr int NF = NP * 2, D = 3, RING = D + 1;
+    static_assert(RB * 16 % KW == 0, "the waves share the adding");
+    __shared__ float part[KW][RB * 16][64];
+    const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = lane >> 5;
+    const int groups = (a.Ct + RB - 1) / RB;
+    const int id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), rt = id / groups, grp = id % groups;
     int t0, t1;
     split_range(a.T, KW, kw, &t0, &t1);
     // (a fragment past the wave's range reads as zeros, a code past the operand's end too)
     const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(a.A + (int64_t)rt * a.T * NP * FRAG_U4), 0,
                                                                          t1 * NP * (FRAG_U4 * 16), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsC = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.C), 0, (int)(a.T * 2 * a.colpad * 4), 0x00020000);
-    const int voff_c = (int)(h * a.colpad * 4) + ct0 * 128 + (lane & 31) * 4, step_c = (int)(a.colpad * 8);
+    const int voff_c = (int)(h * a.colpad * 4) + grp * RB * 128 + (lane & 31) * 4, step_c = (int)(a.colpad * 8);
 
     v16f acc[RB];
 #pragma unroll
     for (int b = 0; b < RB; b++)
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[b][v] = 0.f;
-    v4i fa[DEPTH][NP][2];
-    unsigned fc[DEPTH][RB];
-    auto load = [&](v4i (&A)[NP][2], unsigned (&C)[RB], const int t) {
+    // A ring of D + 1 stages: the tile that is D ahead is requested into the buffers of the one before this, so that nothing is
+    // copied (a copy of a register still being loaded waits for the load)
+    v4i fa[RING][NF];
+    unsigned fc[RING][RB];
+    auto request = [&](v4i (&A)[NF], unsigned (&C)[RB], const int t) {
 #pragma unroll
-        for (int p = 0; p < NP; p++)
+        for (int f = 0; f < NF; f++) A[f] = __builtin_amdgcn_raw_buffer_load_b128(rsA, lane * 16 + (t * NF + f) * 1024, 0, 0);
 #pragma unroll
-            for (int s = 0; s < 2; s++) A[p][s] = __builtin_amdgcn_raw_buffer_load_b128(rsA, lane * 16 + (p * 2 + s) * 1024, t * NP * (FRAG_U4 * 16), 0);
-#pragma unroll
-        for (int b = 0; b < RB; b++) C[b] = __builtin_amdgcn_raw_buffer_load_b32(rsC, voff_c + b * 128, t * step_c, 0);
+        for (int b = 0; b < RB; b++) C[b] = __builtin_amdgcn_raw_buffer_load_b32(rsC, voff_c + t * step_c + b * 128, 0, 0);
     };
-    auto multiply = [&](const v4i (&A)[NP][2], const unsigned (&C)[RB]) {
+    auto multiply = [&](const v4i (&A)[NF], const unsigned (&C)[RB]) {
 #pragma unroll
         for (int s = 0; s < 2; s++)
 #pragma unroll
@@ -366,72 +369,54 @@ __global__ __launch_bounds__(512, 2) void sign_product_kernel(const ProdArgs a)
                 for (int p = 0; p < 4; p++) f[p] = (int)((C[b] << (2 * (4 * s + p))) & 0xc000c000u);
 #pragma unroll
                 for (int p = 0; p < NP; p++) {
-                    if constexpr (NP == 1) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, A[p][s]), __builtin_bit_cast(h8v, f), acc[b], 0, 0, 0);
-                    else acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8v, A[p][s]), __builtin_bit_cast(b8v, f), acc[b], 0, 0, 0);
+                    if constexpr (NP == 1)
+                        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, A[p * 2 + s]), __builtin_bit_cast(h8v, f), acc[b], 0, 0, 0);
+                    else
+                        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8v, A[p * 2 + s]), __builtin_bit_cast(b8v, f), acc[b], 0, 0, 0);
                 }
             }
     };
 #pragma unroll
-    for (int d = 0; d < DEPTH; d++) load(fa[d], fc[d], t0 + d);
-    for (int t = t0; t < t1; t += DEPTH) {
+    for (int d = 0; d < D; d++) request(fa[d], fc[d], t0 + d);
+    for (int t = t0; t < t1;) {
 #pragma unroll
-        for (int d = 0; d < DEPTH; d++) {
-            if (t + d >= t1) break;
+        for (int d = 0; d < RING; d++) {
+            request(fa[(d + D) % RING], fc[(d + D) % RING], t + D);
             multiply(fa[d], fc[d]);
-            load(fa[d], fc[d], t + d + DEPTH);
+            if (++t >= t1) break;
         }
     }
 
-    // the sums meet, one column tile of every set at a time, added in the order of the waves
+    // the sums meet, added in the order of the waves
 #pragma unroll
-    for (int b = 0; b < RB; b++) {
-        if (b) __syncthreads();
+    for (int b = 0; b < RB; b++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) part[wave][v][lane] = acc[b][v];
-        __syncthreads();
+        for (int v = 0; v < 16; v++) part[kw][b * 16 + v][lane] = acc[b][v];
+    __syncthreads();
+    constexpr int SHARE = RB * 16 / KW;
 #pragma unroll
-        for (int o = 0; o < 2 * WC; o++) {
-            const int i = o * 512 + threadIdx.x, set = i >> 10, v = (i >> 6) & 15;
-            float sum = 0.f;
+    for (int o = 0; o < SHARE; o++) {
+        const int e = kw * SHARE + o, b = e >> 4, v = e & 15;
+        float sum = part[0][e][lane];
 #pragma unroll
-            for (int k = 0; k < KW; k++) sum += part[set * KW + k][v][lane];
-            const int r = 8 * (v >> 2) + 4 * h + (v & 3);
-            const int64_t row = a.paired ? (int64_t)(rt >> 1) * 64 + 2 * r + (rt & 1) : (int64_t)rt * 32 + r;
-            const int64_t col = ((int64_t)((id % groups) * WC + set) * RB + b) * 32 + (lane & 31);
-            if (row < a.rows && col < a.cols) prod_store(a, row, col, 0.5f * sum);
-        }
+        for (int k = 1; k < KW; k++) sum += part[k][e][lane];
+        const int r = 8 * (v >> 2) + 4 * h + (v & 3);
+        const int64_t row = a.paired ? (int64_t)(rt >> 1) * 64 + 2 * r + (rt & 1) : (int64_t)rt * 32 + r;
+        const int64_t col = ((int64_t)grp * RB + b) * 32 + (lane & 31);
+        if (row < a.rows && col < a.cols) prod_store(a, row, col, 0.5f * sum);
     }
 }
 
-// Which split of a product: one block (eight waves, two a SIMD) a compute unit, so the cost of a choice is its rounds of blocks
-// times the matrix-core steps of one wave, plus the meetings of the sums.  Among equals the one whose blocks read the
-// fragments for more columns.
+// Three column tiles and four ways on the contraction where that gives every compute unit a block; smaller products one column
+// tile and eight ways.
 template <int NP>
 static int launch_product(const ProdArgs& a, hipStream_t st, const char* who)
 {
     if (a.T * 2 * a.colpad * 4 > 0x7fffffffLL || (int64_t)a.T * NP * FRAG_U4 * 16 > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
-    static const int RBS[3] = {6, 3, 1}, WCS[3] = {4, 2, 1};
-    int best = 0;
-    int64_t best_cost = -1, best_blocks = 0;
-    for (int i = 0; i < 9; i++) {
-        const int rb = RBS[i / 3], wc = WCS[i % 3], kw = 8 / wc;
-        const int64_t blocks = (int64_t)a.R * cdiv(a.Ct, wc * rb);
-        const int64_t cost = cdiv(blocks, 256) * (cdiv(a.T, kw) * 2 * NP * rb * 64 + 1500 + rb * 600);
-        if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = i; best_blocks = blocks; }
-    }
-    if (best_blocks > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: grid of %lld blocks", who, (long long)best_blocks);
-    const dim3 g((unsigned)best_blocks), b(512);
-    switch (best) {
-    case 0: hipLaunchKernelGGL((sign_product_kernel<NP, 6, 4, 2>), g, b, 0, st, a); break;
-    case 1: hipLaunchKernelGGL((sign_product_kernel<NP, 6, 2, 4>), g, b, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((sign_product_kernel<NP, 6, 1, 8>), g, b, 0, st, a); break;
-    case 3: hipLaunchKernelGGL((sign_product_kernel<NP, 3, 4, 2>), g, b, 0, st, a); break;
-    case 4: hipLaunchKernelGGL((sign_product_kernel<NP, 3, 2, 4>), g, b, 0, st, a); break;
-    case 5: hipLaunchKernelGGL((sign_product_kernel<NP, 3, 1, 8>), g, b, 0, st, a); break;
-    case 6: hipLaunchKernelGGL((sign_product_kernel<NP, 1, 4, 2>), g, b, 0, st, a); break;
-    case 7: hipLaunchKernelGGL((sign_product_kernel<NP, 1, 2, 4>), g, b, 0, st, a); break;
-    default: hipLaunchKernelGGL((sign_product_kernel<NP, 1, 1, 8>), g, b, 0, st, a); break;
-    }
+    const int64_t b3 = (int64_t)a.R * cdiv(a.Ct, 3), b1 = (int64_t)a.R * a.Ct;
+    if (b1 > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: grid of %lld blocks", who, (long long)b1);
+    if (b3 >= 256) hipLaunchKernelGGL((sign_product_kernel<NP, 3, 4>), dim3((unsigned)b3), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((sign_product_kernel<NP, 1, 8>), dim3((unsigned)b1), dim3(512), 0, st, a);
     return check_launch(who);
 }
 
@@ -513,8 +498,8 @@ extern "C" int bgemm_linear_backward(const void* W_sign, const void* W_nonzero, 
 
     // the codes of the weight cover as many contraction tiles as the fragments do (an even number): the last may be missing
     const int64_t KT = a.KT;
-    CodeJob jw = {(const uint4*)W_sign, (const uint4*)W_nonzero, (uint32_t*)(base + w.codes_w), KT, grad_x ? (int64_t)a.MT * KT : 0};
-    CodeJob jx = {(const uint4*)X_sign, (const uint4*)X_nonzero, (uint32_t*)(base + w.codes_x), KT, grad_w ? (int64_t)a.NT * KT : 0};
+    CodeJob jw = {(const uint32_t*)W_sign, (const uint32_t*)W_nonzero, (uint32_t*)(base + w.codes_w), KT, grad_x ? (int64_t)a.MT * KT * 4 : 0};
+    CodeJob jx = {(const uint32_t*)X_sign, (const uint32_t*)X_nonzero, (uint32_t*)(base + w.codes_x), KT, grad_w ? (int64_t)a.NT * KT * 4 : 0};
     const int64_t blocks = cdiv(jw.waves + jx.waves, 4);
     if (blocks > 0x3fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
     hipLaunchKernelGGL(sign_codes_kernel, dim3((unsigned)blocks), dim3(256), 0, st, jw, jx);
