@@ -4,6 +4,8 @@ The library must have been built (``python _build.py`` or ``__graft_entry__.buil
 there is no CPU fallback: a missing library raises ImportError.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -94,6 +96,26 @@ def lib():
                               (SO_PATH, L.bgemm_abi_version(), ABI_VERSION))
         _lib = L
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The native host side of the layers (_bgemm_native.so, built with the library)."""
+    global _native
+    if _native is None:
+        lib()                                  # the same library, with its version checked
+        path = os.path.join(_HERE, "_bgemm_native.so")
+        if not os.path.exists(path):
+            raise ImportError("%s is missing: build it with `python %s`" % (path, os.path.join(_HERE, "_build.py")))
+        import torch                           # noqa: F401  (its libraries must be loaded first)
+        loader = importlib.machinery.ExtensionFileLoader("_bgemm_native", path)
+        spec = importlib.util.spec_from_file_location("_bgemm_native", path, loader=loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        _native = module
+    return _native
 
 
 class BgemmError(RuntimeError):

@@ -14,6 +14,7 @@ import math
 import torch
 import torch.nn as nn
 
+import _lib
 import lowbit_kernel
 
 __all__ = ['BNNLinear', 'BGEMMLinear', 'BGEMMChain', 'BGEMMLinear_elastic_signed', 'bgemm_matmul', 'bgemm_attn_matmul',
@@ -154,63 +155,17 @@ class bgemm_linear_bireal(torch.autograd.Function):
         return grad_x * (2 - 2 * x.abs().clamp(max=1)), grad_w, None
 
 
-def _rows_2d(t):
-    """[..., C] as dense rows [R, C]: what the pack kernels read (a row stride larger than C is fine)."""
-    t = t.reshape(-1, t.shape[-1])
-    return t if t.stride(1) == 1 and t.stride(0) >= t.shape[1] else t.contiguous()
-
-
-class _scaled_linear(torch.autograd.Function):
-    """``fn(x - zpa, w - zpw) * sw * sa (+ bias)`` of the binary Linear modules (bgemm_linear.py:479-484) as one node, fn =
-    bgemm_linear or bgemm_linear_bireal: the same values and gradients as the separate operations, in two launches
-    forward and five backward.  What is kept for the backward pass is bits: sign and nonzero planes of both operands."""
-
-    @staticmethod
-    def forward(ctx, x, weight, sw, sa, bias, zpa, zpw, fn):
-        x2, w2 = _rows_2d(x), _rows_2d(weight)
-        N, K, M = x2.shape[0], x2.shape[1], w2.shape[0]
-        xp, wp = lowbit_kernel.pack_linear_operands(x2, w2, zpa, zpw)
-        operand = lambda planes, rows: lowbit_kernel.PackedBits(planes[:1], None, 1, rows, K)
-        out = lowbit_kernel.bgemm_packed_forward(operand(wp, M), operand(xp, N), lowbit_kernel.MODE_XOR, splitK=8,
-                                                 scale=(sw, sa.reshape(1), bias))
-        ctx.fn, ctx.shape, ctx.has_bias, ctx.planes = fn, (N, K, M), bias is not None, (xp, wp)
-        # the scales are read again by the backward pass: the values of now, as with any operation's saved operands
-        ctx.scales, ctx.versions = (sw.detach(), sa.detach()), (sw._version, sa._version)
-        # (only needed to differentiate twice, and by Bi-Real's surrogate)
-        ctx.save_for_backward(x, weight, sw, sa, zpa, zpw, *(() if bias is None else (bias,)))
-        return out.reshape(*x.shape[:-1], M)
-
-    @staticmethod
-    def _twice(ctx, grad_out):
-        # a gradient that will itself be differentiated: the separate operations, whose graph autograd knows
-        x, weight, sw, sa, zpa, zpw, *bias = ctx.saved_tensors
-        with torch.enable_grad():
-            out = ctx.fn.apply(x - zpa, weight - zpw) * sw * sa
-            if bias:
-                out = out + bias[0].view(1, -1)
-        inputs = [x, weight, sw, sa] + bias
-        wanted = [t for t, need in zip(inputs, ctx.needs_input_grad) if need]
-        grads = iter(torch.autograd.grad(out, wanted, grad_out, create_graph=True))
-        got = [next(grads) if need else None for _, need in zip(inputs, ctx.needs_input_grad)]
-        return (*got, *([None] * (8 - len(got))))
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        if torch.is_grad_enabled():
-            return _scaled_linear._twice(ctx, grad_out)
-        (sw, sa), (N, K, M), (xp, wp) = ctx.scales, ctx.shape, ctx.planes
-        if (sw._version, sa._version) != ctx.versions:
-            raise RuntimeError("a scale of the binary layer was modified by an inplace operation between its forward and backward pass")
-        need_x, need_w, need_sw, need_sa, need_b = ctx.needs_input_grad[:5]
-        g = grad_out.reshape(N, M)
-        bireal = None
-        if ctx.fn is bgemm_linear_bireal and need_x:
-            bireal = (_rows_2d(ctx.saved_tensors[0]), ctx.saved_tensors[4])
-        gx, gw, gb, gsw, gsa = lowbit_kernel.linear_backward(xp, wp, g if g.is_contiguous() else g.contiguous(), K, sw, sa, need_x, need_w,
-                                                             ctx.has_bias and need_b, bireal)
-        if need_x:
-            gx = gx.reshape(*grad_out.shape[:-1], K)
-        return gx, gw, gsw if need_sw else None, gsa.reshape(sa.shape) if need_sa else None, gb, None, None, None
+def _scaled_linear_grads(bireal, x, weight, sw, sa, bias, zpa, zpw, grad_out, need):
+    """Gradients of the scaled binary Linear that can be differentiated again: the module's separate operations, whose graph
+    autograd knows.  Called by the backward pass of the one-node form under ``create_graph=True``; entries of the result whose
+    ``need`` is False are None."""
+    with torch.enable_grad():
+        out = (bgemm_linear_bireal if bireal else bgemm_linear).apply(x - zpa, weight - zpw) * sw * sa
+        if bias is not None:
+            out = out + bias.view(1, -1)
+    inputs = (x, weight, sw, sa, bias)
+    grads = iter(torch.autograd.grad(out, [t for t, n in zip(inputs, need) if n], grad_out, create_graph=True))
+    return tuple(next(grads) if n else None for n in need)
 
 
 def ternary(x, is_act=True):
@@ -401,27 +356,16 @@ class BGEMMLinear(_ScaledBinaryLinear):
             out = lowbit_kernel.bgemm_packed_weight_forward(wp, x2, lowbit_kernel.MODE_XOR, scale=(sw, sa, bias), x_zero_point=zpa)
         return out.reshape(*lead, self.weight.shape[0])
 
-    def _one_node(self, x):
-        """Whether a recorded forward is the one-node form: the module's own arithmetic on one device and in one type, zero
-        points that are no parameters, and sizes the kernels take."""
-        w, dt = self.weight, self.weight.dtype
-        if not (self.fuse_training and self._fn in (bgemm_linear, bgemm_linear_bireal) and torch.is_grad_enabled() and x.is_cuda
-                and dt in (torch.float32, torch.half) and 2 <= w.shape[0] <= 2 ** 20 and 1 <= w.shape[1] < 2 ** 24
-                and x.dim() >= 1 and x.shape[-1] == w.shape[1] and 0 < x.numel() // w.shape[1] <= 2 ** 20):
-            return False
-        scalars = (self.sa, self.zpa, self.zpw)
-        return (all(t.dtype == dt and t.device == x.device for t in (x, w, self.sw, *scalars))
-                and all(t.numel() == 1 and t.dim() <= 1 for t in scalars) and self.sw.shape == w.shape[:1] and self.sw.is_contiguous()
-                and not self.zpa.requires_grad and not self.zpw.requires_grad
-                and (self.bias is None or (self.bias.dtype == dt and self.bias.device == x.device and self.bias.is_contiguous())))
-
     def forward(self, x):
         if not self.initialized:
             self._initialize(x, self.weight)
         if self._fusable(x):
             return self._fused_forward(x)
-        if self._one_node(x):
-            return _scaled_linear.apply(x, self.weight, self.sw, self.sa, self.bias, self.zpa, self.zpw, self._fn)
+        if self.fuse_training and x.is_cuda and (self._fn is bgemm_linear or self._fn is bgemm_linear_bireal):
+            # recorded: one autograd node for the whole layer (two launches forward, five backward) where its types and sizes allow
+            out = _lib.native().linear_train(x, self.weight, self.sw, self.sa, self.bias, self.zpa, self.zpw, self._fn is bgemm_linear_bireal)
+            if out is not None:
+                return out
         out = self._fn.apply(x - self.zpa, self.weight - self.zpw) * self.sw * self.sa
         return self._add_bias(out)
 

@@ -467,46 +467,6 @@ class DecodeChain:
             _b.check(_b.lib().bgemm_chain_status(self.workspace(N).data_ptr(), _stream()))
 
 
-# ---- training the binary Linear (bgemm_linear.py's layers call these) -----------------------------------------
-def pack_linear_operands(x, w, zpa, zpw):
-    """Sign and nonzero planes of ``(x - zpa).to(half)`` [N, K] and ``(w - zpw).to(half)`` [M, K], one launch for both
-    operands.  Returns two int32 tensors [2, words]: row 0 the sign plane, row 1 the nonzero plane."""
-    L = _b.lib()
-    xp = torch.empty((2, L.bgemm_tiled_words(x.shape[0], x.shape[1])), dtype=torch.int32, device=x.device)
-    wp = torch.empty((2, L.bgemm_tiled_words(w.shape[0], w.shape[1])), dtype=torch.int32, device=x.device)
-    with _on(x.device):
-        a, b = xp.data_ptr(), wp.data_ptr()
-        _b.check(L.bgemm_pack_sign_nonzero_pair(
-            x.data_ptr(), x.shape[0], x.stride(0), zpa.data_ptr(), a, a + 4 * xp.shape[1],
-            w.data_ptr(), w.shape[0], w.stride(0), zpw.data_ptr(), b, b + 4 * wp.shape[1],
-            SRC_F32 if x.dtype == torch.float32 else SRC_F16, x.shape[1], _stream()))
-    return xp, wp
-
-
-def linear_backward(xp, wp, g, K, sw, sa, need_x=True, need_w=True, bias_grad=True, bireal=None):
-    """Gradients of the scaled binary Linear from the planes of ``pack_linear_operands`` and the upstream gradient ``g`` [N, M]:
-    ``(grad_x [N, K], grad_w [M, K], grad_bias, grad_sw, grad_sa)``, None where not needed.  ``bireal=(x, zpa)`` multiplies the
-    input gradient by Bi-Real's surrogate of ``(x - zpa).half()``."""
-    N, M = g.shape
-    L = _b.lib()
-    dt, dev = g.dtype, g.device
-    gx = torch.empty((N, K), dtype=dt, device=dev) if need_x else None
-    gw = torch.empty((M, K), dtype=dt, device=dev) if need_w else None
-    gsw = torch.empty(M, dtype=dt, device=dev)
-    gb = torch.empty(M, dtype=dt, device=dev) if bias_grad else None
-    gsa = torch.empty((), dtype=dt, device=dev)
-    x, zpa = bireal if bireal is not None else (None, None)
-    with _on(dev):
-        ws = torch.empty(L.bgemm_linear_backward_workspace_bytes(N, M, K, need_x, need_w), dtype=torch.uint8, device=dev)
-        w0, x0 = wp.data_ptr(), xp.data_ptr()
-        _b.check(L.bgemm_linear_backward(
-            w0, w0 + 4 * wp.shape[1], x0, x0 + 4 * xp.shape[1], g.data_ptr(), SRC_F32 if dt == torch.float32 else SRC_F16, N, M, K,
-            sw.data_ptr(), sa.data_ptr(), x.data_ptr() if x is not None else None, x.stride(0) if x is not None else 0,
-            zpa.data_ptr() if x is not None else None, gx.data_ptr() if need_x else None, gw.data_ptr() if need_w else None,
-            gb.data_ptr() if bias_grad else None, gsw.data_ptr(), gsa.data_ptr(), ws.data_ptr(), ws.numel(), _stream()))
-    return gx, gw, gb, gsw, gsa
-
-
 # Opt-in cache of packed weights for the drop-in call.  The reference's interface takes fp16 weights
 # on every call, so every call packs them again: at decode shapes that is most of the time (reading
 # 90 MB of fp16 to produce 5.6 MB of bits).  With the cache on, a weight tensor that is the same object,
