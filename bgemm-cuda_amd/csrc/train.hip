@@ -53,6 +53,31 @@ __device__ __forceinline__ float param(const void* p, const int64_t i)
     else return __half2float(reinterpret_cast<const __half*>(p)[i]);
 }
 
+// Sign and nonzero planes (tiled) of an operand -> codes.  A wave takes one word per row and half of a tile of 32 rows x
+// 256 columns (2 x 32 columns): the rows are the contraction, so the 32 x 32 bit matrices are transposed in registers.
+struct CodeJob { const uint32_t* sg; const uint32_t* nz; uint32_t* dst; int64_t KT, waves; };
+
+__device__ __forceinline__ void sign_codes(const CodeJob& j, const uint32_t gw, const int lane)
+{
+    if (gw >= j.waves) return;
+    const uint32_t tile = gw >> 2, q = gw & 3, rt = tile / (uint32_t)j.KT, kt = tile % (uint32_t)j.KT;
+    const int64_t at = (int64_t)tile * TILE_WORDS + lane * 4 + q;
+    const unsigned ts = transpose32(__brev(j.sg[at]), lane), tz = transpose32(__brev(j.nz[at]), lane);      // bit r: row r of the lane's column
+    const int64_t colpad = j.KT * TILE_KBITS;
+    uint32_t* const dst = j.dst + (int64_t)rt * 2 * colpad + kt * TILE_KBITS + (lane >> 5) * 128 + q * 32 + (lane & 31);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        unsigned v = 0;
+#pragma unroll
+        for (int P = 0; P < 8; P++) {
+            const int s = P >> 2, p = P & 3, r = 16 * s + 4 * h + (p & 1) * 2 + 8 * (p >> 1);      // element 2 p; 2 p + 1 is r + 1
+            v |= ((ts >> r) & 1u) << (15 - 2 * P) | ((tz >> r) & 1u) << (14 - 2 * P);
+            v |= ((ts >> (r + 1)) & 1u) << (31 - 2 * P) | ((tz >> (r + 1)) & 1u) << (30 - 2 * P);
+        }
+        dst[h * colpad] = v;
+    }
+}
+
 // A wave owns 64 columns (weight rows) and walks rt_per_chunk row tiles of 32: a lane holds the two neighbouring columns 2c
 // and 2c + 1 of sixteen rows, so G arrives as 8 (fp16: 4) bytes a lane and g16 leaves as 4, a half-wave a whole line; the
 // column sums stay in registers to the end.  A row tile's G is requested before its bits are multiplied.
@@ -60,13 +85,21 @@ __device__ __forceinline__ float param(const void* p, const int64_t i)
 // +1 * +1 each: no popcounts, no row terms.  Bound by reading G and writing g16: [8192][3072] fp32
 // (150 MB), K = 768, 40.7 us = 3.7 TB/s on three waves a SIMD; with the next tile's G held in registers as well, on two, 54.2.
 template <bool F32>
-__global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArgs a)
+__global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArgs a, const int grid_x, const int grad_blocks, const CodeJob jw,
+                                                             const CodeJob jx)
 {
     typedef typename std::conditional<F32, float, __half>::type E;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, c = lane & 31;
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.ticket = 0;      // for the kernel that adds the chunks up
-    const int mg = blockIdx.x * 4 + wave, chunk = blockIdx.y;
+    // the blocks behind the gradient's make the products' other operands: short ones, while the last of the long ones finish
+    if ((int)blockIdx.x >= grad_blocks) {
+        const uint32_t gw = (blockIdx.x - grad_blocks) * 4 + wave, ww = (uint32_t)(jw.waves + 3) / 4 * 4;
+        if (gw < ww) sign_codes(jw, gw, lane);
+        else sign_codes(jx, gw - ww, lane);
+        return;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.ticket = 0;      // for the launch that adds the chunks up
+    const int mg = blockIdx.x % grid_x * 4 + wave, chunk = blockIdx.x / grid_x;
     if ((int64_t)mg * 64 >= a.M) return;
     const int64_t m = (int64_t)mg * 64 + 2 * c, mc = m < a.M - 2 ? m : a.M - 2;      // (M >= 2)
     const bool ok0 = m < a.M, ok1 = m + 1 < a.M, moved = m != mc;                    // the last column of an odd M: loaded as a pair's second
@@ -195,90 +228,11 @@ __global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArg
     }
 }
 
-// Adds the chunks up: a block of 1024 threads takes 64 columns, sixteen threads a column; the last block to finish adds the
-// blocks' shares of the scalar.
-template <bool F32>
-__global__ __launch_bounds__(1024) void linear_grad_sum_kernel(const float* __restrict__ part, float* __restrict__ block_sa,
-                                                              uint32_t* ticket, const int chunks, const int64_t mpad, const int64_t M,
-                                                              void* grad_bias, void* grad_sw, void* grad_sa)
-{
-    __shared__ float sum[3][16][64];
-    __shared__ bool last;
-    const int c = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int64_t m = (int64_t)blockIdx.x * 64 + c;
-    float s[3] = {0.f, 0.f, 0.f};
-    for (int k = q; k < chunks; k += 16)
-#pragma unroll
-        for (int i = 0; i < 3; i++) s[i] += part[((int64_t)k * 3 + i) * mpad + m];
-#pragma unroll
-    for (int i = 0; i < 3; i++) sum[i][q][c] = s[i];
-    __syncthreads();
-    auto put = [](void* to, const int64_t i, const float v) {
-        if constexpr (F32) reinterpret_cast<float*>(to)[i] = v;
-        else reinterpret_cast<__half*>(to)[i] = __float2half_rn(v);
-    };
-    if (q < 3) {
-        float t = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; i++) t += sum[q][i][c];
-        if (q < 2) {
-            void* const to = q == 0 ? grad_bias : grad_sw;
-            if (to && m < M) put(to, m, t);
-        } else {
-#pragma unroll
-            for (int d = 32; d; d >>= 1) t += __shfl_xor(t, d);
-            if (c == 0) {
-                __hip_atomic_store(&block_sa[blockIdx.x], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
-            }
-        }
-    }
-    __syncthreads();
-    if (last && threadIdx.x < 64) {
-        float t = 0.f;
-        for (unsigned i = threadIdx.x; i < gridDim.x; i += 64) t += __hip_atomic_load(&block_sa[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-        for (int d = 32; d; d >>= 1) t += __shfl_xor(t, d);
-        if (threadIdx.x == 0 && grad_sa) put(grad_sa, 0, t);
-    }
-}
-
 // Row tiles a wave walks: enough waves for about three on every SIMD, at most 16 row tiles (the fewer chunks, the less there is to add up).
 static int grad_rows_per_chunk(int64_t N, int64_t M)
 {
     const int64_t want = row_tiles(N) * cdiv(M, 64) / 3072;
     return (int)(want < 1 ? 1 : want > 16 ? 16 : want);
-}
-
-// Sign and nonzero planes (tiled) of up to two operands -> codes.  A wave takes one word per row and half of a tile of 32 rows x
-// 256 columns (2 x 32 columns): the rows are the contraction, so the 32 x 32 bit matrices are transposed in registers.  A
-// launch of this size is latency: a wave a tile, four words a lane, took 12.8 us for [8192 + 3072, 768].
-struct CodeJob { const uint32_t* sg; const uint32_t* nz; uint32_t* dst; int64_t KT, waves; };
-
-__global__ __launch_bounds__(256) void sign_codes_kernel(const CodeJob j0, const CodeJob j1)
-{
-    const int lane = threadIdx.x & 63;
-    int64_t gw = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const bool first = gw < j0.waves;
-    const CodeJob& j = first ? j0 : j1;
-    if (!first) gw -= j0.waves;
-    if (gw >= j.waves) return;
-    const uint32_t tile = (uint32_t)gw >> 2, q = (uint32_t)gw & 3, rt = tile / (uint32_t)j.KT, kt = tile % (uint32_t)j.KT;
-    const int64_t at = (int64_t)tile * TILE_WORDS + lane * 4 + q;
-    const unsigned ts = transpose32(__brev(j.sg[at]), lane), tz = transpose32(__brev(j.nz[at]), lane);      // bit r: row r of the lane's column
-    const int64_t colpad = j.KT * TILE_KBITS;
-    uint32_t* const dst = j.dst + (int64_t)rt * 2 * colpad + kt * TILE_KBITS + (lane >> 5) * 128 + q * 32 + (lane & 31);
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        unsigned v = 0;
-#pragma unroll
-        for (int P = 0; P < 8; P++) {
-            const int s = P >> 2, p = P & 3, r = 16 * s + 4 * h + (p & 1) * 2 + 8 * (p >> 1);      // element 2 p; 2 p + 1 is r + 1
-            v |= ((ts >> r) & 1u) << (15 - 2 * P) | ((tz >> r) & 1u) << (14 - 2 * P);
-            v |= ((ts >> (r + 1)) & 1u) << (31 - 2 * P) | ((tz >> (r + 1)) & 1u) << (30 - 2 * P);
-        }
-        dst[h * colpad] = v;
-    }
 }
 
 // ---- the products -----------------------------------------------------------------------------------------------------------
@@ -316,6 +270,60 @@ __device__ __forceinline__ void prod_store(const ProdArgs& a, const int64_t row,
     }
 }
 
+// The scales' and the bias gradients from the chunk sums: a block takes 64 columns, its waves the chunks in turn; the last block
+// to finish adds the blocks' shares of the scalar (device-scope stores and loads: the blocks may sit on different XCDs).
+struct SumArgs {
+    const float* part; float* block_sa; uint32_t* ticket;
+    int chunks, blocks, f32;
+    int64_t mpad, M;
+    void* grad_bias; void* grad_sw; void* grad_sa;
+};
+
+template <int WAVES>
+__device__ __forceinline__ void linear_sums(const SumArgs& a, const int block, float* lds)
+{
+    const int c = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int64_t m = (int64_t)block * 64 + c;
+    float s[3] = {0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int k = q; k < a.chunks; k += WAVES)
+#pragma unroll
+        for (int i = 0; i < 3; i++) s[i] += a.part[((int64_t)k * 3 + i) * a.mpad + m];
+#pragma unroll
+    for (int i = 0; i < 3; i++) lds[(i * WAVES + q) * 64 + c] = s[i];
+    __syncthreads();
+    auto put = [&](void* to, const int64_t i, const float v) {
+        if (a.f32) reinterpret_cast<float*>(to)[i] = v;
+        else reinterpret_cast<__half*>(to)[i] = __float2half_rn(v);
+    };
+    if (q >= 3) return;
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < WAVES; i++) t += lds[(q * WAVES + i) * 64 + c];
+    if (q < 2) {
+        void* const to = q == 0 ? a.grad_bias : a.grad_sw;
+        if (to && m < a.M) put(to, m, t);
+        return;
+    }
+#pragma unroll
+    for (int d = 32; d; d >>= 1) t += __shfl_xor(t, d);
+    unsigned n = 0;
+    if (c == 0) {
+        __hip_atomic_store(&a.block_sa[block], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");           // the store has been acknowledged before the ticket is taken
+        n = __hip_atomic_fetch_add(a.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (__shfl(n, 0) != (unsigned)a.blocks - 1u) return;
+    t = 0.f;
+    for (int i = c; i < a.blocks; i += 64) t += __hip_atomic_load(&a.block_sa[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int d = 32; d; d >>= 1) t += __shfl_xor(t, d);
+    if (c == 0 && a.grad_sa) put(a.grad_sa, 0, t);
+}
+
+// Both products and the sums of one backward pass as one launch: blocks of the first product, of the second, of the sums.
+struct ProdLaunch { ProdArgs p[2]; int blocks[2]; SumArgs sums; };
+
 // A block owns one row tile and RB column tiles, its KW waves split the contraction and their sums meet in LDS.  A wave multiplies
 // its fragments from the registers they were loaded into, three contraction tiles ahead, and makes the other operand's from one
 // word per lane, contraction tile and column tile: no barrier before the meeting, three blocks of four waves a compute unit.
@@ -327,15 +335,22 @@ __device__ __forceinline__ void prod_store(const ProdArgs& a, const int64_t row,
 // half the vector instructions, a barrier a stage): 42.1 and 46.5; two row tiles a wave without: 43.1 and 40.4; six column tiles a
 // wave, the vector cache read at 37 of its 64 bytes a cycle: 46.6 and 59.8; eight waves a block (one block a unit): 55.1 and 42.0.
 template <int NP, int RB, int KW>
-__global__ __launch_bounds__(KW * 64, 2) void sign_product_kernel(const ProdArgs a)
+__global__ __launch_bounds__(KW * 64, 2) void sign_product_kernel(const ProdLaunch l)
 {
     constexpr int NF = NP * 2, D = 3, RING = D + 1;
     static_assert(RB * 16 % KW == 0, "the waves share the adding");
     __shared__ float part[KW][RB * 16][64];
+    const int b0 = l.blocks[0], b1 = b0 + l.blocks[1];
+    if ((int)blockIdx.x >= b1) {
+        linear_sums<KW>(l.sums, blockIdx.x - b1, &part[0][0][0]);
+        return;
+    }
+    const bool second = (int)blockIdx.x >= b0;
+    const ProdArgs& a = l.p[second];
     const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5;
     const int groups = (a.Ct + RB - 1) / RB;
-    const int id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), rt = id / groups, grp = id % groups;
+    const int id = (int)xcd_contiguous_id(blockIdx.x - (second ? b0 : 0), l.blocks[second]), rt = id / groups, grp = id % groups;
     int t0, t1;
     split_range(a.T, KW, kw, &t0, &t1);
     // (a fragment past the wave's range reads as zeros, a code past the operand's end too)
@@ -408,15 +423,23 @@ __global__ __launch_bounds__(KW * 64, 2) void sign_product_kernel(const ProdArgs
 }
 
 // Three column tiles and four ways on the contraction where that gives every compute unit a block; smaller products one column
-// tile and eight ways.
+// tile and eight ways.  (A product that is not wanted has R = 0.)
 template <int NP>
-static int launch_product(const ProdArgs& a, hipStream_t st, const char* who)
+static int launch_products(ProdLaunch& l, hipStream_t st, const char* who)
 {
-    if (a.T * 2 * a.colpad * 4 > 0x7fffffffLL || (int64_t)a.T * NP * FRAG_U4 * 16 > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
-    const int64_t b3 = (int64_t)a.R * cdiv(a.Ct, 3), b1 = (int64_t)a.R * a.Ct;
-    if (b1 > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: grid of %lld blocks", who, (long long)b1);
-    if (b3 >= 256) hipLaunchKernelGGL((sign_product_kernel<NP, 3, 4>), dim3((unsigned)b3), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((sign_product_kernel<NP, 1, 8>), dim3((unsigned)b1), dim3(512), 0, st, a);
+    int64_t b3 = 0, b1 = 0;
+    for (const ProdArgs& a : l.p) {
+        if (!a.R) continue;
+        if (a.T * 2 * a.colpad * 4 > 0x7fffffffLL || (int64_t)a.T * NP * FRAG_U4 * 16 > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
+        b3 += (int64_t)a.R * cdiv(a.Ct, 3);
+        b1 += (int64_t)a.R * a.Ct;
+    }
+    if (b1 > 0x3fffffffLL) return fail(BGEMM_EINVAL, "%s: grid of %lld blocks", who, (long long)b1);
+    const bool wide = b3 >= 256;
+    for (int i = 0; i < 2; i++) l.blocks[i] = l.p[i].R ? (int)(l.p[i].R * cdiv(l.p[i].Ct, wide ? 3 : 1)) : 0;
+    const unsigned grid = (unsigned)(l.blocks[0] + l.blocks[1] + l.sums.blocks);
+    if (wide) hipLaunchKernelGGL((sign_product_kernel<NP, 3, 4>), dim3(grid), dim3(256), 0, st, l);
+    else hipLaunchKernelGGL((sign_product_kernel<NP, 1, 8>), dim3(grid), dim3(512), 0, st, l);
     return check_launch(who);
 }
 
@@ -482,42 +505,34 @@ extern "C" int bgemm_linear_backward(const void* W_sign, const void* W_nonzero, 
     a.ticket = (uint32_t*)ws;
     float* const block_sa = (float*)(base + w.block_sa);
     a.part = (float*)(base + w.part);
-    if (w.chunks > 65535) return fail(BGEMM_EINVAL, "%s: too many rows", who);
-    const dim3 grid((unsigned)cdiv(w.cols, 4), (unsigned)w.chunks);
-    if (f32) {
-        hipLaunchKernelGGL(linear_grad_kernel<true>, grid, dim3(256), 0, st, a);
-        hipLaunchKernelGGL(linear_grad_sum_kernel<true>, dim3((unsigned)w.cols), dim3(1024), 0, st, a.part, block_sa, a.ticket, (int)w.chunks, a.mpad, M,
-                           grad_bias, grad_sw, grad_sa);
-    } else {
-        hipLaunchKernelGGL(linear_grad_kernel<false>, grid, dim3(256), 0, st, a);
-        hipLaunchKernelGGL(linear_grad_sum_kernel<false>, dim3((unsigned)w.cols), dim3(1024), 0, st, a.part, block_sa, a.ticket, (int)w.chunks, a.mpad, M,
-                           grad_bias, grad_sw, grad_sa);
-    }
-    int rc = check_launch(who);
-    if (rc || (!grad_x && !grad_w)) return rc;
-
-    // the codes of the weight cover as many contraction tiles as the fragments do (an even number): the last may be missing
+    // the codes of the weight cover as many contraction tiles as the fragments do (an even number): the last may be missing,
+    // and is then multiplied by zeros
     const int64_t KT = a.KT;
     CodeJob jw = {(const uint32_t*)W_sign, (const uint32_t*)W_nonzero, (uint32_t*)(base + w.codes_w), KT, grad_x ? (int64_t)a.MT * KT * 4 : 0};
     CodeJob jx = {(const uint32_t*)X_sign, (const uint32_t*)X_nonzero, (uint32_t*)(base + w.codes_x), KT, grad_w ? (int64_t)a.NT * KT * 4 : 0};
-    const int64_t blocks = cdiv(jw.waves + jx.waves, 4);
+    const int64_t gx = cdiv(w.cols, 4), grad_blocks = gx * w.chunks, blocks = grad_blocks + cdiv(jw.waves, 4) + cdiv(jx.waves, 4);
     if (blocks > 0x3fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
-    hipLaunchKernelGGL(sign_codes_kernel, dim3((unsigned)blocks), dim3(256), 0, st, jw, jx);
-    rc = check_launch(who);
+    if (f32) hipLaunchKernelGGL(linear_grad_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, a, (int)gx, (int)grad_blocks, jw, jx);
+    else hipLaunchKernelGGL(linear_grad_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st, a, (int)gx, (int)grad_blocks, jw, jx);
+    const int rc = check_launch(who);
+    if (rc) return rc;
 
-    ProdArgs p;
-    p.colpad = KT * TILE_KBITS; p.cols = K; p.Ct = (int)cdiv(K, 32);
-    p.x = nullptr; p.ldx = 0; p.zp = nullptr;
-    if (!rc && grad_x) {
+    ProdLaunch l;
+    for (ProdArgs& p : l.p) {
+        p.R = 0;
+        p.colpad = KT * TILE_KBITS; p.cols = K; p.Ct = (int)cdiv(K, 32);
+        p.kind = f32 ? PROD_F32 : PROD_F16;
+        p.x = nullptr; p.ldx = 0; p.zp = nullptr;
+    }
+    if (grad_x) {
+        ProdArgs& p = l.p[0];
         p.A = a.ga; p.C = jw.dst; p.R = a.NT; p.T = (int)(w.cols * 2); p.rows = N; p.paired = 0; p.out = grad_x;
-        p.kind = f32 ? PROD_F32 : PROD_F16;
         if (bireal_x) { p.kind = f32 ? PROD_BIREAL_F32 : PROD_BIREAL_F16; p.x = bireal_x; p.ldx = ldx; p.zp = zero_point; }
-        rc = launch_product<1>(p, st, who);
     }
-    if (!rc && grad_w) {
+    if (grad_w) {
+        ProdArgs& p = l.p[1];
         p.A = a.gt; p.C = jx.dst; p.R = (int)(w.cols * 2); p.T = a.NT; p.rows = M; p.paired = 1; p.out = grad_w;
-        p.kind = f32 ? PROD_F32 : PROD_F16;
-        rc = launch_product<1>(p, st, who);
     }
-    return rc;
+    l.sums = {a.part, block_sa, a.ticket, (int)w.chunks, (int)w.cols, f32, a.mpad, M, grad_bias, grad_sw, grad_sa};
+    return launch_products<1>(l, st, who);
 }
