@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArg
                     G1 = row && ok1 ? G1 : 0.f;
                 }
                 const float a0 = __half2float(__float2half_rn(acc[0][v])), a1 = __half2float(__float2half_rn(acc[1][v]));
-                float p0, p1;                         // (G * sa), then times sw, every step rounded to the parameters' type
+                [[maybe_unused]] float p0, p1;        // (G * sa), then times sw, every step rounded to the parameters' type
                 __half h0, h1;
                 {
 #pragma clang fp contract(off)
@@ -171,13 +171,18 @@ __global__ __launch_bounds__(256, 3) void linear_grad_kernel(const LinearGradArg
                     } else {
                         const _Float16 q0 = (_Float16)G0 * (_Float16)sa, q1 = (_Float16)G1 * (_Float16)sa;
                         const _Float16 r0 = q0 * (_Float16)sw0, r1 = q1 * (_Float16)sw1;
-                        p0 = (float)q0; p1 = (float)q1;
                         __half_raw hr; hr.data = r0; h0 = __half(hr); hr.data = r1; h1 = __half(hr);
+                        // (the sums' terms are rounded, too, as the elementwise products of torch are)
+                        s_w[0] += (float)(_Float16)(q0 * (_Float16)a0); s_w[1] += (float)(_Float16)(q1 * (_Float16)a1);
+                        s_a[0] += (float)(_Float16)((_Float16)G0 * (_Float16)((_Float16)a0 * (_Float16)sw0));
+                        s_a[1] += (float)(_Float16)((_Float16)G1 * (_Float16)((_Float16)a1 * (_Float16)sw1));
                     }
                     s_b[0] += G0; s_b[1] += G1;
                 }
-                s_w[0] += p0 * a0; s_w[1] += p1 * a1;
-                s_a[0] += G0 * (a0 * sw0); s_a[1] += G1 * (a1 * sw1);
+                if constexpr (F32) {
+                    s_w[0] += p0 * a0; s_w[1] += p1 * a1;
+                    s_a[0] += G0 * (a0 * sw0); s_a[1] += G1 * (a1 * sw1);
+                }
                 hp[v] = (uint32_t)__half_as_ushort(h0) | (uint32_t)__half_as_ushort(h1) << 16;
             }
         };
