@@ -66,6 +66,9 @@ SIGNATURES = {
     "bgemm_pack_sign_nonzero_pair": (_int, [_p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _p, _p, _p, _int, _i64, _p]),
     "bgemm_linear_backward_workspace_bytes": (_sz, [_i64, _i64, _i64, _int, _int]),
     "bgemm_linear_backward": (_int, [_p, _p, _p, _p, _p, _int, _i64, _i64, _i64, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _sz, _p]),
+    "bgemm_elastic_forward": (_int, [_p, _p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
+    "bgemm_elastic_backward_workspace_bytes": (_sz, [_i64, _i64, _i64, _int, _int]),
+    "bgemm_elastic_backward": (_int, [_p, _p, _p, _p, _p, _p, _p, _p, _p, ctypes.c_float, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "bgemm_chain_workspace_bytes": (_sz, [_int, _p, _int, _i64]),
     "bgemm_chain_forward": (_int, [_int, _p, _p, _int, _p, _p, _i64, _p, _int, _int, _p, _sz, _int, _p]),
     "bgemm_chain_status": (_int, [_p, _p]),

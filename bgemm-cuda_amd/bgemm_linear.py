@@ -234,6 +234,17 @@ class bgemm_linear_elastic_signed(torch.autograd.Function):
         return _elastic_backward(ctx, grad_output, lambda t: 2 / torch.cosh(t) ** 2, 4)
 
 
+def _elastic_grads(x, weight, sa, sw, bias, grad_scale, grad_out, need):
+    """As _scaled_linear_grads, of the learned-scale layer."""
+    with torch.enable_grad():
+        out = bgemm_linear_elastic_signed.apply(x, weight, sa, sw, grad_scale)
+        if bias is not None:
+            out = out + bias.view(1, -1)
+    inputs = (x, weight, sa, sw, bias)
+    grads = iter(torch.autograd.grad(out, [t for t, n in zip(inputs, need) if n], grad_out, create_graph=True))
+    return tuple(next(grads) if n else None for n in need)
+
+
 class BinActive(torch.autograd.Function):
     """sign with 0 -> +1, identity gradient (bgemm_linear.py:599-616)."""
 
@@ -453,6 +464,7 @@ class BGEMMLinear_elastic_signed(_ScaledBinaryLinear):
     packed once per weight version; the scaling stays in torch, in the reference's order ``out * sa * sw``."""
     _fn = bgemm_linear_elastic_signed
     fuse_inference = True
+    fuse_training = True
 
     def __init__(self, in_channels, out_channels, bias=True):
         super().__init__(in_channels, out_channels, bias)
@@ -485,6 +497,11 @@ class BGEMMLinear_elastic_signed(_ScaledBinaryLinear):
             self._initialize(x, self.weight)
         if self._fusable(x):
             return self._add_bias(self._fused_forward(x))
+        if self.fuse_training and x.is_cuda and self._fn is bgemm_linear_elastic_signed:
+            # recorded: one autograd node for the whole layer (three launches forward, two backward) where its types and sizes allow
+            out = _lib.native().elastic_train(x, self.weight, self.sa, self.sw, self.bias, self.grad_scale)
+            if out is not None:
+                return out
         return self._add_bias(self._fn.apply(x, self.weight, self.sa, self.sw, self.grad_scale))
 
 

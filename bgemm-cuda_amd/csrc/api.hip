@@ -143,10 +143,10 @@ static int packed_forward(int mode, const void* W_tiled, const void* X_tiled, co
     GemmArgs a;
     memset(&a, 0, sizeof a);
     if (!mode_coef(mode, &a.mc)) return fail(BGEMM_EINVAL, "bgemm_packed_forward: unknown mode %d", mode);
-    if (out_dtype < BGEMM_OUT_I32 || out_dtype > BGEMM_OUT_BITS_F16)
+    if (out_dtype < BGEMM_OUT_I32 || out_dtype > OUT_F32_ELASTIC)
         return fail(BGEMM_EINVAL, "bgemm_packed_forward: unknown output dtype %d", out_dtype);
     const bool bits = out_dtype == BGEMM_OUT_BITS_F32 || out_dtype == BGEMM_OUT_BITS_F16;
-    const bool scaled = bits || out_dtype == BGEMM_OUT_F32_SCALED || out_dtype == BGEMM_OUT_F16_SCALED;
+    const bool scaled = bits || out_dtype == BGEMM_OUT_F32_SCALED || out_dtype == BGEMM_OUT_F16_SCALED || out_dtype == OUT_F32_ELASTIC;
     int family, force;
     if (!split_variant(variant, &family, &force))
         return fail(BGEMM_EINVAL, "bgemm_packed_forward: unknown variant %d", variant);
@@ -251,12 +251,22 @@ static int packed_forward(int mode, const void* W_tiled, const void* X_tiled, co
     return launch_gemm_mfma(a, (hipStream_t)stream, fp4);
 }
 
+namespace bgemm {
+int packed_forward_elastic(const void* W_tiled, const void* X_tiled, float* out, int64_t M, int64_t N, int64_t K, const float* sw, const float* sa,
+                           const float* bias, hipStream_t st)
+{
+    return packed_forward(BGEMM_MODE_XOR, W_tiled, X_tiled, nullptr, out, OUT_F32_ELASTIC, 1, M, N, K, 0, 0, N * M, 8, BGEMM_VARIANT_AUTO, nullptr, 0,
+                          nullptr, 0, sw, sa, bias, nullptr, st);
+}
+}  // namespace bgemm
+
 extern "C" int bgemm_packed_kernel_id(int mode, int out_dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int splitK,
                                       int variant)
 {
     // the same checks and the same choice as a call, with stand-in pointers that are never dereferenced
     // and a workspace that is never too small
     alignas(16) static char stand_in[16];
+    if (out_dtype > BGEMM_OUT_BITS_F16) return fail(BGEMM_EINVAL, "bgemm_packed_kernel_id: unknown output dtype %d", out_dtype);
     return packed_forward(mode, stand_in, stand_in, stand_in, stand_in, out_dtype, batch, M, N, K, 0, 0, M * N,
                           splitK, variant, stand_in, (size_t)-1, stand_in, (size_t)-1, stand_in, stand_in, nullptr, nullptr,
                           nullptr, nullptr, true);
@@ -332,6 +342,7 @@ extern "C" int bgemm_packed_weight_forward(int mode, const void* W_tiled, const 
 {
     if (x_dtype != BGEMM_SRC_F16 && x_dtype != BGEMM_SRC_F32)
         return fail(BGEMM_EINVAL, "bgemm_packed_weight_forward: unknown activation type %d", x_dtype);
+    if (out_dtype > BGEMM_OUT_BITS_F16) return fail(BGEMM_EINVAL, "bgemm_packed_weight_forward: unknown output dtype %d", out_dtype);
     if (K == 0 || M == 0 || N == 0)      // nothing to pack: the packed entry point's empty cases
         return packed_forward(mode, W_tiled, nullptr, nullptr, out, out_dtype, 1, M, N, K, 0, 0, 0, 1, variant, nullptr, 0,
                               nullptr, 0, sw, sa, bias, next_zero_point, stream);

@@ -71,6 +71,9 @@ __device__ __forceinline__ int skinny_value(const ModeCoef& mc, const bool two, 
     return two ? val + mc.cb2 * pb2 + dot_terms2(mc, d, d2) : val + dot_term(mc, d);
 }
 
+// An output kind of the library's own, beside the public ones: fp32, scaled in the learned-scale layer's order (elastic_f32).
+constexpr int OUT_F32_ELASTIC = 6;
+
 struct GemmArgs {
     const uint4* W; const uint4* X; const uint4* X2;
     void* out; int out_kind;       // BGEMM_OUT_*
@@ -194,10 +197,25 @@ __device__ __forceinline__ __half scaled_f16(const GemmArgs& a, const int64_t m,
     __half_raw h; h.data = r;
     return __half(h);
 }
+// The learned-scale layer's order, (half(acc) * sa) * sw (+ bias) with fp32 parameters and sa a 0-dim tensor: torch takes a 0-dim
+// tensor in the other operand's type, so sa is rounded to fp16 and the first product is an fp16 one (tests/python/bgemm_linear.py:374).
+__device__ __forceinline__ float elastic_f32(const int v, const float sw, const float sa, const bool has_bias, const float bias)
+{
+#pragma clang fp contract(off)
+    const _Float16 t = (_Float16)(float)v * (_Float16)sa;
+    float r = (float)t * sw;
+    if (has_bias) r = r + bias;
+    return r;
+}
+__device__ __forceinline__ float elastic_f32(const GemmArgs& a, const int64_t m, const int v)
+{
+    return elastic_f32(v, reinterpret_cast<const float*>(a.ep_sw)[m], *reinterpret_cast<const float*>(a.ep_sa), a.ep_bias != nullptr,
+                       a.ep_bias ? reinterpret_cast<const float*>(a.ep_bias)[m] : 0.f);
+}
 // The same with the column's parameters already in registers (a store loop walks rows of fixed columns:
 // the parameters are fetched once per column, not once per element), fp16 parameters widened to fp32.
 struct ColParams { float sw, bias; };
-__device__ __forceinline__ bool f32_params(const int kind) { return kind == BGEMM_OUT_F32_SCALED || kind == BGEMM_OUT_BITS_F32; }
+__device__ __forceinline__ bool f32_params(const int kind) { return kind == BGEMM_OUT_F32_SCALED || kind == BGEMM_OUT_BITS_F32 || kind == OUT_F32_ELASTIC; }
 __device__ __forceinline__ float ep_scalar(const int kind, const void* p)
 {
     return f32_params(kind) ? *reinterpret_cast<const float*>(p) : __half2float(*reinterpret_cast<const __half*>(p));
@@ -254,7 +272,7 @@ __host__ __device__ __forceinline__ int out_elem_shift(const int kind) { return 
 // Bits kinds: the scaled output is not stored; the next binary layer's operand is, i.e. the sign bit
 // of half_rn(y - zp) with y evaluated as above.  The subtraction is exact enough for its sign to
 // survive the rounding to fp16, so the sign bit of the fp32 difference is taken.
-__device__ __forceinline__ bool bits_kind(const int kind) { return kind >= BGEMM_OUT_BITS_F32; }
+__device__ __forceinline__ bool bits_kind(const int kind) { return kind == BGEMM_OUT_BITS_F32 || kind == BGEMM_OUT_BITS_F16; }
 __device__ __forceinline__ unsigned next_sign_bit(const GemmArgs& a, const int64_t m, const int v)
 {
 #pragma clang fp contract(off)      // every step rounds by itself, as torch's separate kernels do
@@ -285,6 +303,7 @@ __device__ __forceinline__ void store_out_as(const GemmArgs& a, const int64_t ro
     if constexpr (KIND == BGEMM_OUT_I32) reinterpret_cast<int*>(a.out)[row0 + m] = v;
     else if constexpr (KIND == BGEMM_OUT_F16) reinterpret_cast<__half*>(a.out)[row0 + m] = __float2half_rn((float)v);
     else if constexpr (KIND == BGEMM_OUT_F32_SCALED) reinterpret_cast<float*>(a.out)[row0 + m] = scaled_f32(a, m, v);
+    else if constexpr (KIND == OUT_F32_ELASTIC) reinterpret_cast<float*>(a.out)[row0 + m] = elastic_f32(a, m, v);
     else reinterpret_cast<__half*>(a.out)[row0 + m] = scaled_f16(a, m, v);
 }
 __device__ __forceinline__ void store_out(const GemmArgs& a, const int64_t row0, const int64_t m, const int v)
@@ -293,6 +312,7 @@ __device__ __forceinline__ void store_out(const GemmArgs& a, const int64_t row0,
     case BGEMM_OUT_I32: store_out_as<BGEMM_OUT_I32>(a, row0, m, v); break;
     case BGEMM_OUT_F16: store_out_as<BGEMM_OUT_F16>(a, row0, m, v); break;
     case BGEMM_OUT_F32_SCALED: store_out_as<BGEMM_OUT_F32_SCALED>(a, row0, m, v); break;
+    case OUT_F32_ELASTIC: store_out_as<OUT_F32_ELASTIC>(a, row0, m, v); break;
     default: store_out_as<BGEMM_OUT_F16_SCALED>(a, row0, m, v); break;
     }
 }
@@ -300,6 +320,14 @@ __device__ __forceinline__ void store_out(const GemmArgs& a, const int64_t row0,
 // Sign-packs two fp16 [rows][K] operands (row stride K) into tiled buffers with one launch.
 int pack_sign_pair(const void* srcA, int64_t rowsA, void* dstA, const void* srcB, int64_t rowsB, void* dstB,
                    int64_t K, hipStream_t st, const char* who);
+
+// bgemm_packed_forward with the kind OUT_F32_ELASTIC on one bit plane a side.
+int packed_forward_elastic(const void* W_tiled, const void* X_tiled, float* out, int64_t M, int64_t N, int64_t K, const float* sw, const float* sa,
+                           const float* bias, hipStream_t st);
+// Sign and nonzero planes of the learned-scale layer's operands, (x - mean(x)) / sa and w - mean(w), fp32 rows of K: the means come as
+// `nparts` partial sums each (parts: x's, then w's) and are left in means[0], means[1].
+int pack_elastic_pair(const float* x, int64_t N, void* x_sign, void* x_nonzero, const float* w, int64_t M, void* w_sign, void* w_nonzero, int64_t K,
+                      const float* parts, int nparts, const float* sa, float* means, hipStream_t st, const char* who);
 
 // Kernel families (each in its own translation unit).
 int launch_gemm_mfma(const GemmArgs& a, hipStream_t st, bool fp4);

@@ -571,7 +571,7 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
     }
     // (the same for the scaled kinds stored four elements a lane: fp32, and fp16 rows that are no multiple of eight long)
     ColParams cp4[4];
-    if (a.vec_store && a.vec_store != 8 && (a.out_kind == BGEMM_OUT_F32_SCALED || a.out_kind == BGEMM_OUT_F16_SCALED)) {
+    if (a.vec_store && a.vec_store != 8 && (a.out_kind == BGEMM_OUT_F32_SCALED || a.out_kind == BGEMM_OUT_F16_SCALED || a.out_kind == OUT_F32_ELASTIC)) {
         saf8 = ep_scalar(a.out_kind, a.ep_sa);
 #pragma unroll
         for (int e = 0; e < 4; e++) cp4[e] = col_params(a, (int64_t)mt0 * 32 + (lane % (WM * 8)) * 4 + e);
@@ -701,6 +701,11 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
                                                __float_as_int(scaled_f32(q.z, cp[2], saf, has_bias)), __float_as_int(scaled_f32(q.w, cp[3], saf, has_bias))),
                                 (a.nt_store != 0 || (a.KT >= 8 && a.KT < 32)));
                         break;
+                    case OUT_F32_ELASTIC: {
+                        auto e = [&](const int v, const ColParams c) { return __float_as_int(elastic_f32(v, c.sw, saf, has_bias, c.bias)); };
+                        store16(dst, make_int4(e(q.x, cp[0]), e(q.y, cp[1]), e(q.z, cp[2]), e(q.w, cp[3])), (a.nt_store != 0 || (a.KT >= 8 && a.KT < 32)));
+                        break;
+                    }
                     default:
                         pk.h[0] = scaled_f16(q.x, cp[0], saf, has_bias); pk.h[1] = scaled_f16(q.y, cp[1], saf, has_bias);
                         pk.h[2] = scaled_f16(q.z, cp[2], saf, has_bias); pk.h[3] = scaled_f16(q.w, cp[3], saf, has_bias);

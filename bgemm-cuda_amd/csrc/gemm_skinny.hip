@@ -444,6 +444,7 @@ __global__ __launch_bounds__(KW * 64, FUSEX && KW <= 8 ? 4 : 2) void gemm_skinny
     case BGEMM_OUT_F16: elements(std::integral_constant<int, BGEMM_OUT_F16>{}); break;
     case BGEMM_OUT_F32_SCALED: elements(std::integral_constant<int, BGEMM_OUT_F32_SCALED>{}); break;
     case BGEMM_OUT_F16_SCALED: elements(std::integral_constant<int, BGEMM_OUT_F16_SCALED>{}); break;
+    case OUT_F32_ELASTIC: elements(std::integral_constant<int, OUT_F32_ELASTIC>{}); break;
     default:        // the bits kinds: every lane takes part in the ballot
         outputs([&](const int n, const int m, const int val) {
             store_bits_word(a, b, n, (int64_t)rt * 32, m < M ? next_sign_bit(a, m, val) : 0u);
@@ -617,6 +618,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_popc_kernel(const GemmArg
     case BGEMM_OUT_F16: elements(std::integral_constant<int, BGEMM_OUT_F16>{}); break;
     case BGEMM_OUT_F32_SCALED: elements(std::integral_constant<int, BGEMM_OUT_F32_SCALED>{}); break;
     case BGEMM_OUT_F16_SCALED: elements(std::integral_constant<int, BGEMM_OUT_F16_SCALED>{}); break;
+    case OUT_F32_ELASTIC: elements(std::integral_constant<int, OUT_F32_ELASTIC>{}); break;
     default:        // the bits kinds: every lane takes part in the ballot
         outputs([&](const int n, const int m, const int val) {
             store_bits_word(a, b, n, (int64_t)rt * 32, m < M ? next_sign_bit(a, m, val) : 0u);
@@ -777,6 +779,7 @@ __global__ __launch_bounds__(KW * 64, 2) void gemm_skinny_splitk_quad_kernel(con
     case BGEMM_OUT_F16: elements(std::integral_constant<int, BGEMM_OUT_F16>{}); break;
     case BGEMM_OUT_F32_SCALED: elements(std::integral_constant<int, BGEMM_OUT_F32_SCALED>{}); break;
     case BGEMM_OUT_F16_SCALED: elements(std::integral_constant<int, BGEMM_OUT_F16_SCALED>{}); break;
+    case OUT_F32_ELASTIC: elements(std::integral_constant<int, OUT_F32_ELASTIC>{}); break;
     default:        // the bits kinds: a half-wave holds the 32 columns of one weight row tile, every lane takes part
         outputs([&](const int n, const int m, const int i, const int val) {
             store_bits_word(a, b, n, (int64_t)(rt0 + i) * 32, m < M ? next_sign_bit(a, m, val) : 0u);

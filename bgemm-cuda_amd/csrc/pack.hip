@@ -21,6 +21,10 @@ struct PackJob {
     const void* src; int64_t rows, K, ld;
     uint32_t* dst0; uint32_t* dst1; int mode;
     const void* zp;
+    // the zero point as a mean of the operand itself, fp32: `nparts` partial sums (up to 128), 1 / elements, and where to leave it
+    const float* parts; float* mean_out; int nparts; float inv_n;
+    const float* divisor;          // the values are divided by this scalar: its sign turns theirs
+    NonzeroRule nonzero;
     int64_t rows_out, nseg, KT, Kw, waves;
     int64_t nmat, inner, so, si, mtiles;
 };
@@ -35,6 +39,33 @@ __device__ __forceinline__ int64_t source_row(const PackJob& j, const int64_t ro
     return o * j.so + i * j.si + rl * j.ld;
 }
 
+// Elements k0 .. k0 + 7 of a source row, centred (and turned), those from K on as +0.0.
+__device__ __forceinline__ void load8_as_float(const void* row, const bool f32, const int64_t k0, const int64_t K, const float zf, const bool turn, float (&f)[8])
+{
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        f[e] = 0.f;
+        if (k0 + e < K) {
+            const float v = f32 ? reinterpret_cast<const float*>(row)[k0 + e] : __half2float(reinterpret_cast<const __half*>(row)[k0 + e]);
+            f[e] = turn ? -__fsub_rn(v, zf) : __fsub_rn(v, zf);
+        }
+    }
+}
+
+// The scalar an operand is centred by, and whether it is; wave-uniform.
+__device__ __forceinline__ float job_center(const PackJob& j, const bool f32, const int lane)
+{
+    if (j.parts) {
+        float s = lane < j.nparts ? j.parts[lane] : 0.f;
+        if (lane + 64 < j.nparts) s += j.parts[lane + 64];
+#pragma unroll
+        for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d);
+        return s * j.inv_n;
+    }
+    return !j.zp ? 0.f : f32 ? *reinterpret_cast<const float*>(j.zp) : __half2float(*reinterpret_cast<const __half*>(j.zp));
+}
+__device__ __forceinline__ bool job_centred(const PackJob& j) { return j.zp != nullptr || (j.mode & 16); }
+
 // Logical output: one wave packs 512 consecutive K elements of one row (16 words).
 __device__ __forceinline__ void pack_wave(const PackJob& j, const int64_t gw, const int lane)
 {
@@ -44,21 +75,24 @@ __device__ __forceinline__ void pack_wave(const PackJob& j, const int64_t gw, co
 
     uint32_t sg = 0, nz = 0;              // elements past K stay +0.0
     const int64_t soff = source_row(j, row);
+    const float zf = job_center(j, j.mode & 4, lane);
+    const bool turn = j.divisor && *j.divisor < 0.f;
+    if (j.mean_out && gw == 0 && lane == 0) *j.mean_out = zf;
     if (soff >= 0 && k0 < j.K) {
-        const bool f32 = j.mode & 4, centred = j.zp != nullptr;
-        const float zf = !centred ? 0.f : f32 ? *reinterpret_cast<const float*>(j.zp) : __half2float(*reinterpret_cast<const __half*>(j.zp));
+        const bool f32 = j.mode & 4, centred = job_centred(j);
         const char* const src = reinterpret_cast<const char*>(j.src) + soff * (f32 ? 4 : 2);
         if (j.K >= 8) {
             // the row's last chunk is read as its last eight elements, and the bits shifted into place
             const int64_t kc = k0 + 8 <= j.K ? k0 : j.K - 8;
-            if (f32) bits8(load_raw8<true>(src, kc), centred, zf, sg, nz);
-            else bits8(load_raw8<false>(src, kc), centred, zf, sg, nz);
+            if (f32) bits8(load_raw8<true>(src, kc), centred, zf, j.nonzero, sg, nz);
+            else bits8(load_raw8<false>(src, kc), centred, zf, j.nonzero, sg, nz);
+            if (turn) sg ^= 0xffu;
             sg = (sg << (k0 - kc)) & 0xffu;
             nz = (nz << (k0 - kc)) & 0xffu;
         } else {
-            uint16_t h[8];
-            load8_as_half(src, f32, k0, j.K, centred, zf, h);
-            bits8(h, sg, nz);
+            float f[8];
+            load8_as_float(src, f32, k0, j.K, zf, turn, f);
+            bits8(f, j.nonzero, sg, nz);
         }
     }
     const bool ternary = j.mode & (1 | 16);
@@ -99,10 +133,11 @@ __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, co
         off0 = o * j.so + i * j.si + rtl * TILE_ROWS * j.ld;
         rows_left = j.rows - rtl * TILE_ROWS;
     }
-    const bool ternary = j.mode & (1 | 16), centred = j.zp != nullptr;      // two planes are written
+    const bool ternary = j.mode & (1 | 16), centred = job_centred(j);      // two planes are written
     const bool nz_first = j.mode & 1, nz_second = j.mode & 16;
-    float zf = 0.f;
-    if (centred) zf = F32 ? *reinterpret_cast<const float*>(j.zp) : __half2float(*reinterpret_cast<const __half*>(j.zp));
+    const float zf = job_center(j, F32, lane);
+    const bool turn = j.divisor && *j.divisor < 0.f;
+    if (j.mean_out && gw == 0 && lane == 0) *j.mean_out = zf;
     const int64_t left = j.K - kt * TILE_KBITS;
     typedef typename std::conditional<F32, uint32_t, uint16_t>::type E;
     const E* const src = reinterpret_cast<const E*>(j.src) + off0;
@@ -128,7 +163,8 @@ __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, co
                 for (int jj = 0; jj < G; jj++) {
                     const int r = RI * (g + jj) + rs, at = slot_byte(c, r);
                     uint32_t sg, nz;
-                    bits8(raw[jj], centred, zf, sg, nz);
+                    bits8(raw[jj], centred, zf, j.nonzero, sg, nz);
+                    if (turn) sg ^= 0xffu;
                     const uint32_t keep = row0 + r <= last_row ? 0xffu : 0u;
                     sg = (sg << shift) & keep; nz = (nz << shift) & keep;
                     lds[at] = (unsigned char)(nz_first ? nz : sg);
@@ -144,10 +180,10 @@ __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, co
         const int c = lane & 31;
         for (int jj = 0; jj < RW / 2; jj++) {
             const int rl = 2 * jj + (lane >> 5), r = row0 + rl, at = slot_byte(c, rl);
-            uint16_t h[8];
+            float f[8];
             uint32_t sg, nz;
-            load8_as_half(src + (int64_t)(r < last_row ? r : last_row) * j.ld, F32, r <= last_row ? 8 * c : j.K, j.K, centred, zf, h);
-            bits8(h, sg, nz);
+            load8_as_float(src + (int64_t)(r < last_row ? r : last_row) * j.ld, F32, r <= last_row ? 8 * c : j.K, j.K, zf, turn, f);
+            bits8(f, j.nonzero, sg, nz);
             lds[at] = (unsigned char)(nz_first ? nz : sg);
             if (ternary) lds[PLANE + at] = (unsigned char)(nz_second ? nz : sg & nz);
         }
@@ -210,6 +246,7 @@ static int make_job(PackJob* j, const void* src, int64_t rows, int64_t K, int64_
     if (rows == 0 || K == 0 || outer * inner == 0) return BGEMM_OK;
     if (!src || !d0 || ((mode & (1 | 16)) && !d1)) return fail(BGEMM_ENULL, "%s: null pointer", who);
     if (((uintptr_t)d0 & 15) || ((uintptr_t)d1 & 15)) return fail(BGEMM_EALIGN, "%s: destination not 16-byte aligned", who);
+    j->nonzero = mode & 16 ? nonzero_sign_half() : nonzero_half();
     j->src = src; j->zp = zp; j->rows = rows; j->K = K; j->ld = ld;
     j->dst0 = (uint32_t*)d0; j->dst1 = (uint32_t*)d1; j->mode = mode;
     j->KT = k_tiles(K); j->Kw = cdiv(K, 32);
@@ -257,6 +294,21 @@ int pack_sign_pair(const void* srcA, int64_t rowsA, void* dstA, const void* srcB
     int rc = make_job(&j0, srcA, rowsA, K, K, dstA, nullptr, 0, nullptr, who);
     if (!rc) rc = make_job(&j1, srcB, rowsB, K, K, dstB, nullptr, 0, nullptr, who);
     return rc ? rc : launch_jobs(j0, j1, st, who);
+}
+
+// Sign and nonzero planes of the learned-scale layer's operands, centred by their own means (see common.h).
+int pack_elastic_pair(const float* x, int64_t N, void* x_sign, void* x_nonzero, const float* w, int64_t M, void* w_sign, void* w_nonzero, int64_t K,
+                      const float* parts, int nparts, const float* sa, float* means, hipStream_t st, const char* who)
+{
+    PackJob j0, j1;
+    int rc = make_job(&j0, x, N, K, K, x_sign, x_nonzero, 16 | 4, nullptr, who);
+    if (!rc) rc = make_job(&j1, w, M, K, K, w_sign, w_nonzero, 16 | 4, nullptr, who);
+    if (rc) return rc;
+    j0.parts = parts; j0.inv_n = 1.f / (float)(N * K); j0.mean_out = means; j0.divisor = sa;
+    j1.parts = parts + nparts; j1.inv_n = 1.f / (float)(M * K); j1.mean_out = means + 1;
+    j0.nparts = j1.nparts = nparts;
+    j0.nonzero = j1.nonzero = nonzero_sign_float();
+    return launch_jobs(j0, j1, st, who);
 }
 
 }  // namespace bgemm

@@ -39,16 +39,24 @@ __device__ __forceinline__ void bits8(const uint4 v, uint32_t& sg, uint32_t& nz)
     sg &= 0xffu; nz &= 0xffu;
 }
 
-// Sign (and nonzero) bits of eight fp32 values as their fp16 roundings have them (`.to(torch.half)`): the rounding keeps
-// the sign, and gives zero up to and including 2^-25 (half the smallest fp16 number, a tie that goes to even).
-__device__ __forceinline__ void bits8(const float (&f)[8], uint32_t& sg, uint32_t& nz)
+// Which magnitudes (fp32 bit patterns without the sign) count as nonzero: lo .. lo + span.
+struct NonzeroRule { uint32_t lo, span; };
+// of a value's fp16 rounding (`.to(torch.half)`): zero up to and including 2^-25, half the smallest fp16 number, a tie that goes to even
+constexpr uint32_t HALF_NONZERO = 0x33000001u, INF_BITS = 0x7f800000u;
+__host__ __device__ static inline NonzeroRule nonzero_half() { return {HALF_NONZERO, 0x7fffffffu - HALF_NONZERO}; }
+// the same as torch.sign has it, for which NaN is zero, and that of the fp32 value itself
+__host__ __device__ static inline NonzeroRule nonzero_sign_half() { return {HALF_NONZERO, INF_BITS - HALF_NONZERO}; }
+__host__ __device__ static inline NonzeroRule nonzero_sign_float() { return {1u, INF_BITS - 1u}; }
+
+// Sign (and nonzero) bits of eight fp32 values, element e at bit 7 - e (rounding to fp16 keeps the sign).
+__device__ __forceinline__ void bits8(const float (&f)[8], const NonzeroRule rule, uint32_t& sg, uint32_t& nz)
 {
     sg = 0; nz = 0;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
         const uint32_t u = __float_as_uint(f[e]);
         sg = (sg << 1) | (u >> 31);
-        nz = (nz << 1) | (uint32_t)((u & 0x7fffffffu) > 0x33000000u);
+        nz = (nz << 1) | (uint32_t)((u & 0x7fffffffu) - rule.lo <= rule.span);
     }
 }
 
@@ -67,21 +75,21 @@ __device__ __forceinline__ Raw8<F32> load_raw8(const void* row, const int64_t k)
 
 // Their sign and nonzero bits, element e at bit 7 - e, after subtracting the zero point if there is one.
 template <bool F32>
-__device__ __forceinline__ void bits8(const Raw8<F32>& r, const bool centred, const float zf, uint32_t& sg, uint32_t& nz)
+__device__ __forceinline__ void bits8(const Raw8<F32>& r, const bool centred, const float zf, const NonzeroRule rule, uint32_t& sg, uint32_t& nz)
 {
     if constexpr (F32) {
         const uint32_t d[8] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w, r.v[1].x, r.v[1].y, r.v[1].z, r.v[1].w};
         float f[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) f[e] = centred ? __fsub_rn(__uint_as_float(d[e]), zf) : __uint_as_float(d[e]);
-        bits8(f, sg, nz);
+        bits8(f, rule, sg, nz);
     } else if (centred) {
         const uint32_t d[4] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w};
         float f[8];
 #pragma unroll
         for (int e = 0; e < 8; e++)
             f[e] = __fsub_rn(__half2float(__ushort_as_half((uint16_t)(d[e >> 1] >> (16 * (e & 1))))), zf);
-        bits8(f, sg, nz);
+        bits8(f, rule, sg, nz);
     } else
         bits8(r.v[0], sg, nz);
 }

@@ -206,7 +206,140 @@ PyObject* linear_train(PyObject*, PyObject* const* args, const Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
+// ---- the learned-scale layer as one autograd node ----------------------------------------------------------------------------------
+// (half(acc) * sa) * sw (+ bias) of (x - mean(x)) / sa and w - mean(w) (tests/python/bgemm_linear.py:350-457, :538-564): three launches
+// forward, two backward.  Kept: sign and nonzero planes of both operands, the means, and the operands themselves (as references).
+struct ElasticNode : public torch::autograd::Node {
+    int64_t N, K, M, words_x, words_w;
+    double grad_scale;
+    Tensor planes;                                  // [x sign | x nonzero | w sign | w nonzero | stats]
+    SavedVariable x_, weight_, sa_, sw_, bias_;
+    bool has_bias;
+
+    std::string name() const override { return "ElasticBinaryLinearBackward"; }
+
+    void release_variables() override
+    {
+        std::lock_guard<std::mutex> lock(mutex_);
+        planes.reset();
+        for (SavedVariable* s : {&x_, &weight_, &sa_, &sw_, &bias_}) s->reset_data();
+    }
+
+    variable_list differentiable(const Tensor& grad)
+    {
+        pybind11::gil_scoped_acquire gil;
+        const Tensor bias = has_bias ? bias_.unpack() : Tensor();
+        PyObject* const module = PyImport_ImportModule("bgemm_linear");
+        if (!module) throw python_error();
+        PyObject* const need = PyTuple_New(5);
+        for (int i = 0; i < 5; i++) PyTuple_SET_ITEM(need, i, PyBool_FromLong(i < (has_bias ? 5 : 4) && task_should_compute_output(i)));
+        PyObject* const got = PyObject_CallMethod(module, "_elastic_grads", "NNNNNdNN", THPVariable_Wrap(x_.unpack()), THPVariable_Wrap(weight_.unpack()),
+                                                  THPVariable_Wrap(sa_.unpack()), THPVariable_Wrap(sw_.unpack()), THPVariable_Wrap(bias), grad_scale,
+                                                  THPVariable_Wrap(grad), need);
+        Py_DECREF(module);
+        if (!got) throw python_error();
+        variable_list r;
+        for (int i = 0; i < (has_bias ? 5 : 4); i++) r.push_back(tensor_or_none(PyTuple_GET_ITEM(got, i)));
+        Py_DECREF(got);
+        return r;
+    }
+
+    variable_list apply(variable_list&& grads) override
+    {
+        std::lock_guard<std::mutex> lock(mutex_);
+        const size_t inputs = has_bias ? 5 : 4;
+        if (!grads[0].defined()) return variable_list(inputs);
+        TORCH_CHECK(planes.defined(), torch::autograd::ERR_BACKWARD_TWICE);
+        if (c10::GradMode::is_enabled()) return differentiable(grads[0]);
+        const c10::OptionalDeviceGuard guard(planes.device());
+        const bool want_x = task_should_compute_output(0), want_sa = task_should_compute_output(2);
+        const bool need_x = want_x || want_sa, need_w = task_should_compute_output(1) || task_should_compute_output(3);
+        const Tensor g = grads[0].contiguous(), x = x_.unpack().contiguous(), w = weight_.unpack().contiguous(), sa = sa_.unpack();
+        Tensor gx, gw, gb, gsw, gsa;
+        const bool need_b = has_bias && task_should_compute_output(4);
+        if (!need_x && !need_w) {
+            if (need_b) gb = g.reshape({N, M}).sum(0);
+        } else {
+            if (need_x) gx = at::empty(x.sizes(), g.options());
+            if (want_sa) gsa = at::empty({}, g.options());
+            if (need_w) {
+                gw = at::empty({M, K}, g.options());
+                gsw = at::empty({M}, g.options());
+            }
+            if (need_b) gb = at::empty({M}, g.options());
+            const size_t bytes = bgemm_elastic_backward_workspace_bytes(N, M, K, need_x, need_w);
+            const Tensor ws = at::empty({(int64_t)bytes}, g.options().dtype(at::kByte));
+            const int32_t* const p = planes.data_ptr<int32_t>();
+            const int32_t* const pw = p + 2 * words_x;
+            check(bgemm_elastic_backward(p, p + words_x, pw, pw + words_w, g.data_ptr(), x.data_ptr(), w.data_ptr(), pw + 2 * words_w, sa.data_ptr(),
+                                         (float)grad_scale, N, M, K, data_or_null(gx), data_or_null(gw), data_or_null(gb), data_or_null(gsw),
+                                         data_or_null(gsa), ws.data_ptr(), bytes, stream_of(g)));
+        }
+        variable_list r = {want_x ? gx : Tensor(), gw, gsa, gsw};
+        if (has_bias) r.push_back(gb);
+        return r;
+    }
+};
+
+// elastic_train(x, weight, sa, sw, bias | None, grad_scale) -> y, or None where the separate operations have to run
+PyObject* elastic_train(PyObject*, PyObject* const* args, const Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    TORCH_CHECK_TYPE(n == 6, "elastic_train takes 6 arguments");
+    for (int i = 0; i < 5; i++)
+        if (!THPVariable_Check(args[i]) && !(i == 4 && args[i] == Py_None)) Py_RETURN_NONE;
+    const Tensor &x = tensor_at(args[0]), &w = tensor_at(args[1]), &sa = tensor_at(args[2]), &sw = tensor_at(args[3]);
+    const Tensor bias = tensor_or_none(args[4]);
+    const double grad_scale = PyFloat_AsDouble(args[5]);
+    if (grad_scale == -1.0 && PyErr_Occurred()) throw python_error();
+    if (!c10::GradMode::is_enabled() || !x.is_cuda() || w.dim() != 2 || x.dim() < 1 || x.numel() == 0 || sa.dim() != 0) Py_RETURN_NONE;
+    const int64_t M = w.size(0), K = w.size(1), N = x.numel() / (K ? K : 1);
+    if (M < 2 || M > (1 << 20) || K < 1 || K >= (1 << 24) || x.size(-1) != K || N > (1 << 20)) Py_RETURN_NONE;
+    for (const Tensor* t : {&x, &w, &sa, &sw})
+        if (t->scalar_type() != at::kFloat || t->device() != x.device() || t->layout() != at::kStrided) Py_RETURN_NONE;
+    if (sw.dim() != 1 || sw.size(0) != M || !sw.is_contiguous()) Py_RETURN_NONE;
+    if (bias.defined() && (bias.scalar_type() != at::kFloat || bias.device() != x.device() || bias.dim() != 1 || bias.size(0) != M || !bias.is_contiguous())) Py_RETURN_NONE;
+    Tensor out;
+    {
+        const WithoutGil no_gil;
+        bool recorded = bias.defined() && bias.requires_grad();
+        for (const Tensor* t : {&x, &w, &sa, &sw}) recorded |= t->requires_grad();
+        const int64_t words_x = bgemm_tiled_words(N, K), words_w = bgemm_tiled_words(M, K);
+        Tensor planes;
+        {
+            const c10::NoGradGuard no_grad;
+            const c10::OptionalDeviceGuard guard(x.device());
+            const Tensor x2 = x.contiguous(), w2 = w.contiguous();
+            planes = at::empty({2 * (words_x + words_w) + BGEMM_ELASTIC_STATS}, x.options().dtype(at::kInt));
+            std::vector<int64_t> shape = x.sizes().vec();
+            shape.back() = M;
+            out = at::empty(shape, x.options());
+            int32_t* const p = planes.data_ptr<int32_t>();
+            int32_t* const pw = p + 2 * words_x;
+            check(bgemm_elastic_forward(x2.data_ptr(), w2.data_ptr(), N, M, K, sa.data_ptr(), sw.data_ptr(), data_or_null(bias), p, p + words_x, pw,
+                                        pw + words_w, pw + 2 * words_w, out.data_ptr(), stream_of(x)));
+        }
+        if (recorded) {
+            auto node = std::shared_ptr<ElasticNode>(new ElasticNode(), torch::autograd::deleteNode);
+            node->N = N; node->K = K; node->M = M; node->words_x = words_x; node->words_w = words_w;
+            node->grad_scale = grad_scale; node->has_bias = bias.defined();
+            node->planes = planes;
+            node->x_ = SavedVariable(x, false); node->weight_ = SavedVariable(w, false);
+            node->sa_ = SavedVariable(sa, false); node->sw_ = SavedVariable(sw, false);
+            if (bias.defined()) {
+                node->bias_ = SavedVariable(bias, false);
+                node->set_next_edges(torch::autograd::collect_next_edges(x, w, sa, sw, bias));
+            } else
+                node->set_next_edges(torch::autograd::collect_next_edges(x, w, sa, sw));
+            torch::autograd::set_history(out, node);
+        }
+    }
+    return THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"elastic_train", (PyCFunction)(void (*)(void))elastic_train, METH_FASTCALL, "forward of a learned-scale binary Linear, recorded as one autograd node"},
     {"linear_train", (PyCFunction)(void (*)(void))linear_train, METH_FASTCALL, "forward of a scaled binary Linear, recorded as one autograd node"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -9,6 +9,13 @@
 // kernels this is a dozen passes over [N][M] fp32 matrices.  Here it is one: acc is not kept from the forward pass but
 // multiplied again from the two operands' sign bits (a hundredth of the bytes), in the shadow of the read of G; g16 leaves
 // in the order in which the matrix cores of the two products read it, and their other operand stays packed.
+//
+// The learned-scale layer (BGEMMLinear_elastic_signed; tests/python/bgemm_linear.py:350-457, 519-564), all in fp32:
+//   forward   xs = (x - mean(x)) / sa, ws = w - mean(w), y = half(half(acc) * sa) * sw (+ bias), acc = sum_k sign(xs) sign(ws)
+//   backward  f[n,k] = sum_m G[n,m] sign(ws)[m,k],  g[m,k] = sum_n G[n,m] sign(xs)[n,k]
+//             grad_x = f * 2 / cosh(min(|xs|, 4))^2,  grad_w = g * 2 / cosh(min(|ws|, 4))^2
+//             grad_sa = c sum_n,k inner(xs) f,  grad_sw[m] = c sum_k sign(ws) g,  grad_bias[m] = sum_n G
+// G stays fp32: the same products with G split into three bf16 planes (8 significant bits each, all 24).
 #include "common.h"
 #include "mfma_engines.h"
 #include "pack_bits.h"
@@ -240,8 +247,128 @@ static int grad_rows_per_chunk(int64_t N, int64_t M)
     return (int)(want < 1 ? 1 : want > 16 ? 16 : want);
 }
 
+// ---- the learned-scale layer's own passes -----------------------------------------------------------------------------------
+// Partial sums of x and w for their means: `parts` blocks each.
+__global__ __launch_bounds__(256) void elastic_sums_kernel(const float* __restrict__ x, const int64_t nx, const float* __restrict__ w, const int64_t nw,
+                                                           const int parts, float* __restrict__ out)
+{
+    __shared__ float lds[4];
+    const bool second = (int)blockIdx.x >= parts;
+    const float* const p = second ? w : x;
+    const int64_t n = second ? nw : nx;
+    const int b = blockIdx.x - (second ? parts : 0);
+    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
+    const int64_t step = (int64_t)parts * 1024;
+    int64_t i = (int64_t)b * 1024 + threadIdx.x * 4;
+    if ((((uintptr_t)p) & 15) == 0)
+        for (; i + 4 <= n; i += step) {
+            const float4 v = *reinterpret_cast<const float4*>(p + i);
+            s0 += v.x; s1 += v.y; s2 += v.z; s3 += v.w;
+        }
+    for (; i < n; i += step)                       // the last elements, or all of them where a row of four is not aligned
+        for (int e = 0; e < 4; e++)
+            if (i + e < n) s0 += p[i + e];
+    float s = (s0 + s1) + (s2 + s3);
+#pragma unroll
+    for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
+}
+
+struct ElasticPrepArgs {
+    const float* g;                       // [N][M]
+    uint4* ga; uint4* gt;                 // three planes of G as fragments of rows n and of rows m, or null
+    float* part;                          // [chunks][mpad] column sums
+    uint32_t* ticket;
+    int64_t N, M, mpad;
+    int NT, rt_per_chunk, grid_x, grad_blocks;
+};
+
+// G, fp32, into fragments of both products, with its column sums on the way; as linear_grad_kernel, without the bits.
+__global__ __launch_bounds__(256, 3) void elastic_prep_kernel(const ElasticPrepArgs a, const CodeJob jw, const CodeJob jx)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = lane >> 5, c = lane & 31;
+    if ((int)blockIdx.x >= a.grad_blocks) {
+        const uint32_t gw = (blockIdx.x - a.grad_blocks) * 4 + wave, ww = (uint32_t)(jw.waves + 3) / 4 * 4;
+        if (gw < ww) sign_codes(jw, gw, lane);
+        else sign_codes(jx, gw - ww, lane);
+        return;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.ticket = 0;
+    const int mg = blockIdx.x % a.grid_x * 4 + wave, chunk = blockIdx.x / a.grid_x;
+    if ((int64_t)mg * 64 >= a.M) return;
+    const int64_t m = (int64_t)mg * 64 + 2 * c, mc = m < a.M - 2 ? m : a.M - 2;      // (M >= 2)
+    const bool ok0 = m < a.M, ok1 = m + 1 < a.M, moved = m != mc;
+    const int CT = (int)(a.mpad / 32);
+    __shared__ __align__(16) unsigned char s_tile[4][32 * GA_STRIDE];
+    unsigned char* const st = s_tile[wave];
+    float sum0 = 0.f, sum1 = 0.f;
+    for (int t = chunk * a.rt_per_chunk; t < min(a.NT, (chunk + 1) * a.rt_per_chunk); t++) {
+        uint2 g[16];
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int64_t n = (int64_t)t * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+            __builtin_memcpy(&g[v], a.g + (n < a.N ? n : a.N - 1) * a.M + mc, 8);
+        }
+        // plane p of a value: its next eight significant bits (the first plane alone where it is not finite)
+        float r0[16], r1[16];
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const bool row = (int64_t)t * 32 + 8 * (v >> 2) + 4 * h + (v & 3) < a.N;
+            const float u0 = __uint_as_float(g[v].x), u1 = __uint_as_float(g[v].y);
+            r0[v] = row && ok0 ? (moved ? u1 : u0) : 0.f;
+            r1[v] = row && ok1 ? u1 : 0.f;
+            sum0 += r0[v]; sum1 += r1[v];
+        }
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            uint32_t hp[16];
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const uint32_t b0 = __float_as_uint(r0[v]), b1 = __float_as_uint(r1[v]);
+                hp[v] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+                r0[v] = (b0 & 0x7f800000u) == 0x7f800000u ? 0.f : r0[v] - __uint_as_float(b0 & 0xffff0000u);
+                r1[v] = (b1 & 0x7f800000u) == 0x7f800000u ? 0.f : r1[v] - __uint_as_float(b1 & 0xffff0000u);
+            }
+            if (a.gt) {
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int s = 0; s < 2; s++) {
+                        uint32_t w[4];
+#pragma unroll
+                        for (int q = 0; q < 4; q++)
+                            w[q] = __builtin_amdgcn_perm(hp[8 * s + 2 * q + 1], hp[8 * s + 2 * q], j ? 0x07060302u : 0x05040100u);
+                        a.gt[((((int64_t)mg * 2 + j) * a.NT + t) * 3 + p) * FRAG_U4 + s * 64 + lane] = make_uint4(w[0], w[1], w[2], w[3]);
+                    }
+            }
+            if (a.ga) {
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    *reinterpret_cast<uint32_t*>(st + (8 * (v >> 2) + 4 * h + (v & 3)) * GA_STRIDE + c * 4) = hp[v];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const unsigned char* const from = st + c * GA_STRIDE + (16 * i + 4 * h) * 2;
+                    const uint2 lo = *reinterpret_cast<const uint2*>(from), hi = *reinterpret_cast<const uint2*>(from + 16);
+                    a.ga[(((int64_t)t * CT + mg * 2 + (i >> 1)) * 3 + p) * FRAG_U4 + (i & 1) * 64 + lane] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+    }
+    sum0 += __shfl_xor(sum0, 32);
+    sum1 += __shfl_xor(sum1, 32);
+    if (h == 0) *reinterpret_cast<float2*>(a.part + (int64_t)chunk * a.mpad + m) = make_float2(sum0, sum1);
+}
+
 // ---- the products -----------------------------------------------------------------------------------------------------------
-enum { PROD_F32 = 0, PROD_F16 = 1, PROD_BIREAL_F32 = 2, PROD_BIREAL_F16 = 3 };
+enum { PROD_F32 = 0, PROD_F16 = 1, PROD_BIREAL_F32 = 2, PROD_BIREAL_F16 = 3, PROD_ELASTIC_X = 4, PROD_ELASTIC_W = 5 };
 
 struct ProdArgs {
     const uint4* A; const uint32_t* C;
@@ -249,7 +376,9 @@ struct ProdArgs {
     int64_t colpad, rows, cols;
     int kind, paired;                     // paired: row tile 2 i + j holds rows 64 i + 2 * (row) + j
     void* out;                            // [rows][cols]
-    const void* x; int64_t ldx; const void* zp;      // Bi-Real: the layer's input and its zero point
+    const void* x; int64_t ldx; const void* zp;      // Bi-Real: the layer's input and its zero point; elastic: x or w and its mean
+    const float* sa; float scale;         // elastic: the divisor (x), the scale gradients' factor
+    float* shares;                        // elastic: x: a value per block, w: [rows][column groups], of the scale gradients' sums
 };
 
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
@@ -262,6 +391,22 @@ __device__ __forceinline__ _Float16 bireal_factor(const ProdArgs& a, const int64
 {
     const _Float16 ax = (_Float16)fabsf(__fsub_rn(param<F32>(a.x, row * a.ldx + col), param<F32>(a.zp, 0)));
     return (_Float16)2.0f - (_Float16)2.0f * (ax > (_Float16)1.0f ? (_Float16)1.0f : ax);
+}
+
+// The learned-scale layers' gradient of one element from the straight-through one, and that element's share of the scale's
+// (calculate_gradient_signed, tests/python/bgemm_linear.py:519-535, with Qn = -1, Qp = 1).
+__device__ __forceinline__ float elastic_grad(const ProdArgs& a, const int64_t row, const int64_t col, const float v, float& share)
+{
+    float q = reinterpret_cast<const float*>(a.x)[row * a.ldx + col] - *reinterpret_cast<const float*>(a.zp);
+    float inner;
+    if (a.kind == PROD_ELASTIC_X) {
+        q = q / *a.sa;
+        inner = q > 1.f ? 1.f : q < -1.f ? -1.f : (q > 0.f ? 1.f : q < 0.f ? -1.f : 0.f) - q;
+    } else
+        inner = q > 0.f ? 1.f : q < 0.f ? -1.f : 0.f;
+    share = inner * v * a.scale;
+    const float t = coshf(fminf(fabsf(q), 4.f));
+    return v * (2.f / (t * t));
 }
 
 __device__ __forceinline__ void prod_store(const ProdArgs& a, const int64_t row, const int64_t col, const float v)
@@ -414,16 +559,109 @@ __global__ __launch_bounds__(KW * 64, 2) void sign_product_kernel(const ProdLaun
         for (int v = 0; v < 16; v++) part[kw][b * 16 + v][lane] = acc[b][v];
     __syncthreads();
     constexpr int SHARE = RB * 16 / KW;
-#pragma unroll
-    for (int o = 0; o < SHARE; o++) {
-        const int e = kw * SHARE + o, b = e >> 4, v = e & 15;
+    auto result = [&](const int e, int& r, int64_t& row, int64_t& col) {
+        const int b = e >> 4, v = e & 15;
         float sum = part[0][e][lane];
 #pragma unroll
         for (int k = 1; k < KW; k++) sum += part[k][e][lane];
-        const int r = 8 * (v >> 2) + 4 * h + (v & 3);
-        const int64_t row = a.paired ? (int64_t)(rt >> 1) * 64 + 2 * r + (rt & 1) : (int64_t)rt * 32 + r;
-        const int64_t col = ((int64_t)grp * RB + b) * 32 + (lane & 31);
-        if (row < a.rows && col < a.cols) prod_store(a, row, col, 0.5f * sum);
+        r = 8 * (v >> 2) + 4 * h + (v & 3);
+        row = a.paired ? (int64_t)(rt >> 1) * 64 + 2 * r + (rt & 1) : (int64_t)rt * 32 + r;
+        col = ((int64_t)grp * RB + b) * 32 + (lane & 31);
+        return 0.5f * sum;
+    };
+    if constexpr (NP == 1) {
+#pragma unroll
+        for (int o = 0; o < SHARE; o++) {
+            int r;
+            int64_t row, col;
+            const float v = result(kw * SHARE + o, r, row, col);
+            if (row < a.rows && col < a.cols) prod_store(a, row, col, v);
+        }
+    } else {
+        // elastic: the block's share of the scale's gradient, one value (x) or one a row (w), added in a fixed order
+        float total = 0.f, of_row[SHARE];
+#pragma unroll
+        for (int o = 0; o < SHARE; o++) {
+            int r;
+            int64_t row, col;
+            const float v = result(kw * SHARE + o, r, row, col);
+            float share = 0.f;
+            if (row < a.rows && col < a.cols) reinterpret_cast<float*>(a.out)[row * a.cols + col] = elastic_grad(a, row, col, v, share);
+            total += share;
+            of_row[o] = share;
+        }
+        __shared__ float rows_lds[RB][32], blk[KW];
+        __shared__ bool last;
+        if (a.kind == PROD_ELASTIC_X) {
+#pragma unroll
+            for (int d = 32; d; d >>= 1) total += __shfl_xor(total, d);
+            if (lane == 0) blk[kw] = total;
+        } else {
+#pragma unroll
+            for (int o = 0; o < SHARE; o++) {
+                const int e = kw * SHARE + o;
+#pragma unroll
+                for (int d = 16; d; d >>= 1) of_row[o] += __shfl_xor(of_row[o], d);
+                if ((lane & 31) == 0) rows_lds[e >> 4][8 * ((e & 15) >> 2) + 4 * h + (e & 3)] = of_row[o];
+            }
+        }
+        __syncthreads();
+        auto device_store = [](float* p, const float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+        if (a.kind == PROD_ELASTIC_X) {
+            if (threadIdx.x == 0) {
+                float t = 0.f;
+#pragma unroll
+                for (int k = 0; k < KW; k++) t += blk[k];
+                device_store(a.shares + id, t);
+            }
+        } else if (threadIdx.x < 32) {
+            float t = 0.f;
+#pragma unroll
+            for (int b = 0; b < RB; b++) t += rows_lds[b][threadIdx.x];
+            const int64_t row = (int64_t)(rt >> 1) * 64 + 2 * threadIdx.x + (rt & 1);
+            if (row < a.rows) device_store(a.shares + row * groups + grp, t);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");           // every share has been acknowledged before the ticket is taken
+        __syncthreads();
+        if (threadIdx.x == 0)
+            last = __hip_atomic_fetch_add(l.sums.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)b1 - 1u;
+        __syncthreads();
+        if (!last) return;
+        // the last block adds all shares up
+        auto device_load = [](const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+        const SumArgs& f = l.sums;
+        const ProdArgs &px = l.p[0], &pw = l.p[1];
+        if (f.grad_bias)
+            for (int64_t m = threadIdx.x; m < f.M; m += KW * 64) {
+                float t = 0.f;
+#pragma unroll 8
+                for (int k = 0; k < f.chunks; k++) t += f.part[(int64_t)k * f.mpad + m];
+                reinterpret_cast<float*>(f.grad_bias)[m] = t;
+            }
+        if (f.grad_sw) {
+            const int wg = (pw.Ct + RB - 1) / RB;
+            for (int64_t m = threadIdx.x; m < f.M; m += KW * 64) {
+                float t = 0.f;
+#pragma unroll 8
+                for (int k = 0; k < wg; k++) t += device_load(pw.shares + m * wg + k);
+                reinterpret_cast<float*>(f.grad_sw)[m] = t;
+            }
+        }
+        if (f.grad_sa) {
+            float t = 0.f;
+#pragma unroll 4
+            for (int i = threadIdx.x; i < b0; i += KW * 64) t += device_load(px.shares + i);
+#pragma unroll
+            for (int d = 32; d; d >>= 1) t += __shfl_xor(t, d);
+            if (lane == 0) blk[kw] = t;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                t = 0.f;
+#pragma unroll
+                for (int k = 0; k < KW; k++) t += blk[k];
+                *reinterpret_cast<float*>(f.grad_sa) = t;
+            }
+        }
     }
 }
 
@@ -442,6 +680,7 @@ static int launch_products(ProdLaunch& l, hipStream_t st, const char* who)
     if (b1 > 0x3fffffffLL) return fail(BGEMM_EINVAL, "%s: grid of %lld blocks", who, (long long)b1);
     const bool wide = b3 >= 256;
     for (int i = 0; i < 2; i++) l.blocks[i] = l.p[i].R ? (int)(l.p[i].R * cdiv(l.p[i].Ct, wide ? 3 : 1)) : 0;
+    if (NP == 3 && !l.p[0].R) l.sums.grad_sa = nullptr;
     const unsigned grid = (unsigned)(l.blocks[0] + l.blocks[1] + l.sums.blocks);
     if (wide) hipLaunchKernelGGL((sign_product_kernel<NP, 3, 4>), dim3(grid), dim3(256), 0, st, l);
     else hipLaunchKernelGGL((sign_product_kernel<NP, 1, 8>), dim3(grid), dim3(512), 0, st, l);
@@ -540,4 +779,103 @@ extern "C" int bgemm_linear_backward(const void* W_sign, const void* W_nonzero, 
     }
     l.sums = {a.part, block_sa, a.ticket, (int)w.chunks, (int)w.cols, f32, a.mpad, M, grad_bias, grad_sw, grad_sa};
     return launch_products<1>(l, st, who);
+}
+
+// ---- the learned-scale layer ------------------------------------------------------------------------------------------------
+// stats: [0] mean(x), [1] mean(w), then the partial sums of both (ELASTIC_PARTS each).
+static constexpr int ELASTIC_PARTS = 128;
+
+extern "C" int bgemm_elastic_forward(const void* x, const void* w, int64_t N, int64_t M, int64_t K, const void* sa, const void* sw, const void* bias,
+                                     void* x_sign, void* x_nonzero, void* w_sign, void* w_nonzero, void* stats, void* out, void* stream)
+{
+    const char* who = "bgemm_elastic_forward";
+    if (N < 1 || M < 1 || K < 1 || K >= (1LL << 24) || N > (1 << 20) || M > (1 << 20))
+        return fail(BGEMM_EINVAL, "%s: bad shape N=%lld M=%lld K=%lld", who, (long long)N, (long long)M, (long long)K);
+    if (!x || !w || !sa || !sw || !x_sign || !x_nonzero || !w_sign || !w_nonzero || !stats || !out) return fail(BGEMM_ENULL, "%s: null pointer", who);
+    if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)stats) & 3)) return fail(BGEMM_EALIGN, "%s: an operand is not aligned", who);
+    const hipStream_t st = (hipStream_t)stream;
+    float* const means = (float*)stats;
+    const int64_t most = (N > M ? N : M) * K, want = cdiv(most, 4096);
+    const int parts = (int)(want < ELASTIC_PARTS ? want : ELASTIC_PARTS);
+    hipLaunchKernelGGL(elastic_sums_kernel, dim3(2 * parts), dim3(256), 0, st, (const float*)x, N * K, (const float*)w, M * K, parts, means + 2);
+    int rc = check_launch(who);
+    if (!rc) rc = pack_elastic_pair((const float*)x, N, x_sign, x_nonzero, (const float*)w, M, w_sign, w_nonzero, K, means + 2, parts, (const float*)sa, means, st, who);
+    return rc ? rc : packed_forward_elastic(w_sign, x_sign, (float*)out, M, N, K, (const float*)sw, (const float*)sa, (const float*)bias, st);
+}
+
+// Workspace: [ticket] [chunk sums of G] [shares of grad_sa] [shares of grad_sw] [codes of w, fragments of rows n] [codes of x, fragments of rows m].
+struct ElasticWs { size_t part, share_x, share_w, codes_w, ga, codes_x, gt, total; int64_t chunks, cols; };
+
+static ElasticWs elastic_ws(int64_t N, int64_t M, int64_t K, bool need_x, bool need_w)
+{
+    ElasticWs w;
+    w.chunks = cdiv(row_tiles(N), grad_rows_per_chunk(N, M));
+    w.cols = cdiv(M, 64);
+    const size_t frags = (size_t)row_tiles(N) * w.cols * 2 * FRAG_U4 * 16 * 3, words = (size_t)k_tiles(K) * TILE_KBITS * 2 * 4, kt32 = (size_t)cdiv(K, 32);
+    w.part = 256;
+    w.share_x = w.part + grad_round((size_t)w.chunks * w.cols * 64 * 4);
+    w.share_w = w.share_x + grad_round((size_t)row_tiles(N) * kt32 * 4);
+    w.codes_w = w.share_w + grad_round((size_t)M * kt32 * 4);
+    w.ga = w.codes_w + (need_x ? grad_round(w.cols * 2 * words) : 0);
+    w.codes_x = w.ga + (need_x ? frags : 0);
+    w.gt = w.codes_x + (need_w ? grad_round(row_tiles(N) * words) : 0);
+    w.total = w.gt + (need_w ? frags : 0);
+    return w;
+}
+
+extern "C" size_t bgemm_elastic_backward_workspace_bytes(int64_t N, int64_t M, int64_t K, int need_x, int need_w)
+{
+    return N <= 0 || M <= 0 || K <= 0 ? 0 : elastic_ws(N, M, K, need_x, need_w).total;
+}
+
+extern "C" int bgemm_elastic_backward(const void* x_sign, const void* x_nonzero, const void* w_sign, const void* w_nonzero, const void* grad_out,
+                                      const void* x, const void* w, const void* stats, const void* sa, float grad_scale, int64_t N, int64_t M,
+                                      int64_t K, void* grad_x, void* grad_w, void* grad_bias, void* grad_sw, void* grad_sa, void* ws,
+                                      size_t ws_bytes, void* stream)
+{
+    const char* who = "bgemm_elastic_backward";
+    if (N < 1 || M < 2 || K < 1 || K >= (1LL << 24) || N > (1 << 20) || M > (1 << 20))
+        return fail(BGEMM_EINVAL, "%s: bad shape N=%lld M=%lld K=%lld", who, (long long)N, (long long)M, (long long)K);
+    if (!grad_out || !stats || !sa || !ws || ((grad_x || grad_sa) && (!x || !w_sign || !w_nonzero || !grad_x)) ||
+        ((grad_w || grad_sw) && (!w || !x_sign || !x_nonzero || !grad_w)))
+        return fail(BGEMM_ENULL, "%s: null pointer", who);
+    if ((((uintptr_t)x_sign | (uintptr_t)x_nonzero | (uintptr_t)w_sign | (uintptr_t)w_nonzero) & 15) || ((uintptr_t)ws & 255) ||
+        (((uintptr_t)grad_out | (uintptr_t)x | (uintptr_t)w | (uintptr_t)grad_x | (uintptr_t)grad_w) & 3))
+        return fail(BGEMM_EALIGN, "%s: an operand is not aligned", who);
+    const ElasticWs f = elastic_ws(N, M, K, grad_x, grad_w);
+    if (ws_bytes < f.total) return fail(BGEMM_EWORKSPACE, "%s: workspace of %zu bytes, %zu needed", who, ws_bytes, f.total);
+    if (!grad_x && !grad_w) return fail(BGEMM_EINVAL, "%s: neither operand's gradient is wanted", who);
+    char* const base = (char*)ws;
+    const hipStream_t st = (hipStream_t)stream;
+    const int64_t KT = k_tiles(K), MT = row_tiles(M), NT = row_tiles(N);
+    ElasticPrepArgs a;
+    a.g = (const float*)grad_out; a.ga = grad_x ? (uint4*)(base + f.ga) : nullptr; a.gt = grad_w ? (uint4*)(base + f.gt) : nullptr;
+    a.part = (float*)(base + f.part); a.ticket = (uint32_t*)ws;
+    a.N = N; a.M = M; a.mpad = f.cols * 64; a.NT = (int)NT; a.rt_per_chunk = grad_rows_per_chunk(N, M);
+    a.grid_x = (int)cdiv(f.cols, 4);
+    CodeJob jw = {(const uint32_t*)w_sign, (const uint32_t*)w_nonzero, (uint32_t*)(base + f.codes_w), KT, grad_x ? MT * KT * 4 : 0};
+    CodeJob jx = {(const uint32_t*)x_sign, (const uint32_t*)x_nonzero, (uint32_t*)(base + f.codes_x), KT, grad_w ? NT * KT * 4 : 0};
+    const int64_t grad_blocks = a.grid_x * f.chunks, blocks = grad_blocks + cdiv(jw.waves, 4) + cdiv(jx.waves, 4);
+    if (blocks > 0x3fffffffLL) return fail(BGEMM_EINVAL, "%s: operand too large", who);
+    a.grad_blocks = (int)grad_blocks;
+    hipLaunchKernelGGL(elastic_prep_kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, jw, jx);
+    int rc = check_launch(who);
+    if (rc) return rc;
+    ProdLaunch l;
+    for (ProdArgs& p : l.p) {
+        p.R = 0;
+        p.colpad = KT * TILE_KBITS; p.cols = K; p.Ct = (int)cdiv(K, 32); p.ldx = K; p.sa = (const float*)sa; p.scale = grad_scale;
+    }
+    if (grad_x) {
+        ProdArgs& p = l.p[0];
+        p.A = a.ga; p.C = jw.dst; p.R = (int)NT; p.T = (int)(f.cols * 2); p.rows = N; p.paired = 0; p.out = grad_x; p.kind = PROD_ELASTIC_X;
+        p.x = x; p.zp = stats; p.shares = (float*)(base + f.share_x);
+    }
+    if (grad_w) {
+        ProdArgs& p = l.p[1];
+        p.A = a.gt; p.C = jx.dst; p.R = (int)(f.cols * 2); p.T = (int)NT; p.rows = M; p.paired = 1; p.out = grad_w; p.kind = PROD_ELASTIC_W;
+        p.x = w; p.zp = (const float*)stats + 1; p.shares = (float*)(base + f.share_w);
+    }
+    l.sums = {a.part, nullptr, a.ticket, (int)f.chunks, 0, 1, a.mpad, M, grad_bias, grad_w ? grad_sw : nullptr, grad_sa};
+    return launch_products<3>(l, st, who);
 }

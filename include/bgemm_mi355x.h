@@ -296,6 +296,23 @@ int bgemm_linear_backward(const void* W_sign, const void* W_nonzero, const void*
                           const void* bireal_x, int64_t ldx, const void* zero_point, void* grad_x, void* grad_w,
                           void* grad_bias, void* grad_sw, void* grad_sa, void* ws, size_t ws_bytes, void* stream);
 
+/* The learned-scale layer (:350-457, :519-564), fp32, dense rows, three launches: sign and nonzero planes (tiled) of
+ * (x - mean(x)) / sa and w - mean(w), and out [N][M] = half(half(acc) * sa) * sw (+ bias), acc their product of signs.
+ * stats: BGEMM_ELASTIC_STATS floats, left for the backward pass (the means, partial sums). */
+#define BGEMM_ELASTIC_STATS 512
+int bgemm_elastic_forward(const void* x, const void* w, int64_t N, int64_t M, int64_t K, const void* sa, const void* sw, const void* bias,
+                          void* x_sign, void* x_nonzero, void* w_sign, void* w_nonzero, void* stats, void* out, void* stream);
+/* Its backward pass, two launches: grad_x [N][K] and grad_w [M][K] = the straight-through products (fp32 products and sums) times
+ * 2 / cosh(min(|.|, 4))^2 of the centred operands, grad_bias [M] = column sums of grad_out, grad_sw [M] and grad_sa from
+ * calculate_gradient_signed with factor grad_scale.  NULL where not wanted (grad_sa needs grad_x, grad_sw needs
+ * grad_w, and one of those two has to be).
+ * M >= 2; N, M <= 2^20.  ws: 256-byte aligned, no initialisation needed. */
+size_t bgemm_elastic_backward_workspace_bytes(int64_t N, int64_t M, int64_t K, int need_x, int need_w);
+int bgemm_elastic_backward(const void* x_sign, const void* x_nonzero, const void* w_sign, const void* w_nonzero, const void* grad_out,
+                           const void* x, const void* w, const void* stats, const void* sa, float grad_scale, int64_t N, int64_t M,
+                           int64_t K, void* grad_x, void* grad_w, void* grad_bias, void* grad_sw, void* grad_sa, void* ws,
+                           size_t ws_bytes, void* stream);
+
 /* ---- a chain of dependent decode-shaped layers in one launch ------------------------------------
  * Layer l computes acc = MODE(W_l [M_l][K_l], x_l [N][K_l]) and hands layer l + 1 the bits of
  * half_rn(y - *next_zero_point), y = half(acc) * sw * sa (+ bias) evaluated as in bgemm_packed_forward_scaled

@@ -112,3 +112,49 @@ def test_gradients_can_be_differentiated_and_modified_scales_are_refused():
         lin.sw.mul_(2.0)
     with pytest.raises(RuntimeError):
         torch.autograd.grad(y, x, g)
+
+
+@pytest.mark.parametrize("N, K, M", SHAPES)
+def test_learned_scale_layer_as_one_node(N, K, M):
+    """Against the separate operations (torch's own means, fp32 matmul).  The upstream gradient's three bf16 planes hold all of its bits
+    and the products' terms are exact, so the two sides differ by the order of fp32 sums of R terms (R * 2^-24 * sum|terms|), the means'
+    last bits (an element within 2^-22 of its operand's mean would flip: none does here), and a few roundings of the surrogate (cosh
+    within 4 ulp on either side: 2^-20)."""
+    torch.manual_seed(N + K)
+    lin = bl.BGEMMLinear_elastic_signed(K, M).to(DEV)
+    x = torch.randn(N, K, device=DEV) * 1.5 + 0.25
+    lin(torch.randn(64, K, device=DEV))
+    with torch.no_grad():
+        lin.sw.copy_(torch.rand_like(lin.sw) + 0.5)
+        lin.sa.fill_(0.75 if M % 2 else -0.75)
+    x.requires_grad_(True)
+    g = torch.randn(N, M, device=DEV) * torch.logspace(-6, 2, M, device=DEV)
+    wanted = [x, lin.weight, lin.sa, lin.sw, lin.bias]
+    assert lin(x).grad_fn.name() == "ElasticBinaryLinearBackward"
+    got = grads(lin, x, g, wanted)
+    lin.fuse_training = False
+    want = grads(lin, x, g, wanted)
+    assert torch.equal(got[0], want[0])
+    d = lambda t: t.detach().double()
+    xs, ws = (d(x) - d(x).mean()) / d(lin.sa), d(lin.weight) - d(lin.weight).mean()
+    ga = d(g).abs()
+    sur = lambda t: 2 / torch.cosh(t.abs().clamp(max=4)) ** 2
+    assert ((d(got[1]) - d(want[1])).abs() <= sur(xs) * (M + 8) * 2.0 ** -23 * ga.sum(1, keepdim=True) + 2.0 ** -19 * d(want[1]).abs()).all()
+    assert ((d(got[2]) - d(want[2])).abs() <= sur(ws) * (N + 8) * 2.0 ** -23 * ga.sum(0)[:, None] + 2.0 ** -19 * d(want[2]).abs()).all()
+    f, h = d(g) @ ws.sign(), d(g).T @ xs.sign()
+    inner = (xs > 1).double() - (xs < -1).double() + (xs.abs() <= 1) * (xs.sign() - xs)
+    c = lin.grad_scale
+    slack = 2.0 ** -20 * (N + M + K)
+    assert float((d(got[3]) - (inner * f * c).sum()).abs()) <= slack * float((inner.abs() * ga.sum(1, keepdim=True) * c).sum())
+    assert ((d(got[4]) - (ws.sign() * h * c).sum(1)).abs() <= slack * c * K * ga.sum(0)).all()
+    assert ((d(got[5]) - d(g).sum(0)).abs() <= N * 2.0 ** -24 * ga.sum(0)).all()
+    lin.fuse_training = True
+    x3 = x.detach()[: N // 2 * 2].reshape(2, N // 2, K).requires_grad_(True) if N > 1 else x
+    if N > 1:                                                # leading dimensions, a subset of gradients
+        y3 = lin(x3)
+        assert y3.shape == (2, N // 2, M)
+        a = torch.autograd.grad(y3, [lin.weight, lin.bias], g[: N // 2 * 2].reshape(2, N // 2, M))
+        lin.fuse_training = False
+        b = torch.autograd.grad(lin(x3), [lin.weight, lin.bias], g[: N // 2 * 2].reshape(2, N // 2, M))
+        for p, q in zip(a, b):
+            assert torch.allclose(p, q, rtol=1e-4, atol=1e-4 * float(q.abs().max()))
