@@ -19,10 +19,13 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-u
 
 
 def native_command():
-    """The host compiler's command for _bgemm_native.so (torch is located, not imported)."""
+    """The host compiler's command for _bgemm_native.so (torch is located, not imported).  NDEBUG, as torch itself is built: pybind11's
+    debug counter would give the library a TLS segment.  One that is loaded after torch and never touched leaves every access to
+    torch's own thread-local variables on the slow path of glibc's __tls_get_addr: an attention block of small kernels took
+    291 us instead of 262, a packed product 9.7 instead of 8.8."""
     torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
-    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+    return [os.environ.get("CXX", "g++"), "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
             "-I" + os.path.join(torch_dir, "include"), "-I" + os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
             "-I" + os.path.join(rocm, "include"), "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "torch_ops.cpp"), "-o", NATIVE_SO,
             "-L" + os.path.join(torch_dir, "lib"), "-lc10", "-ltorch_cpu", "-ltorch_python", "-lc10_hip", "-L" + HERE, "-l:" + os.path.basename(SO),

@@ -4,6 +4,7 @@ import ctypes
 import os
 import re
 import shutil
+import struct
 import subprocess
 
 import pytest
@@ -364,3 +365,13 @@ def test_chain_entry_point_rejects_bad_arguments_on_the_host():
     assert b"activation rows" in L.bgemm_last_error()
     assert L.bgemm_chain_workspace_bytes(9, layers, 2, 4) == 0
     assert L.bgemm_chain_status(None, None) == _lib.ENULL
+
+
+def test_native_host_side_has_no_tls_segment():
+    """A TLS segment that is loaded after torch and never touched slows every access to torch's thread-local variables."""
+    path = os.path.join(os.path.dirname(os.path.abspath(_lib.__file__)), "_bgemm_native.so")
+    with open(path, "rb") as f:
+        data = f.read()
+    phoff, phentsize, phnum = struct.unpack_from("<Q", data, 32)[0], *struct.unpack_from("<HH", data, 54)
+    kinds = [struct.unpack_from("<I", data, phoff + i * phentsize)[0] for i in range(phnum)]
+    assert 1 in kinds and 7 not in kinds            # PT_LOAD, PT_TLS
