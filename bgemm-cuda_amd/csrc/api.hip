@@ -211,8 +211,8 @@ static int packed_forward(int mode, const void* W_tiled, const void* X_tiled, co
     a.MT = (int)row_tiles(M); a.NT = (int)row_tiles(N); a.KT = (int)k_tiles(K);
     a.strideW = strideW / 4; a.strideX = strideX / 4;
     a.splitK = splitK;
-    a.vec_store = !bits && (M % 4 == 0) && (strideC % 4 == 0) && (((uintptr_t)out & 15) == 0) ? 4 : 0;
-    if (a.vec_store && out_elem_shift(a.out_kind) == 1 && M % 8 == 0 && strideC % 8 == 0) a.vec_store = 8;
+    const int per16 = 16 >> out_elem_shift(a.out_kind);
+    a.row_aligned = !bits && M % per16 == 0 && strideC % per16 == 0 && ((uintptr_t)out & 15) == 0;
     a.nt_store = batch * N * M * 4 <= (32LL << 20);
     const int v = family == BGEMM_VARIANT_AUTO ? pick_variant(mode, batch, M, N, K) : family;
     const bool fp4 = v == BGEMM_VARIANT_MFMA_F4;

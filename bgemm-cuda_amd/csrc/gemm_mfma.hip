@@ -99,8 +99,7 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
     // pair take the even and the odd rows of the pair's 64 weight rows (lane l: rows 2l and 2l + 1), so that a
     // lane ends up with two neighbouring outputs of a row, one 4-byte store of two halves, and a half-wave
     // with a whole 128-byte line (see the epilogue).  The popcounts travel with the lane, nothing else changes.
-    const bool pair_cols = !PIPE && WM % 2 == 0 && a.out_kind == BGEMM_OUT_F16 && a.vec_store == 8 &&
-                           a.K <= (1 << 20) && a.M < (1 << 28);
+    const bool pair_cols = !PIPE && WM % 2 == 0 && a.out_kind == BGEMM_OUT_F16 && a.row_aligned && a.K <= (1 << 20) && a.M < (1 << 28);
 #pragma unroll
     for (int j = 0; j < WM; j++) {
         if (pair_cols) {
@@ -514,7 +513,7 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
     char* const out_base = reinterpret_cast<char*>(a.out) + (out_off << esz_shift);
     const int64_t row_bytes = a.M << esz_shift;
     int* const st = stage + wave * (32 * ROW_I);
-    // Stores past the caches (non-temporal) where timing favours them: always for the 2-byte kinds, for the
+    // Stores past the caches (non-temporal) where timing favours them (on rows that suit, see below): always for the 2-byte kinds, for the
     // 4-byte kinds on outputs of up to 32 MiB (a.nt_store) and on larger ones on 8 to 31 K-tiles (see the int32 path above;
     // fp32 scaled: 16384 x 8192 x 4096 252.2 -> 238.3 us, 4096^3 36.0 -> 34.6); else ordinary stores are faster.
     // (The non-temporal store is written as an instruction: as a builtin next to an ordinary store of the same
@@ -526,11 +525,18 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
             const v4i x = {v.x, v.y, v.z, v.w};
             asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" : : "v"(to), "v"(x) : "memory");
         } else
-            *reinterpret_cast<int4*>(to) = v;
+            __builtin_memcpy(to, &v, 16);
     };
-    // Plain fp16 with rows a multiple of eight long: the integers are rounded once, staged as halves, and a
+    // Rows at any address take the same vector stores (the hardware stores vectors at any element address); only the piece that
+    // reaches past a row's end is stored element by element.  Past the caches only where rows are a whole number of 64-byte
+    // pieces, or aligned and few: elsewhere neighbouring blocks share lines, which the L2 puts together (8192 x 4096 x 8200 ->
+    // fp16: 121 -> 99 us, fp32 scaled 148 -> 130; 4096 x 768 x 3080 fp16 scaled (25 MB) 18.0 -> 15.7; but 2048 x 4096 x 4104
+    // (17 MB) 21.7 past the caches against 22.8).  Stored element by element, ragged rows took
+    // 64 us instead of 43 (2053 x 4345 x 8195 -> fp16), scaled 98 instead of 44, 8192 x 768 x 3075 37 instead of 20.
+    const bool past = a.row_aligned && ((row_bytes & 63) == 0 || a.batch * a.N * row_bytes <= (20 << 20));
+    // Plain fp16: the integers are rounded once, staged as halves, and a
     // lane reads back the eight it stores with one 16-byte LDS read (no conversion behind the staging).
-    if (a.out_kind == BGEMM_OUT_F16 && a.vec_store == 8) {
+    if (a.out_kind == BGEMM_OUT_F16) {
         constexpr int ROW_H = WM * 32 + 8;       // staged row stride in halves (+8: rows four apart, the two
                                                  // lane halves, fall on different LDS banks)
         constexpr int C8 = WM * 4, RSTEP = 64 / C8;              // lanes per staged row, rows per store instruction
@@ -549,30 +555,37 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
                 for (int j = 0; j < WM; j++)
                     sh[(8 * (v >> 2) + 4 * half + (v & 3)) * ROW_H + j * 32 + col] = __float2half_rn((float)val[j][v]);
             wave_sync();
-            if (m < a.M) {
+            auto rows_out = [&](auto past_cache) {
                 char* dst = out_base + (nrow0 + row0) * row_bytes + (m << 1);
                 const __half* sp = sh + row0 * ROW_H + c8 * 8;
 #pragma unroll
                 for (int row = row0; row < 32; row += RSTEP, sp += RSTEP * ROW_H, dst += RSTEP * row_bytes)
-                    if (nrow0 + row < a.N) store16(dst, *reinterpret_cast<const int4*>(sp), true);
+                    if (nrow0 + row < a.N) store16(dst, *reinterpret_cast<const int4*>(sp), past_cache);
+            };
+            if (m + 8 <= a.M) {
+                if (past) rows_out(std::true_type{});
+                else rows_out(std::false_type{});
+            } else if (m < a.M) {
+                for (int row = row0; row < 32 && nrow0 + row < a.N; row += RSTEP)
+                    for (int e = 0; m + e < a.M; e++)
+                        reinterpret_cast<__half*>(out_base + (nrow0 + row) * row_bytes)[m + e] = sh[row * ROW_H + c8 * 8 + e];
             }
             wave_sync();                                 // the next strip overwrites the staging area
         }
         return;
     }
-    // fp16 scaled, eight elements a lane: the lane's eight columns are the same for every strip, so their parameters are
+    // Scaled kinds: a lane's columns (eight of fp16, four of fp32) are the same for every strip, so their parameters are
     // fetched once, before the strips (inside the strip loop the stores between them keep the compiler from reusing them)
     ColParams cp8[8];
     float saf8 = 0.f;
-    if (a.vec_store == 8 && a.out_kind == BGEMM_OUT_F16_SCALED) {
-        saf8 = ep_scalar(a.out_kind, a.ep_sa);
+    const bool f16_scaled = a.out_kind == BGEMM_OUT_F16_SCALED;
+    if (f16_scaled || a.out_kind == BGEMM_OUT_F32_SCALED || a.out_kind == OUT_F32_ELASTIC) saf8 = ep_scalar(a.out_kind, a.ep_sa);
+    if (f16_scaled) {
 #pragma unroll
         for (int e = 0; e < 8; e++) cp8[e] = col_params(a, (int64_t)mt0 * 32 + (lane % (WM * 4)) * 8 + e);
     }
-    // (the same for the scaled kinds stored four elements a lane: fp32, and fp16 rows that are no multiple of eight long)
     ColParams cp4[4];
-    if (a.vec_store && a.vec_store != 8 && (a.out_kind == BGEMM_OUT_F32_SCALED || a.out_kind == BGEMM_OUT_F16_SCALED || a.out_kind == OUT_F32_ELASTIC)) {
-        saf8 = ep_scalar(a.out_kind, a.ep_sa);
+    if (a.out_kind == BGEMM_OUT_F32_SCALED || a.out_kind == OUT_F32_ELASTIC) {
 #pragma unroll
         for (int e = 0; e < 4; e++) cp4[e] = col_params(a, (int64_t)mt0 * 32 + (lane % (WM * 8)) * 4 + e);
     }
@@ -586,45 +599,14 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
             for (int j = 0; j < WM; j++) st[(8 * (v >> 2) + 4 * half + (v & 3)) * ROW_I + j * 32 + col] = val[j][v];
         wave_sync();
         const int64_t nrow0 = (int64_t)x_tile(i) * 32, mcol0 = (int64_t)mt0 * 32;
-        constexpr int C4 = WM * 8;               // int4 per staged row
-        constexpr int NP = 32 * C4 / 64;
-        if (a.vec_store && a.out_kind == BGEMM_OUT_I32) {
-            // 16-byte stores: one instruction covers 64 * 4 consecutive elements of the strip.  Eight
-            // LDS reads are issued together, then their stores; the address advances by whole rows.
-            constexpr int RSTEP = 64 / C4, CHUNK = NP < 8 ? NP : 8;
-            const int c4 = lane % C4, row0 = lane / C4;
-            const int* sp = st + row0 * ROW_I + c4 * 4;
-            const int64_t m = mcol0 + c4 * 4, dstep = RSTEP * row_bytes;
-            char* dst = out_base + (nrow0 + row0) * row_bytes + (m << 2);
-            if (m < a.M) {
-                if (nrow0 + 32 <= a.N) {             // uniform: the whole strip exists, nothing to mask
-#pragma unroll
-                    for (int p0 = 0; p0 < NP; p0 += CHUNK) {
-                        int4 q[CHUNK];
-#pragma unroll
-                        for (int p = 0; p < CHUNK; p++) q[p] = *reinterpret_cast<const int4*>(sp + (p0 + p) * RSTEP * ROW_I);
-                        if (a.nt_store || (a.KT >= 8 && a.KT < 32)) {
-#pragma unroll
-                            for (int p = 0; p < CHUNK; p++, dst += dstep) store16(dst, q[p], true);
-                        } else {
-#pragma unroll
-                            for (int p = 0; p < CHUNK; p++, dst += dstep) store16(dst, q[p], false);
-                        }
-                    }
-                } else {
-                    for (int row = row0; nrow0 + row < a.N; row += RSTEP, sp += RSTEP * ROW_I, dst += dstep)
-                        store16(dst, *reinterpret_cast<const int4*>(sp), (a.nt_store != 0 || (a.KT >= 8 && a.KT < 32)));
-                }
-            }
-        } else if (a.vec_store == 8) {
-            // fp16 kinds, rows a multiple of eight long: eight elements and one 16-byte store per lane
+        if (f16_scaled) {
+            // eight elements and one 16-byte store per lane
             constexpr int C8 = WM * 4, RSTEP = 64 / C8;          // lanes per staged row, rows per step
             const int c8 = lane % C8, row0 = lane / C8;
             const int64_t m = mcol0 + c8 * 8;
             const int* sp = st + row0 * ROW_I + c8 * 8;
             char* dst = out_base + (nrow0 + row0) * row_bytes + (m << 1);
             const int64_t dstep = RSTEP * row_bytes;
-            const bool scaled = a.out_kind == BGEMM_OUT_F16_SCALED;
             const ColParams (&cp)[8] = cp8;      // this lane's eight columns, the same for every row of every strip
             const float saf = saf8;
             const bool has_bias = a.ep_bias != nullptr;
@@ -636,128 +618,115 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
             const __half2 sah = __float2half2_rn(saf);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                swh[e] = scaled ? __floats2half2_rn(cp[2 * e].sw, cp[2 * e + 1].sw) : sah;
-                biash[e] = scaled && has_bias ? __floats2half2_rn(cp[2 * e].bias, cp[2 * e + 1].bias) : sah;
+                swh[e] = __floats2half2_rn(cp[2 * e].sw, cp[2 * e + 1].sw);
+                biash[e] = __floats2half2_rn(cp[2 * e].bias, cp[2 * e + 1].bias);
             }
-            auto put8 = [&](const int4 q0, const int4 q1, char* const to, const bool sc) {
+            auto eight = [&](const int4 q0, const int4 q1) {
 #pragma clang fp contract(off)
                 const int q[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-                union { __half h[8]; __half2 h2[4]; uint4 u; } pk;
+                union { __half h[8]; __half2 h2[4]; int4 u; } pk;
 #pragma unroll
                 for (int e = 0; e < 8; e++) pk.h[e] = __float2half_rn((float)q[e]);
-                if (sc) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) pk.h2[e] = __hmul2(__hmul2(pk.h2[e], swh[e]), sah);
-                    if (has_bias) {
+                for (int e = 0; e < 4; e++) pk.h2[e] = __hmul2(__hmul2(pk.h2[e], swh[e]), sah);
+                if (has_bias) {
 #pragma unroll
-                        for (int e = 0; e < 4; e++) pk.h2[e] = __hadd2(pk.h2[e], biash[e]);
-                    }
+                    for (int e = 0; e < 4; e++) pk.h2[e] = __hadd2(pk.h2[e], biash[e]);
                 }
-                store16(to, make_int4((int)pk.u.x, (int)pk.u.y, (int)pk.u.z, (int)pk.u.w), true);
+                return pk.u;
             };
-            if (m < a.M) {
+            auto rows_out = [&](auto past_cache) {
                 if (nrow0 + 32 <= a.N) {             // uniform: whole strip: reads issued in pairs of rows
 #pragma unroll
                     for (int r = 0; r < 32 / RSTEP; r += 2, dst += 2 * dstep) {
                         const int* s0 = sp + r * RSTEP * ROW_I, * s1 = s0 + RSTEP * ROW_I;
                         const int4 a0 = *reinterpret_cast<const int4*>(s0), a1 = *reinterpret_cast<const int4*>(s0 + 4);
                         const int4 b0 = *reinterpret_cast<const int4*>(s1), b1 = *reinterpret_cast<const int4*>(s1 + 4);
-                        put8(a0, a1, dst, scaled);
-                        put8(b0, b1, dst + dstep, scaled);
+                        store16(dst, eight(a0, a1), past_cache);
+                        store16(dst + dstep, eight(b0, b1), past_cache);
                     }
                 } else {
 #pragma unroll 2
                     for (int row = row0; row < 32 && nrow0 + row < a.N; row += RSTEP, sp += RSTEP * ROW_I, dst += dstep)
-                        put8(*reinterpret_cast<const int4*>(sp), *reinterpret_cast<const int4*>(sp + 4), dst, scaled);
+                        store16(dst, eight(*reinterpret_cast<const int4*>(sp), *reinterpret_cast<const int4*>(sp + 4)), past_cache);
+                }
+            };
+            if (m + 8 <= a.M) {
+                if (past) rows_out(std::true_type{});
+                else rows_out(std::false_type{});
+            } else if (m < a.M) {
+#pragma unroll 1
+                for (int row = row0; row < 32 && nrow0 + row < a.N; row += RSTEP, sp += RSTEP * ROW_I, dst += dstep) {
+                    const int4 u = eight(*reinterpret_cast<const int4*>(sp), *reinterpret_cast<const int4*>(sp + 4));
+                    const int w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                    for (int e = 0; e < 7; e++)
+                        if (m + e < a.M) reinterpret_cast<uint16_t*>(dst)[e] = (uint16_t)((unsigned)w[e >> 1] >> (16 * (e & 1)));
                 }
             }
-        } else if (a.vec_store) {
-            // four elements per lane; the address advances by whole rows from step to step
-            constexpr int RSTEP = 64 / C4;
+        } else if (!bits_kind(a.out_kind)) {
+            // 4-byte kinds, four elements per lane; the address advances by whole rows from step to step
+            constexpr int C4 = WM * 8, RSTEP = 64 / C4;
             const int c4 = lane % C4, row0 = lane / C4;
             const int64_t m = mcol0 + c4 * 4;
             const int* sp = st + row0 * ROW_I + c4 * 4;
-            char* dst = out_base + (nrow0 + row0) * row_bytes + (m << esz_shift);
+            char* dst = out_base + (nrow0 + row0) * row_bytes + (m << 2);
             const int64_t dstep = RSTEP * row_bytes;
-            const bool has_bias = a.ep_bias != nullptr;
+            const bool has_bias = a.ep_bias != nullptr, past_cache = past && (a.nt_store != 0 || (a.KT >= 8 && a.KT < 32));
             const ColParams (&cp)[4] = cp4;
             const float saf = saf8;
-            if (m < a.M) {
+            auto four = [&](const int4 q) {
+                if (a.out_kind == BGEMM_OUT_I32) return q;
+                if (a.out_kind == BGEMM_OUT_F32_SCALED)
+                    return make_int4(__float_as_int(scaled_f32(q.x, cp[0], saf, has_bias)), __float_as_int(scaled_f32(q.y, cp[1], saf, has_bias)),
+                                     __float_as_int(scaled_f32(q.z, cp[2], saf, has_bias)), __float_as_int(scaled_f32(q.w, cp[3], saf, has_bias)));
+                auto e = [&](const int v, const ColParams c) { return __float_as_int(elastic_f32(v, c.sw, saf, has_bias, c.bias)); };
+                return make_int4(e(q.x, cp[0]), e(q.y, cp[1]), e(q.z, cp[2]), e(q.w, cp[3]));
+            };
+            if (m + 4 <= a.M) {
 #pragma unroll 2
+                for (int row = row0; row < 32 && nrow0 + row < a.N; row += RSTEP, sp += RSTEP * ROW_I, dst += dstep)
+                    store16(dst, four(*reinterpret_cast<const int4*>(sp)), past_cache);
+            } else if (m < a.M) {
+#pragma unroll 1
                 for (int row = row0; row < 32 && nrow0 + row < a.N; row += RSTEP, sp += RSTEP * ROW_I, dst += dstep) {
-                    const int4 q = *reinterpret_cast<const int4*>(sp);
-                    union { __half h[4]; uint2 u; } pk;
-                    switch (a.out_kind) {
-                    case BGEMM_OUT_I32:
-                        store16(dst, q, (a.nt_store != 0 || (a.KT >= 8 && a.KT < 32)));
-                        break;
-                    case BGEMM_OUT_F16:
-                        pk.h[0] = __float2half_rn((float)q.x); pk.h[1] = __float2half_rn((float)q.y);
-                        pk.h[2] = __float2half_rn((float)q.z); pk.h[3] = __float2half_rn((float)q.w);
-                        *reinterpret_cast<uint2*>(dst) = pk.u;
-                        break;
-                    case BGEMM_OUT_F32_SCALED:
-                        store16(dst, make_int4(__float_as_int(scaled_f32(q.x, cp[0], saf, has_bias)), __float_as_int(scaled_f32(q.y, cp[1], saf, has_bias)),
-                                               __float_as_int(scaled_f32(q.z, cp[2], saf, has_bias)), __float_as_int(scaled_f32(q.w, cp[3], saf, has_bias))),
-                                (a.nt_store != 0 || (a.KT >= 8 && a.KT < 32)));
-                        break;
-                    case OUT_F32_ELASTIC: {
-                        auto e = [&](const int v, const ColParams c) { return __float_as_int(elastic_f32(v, c.sw, saf, has_bias, c.bias)); };
-                        store16(dst, make_int4(e(q.x, cp[0]), e(q.y, cp[1]), e(q.z, cp[2]), e(q.w, cp[3])), (a.nt_store != 0 || (a.KT >= 8 && a.KT < 32)));
-                        break;
-                    }
-                    default:
-                        pk.h[0] = scaled_f16(q.x, cp[0], saf, has_bias); pk.h[1] = scaled_f16(q.y, cp[1], saf, has_bias);
-                        pk.h[2] = scaled_f16(q.z, cp[2], saf, has_bias); pk.h[3] = scaled_f16(q.w, cp[3], saf, has_bias);
-                        *reinterpret_cast<uint2*>(dst) = pk.u;
-                        break;
-                    }
+                    const int4 u = four(*reinterpret_cast<const int4*>(sp));
+                    int* const to = reinterpret_cast<int*>(dst);
+                    to[0] = u.x;
+                    if (m + 1 < a.M) to[1] = u.y;
+                    if (m + 2 < a.M) to[2] = u.z;
                 }
             }
         } else {
-            // ragged or unaligned rows, and the bits kinds: one element per lane and step.  A lane meets one
+            // bits kinds: one element per lane and step.  A lane meets one
             // column (two where the strip is 128 wide), whose parameters it fetches once.
             constexpr int NC = WM == 4 ? 2 : 1;
-            const bool bits = bits_kind(a.out_kind);
             const bool has_bias = a.ep_bias != nullptr;
             ColParams cp[NC];
-            float saf = 0.f, zpf = 0.f;
-            if (bits) {
-                saf = ep_scalar(a.out_kind, a.ep_sa);
-                if (a.ep_zp) zpf = ep_scalar(a.out_kind, a.ep_zp);
+            const float saf = ep_scalar(a.out_kind, a.ep_sa), zpf = a.ep_zp ? ep_scalar(a.out_kind, a.ep_zp) : 0.f;
 #pragma unroll
-                for (int k = 0; k < NC; k++) cp[k] = col_params(a, mcol0 + (lane + 64 * k) % (32 * WM));
+            for (int k = 0; k < NC; k++) cp[k] = col_params(a, mcol0 + (lane + 64 * k) % (32 * WM));
+            // half-waves hold 32 consecutive columns of one row: a ballot makes the output word.  The strip
+            // starts on a row tile of the output operand, so its words sit at fixed steps from one base.
+            uint32_t* const obase = reinterpret_cast<uint32_t*>(a.out) + (int64_t)b * a.strideC;
+            const int64_t okt = k_tiles(a.M);
+            int64_t wbase[NC];
+            bool col_ok[NC], word_ok[NC];
+#pragma unroll
+            for (int k = 0; k < NC; k++) {
+                const int c = (lane + 64 * k) % (32 * WM);
+                col_ok[k] = mcol0 + c < a.M;
+                word_ok[k] = mcol0 + (c & ~31) < a.M;
+                wbase[k] = tiled_word_offset(nrow0, (mcol0 + c) >> 5, okt);
             }
-            if (bits) {
-                // half-waves hold 32 consecutive columns of one row: a ballot makes the output word.  The strip
-                // starts on a row tile of the output operand, so its words sit at fixed steps from one base.
-                uint32_t* const obase = reinterpret_cast<uint32_t*>(a.out) + (int64_t)b * a.strideC;
-                const int64_t okt = k_tiles(a.M);
-                int64_t wbase[NC];
-                bool col_ok[NC], word_ok[NC];
-#pragma unroll
-                for (int k = 0; k < NC; k++) {
-                    const int c = (lane + 64 * k) % (32 * WM);
-                    col_ok[k] = mcol0 + c < a.M;
-                    word_ok[k] = mcol0 + (c & ~31) < a.M;
-                    wbase[k] = tiled_word_offset(nrow0, (mcol0 + c) >> 5, okt);
-                }
 #pragma unroll 4
-                for (int p = 0; p < 16 * WM; p++) {
-                    const int idx = p * 64 + lane, row = idx / (32 * WM), c = idx % (32 * WM), k = NC == 2 ? (p & 1) : 0;
-                    const bool row_ok = nrow0 + row < a.N;
-                    const unsigned bit = next_sign_bit(a.out_kind, st[row * ROW_I + c], cp[k], saf, has_bias, zpf);
-                    const unsigned long long bal = __ballot(bit != 0 && row_ok && col_ok[k]);
-                    const unsigned w = __brev((unsigned)(lane < 32 ? bal : bal >> 32));
-                    if ((lane & 31) == 0 && row_ok && word_ok[k]) obase[wbase[k] + row * 4] = w;
-                }
-            } else {
-#pragma unroll 4
-                for (int p = 0; p < 16 * WM; p++) {
-                    const int idx = p * 64 + lane, row = idx / (32 * WM), c = idx % (32 * WM);
-                    const int64_t n = nrow0 + row, m = mcol0 + c;
-                    if (n < a.N && m < a.M) store_out(a, out_off + n * a.M, m, st[row * ROW_I + c]);
-                }
+            for (int p = 0; p < 16 * WM; p++) {
+                const int idx = p * 64 + lane, row = idx / (32 * WM), c = idx % (32 * WM), k = NC == 2 ? (p & 1) : 0;
+                const bool row_ok = nrow0 + row < a.N;
+                const unsigned bit = next_sign_bit(a.out_kind, st[row * ROW_I + c], cp[k], saf, has_bias, zpf);
+                const unsigned long long bal = __ballot(bit != 0 && row_ok && col_ok[k]);
+                const unsigned w = __brev((unsigned)(lane < 32 ? bal : bal >> 32));
+                if ((lane & 31) == 0 && row_ok && word_ok[k]) obase[wbase[k] + row * 4] = w;
             }
         }
         wave_sync();                                 // the next strip overwrites the staging area
@@ -837,7 +806,7 @@ static int launch_cfg(const GemmArgs& a, hipStream_t st)
             // two weight tiles, four MFMAs a step; W[11008,4096] x 128 ternary rows 10.3 -> 9.1 us, W[22016,4096] x 128 17.5 ->
             // 14.8, W[11008,8192] x 320 28.5 -> 24.0)
             if constexpr ((WGN == 2 && WGM == 2 && WN == 2 && WM == 2) || (WGN == 1 && WGM == 4 && WN == 1 && WM == 2)) {
-                const bool pairs2 = a.out_kind == BGEMM_OUT_F16 && a.vec_store == 8;
+                const bool pairs2 = a.out_kind == BGEMM_OUT_F16 && a.row_aligned;
                 if (a.KT >= 8 && (!pairs2 || a.KT >= 16)) {
                     hipLaunchKernelGGL((gemm_mfma_kernel<Eng, WGN, WGM, WN, WM, 2, true>), dim3((unsigned)grid),
                                        dim3(WGN * WGM * 64), 0, st, a, tiles_n, tiles_m);
@@ -854,7 +823,7 @@ static int launch_cfg(const GemmArgs& a, hipStream_t st)
         // loop is 4 % ahead); where the output is fp16 pairs, which only the plain loop stores straight from registers, from
         // sixteen K-tiles on (5120 x 2048 x 8192 -> fp16: 33.5 against 37.3 us, 6144 x 3072 x 4096: 31.2 against 33.8; level at eight).
         constexpr bool MUST_PIPE = WN * WM >= 8, CAN_PIPE = WN * WM >= 4 && WGM == 2 && WN % 2 == 0;
-        const bool pairs = a.out_kind == BGEMM_OUT_F16 && a.vec_store == 8 && WM % 2 == 0;
+        const bool pairs = a.out_kind == BGEMM_OUT_F16 && a.row_aligned && WM % 2 == 0;
         const dim3 g((unsigned)grid), blk(WGN * WGM * 64);
         if constexpr (CAN_PIPE) {
             if (MUST_PIPE || (a.KT >= 8 && (!pairs || a.KT >= 16))) {
