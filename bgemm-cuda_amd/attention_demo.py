@@ -17,6 +17,7 @@ import time
 import torch
 import torch.nn as nn
 
+import lowbit_kernel
 from bgemm_linear import BGEMMLinear, GraphedInference, bgemm_attn_matmul, bgemm_matmul
 
 
@@ -45,7 +46,18 @@ class BinarySelfAttention(nn.Module):
     def transpose_for_scores(self, x):
         return x.view(*x.shape[:-1], self.num_attention_heads, self.attention_head_size).permute(0, 2, 1, 3)
 
+    def _fusable(self, x):
+        return (not torch.is_grad_enabled() and x.dim() == 3 and x.numel() > 0 and not torch.is_autocast_enabled()
+                and all(layer._bits_fusable(x) for layer in (self.query, self.key, self.value))
+                and lowbit_kernel.attention_supported(x.shape[0], x.shape[1], self.num_attention_heads, self.attention_head_size))
+
     def forward(self, hidden_states, attention_mask=None):
+        if self.kernels and attention_mask is None and self._fusable(hidden_states):
+            # nothing but the projections' signs is read: they leave their GEMMs as bits, and one kernel does the rest
+            scores, context = lowbit_kernel.attention_forward(self.query._fused_bits(hidden_states), self.key._fused_bits(hidden_states),
+                                                              self.value._fused_bits(hidden_states), hidden_states.shape[0],
+                                                              self.num_attention_heads, hidden_states.dtype)
+            return self.LayerNorm(self.dense(context) + hidden_states), scores
         q = self.transpose_for_scores(self.query(hidden_states))
         k = self.transpose_for_scores(self.key(hidden_states))
         v = self.transpose_for_scores(self.value(hidden_states))

@@ -367,6 +367,20 @@ class BGEMMLinear(_ScaledBinaryLinear):
             out = lowbit_kernel.bgemm_packed_weight_forward(wp, x2, lowbit_kernel.MODE_XOR, scale=(sw, sa, bias), x_zero_point=zpa)
         return out.reshape(*lead, self.weight.shape[0])
 
+    def _bits_fusable(self, x):
+        """Whether ``_fused_bits(x)`` may stand for calling this layer: nothing listens to the call."""
+        return (type(self) is BGEMMLinear and self.initialized and self._fusable(x) and "forward" not in self.__dict__
+                and not self._forward_hooks and not self._forward_pre_hooks and not nn.modules.module._has_any_global_hook())
+
+    def _fused_bits(self, x):
+        """The sign bits of ``self(x)``, [rows of x] x [features], for a consumer that reads nothing else of it."""
+        _, sw, sa, bias, zpa = self._inference_state()
+        if zpa is None:
+            zpa = self.zpa.detach().to(x.dtype).reshape(1)
+        xp = lowbit_kernel.pack_sign(x.reshape(-1, x.shape[-1]), zero_point=zpa)
+        bits = lowbit_kernel.empty_packed(xp.rows, self.weight.shape[0], x.device)
+        return lowbit_kernel.bgemm_packed_forward(self._packed_weight(), xp, lowbit_kernel.MODE_XOR, scale=(sw, sa, bias), bits_out=bits)
+
     def forward(self, x):
         if not self.initialized:
             self._initialize(x, self.weight)

@@ -1,0 +1,258 @@
+// Binary self-attention without a gradient, one launch: what tests/python/bert/bert.py:245-259 does with dense matrices, on sign bits.
+//
+//   scores[q,k] = half(half(sum_c sign(Q)[q,c] sign(K)[k,c]) / sqrt(D))              stored: the block returns them
+//   p[q,k]      = half(softmax_k(scores[q,:]))                                       never stored
+//   context[q,c] = half(sum over the k with p[q,k] >= 1/S of sign(V)[k,c])           stored in the layer's own order, heads merged
+//
+// As separate kernels (a GEMM, the division, the softmax, the shift by 1/S, a pack, the second GEMM, and packs and copies of
+// head-split views around them) the probabilities cross memory seven times: 12 heads of 64, 16 x 512 tokens 225 us, of which the one
+// pass over the scores that is needed takes 20.  A score is one of D + 1 numbers (matching bits, 0 .. D), so everything the softmax
+// needs of it comes from a table of D + 1 entries in LDS (exponential and rounded score), shifted by the largest score there can
+// be instead of the row's: no pass for the maximum, and the table is the same for every row.  The probabilities rise with the
+// score, so the bits of a row are a comparison with one number, found by bisection with the very division and rounding.
+//
+// A wave owns 32 queries.  Keys are the rows of the MFMA and queries its columns: a lane then holds one query's scores, row sums
+// stay in the lane, and the order of the keys in a fragment is chosen such that a lane holds 32 consecutive ones: its bits are a
+// word, and that word, four ways shifted, is the second product's operand as it stands.  The scores are multiplied twice, once for
+// the sums and once for the bits: one MFMA per 32 x 32 tile and 64 of D, cheaper than keeping S of them a lane.
+#include "common.h"
+#include "mfma_engines.h"
+#include "pack_bits.h"
+#include <math.h>
+#include <type_traits>
+
+namespace bgemm {
+
+struct AttnArgs {
+    const uint32_t* q; const uint32_t* k; const uint32_t* v;      // sign bits [batch * S][heads * D], tiled
+    __half* scores; void* context;
+    int64_t KT;                       // of the operands
+    int S, heads, groups, qblocks, f32;
+    float scale, level;               // 1 / sqrt(D), 1 / S
+};
+
+constexpr int ATTN_STAGE = 144;       // bytes of a staged row of 64 scores (padded)
+
+// One word of signed fp4 operands at step s: +1.0, or -1.0 where the bit is set; the same with 1.0 where it is set and 0 elsewhere.
+__device__ __forceinline__ unsigned attn_pm1(const unsigned w, const int s) { return (s == 3 ? w & 0x88888888u : (w << (3 - s)) & 0x88888888u) | 0x22222222u; }
+__device__ __forceinline__ unsigned attn_01(const unsigned w, const int s) { return (s == 0 ? w << 1 : w >> (s - 1)) & 0x22222222u; }
+
+// W: words a head (D = 32 W).
+template <int W>
+__global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
+{
+    constexpr int D = W * 32, CH = (W + 1) / 2, PAD = CH * 64 - D;       // chunks of 64 bits, the last half a one if W is odd
+    // a sum comes out as 2^23 + 2 * (matching bits): its bit pattern is an index
+    constexpr unsigned BASE = 0x4b000000u;
+    constexpr float C0 = 8388608.f + (D - PAD);
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int h = lane >> 5, c = lane & 31;
+    const int S = a.S, S64 = a.groups * 64;
+    unsigned char* const stage = smem + wave * (32 * ATTN_STAGE);
+    uint2* const tbl = reinterpret_cast<uint2*>(smem + waves * (32 * ATTN_STAGE));           // [D + 2]
+    uint32_t* const kb = reinterpret_cast<uint32_t*>(tbl + D + 2);                           // [W][S64]
+    uint32_t* const vt = kb + W * S64;                                                       // [2 groups][D]: words of 32 keys
+
+    const int bh = blockIdx.x / a.qblocks, qb = blockIdx.x % a.qblocks, b = bh / a.heads, head = bh % a.heads;
+    const int64_t row0 = (int64_t)b * S;
+    auto word = [&](const uint32_t* p, const int row, const int w) { return p[tiled_word_offset(row0 + row, head * W + w, a.KT)]; };
+
+    // ---- the block's shared operands: table, key bits, value bits transposed -----------------------------------------------------
+    auto score16 = [&](const int idx) { return __float2half_rn((float)(2 * idx - D) * a.scale); };
+    for (int i = threadIdx.x; i <= D; i += blockDim.x) {
+        const __half s = score16(i);
+        tbl[i] = make_uint2(__float_as_uint(expf(__half2float(s) - __half2float(score16(D)))), __half_as_ushort(s));
+    }
+    for (int key = threadIdx.x; key < S64; key += blockDim.x)
+#pragma unroll
+        for (int w = 0; w < W; w++) kb[w * S64 + key] = key < S ? word(a.k, key, w) : 0u;
+    for (int u0 = wave * 2; u0 < a.groups * 2 * W; u0 += waves * 2) {
+        const int u = u0 + h, kw = u / W, w = u % W, key = kw * 32 + c;
+        const unsigned t = transpose32(__brev(key < S ? word(a.v, key, w) : 0u), lane);       // bit r: key r of the lane's column
+        vt[kw * D + w * 32 + c] = __brev(t);
+    }
+    __syncthreads();
+
+    const int q0 = (qb * waves + wave) * 32;
+    if (q0 >= S) return;
+    unsigned qf[CH][4];
+#pragma unroll
+    for (int ch = 0; ch < CH; ch++) {
+        const int w = 2 * ch + h;
+        const unsigned x = w < W ? word(a.q, min(q0 + c, S - 1), w < W ? w : 0) : 0u;
+#pragma unroll
+        for (int s = 0; s < 4; s++) qf[ch][s] = attn_pm1(x, s);
+    }
+    // MFMA row r = 8 g + 4 half + i of tile j is key 32 half + 16 j + 4 g + i of the group's 64: register v of a lane is then key
+    // 32 h + 16 j + v.  (The second product's rows, columns of V, likewise: register v is column 16 h + v.)
+    const int row_key = 32 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3), row_col = 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3);
+    auto tile = [&](const int grp, const int j) {
+        EngF4::Acc acc;
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[v] = C0;
+#pragma unroll
+        for (int ch = 0; ch < CH; ch++) {
+            const int w = 2 * ch + h;
+            unsigned x = kb[(w < W ? w : 0) * S64 + grp * 64 + 16 * j + row_key];
+            if (W % 2 && ch == CH - 1 && h) x = 0;
+            unsigned kf[4];
+#pragma unroll
+            for (int s = 0; s < 4; s++) kf[s] = attn_pm1(x, s);
+            acc = EngF4::mma(EngF4::make(kf), EngF4::make(qf[ch]), acc);
+        }
+        return acc;
+    };
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+
+    // ---- scores out, sums of the exponentials --------------------------------------------------------------------------------------
+    float s0 = 0.f, s1 = 0.f;
+    const int r8 = lane >> 3, c8 = lane & 7;
+    __half* const srow = a.scores + ((int64_t)bh * S + q0 + r8) * S + c8 * 8;
+    auto group_scores = [&](const int grp, auto tail_c) {
+        constexpr bool TAIL = decltype(tail_c)::value;       // some of the group's keys do not exist
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const EngF4::Acc acc = tile(grp, j);
+            unsigned hs[8];
+#pragma unroll
+            for (int p = 0; p < 8; p++) {
+                const unsigned o0 = (__float_as_uint(acc[2 * p]) - BASE) << 2, o1 = (__float_as_uint(acc[2 * p + 1]) - BASE) << 2;
+                const uint2 e0 = *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(tbl) + o0);
+                const uint2 e1 = *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(tbl) + o1);
+                const int key = grp * 64 + 32 * h + 16 * j + 2 * p;
+                s0 += !TAIL || key < S ? __uint_as_float(e0.x) : 0.f;
+                s1 += !TAIL || key + 1 < S ? __uint_as_float(e1.x) : 0.f;
+                hs[p] = __builtin_amdgcn_perm(e1.y, e0.y, 0x05040100u);
+            }
+            uint4* const to = reinterpret_cast<uint4*>(stage + c * ATTN_STAGE + 64 * h + 32 * j);
+            to[0] = make_uint4(hs[0], hs[1], hs[2], hs[3]);
+            to[1] = make_uint4(hs[4], hs[5], hs[6], hs[7]);
+        }
+        wave_sync();
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint4 x = *reinterpret_cast<const uint4*>(stage + (r8 + 8 * i) * ATTN_STAGE + c8 * 16);
+            __half* const to = srow + (int64_t)(8 * i) * S + grp * 64;
+            if (q0 + r8 + 8 * i < S) {
+                if (!TAIL || grp * 64 + c8 * 8 + 8 <= S) __builtin_memcpy(to, &x, 16);
+                else {
+                    const unsigned d[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                    for (int e = 0; e < 7; e++)
+                        if (grp * 64 + c8 * 8 + e < S) to[e] = __ushort_as_half((uint16_t)(d[e >> 1] >> (16 * (e & 1))));
+                }
+            }
+        }
+        wave_sync();
+    };
+    const int whole = S / 64;
+#pragma unroll 1
+    for (int grp = 0; grp < whole; grp++) group_scores(grp, std::false_type{});
+    if (whole < a.groups) group_scores(whole, std::true_type{});
+    float total = s0 + s1;
+    total += __shfl_xor(total, 32);
+
+    // the fewest matching bits whose probability, rounded to fp16, reaches the level (D + 1: none does)
+    int lo = 0, hi = D + 1;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (__half2float(__float2half_rn(__fdiv_rn(__uint_as_float(tbl[mid].x), total))) >= a.level) hi = mid;
+        else lo = mid + 1;
+    }
+    const unsigned first = BASE + 2 * lo;
+
+    // ---- bits of the probabilities, context --------------------------------------------------------------------------------------
+    EngF4::Acc ctx[W];
+#pragma unroll
+    for (int t = 0; t < W; t++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) ctx[t][v] = 0.f;
+#pragma unroll 1
+    for (int grp = 0; grp < a.groups; grp++) {
+        unsigned below = 0;               // key 32 h + r of the group at bit 31 - r: set where its probability counts as 0
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const EngF4::Acc acc = tile(grp, j);
+#pragma unroll
+            for (int v = 0; v < 16; v++) below = __builtin_amdgcn_alignbit(below, __float_as_uint(acc[v]) - first, 31);
+        }
+        const int left = S - (grp * 64 + 32 * h);
+        if (left < 32) below |= left <= 0 ? 0xffffffffu : 0xffffffffu >> left;
+        unsigned pf[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) pf[s] = attn_01(~below, s);
+#pragma unroll
+        for (int t = 0; t < W; t++) {
+            const unsigned x = vt[(2 * grp + h) * D + t * 32 + row_col];
+            unsigned vf[4];
+#pragma unroll
+            for (int s = 0; s < 4; s++) vf[s] = attn_pm1(x, s);
+            ctx[t] = EngF4::mma(EngF4::make(vf), EngF4::make(pf), ctx[t]);
+        }
+    }
+    if (q0 + c < S) {
+        const int64_t at = ((row0 + q0 + c) * a.heads + head) * D + 16 * h;
+#pragma unroll
+        for (int t = 0; t < W; t++) {
+            if (a.f32) {
+                float4* const to = reinterpret_cast<float4*>(reinterpret_cast<float*>(a.context) + at + t * 32);
+                auto f = [&](const int v) { return __half2float(__float2half_rn(ctx[t][v])); };
+#pragma unroll
+                for (int g = 0; g < 4; g++) to[g] = make_float4(f(4 * g), f(4 * g + 1), f(4 * g + 2), f(4 * g + 3));
+            } else {
+                union { __half x[16]; uint4 u[2]; } pk;
+#pragma unroll
+                for (int v = 0; v < 16; v++) pk.x[v] = __float2half_rn(ctx[t][v]);
+                uint4* const to = reinterpret_cast<uint4*>(reinterpret_cast<__half*>(a.context) + at + t * 32);
+                to[0] = pk.u[0]; to[1] = pk.u[1];
+            }
+        }
+    }
+}
+
+}  // namespace bgemm
+
+using namespace bgemm;
+
+// Heads of 32, 64, 96 or 128 (whole words), and as many keys as leave a block's key and value bits within 32 KiB of LDS.
+extern "C" int bgemm_attention_supported(int64_t batch, int64_t seq, int64_t heads, int64_t head_size)
+{
+    return batch >= 1 && seq >= 1 && heads >= 1 && head_size >= 32 && head_size <= 128 && head_size % 32 == 0 && seq * head_size <= (1 << 17) &&
+           heads <= (1 << 17) && batch <= (1 << 24) && batch * heads * cdiv(seq, 32) <= 0x7fffffffLL && batch * seq <= 0x7fffffffLL;
+}
+
+extern "C" int bgemm_attention_forward(const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
+                                       void* scores, void* context, int context_type, void* stream)
+{
+    if (context_type != BGEMM_SRC_F16 && context_type != BGEMM_SRC_F32) return fail(BGEMM_EINVAL, "bgemm_attention_forward: context type %d", context_type);
+    if (!bgemm_attention_supported(batch, seq, heads, head_size))
+        return fail(BGEMM_EINVAL, "bgemm_attention_forward: %lld x %lld tokens, %lld heads of %lld", (long long)batch, (long long)seq, (long long)heads,
+                    (long long)head_size);
+    if (!q || !k || !v || !scores || !context) return fail(BGEMM_ENULL, "bgemm_attention_forward: null pointer");
+    if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)context) & 15 || (uintptr_t)scores & 1)
+        return fail(BGEMM_EALIGN, "bgemm_attention_forward: operands and context must be 16-byte aligned");
+    const int W = (int)head_size / 32;
+    AttnArgs a = {(const uint32_t*)q, (const uint32_t*)k, (const uint32_t*)v, (__half*)scores, context, k_tiles(heads * head_size)};
+    a.S = (int)seq; a.heads = (int)heads; a.groups = (int)cdiv(seq, 64); a.f32 = context_type == BGEMM_SRC_F32;
+    a.scale = 1.0f / (float)sqrt((double)head_size);
+    a.level = (float)(1.0 / (double)seq);
+    // four waves share a block's operands; fewer where that leaves the chip without two blocks a compute unit
+    int waves = 4;
+    while (waves > 1 && batch * heads * cdiv(seq, 32 * waves) < 512) waves /= 2;
+    a.qblocks = (int)cdiv(seq, 32 * waves);
+    const size_t lds = (size_t)waves * 32 * ATTN_STAGE + (head_size + 2) * 8 + (size_t)2 * W * a.groups * 64 * 4;
+    const dim3 grid((unsigned)(batch * heads * a.qblocks)), block(waves * 64);
+    const hipStream_t st = (hipStream_t)stream;
+    switch (W) {
+    case 1: hipLaunchKernelGGL(attention_kernel<1>, grid, block, lds, st, a); break;
+    case 2: hipLaunchKernelGGL(attention_kernel<2>, grid, block, lds, st, a); break;
+    case 3: hipLaunchKernelGGL(attention_kernel<3>, grid, block, lds, st, a); break;
+    default: hipLaunchKernelGGL(attention_kernel<4>, grid, block, lds, st, a); break;
+    }
+    return check_launch("bgemm_attention_forward");
+}

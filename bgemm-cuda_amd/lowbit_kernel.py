@@ -157,6 +157,11 @@ def zeros_packed(rows, K, batch=1, device="cuda"):
     return PackedBits(torch.zeros((batch, words), dtype=torch.int32, device=device), None, batch, rows, K)
 
 
+def empty_packed(rows, K, device="cuda"):
+    """The same without the zeros, for a reader that looks at real bits only."""
+    return PackedBits(torch.empty((1, _b.lib().bgemm_tiled_words(rows, K)), dtype=torch.int32, device=device), None, 1, rows, K)
+
+
 def _batch_layout(x):
     """(outer, inner, stride_outer, stride_inner) of the leading dimensions of a 2-D to 4-D tensor."""
     if x.dim() == 2:
@@ -369,6 +374,37 @@ def bgemm_packed_forward(w, x, mode=MODE_XOR, out_dtype=torch.int32, splitK=1, v
             _b.check(L.bgemm_packed_forward_scaled(*args, sw.data_ptr(), sa.data_ptr(),
                                                    bias.data_ptr() if bias is not None else None, _stream()))
     return out
+
+
+def attention_supported(batch, seq, heads, head_size):
+    """Whether ``attention_forward`` takes these sizes."""
+    return bool(_b.lib().bgemm_attention_supported(batch, seq, heads, head_size))
+
+
+def attention_forward(q, k, v, batch, heads, dtype):
+    """Binary self-attention on packed operands (bert.py:245-259), one launch.  ``q``, ``k``, ``v``: sign bits of ``batch * seq`` rows
+    and ``heads * head_size`` columns.  Returns the scores ``half(q . k) / sqrt(head_size)``, fp16 ``[batch, heads, seq, seq]``, and
+    the context in ``dtype``, ``[batch, seq, heads * head_size]``: the sum of sign(v) over the keys whose probability (softmax in
+    fp16 storage) is at least ``1 / seq``."""
+    rows, hidden = q.rows, q.K
+    for name, p in (("q", q), ("k", k), ("v", v)):
+        if p.ternary or p.batch != 1 or (p.rows, p.K) != (rows, hidden):
+            raise ValueError("%s must be a binary operand of %d x %d" % (name, rows, hidden))
+        _check_packed(p, name)
+        if p.data.device != q.data.device:
+            raise ValueError("%s is on %s, q on %s" % (name, p.data.device, q.data.device))
+    if batch < 1 or heads < 1 or rows % batch or hidden % heads:
+        raise ValueError("%d x %d bits are no %d sequences of %d heads" % (rows, hidden, batch, heads))
+    if dtype not in (torch.float32, torch.half):
+        raise TypeError("dtype must be torch.float32 or torch.half")
+    seq, dev = rows // batch, q.data.device
+    scores = torch.empty((batch, heads, seq, seq), dtype=torch.half, device=dev)
+    context = torch.empty((batch, seq, hidden), dtype=dtype, device=dev)
+    with _on(dev):
+        _b.check(_b.lib().bgemm_attention_forward(q.data.data_ptr(), k.data.data_ptr(), v.data.data_ptr(), batch, seq, heads, hidden // heads,
+                                                  scores.data_ptr(), context.data_ptr(), SRC_F32 if dtype == torch.float32 else SRC_F16,
+                                                  _stream()))
+    return scores, context
 
 
 class DecodeChain:

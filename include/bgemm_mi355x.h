@@ -313,6 +313,16 @@ int bgemm_elastic_backward(const void* x_sign, const void* x_nonzero, const void
                            int64_t K, void* grad_x, void* grad_w, void* grad_bias, void* grad_sw, void* grad_sa, void* ws,
                            size_t ws_bytes, void* stream);
 
+/* ---- binary self-attention without a gradient, one launch -----------------------------------------
+ * (tests/python/bert/bert.py:245-259 on sign bits.)  q, k, v: sign bits [batch * seq][heads * head_size], tiled, 16-byte aligned.
+ *   scores  [batch][heads][seq][seq] fp16 = half(half(sign(q) . sign(k)) / sqrt(head_size))
+ *   context [batch][seq][heads * head_size] (context_type BGEMM_SRC_F16 / BGEMM_SRC_F32, 16-byte aligned) = half(sum of sign(v)
+ *           over the keys whose probability, half(softmax(scores)), is at least 1 / seq)
+ * Supported: head_size 32, 64, 96 or 128 with seq * head_size <= 2^17; EINVAL otherwise. */
+int bgemm_attention_supported(int64_t batch, int64_t seq, int64_t heads, int64_t head_size);
+int bgemm_attention_forward(const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
+                            void* scores, void* context, int context_type, void* stream);
+
 /* ---- a chain of dependent decode-shaped layers in one launch ------------------------------------
  * Layer l computes acc = MODE(W_l [M_l][K_l], x_l [N][K_l]) and hands layer l + 1 the bits of
  * half_rn(y - *next_zero_point), y = half(acc) * sw * sa (+ bias) evaluated as in bgemm_packed_forward_scaled

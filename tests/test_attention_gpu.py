@@ -1,0 +1,65 @@
+"""The one-launch binary self-attention against dense torch: scores bit for bit, the context wherever float64 leaves no doubt about a
+probability's side of the level; the block that uses it against its own general path."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+import attention_demo
+import lowbit_kernel as lk
+
+DEV = "cuda:0"
+
+
+def pm1(t):
+    return torch.where(torch.signbit(t), -1.0, 1.0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.half])
+@pytest.mark.parametrize("B, S, H, d", [(1, 1, 1, 32), (3, 7, 2, 64), (1, 32, 3, 96), (2, 33, 5, 128), (2, 63, 3, 32), (1, 64, 9, 64), (1, 65, 2, 64),
+                                        (2, 127, 4, 96), (5, 129, 7, 64), (4, 512, 12, 64), (1, 1000, 3, 128), (1, 2048, 2, 64), (1, 4096, 1, 32),
+                                        (16, 130, 12, 32)])
+def test_attention_in_one_launch(B, S, H, d, dtype):
+    g = torch.Generator(device=DEV).manual_seed(S * 131 + d)
+    q, k, v = (torch.randn(B * S, H * d, generator=g, device=DEV) for _ in range(3))
+    q = q + 0.4 * k                                     # scores away from their mean as well
+    scores, context = lk.attention_forward(lk.pack_sign(q), lk.pack_sign(k), lk.pack_sign(v), B, H, dtype)
+    assert scores.shape == (B, H, S, S) and context.shape == (B, S, H * d) and context.dtype == dtype
+    split = lambda t: pm1(t).view(B, S, H, d).permute(0, 2, 1, 3)
+    want = (split(q) @ split(k).transpose(-1, -2).contiguous()).half() / math.sqrt(d)
+    assert torch.equal(scores, want)
+    p = torch.softmax(want.double(), -1)
+    # fp32 exponentials, a sum of S of them and a division: within 1e-6 of p (measured bits agree far closer)
+    over = [(p * (1 + e)).half().float() >= torch.tensor(1.0 / S) for e in (-1e-6, 1e-6)]
+    clear = (over[0] == over[1]).all(-1)
+    ref = (over[0].float() @ split(v).contiguous()).half()
+    got = context.view(B, S, H, d).permute(0, 2, 1, 3)
+    assert clear.float().mean() > 0.97
+    assert torch.equal(got[clear], ref.to(dtype)[clear])
+
+
+@pytest.mark.parametrize("hidden, heads, B, S, dtype", [(768, 12, 2, 128, torch.float32), (96, 3, 3, 77, torch.half), (640, 5, 1, 200, torch.float32)])
+def test_block_fused_equals_its_general_path(hidden, heads, B, S, dtype, monkeypatch):
+    torch.manual_seed(S)
+    block = attention_demo.BinarySelfAttention(hidden, heads).to(DEV).to(dtype)
+    x = torch.randn(B, S, hidden, device=DEV, dtype=dtype)
+    calls = []
+    inner = lk.attention_forward
+    monkeypatch.setattr(lk, "attention_forward", lambda *a: calls.append(1) or inner(*a))
+    with torch.no_grad():
+        block(x)                                        # sets the scales
+        assert not calls
+        out, scores = block(x)
+        assert len(calls) == 1
+        seen = []
+        handle = block.key.register_forward_hook(lambda m, i, o: seen.append(o.shape))       # a listener gets its call
+        out2, scores2 = block(x)
+        handle.remove()
+        assert len(calls) == 1 and seen == [(B, S, hidden)]
+        masked, _ = block(x, torch.zeros(B, 1, 1, S, device=DEV))
+    assert out.dtype == out2.dtype and torch.equal(scores, scores2)
+    # a probability on the level may fall either way with the order of the softmax's sum: few rows of the context, if any
+    same = (out == out2).all(-1).float().mean()
+    assert same > 0.98 and torch.equal(masked, out2), float(same)
