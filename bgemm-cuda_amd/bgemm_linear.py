@@ -68,6 +68,19 @@ def _batched_packed(x_rows, right, mode):
     return out.reshape(*lead, x_rows.shape[-2], right.shape[-1])
 
 
+# The longest rows the one-launch gradients take.  The scores' read an [N][M] matrix twice, which beats the separate kernels while the
+# caches hold one (8 x 1024^2, D = 128, twice: 172 -> 90 us; 4 x 2048^2, D = 64: 126 -> 88) and not when each reading comes from
+# memory (16 x 4096^2: 231 -> 264).  The context's were timed ahead up to 4096 (16 x 4096^2: 1553 -> 511).
+SCORES_GRAD_ROWS, CONTEXT_GRAD_ROWS = 2048, 4096
+
+
+def _one_launch_grads(matrix, a, b, longest):
+    """Whether the batched products' gradients go to their one-launch kernels: operands those read where they lie, and nothing that
+    has to see the torch operations (a graph of the gradients, vmap, a tensor subclass)."""
+    return (not torch.is_grad_enabled() and lowbit_kernel.attention_grads_supported(a, b, longest) and type(matrix) is torch.Tensor
+            and matrix.dtype == torch.half and matrix.device == a.device and not lowbit_kernel._wrapped(matrix))
+
+
 class bgemm_matmul(torch.autograd.Function):
     """matA [.., N, K] @ matB [K, M] with both operands binarised by sign (bgemm_linear.py:9-42).
     A matB with leading dimensions ([B, H, K, M], as K^T in attention) is a batched matmul."""
@@ -91,6 +104,10 @@ class bgemm_matmul(torch.autograd.Function):
         matA, matB = ctx.saved_tensors
         if matB.dim() > 2:
             g = grad_output.to(matA.dtype)
+            right = matB.transpose(-1, -2)
+            if _one_launch_grads(g, matA, right, SCORES_GRAD_ROWS):
+                grad_a, grad_bt = lowbit_kernel.scores_backward(g, matA, right, ctx.needs_input_grad[:2])
+                return grad_a, None if grad_bt is None else grad_bt.transpose(-1, -2), None
             return g @ matB.sign().transpose(-1, -2), matA.sign().transpose(-1, -2) @ g, None
         grad_a, grad_bt = _linear_grads(grad_output, matA.sign(), matB.sign().transpose(-1, -2))
         return grad_a, grad_bt.transpose(-1, -2), None
@@ -116,6 +133,10 @@ class bgemm_attn_matmul(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         attn, value = ctx.saved_tensors
+        if attn.dim() > 2:
+            g = grad_output.to(value.dtype)
+            if _one_launch_grads(attn, g, value, CONTEXT_GRAD_ROWS):
+                return (*lowbit_kernel.context_backward(attn, g, value, ctx.needs_input_grad[:2]), None)
         a01 = (attn.sign() + 1) / 2
         a01 = torch.where(a01 == 0, torch.ones_like(a01), a01)     # as the reference does (:70-71)
         v = value.sign()

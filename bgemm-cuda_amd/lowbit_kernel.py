@@ -11,6 +11,7 @@ include/bgemm_mi355x.h; torch supplies device memory and streams only.
 """
 import contextlib
 import collections
+import ctypes
 import struct
 import weakref
 
@@ -405,6 +406,63 @@ def attention_forward(q, k, v, batch, heads, dtype):
                                                   scores.data_ptr(), context.data_ptr(), SRC_F32 if dtype == torch.float32 else SRC_F16,
                                                   _stream()))
     return scores, context
+
+
+def _head_view(t):
+    """(outer, inner, row) strides of [.., rows, D] with up to two leading dimensions, zero where there is one of something."""
+    st = [s if n > 1 else 0 for s, n in zip(t.stride()[:-1], t.shape[:-1])]
+    return [0] * (3 - len(st)) + st
+
+
+def attention_grads_supported(a, b, longest=4096):
+    """Whether ``scores_backward`` / ``context_backward`` read these [.., rows, D] operands where they lie: fp16 tensors of their own
+    on one GPU, D dense and 32, 64, 96 or 128, everything 16-byte aligned, ``longest`` rows at most."""
+    for t in (a, b):
+        if (type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.half or t.dim() not in (3, 4) or not t.numel()
+                or t.shape[-1] not in (32, 64, 96, 128) or t.stride(-1) != 1 or _wrapped(t) or t.data_ptr() % 16
+                or any(s % 8 for s in _head_view(t))):
+            return False
+    N, M, batch = a.shape[-2], b.shape[-2], a.numel() // (a.shape[-2] * a.shape[-1])
+    return a.device == b.device and max(N, M) <= longest and batch * -(-N // 64) * (-(-M // 64) + 1) < 2 ** 31 - 2 ** 24
+
+
+def _wrapped(t):
+    f = torch._C._functorch
+    return f.is_functorch_wrapped_tensor(t) or f.is_legacy_batchedtensor(t)
+
+
+def _grad_like(t):
+    """An uninitialised gradient in the operand's own strides, or dense where those have gaps that end its rows."""
+    g = torch.empty_like(t)
+    return g if g.stride(-1) == 1 else torch.empty_like(t, memory_format=torch.contiguous_format)
+
+
+def _attention_backward(fn, m, a, b, out_a, out_b, strides_of):
+    strides = (ctypes.c_int64 * 12)(*(s for t in strides_of for s in ([0] * 3 if t is None else _head_view(t))))
+    inner = a.shape[-3]
+    ptr = lambda t: None if t is None else t.data_ptr()
+    with _on(a.device):
+        _b.check(fn(ptr(m), a.data_ptr(), b.data_ptr(), strides, inner * (a.shape[0] if a.dim() == 4 else 1), inner, a.shape[-2],
+                    b.shape[-2], a.shape[-1], ptr(out_a), ptr(out_b), _stream()))
+
+
+def scores_backward(grad_scores, a, b, need=(True, True)):
+    """Straight-through gradients of ``sign(a) @ sign(b).T`` (bgemm_linear.py:28-42) in one launch: ``a`` [.., N, D], ``b`` [.., M, D],
+    ``grad_scores`` [.., N, M] fp16.  The gradients have their operands' strides; one not needed is None."""
+    g = grad_scores.contiguous()
+    ga, gb = (_grad_like(t) if wanted else None for t, wanted in zip((a, b), need))
+    _attention_backward(_b.lib().bgemm_scores_backward, g, a, b, ga, gb, (a, b, ga, gb))
+    return ga, gb
+
+
+def context_backward(probs, grad_context, value, need=(True, True)):
+    """Gradients of the attention matmul (bgemm_linear.py:64-86) in one launch: ``probs`` [.., N, M], ``grad_context`` [.., N, D],
+    ``value`` [.., M, D], fp16.  Returns (grad_probs, grad_value), None for one not needed."""
+    gp = torch.empty(probs.shape, dtype=torch.half, device=probs.device) if need[0] else None
+    gv = _grad_like(value) if need[1] else None
+    _attention_backward(_b.lib().bgemm_context_backward, probs.contiguous() if need[1] else None, grad_context, value, gp, gv,
+                        (grad_context, value, None, gv))
+    return gp, gv
 
 
 class DecodeChain:

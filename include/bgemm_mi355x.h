@@ -323,6 +323,21 @@ int bgemm_attention_supported(int64_t batch, int64_t seq, int64_t heads, int64_t
 int bgemm_attention_forward(const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
                             void* scores, void* context, int context_type, void* stream);
 
+/* ---- gradients of both attention products, one launch each ----------------------------------------
+ * (tests/python/bgemm_linear.py:28-42, 64-86 on `batch` matrices, `inner` to an outer one.)  fp16 throughout, sums in fp32; sign(0) = 0.
+ *   scores   a [N][D], b [M][D], grad_scores [N][M] dense:
+ *            grad_a[n] = sum_m grad_scores[n][m] sign(b[m])      grad_b[m] = sum_n grad_scores[n][m] sign(a[n])
+ *   context  probs [N][M] dense, grad_context [N][D], value [M][D]:
+ *            grad_probs[n][m] = half(grad_context[n] . sign(value[m])) / 2, dense
+ *            grad_value[m] = sum_n w(probs[n][m]) grad_context[n],  w = 0.5 where probs is 0, else 1
+ * strides: 12 numbers, the outer, inner and row stride in elements of (a, b, grad_a, grad_b), or of (grad_context, value, unused,
+ * grad_value); all multiples of 8, columns dense, bases 16-byte aligned.  D is 32, 64, 96 or 128.  A null gradient is not computed
+ * (probs may be null where grad_value is). */
+int bgemm_scores_backward(const void* grad_scores, const void* a, const void* b, const int64_t* strides, int64_t batch, int64_t inner,
+                          int64_t N, int64_t M, int64_t D, void* grad_a, void* grad_b, void* stream);
+int bgemm_context_backward(const void* probs, const void* grad_context, const void* value, const int64_t* strides, int64_t batch,
+                           int64_t inner, int64_t N, int64_t M, int64_t D, void* grad_probs, void* grad_value, void* stream);
+
 /* ---- a chain of dependent decode-shaped layers in one launch ------------------------------------
  * Layer l computes acc = MODE(W_l [M_l][K_l], x_l [N][K_l]) and hands layer l + 1 the bits of
  * half_rn(y - *next_zero_point), y = half(acc) * sw * sa (+ bias) evaluated as in bgemm_packed_forward_scaled

@@ -1,0 +1,89 @@
+"""The one-launch gradients of both attention products against float64, and against the torch operations they stand for."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+import bgemm_linear as bl
+import lowbit_kernel as lk
+
+DEV = "cuda:0"
+
+
+def head_split(t, H):
+    return t.view(t.shape[0], t.shape[1], H, -1).permute(0, 2, 1, 3)
+
+
+def bound(terms):
+    """Products of fp16 numbers and +-1 (1/2) are exact in fp32; `terms` sums of them in any order, rounded to fp16 once: half a last
+    place of the result, 2^-24 of the absolute sum for each addition, and the smallest fp16 step."""
+    return lambda got, want, total: bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -11 + total * terms * 2.0 ** -23 + 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("B, H, N, M, d", [(1, 1, 1, 1, 32), (2, 3, 7, 65, 64), (1, 2, 64, 64, 96), (3, 1, 63, 8, 128), (2, 2, 129, 71, 32),
+                                           (1, 5, 130, 200, 64), (4, 12, 512, 512, 64), (1, 1, 4096, 100, 32)])
+def test_gradients(B, H, N, M, d, monkeypatch):
+    g = torch.Generator(device=DEV).manual_seed(N * 131 + M)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).half()
+    q, k, v, p = rnd(B, N, H * d), rnd(B, M, H * d), rnd(B, M, H * d), rnd(B, H, N, M)
+    for t in (q, k, v, p):
+        t.view(-1)[::3] = 0                                       # sign 0 / weight 1/2
+        t.view(-1)[1::7] = -0.0
+        t.view(-1)[2::11] = float("nan")
+        t.view(-1)[5::13] = float("inf")
+    for t in (q, k, v, p):
+        t.requires_grad_(True)
+    gs, gc = rnd(B, H, N, M), rnd(B, H, N, d)
+
+    def grads(**kw):
+        scores = bl.bgemm_matmul.apply(head_split(q, H), head_split(k, H).transpose(-1, -2))
+        context = bl.bgemm_attn_matmul.apply(p, head_split(v, H))
+        return torch.autograd.grad([scores, context], [q, k, v, p], [gs, gc], **kw)
+
+    calls = []
+    for name in ("scores_backward", "context_backward"):
+        monkeypatch.setattr(lk, name, lambda *a, fn=getattr(lk, name): calls.append(1) or fn(*a))
+    got = grads()
+    assert len(calls) == 2
+    general = grads(create_graph=True)                            # needs the torch operations
+    assert len(calls) == 2
+    sign = lambda t: ((t > 0).double() - (t < 0).double())
+    sq, sk, sv = (sign(head_split(t.detach(), H)) for t in (q, k, v))
+    w = 0.5 + 0.5 * sign(p.detach()).abs()
+    gs, gc = gs.double(), gc.double()
+    merge = lambda t: t.permute(0, 2, 1, 3).reshape(B, -1, H * d)
+    T = lambda t: t.transpose(-1, -2).contiguous()
+    want = [merge(gs @ sk), merge(T(gs) @ sq), merge(T(w) @ gc), gc @ T(sv) / 2]
+    total = [merge(gs.abs() @ sk.abs()), merge(T(gs.abs()) @ sq.abs()), merge(T(w) @ gc.abs()), gc.abs() @ T(sv.abs()) / 2]
+    for a, b, x, y, terms in zip(got, (t.detach() for t in general), want, total, (M, N, N, d)):
+        assert a.shape == b.shape and a.dtype == b.dtype and a.is_contiguous()
+        assert bound(terms)(a, x, y)
+        assert float((a.double() - x).norm()) <= 1.02 * float((b.double() - x).norm()) + 1e-9
+
+
+def test_other_forms_take_the_way_they_took(monkeypatch):
+    """fp32 operands, one gradient only, gradients and operands in other strides, an infinite gradient, two dimensions."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    q, k, p = rnd(2, 40, 64), rnd(2, 50, 64), rnd(2, 40, 50)
+    gs, gc = rnd(2, 50, 40).transpose(1, 2), rnd(2, 64, 40).transpose(1, 2)
+    gs[0, 3, 4] = float("inf")
+
+    def run(fn, a, b, up, which):
+        a, b = a.detach().requires_grad_("a" in which), b.detach().requires_grad_("b" in which)
+        leaves = [t for t in (a, b) if t.requires_grad]
+        out = fn.apply(a, b)
+        return torch.autograd.grad(out, leaves, up.to(out.dtype))
+
+    cases = [(bl.bgemm_matmul, q, k.transpose(1, 2), gs), (bl.bgemm_matmul, q.half(), rnd(2, 64, 50).half(), gs),
+             (bl.bgemm_matmul, q.transpose(0, 1).contiguous().transpose(0, 1).half(), k.half().transpose(1, 2), gs),
+             (bl.bgemm_attn_matmul, p, k, gc), (bl.bgemm_attn_matmul, p.half().transpose(1, 2).contiguous().transpose(1, 2), k.half(), gc),
+             (bl.bgemm_matmul, rnd(2, 40, 72).half()[..., 3:67], k.half().transpose(1, 2), gs), (bl.bgemm_matmul, q[0], k[0].T, gs[0])]
+    got = [run(*c, which) for c in cases for which in ("a", "b", "ab")]
+    monkeypatch.setattr(bl, "_one_launch_grads", lambda *a: False)
+    for have, want in zip(got, [run(*c, which) for c in cases for which in ("a", "b", "ab")]):
+        assert len(have) == len(want)
+        for x, y in zip(have, want):
+            assert x.dtype == y.dtype and x.shape == y.shape
+            # both round exact products' fp32 sums (at most 64 terms) to fp16: a last place apart
+            assert torch.allclose(x.double(), y.double(), rtol=2.0 ** -9, atol=2.0 ** -10, equal_nan=True)
