@@ -14,7 +14,7 @@ SO_PATH = os.path.join(_HERE, "libbgemm_mi355x.so")
 OK, EINVAL, ENULL, EWORKSPACE, ELAUNCH, EALIGN, ETIMEOUT = 0, -1, -2, -3, -4, -5, -6
 MODE_AND, MODE_XOR, MODE_ATTN, MODE_BWTA, MODE_ATTN_X = 0, 1, 2, 3, 4
 OUT_I32, OUT_F16, OUT_F32_SCALED, OUT_F16_SCALED, OUT_BITS_F32, OUT_BITS_F16 = 0, 1, 2, 3, 4, 5
-SRC_F16, SRC_F32 = 0, 1
+SRC_F16, SRC_F32, SRC_BITS = 0, 1, 2
 ABI_VERSION = 11
 LAYOUT_VERSION = 6     # of the tiled operand layout, written into packed files; changes only when the layout does
 STATIC_SCRATCH_BYTES = 32 << 20      # BGEMM_STATIC_SCRATCH_BYTES
@@ -70,14 +70,22 @@ SIGNATURES = {
     "bgemm_elastic_forward": (_int, [_p, _p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     "bgemm_elastic_backward_workspace_bytes": (_sz, [_i64, _i64, _i64, _int, _int]),
     "bgemm_elastic_backward": (_int, [_p, _p, _p, _p, _p, _p, _p, ctypes.c_float, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _sz, _p]),
+    "bgemm_linear_rows_supported": (_int, [_i64, _i64, _i64, _int, _int]),
+    "bgemm_linear_rows_forward": (_int, [_p, _int, _i64, _i64, _i64, _i64, _int, _p, _int, _p, _int, _p]),
     "bgemm_attention_supported": (_int, [_i64, _i64, _i64, _i64]),
     "bgemm_attention_forward": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p, _int, _p]),
+    "bgemm_attention_forward_bits": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _int, _p]),
     "bgemm_scores_backward": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p]),
     "bgemm_context_backward": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p]),
     "bgemm_chain_workspace_bytes": (_sz, [_int, _p, _int, _i64]),
     "bgemm_chain_forward": (_int, [_int, _p, _p, _int, _p, _p, _i64, _p, _int, _int, _p, _sz, _int, _p]),
     "bgemm_chain_status": (_int, [_p, _p]),
 }
+
+
+class RowsLayer(ctypes.Structure):
+    """bgemm_rows_layer: one layer of bgemm_linear_rows_forward; every pointer is a device pointer."""
+    _fields_ = [(name, _p) for name in ("W_tiled", "zero_point", "sw", "sa", "bias", "next_zero_point", "out")]
 
 
 class ChainLayer(ctypes.Structure):

@@ -18,7 +18,7 @@ import torch
 import torch.nn as nn
 
 import lowbit_kernel
-from bgemm_linear import BGEMMLinear, GraphedInference, bgemm_attn_matmul, bgemm_matmul
+from bgemm_linear import BGEMMLinear, GraphedInference, bgemm_attn_matmul, bgemm_matmul, fused_bits
 
 
 def _pm1(t):
@@ -60,12 +60,26 @@ class BinarySelfAttention(nn.Module):
                 and splits(self.query) and splits(self.key) and splits(self.value)
                 and lowbit_kernel.attention_supported(x.shape[0], x.shape[1], self.num_attention_heads, self.attention_head_size))
 
+    def _dense_fusable(self, x, rows, hidden):
+        """Whether the last projection may read the context's bits and add the residual: a plain layer of this block's size."""
+        layer = self.dense
+        return (type(layer) is BGEMMLinear and layer.weight.shape == (hidden, hidden) and x.shape[-1] == hidden and layer._bits_fusable(x)
+                and lowbit_kernel.linear_rows_supported(rows, hidden, hidden, 1, lowbit_kernel.OUT_F32_SCALED if x.dtype == torch.float32
+                                                        else lowbit_kernel.OUT_F16_SCALED))
+
     def forward(self, hidden_states, attention_mask=None):
         if self.kernels and attention_mask is None and self._fusable(hidden_states):
             # nothing but the projections' signs is read: they leave their GEMMs as bits, and one kernel does the rest
-            scores, context = lowbit_kernel.attention_forward(self.query._fused_bits(hidden_states), self.key._fused_bits(hidden_states),
-                                                              self.value._fused_bits(hidden_states), hidden_states.shape[0],
-                                                              self.num_attention_heads, hidden_states.dtype)
+            bits = fused_bits([self.query, self.key, self.value], hidden_states)
+            batch, seq, _ = hidden_states.shape
+            rows, hidden = batch * seq, bits[0].K
+            if self._dense_fusable(hidden_states, rows, hidden):
+                # of the context, too, the last projection reads its signs only, and it adds the residual as it stores
+                dense = self.dense._rows_layer(hidden_states.dtype)
+                scores, context = lowbit_kernel.attention_forward(*bits, batch, self.num_attention_heads, hidden_states.dtype, dense[1])
+                out = lowbit_kernel.linear_rows_forward(context, [dense], residual=hidden_states.reshape(rows, hidden).contiguous())[0]
+                return self.LayerNorm(out.view(batch, seq, hidden)), scores
+            scores, context = lowbit_kernel.attention_forward(*bits, batch, self.num_attention_heads, hidden_states.dtype)
             return self.LayerNorm(self.dense(context) + hidden_states), scores
         q = self.transpose_for_scores(self.query(hidden_states))
         k = self.transpose_for_scores(self.key(hidden_states))

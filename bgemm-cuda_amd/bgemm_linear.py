@@ -440,6 +440,11 @@ class BGEMMLinear(_ScaledBinaryLinear):
         return (type(self) is BGEMMLinear and self.initialized and self._fusable(x) and "forward" not in self.__dict__
                 and not self._forward_hooks and not self._forward_pre_hooks and not nn.modules.module._has_any_global_hook())
 
+    def _rows_layer(self, dtype):
+        """The layer as ``lowbit_kernel.linear_rows_forward`` takes it."""
+        _, sw, sa, bias, zpa = self._inference_state()
+        return self._packed_weight(), self.zpa.detach().to(dtype).reshape(1) if zpa is None else zpa, sw, sa, bias
+
     def _fused_bits(self, x):
         """The sign bits of ``self(x)``, [rows of x] x [features], for a consumer that reads nothing else of it."""
         _, sw, sa, bias, zpa = self._inference_state()
@@ -463,6 +468,17 @@ class BGEMMLinear(_ScaledBinaryLinear):
                     return out
         out = self._fn.apply(x - self.zpa, self.weight - self.zpw) * self.sw * self.sa
         return self._add_bias(out)
+
+
+def fused_bits(layers, x):
+    """The sign bits of ``layer(x)`` for every layer of a list, each of which is ``_bits_fusable(x)``: one launch where they are of one
+    size that ``lowbit_kernel.linear_rows_forward`` takes, else two a layer."""
+    w = layers[0].weight
+    kind = lowbit_kernel.OUT_BITS_F32 if x.dtype == torch.float32 else lowbit_kernel.OUT_BITS_F16
+    if (all(l.weight.shape == w.shape for l in layers)
+            and lowbit_kernel.linear_rows_supported(x.numel() // x.shape[-1], w.shape[0], w.shape[1], len(layers), kind)):
+        return lowbit_kernel.linear_rows_forward(x.reshape(-1, x.shape[-1]), [l._rows_layer(x.dtype) for l in layers], bits=True)
+    return [l._fused_bits(x) for l in layers]
 
 
 class BGEMMChain(nn.Sequential):

@@ -26,7 +26,8 @@ namespace bgemm {
 
 struct AttnArgs {
     const uint32_t* q; const uint32_t* k; const uint32_t* v;      // sign bits [batch * S][heads * D], tiled
-    __half* scores; void* context;
+    __half* scores; void* context;    // context: numbers, or the tiled operand of their signs after *zp is subtracted
+    const void* zp;
     int64_t KT;                       // of the operands
     int S, heads, groups, qblocks, f32;
     float scale, level;               // 1 / sqrt(D), 1 / S
@@ -38,8 +39,8 @@ constexpr int ATTN_STAGE = 144;       // bytes of a staged row of 64 scores (pad
 __device__ __forceinline__ unsigned attn_pm1(const unsigned w, const int s) { return (s == 3 ? w & 0x88888888u : (w << (3 - s)) & 0x88888888u) | 0x22222222u; }
 __device__ __forceinline__ unsigned attn_01(const unsigned w, const int s) { return (s == 0 ? w << 1 : w >> (s - 1)) & 0x22222222u; }
 
-// W: words a head (D = 32 W).
-template <int W>
+// W: words a head (D = 32 W).  BITS: the context leaves as the next binary layer's operand.
+template <int W, bool BITS>
 __global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
 {
     constexpr int D = W * 32, CH = (W + 1) / 2, PAD = CH * 64 - D;       // chunks of 64 bits, the last half a one if W is odd
@@ -196,6 +197,22 @@ __global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
             ctx[t] = EngF4::mma(EngF4::make(vf), EngF4::make(pf), ctx[t]);
         }
     }
+    if constexpr (BITS) {
+        // a lane's 16 columns of its query, joined with the other half's: a word a head and 32 columns
+        const float zp = !a.zp ? 0.f : a.f32 ? *reinterpret_cast<const float*>(a.zp) : __half2float(*reinterpret_cast<const __half*>(a.zp));
+        uint32_t* const out = reinterpret_cast<uint32_t*>(a.context);
+#pragma unroll
+        for (int t = 0; t < W; t++) {
+            unsigned w = 0;
+#pragma unroll
+            for (int v = 0; v < 16; v++) w = __builtin_amdgcn_alignbit(w, __float_as_uint(__fsub_rn(__half2float(__float2half_rn(ctx[t][v])), zp)), 31);
+            w = w << 16 | __shfl_xor(w, 32);
+            if (h == 0 && q0 + c < S) out[tiled_word_offset(row0 + q0 + c, head * W + t, a.KT)] = w;
+        }
+        if (head == a.heads - 1 && q0 + c < S)
+            for (int64_t w = a.heads * W + h; w < a.KT * 8; w += 2) out[tiled_word_offset(row0 + q0 + c, w, a.KT)] = 0u;
+        return;
+    }
     if (q0 + c < S) {
         const int64_t at = ((row0 + q0 + c) * a.heads + head) * D + 16 * h;
 #pragma unroll
@@ -227,18 +244,19 @@ extern "C" int bgemm_attention_supported(int64_t batch, int64_t seq, int64_t hea
            heads <= (1 << 17) && batch <= (1 << 24) && batch * heads * cdiv(seq, 32) <= 0x7fffffffLL && batch * seq <= 0x7fffffffLL;
 }
 
-extern "C" int bgemm_attention_forward(const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
-                                       void* scores, void* context, int context_type, void* stream)
+static int attention(const char* who, const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
+                     void* scores, void* context, const void* zero_point, bool bits, int context_type, void* stream)
 {
-    if (context_type != BGEMM_SRC_F16 && context_type != BGEMM_SRC_F32) return fail(BGEMM_EINVAL, "bgemm_attention_forward: context type %d", context_type);
+    if (context_type != BGEMM_SRC_F16 && context_type != BGEMM_SRC_F32) return fail(BGEMM_EINVAL, "%s: context type %d", who, context_type);
     if (!bgemm_attention_supported(batch, seq, heads, head_size))
-        return fail(BGEMM_EINVAL, "bgemm_attention_forward: %lld x %lld tokens, %lld heads of %lld", (long long)batch, (long long)seq, (long long)heads,
+        return fail(BGEMM_EINVAL, "%s: %lld x %lld tokens, %lld heads of %lld", who, (long long)batch, (long long)seq, (long long)heads,
                     (long long)head_size);
-    if (!q || !k || !v || !scores || !context) return fail(BGEMM_ENULL, "bgemm_attention_forward: null pointer");
-    if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)context) & 15 || (uintptr_t)scores & 1)
-        return fail(BGEMM_EALIGN, "bgemm_attention_forward: operands and context must be 16-byte aligned");
+    if (!q || !k || !v || !scores || !context) return fail(BGEMM_ENULL, "%s: null pointer", who);
+    if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)context) & 15 || (uintptr_t)scores & 1 ||
+        (uintptr_t)zero_point & (context_type == BGEMM_SRC_F32 ? 3 : 1))
+        return fail(BGEMM_EALIGN, "%s: operands and context must be 16-byte aligned", who);
     const int W = (int)head_size / 32;
-    AttnArgs a = {(const uint32_t*)q, (const uint32_t*)k, (const uint32_t*)v, (__half*)scores, context, k_tiles(heads * head_size)};
+    AttnArgs a = {(const uint32_t*)q, (const uint32_t*)k, (const uint32_t*)v, (__half*)scores, context, zero_point, k_tiles(heads * head_size)};
     a.S = (int)seq; a.heads = (int)heads; a.groups = (int)cdiv(seq, 64); a.f32 = context_type == BGEMM_SRC_F32;
     a.scale = 1.0f / (float)sqrt((double)head_size);
     a.level = (float)(1.0 / (double)seq);
@@ -249,11 +267,27 @@ extern "C" int bgemm_attention_forward(const void* q, const void* k, const void*
     const size_t lds = (size_t)waves * 32 * ATTN_STAGE + (head_size + 2) * 8 + (size_t)2 * W * a.groups * 64 * 4;
     const dim3 grid((unsigned)(batch * heads * a.qblocks)), block(waves * 64);
     const hipStream_t st = (hipStream_t)stream;
+    auto go = [&](auto numbers, auto as_bits) {
+        if (bits) hipLaunchKernelGGL(as_bits, grid, block, lds, st, a);
+        else hipLaunchKernelGGL(numbers, grid, block, lds, st, a);
+    };
     switch (W) {
-    case 1: hipLaunchKernelGGL(attention_kernel<1>, grid, block, lds, st, a); break;
-    case 2: hipLaunchKernelGGL(attention_kernel<2>, grid, block, lds, st, a); break;
-    case 3: hipLaunchKernelGGL(attention_kernel<3>, grid, block, lds, st, a); break;
-    default: hipLaunchKernelGGL(attention_kernel<4>, grid, block, lds, st, a); break;
+    case 1: go(attention_kernel<1, false>, attention_kernel<1, true>); break;
+    case 2: go(attention_kernel<2, false>, attention_kernel<2, true>); break;
+    case 3: go(attention_kernel<3, false>, attention_kernel<3, true>); break;
+    default: go(attention_kernel<4, false>, attention_kernel<4, true>); break;
     }
-    return check_launch("bgemm_attention_forward");
+    return check_launch(who);
+}
+
+extern "C" int bgemm_attention_forward(const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
+                                       void* scores, void* context, int context_type, void* stream)
+{
+    return attention("bgemm_attention_forward", q, k, v, batch, seq, heads, head_size, scores, context, nullptr, false, context_type, stream);
+}
+
+extern "C" int bgemm_attention_forward_bits(const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
+                                            void* scores, void* context_bits, const void* zero_point, int context_type, void* stream)
+{
+    return attention("bgemm_attention_forward_bits", q, k, v, batch, seq, heads, head_size, scores, context_bits, zero_point, true, context_type, stream);
 }

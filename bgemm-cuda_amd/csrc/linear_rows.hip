@@ -1,0 +1,464 @@
+// Scaled binary Linear layers without a gradient in one launch, activations as they come: what tests/python/bgemm_linear.py:479-484 does
+// in a centring pass, a pack, a GEMM and three elementwise passes.
+//
+//   y_l[n,m] = half(sum_k sign(x - zp_l)[n,k] sign(w_l)[m,k]) * sw_l[m] * sa_l (+ bias_l[m])          for up to three layers l of one input
+//
+// stored as numbers, with a residual added or not, or as the next layer's operand, the sign bits of y - next zero point.
+#include "common.h"
+#include "mfma_engines.h"
+#include "pack_bits.h"
+#include <type_traits>
+
+namespace bgemm {
+
+struct RowsLayer { const uint32_t* W; const void* zp; const void* sw; const void* sa; const void* bias; const void* next_zp; void* out; };
+
+struct RowsArgs {
+    RowsLayer l[3];
+    const void* x; int64_t ld;        // unpacked rows (element stride), or one tiled operand of sign bits
+    const void* residual;             // [N][M], or null
+    int N, M, K, KT, MT, layers;
+    int groups, splits;               // column groups of a layer, blocks a row tile
+    int nt;                           // stores past the caches
+    int first_lds;                    // bytes of the first area
+    int gather;                       // bits of a whole row tile leave together: column tiles of the output, to the end of its last K-tile; else 0
+};
+
+enum { ROWS_BITS_F32 = 0, ROWS_BITS_F16 = 1, ROWS_F32 = 2, ROWS_F16 = 3 };
+enum { ROWS_SRC_PACKED = 0, ROWS_SRC_F32 = 1, ROWS_SRC_F16 = 2 };
+constexpr int ROWS_MAX_WAVES = 16;
+constexpr int ROWS_MAX_K = 2048;      // up to here a sum is exact in fp16, and the rounding to it that the layer does is none
+
+// fp4 operands whose products are -2 x where the weight's bit is set and 0 elsewhere, x = +-1, so that a sum that starts from the row's
+// sum of x is the layer's: sum x (1 - 2 b).  The weight's bit stays where it is (0.5, 1, 2; at step 3 it moves to 1.0), five vector
+// instructions a word; the activation is the sign over 2 / that value, from the inverted word.
+__device__ __forceinline__ unsigned rows_w(const unsigned w, const int s) { return s == 3 ? (w >> 2) & 0x22222222u : w & (0x11111111u << s); }
+__device__ __forceinline__ unsigned rows_x(const unsigned inverted, const int s)
+{
+    return ((inverted << (3 - s)) & 0x88888888u) | (s == 0 ? 0x66666666u : s == 2 ? 0x22222222u : 0x44444444u);
+}
+
+// A block owns one row tile of 32 activation rows.  Its waves turn them into sign bits in LDS, each layer's with that layer's zero
+// point, then into matrix-core operands there (once: every column tile needs them), and take groups of CT column tiles in turn,
+// whose weights come straight from the caches into registers, two K-tiles ahead.  The accumulators leave without a detour: a lane holds a
+// column of sixteen rows (numbers: a half-wave stores a whole line; fp16 in pairs of columns), or with the operands exchanged sixteen
+// columns of a row (bits: one instruction collects a sign, and whole 16-byte pieces of the output's tiles leave behind a barrier).
+// What bounds it: numbers on many rows the stores, 8192 x 768 x 3072 fp32 24.3 us in place of 34 in two launches (101 MB of stores and
+// 25 of reads, 5.2 TB/s; fp16 18.7 for 23.5); bits the vector units, half of them the scaling: three layers 8192 x 768 x 768 14 us
+// where three packs and three GEMMs took 46.7, each reading x and passing its outputs through LDS and a ballot a row; with a residual
+// and a packed operand 8192 x 768 x 768 8.4 for 24.3 with the addition as its own pass.  Few rows: the chain of one row tile, 64 x 512
+// x 512 4.5 for 7.6.
+template <int SRC, int KIND, int CT>
+__global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const RowsArgs a)
+{
+    constexpr bool BITS = KIND == ROWS_BITS_F32 || KIND == ROWS_BITS_F16, F32P = KIND == ROWS_BITS_F32 || KIND == ROWS_F32;
+    static_assert(KIND != ROWS_F16 || CT % 2 == 0, "fp16 outputs leave in pairs of columns of two tiles");
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int h = lane >> 5, c = lane & 31;
+    const unsigned id = xcd_contiguous_id(blockIdx.x, gridDim.x);
+    const int rt = id / a.splits, part = id % a.splits;
+    const int KT = a.KT, tiles_x = (SRC == ROWS_SRC_PACKED ? 1 : a.layers) * KT;
+    uint4* const raw_bits = reinterpret_cast<uint4*>(smem);                 // [layer][K-tile][64]
+    uint32_t* const words = reinterpret_cast<uint32_t*>(smem);              // BITS, in the same place later: [layer][column tile][row], tiles to the end of K-tiles
+    uint4* const operands = reinterpret_cast<uint4*>(smem + a.first_lds);   // [layer][K-tile][step][64]
+    float* const cols = reinterpret_cast<float*>(operands + tiles_x * 4 * TILE_U4);      // BITS: the columns' parameters, [layer][sw | bias][MT * 32]
+    [[maybe_unused]] float* const xsums = cols + wave * 32;                 // else: the wave's row sums
+    auto par = [](const void* p, const int64_t i) {
+        if constexpr (F32P) return reinterpret_cast<const float*>(p)[i];
+        else return __half2float(reinterpret_cast<const __half*>(p)[i]);
+    };
+
+    // ---- the rows' bits ----------------------------------------------------------------------------------------------------------
+    if constexpr (SRC == ROWS_SRC_PACKED) {
+        const uint4* const x = reinterpret_cast<const uint4*>(a.x) + (int64_t)rt * KT * TILE_U4;
+        for (int i = threadIdx.x; i < KT * TILE_U4; i += waves * 64) raw_bits[i] = x[i];
+    } else {
+        constexpr bool F32 = SRC == ROWS_SRC_F32;
+        typedef typename std::conditional<F32, uint32_t, uint16_t>::type E;
+        const int last_row = min(a.N - rt * 32, 32) - 1;
+        const E* const src = reinterpret_cast<const E*>(a.x) + (int64_t)rt * 32 * a.ld;
+        float zf[3] = {0.f, 0.f, 0.f};
+        for (int l = 0; l < a.layers; l++)
+            if (a.l[l].zp) zf[l] = F32 ? *reinterpret_cast<const float*>(a.l[l].zp) : __half2float(*reinterpret_cast<const __half*>(a.l[l].zp));
+        // a unit is two rows of a K-tile, a chunk of eight elements a lane; four of them requested at once
+        // (K >= 8: a row's last chunk is read as its last eight elements, and the bits shifted into place)
+        constexpr int AHEAD = 4;
+        for (int u0 = wave; u0 < 16 * KT; u0 += waves * AHEAD) {
+            Raw8<F32> raw[AHEAD];
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) {
+                const int u = min(u0 + i * waves, 16 * KT - 1), r = (u & 15) * 2 + h;
+                raw[i] = load_raw8<F32>(src + (int64_t)(r < last_row ? r : last_row) * a.ld, min((u >> 4) * TILE_KBITS + 8 * c, a.K - 8));
+            }
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) {
+                const int u = min(u0 + i * waves, 16 * KT - 1), kt = u >> 4;           // (the last unit twice or more: the same bits)
+                const int shift = min(max(kt * TILE_KBITS + 8 * c - (a.K - 8), 0), 8);
+                unsigned char* const at = smem + kt * 1024 + tile_byte_of_chunk(c) + 16 * ((u & 15) * 2 + h);
+                float f[8];
+                centre8<F32>(raw[i], 0.f, f);
+#pragma unroll
+                for (int l = 0; l < 3; l++) {
+                    if (l >= a.layers) break;
+                    uint32_t sg = 0;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) sg = __builtin_amdgcn_alignbit(sg, __float_as_uint(__fsub_rn(f[e], zf[l])), 31);
+                    at[l * KT * 1024] = (unsigned char)(sg << shift);
+                }
+            }
+        }
+    }
+    if constexpr (BITS) {
+        for (int l = 0; l < a.layers; l++)
+            for (int m = threadIdx.x; m < a.MT * 32; m += waves * 64) {
+                cols[(2 * l) * a.MT * 32 + m] = m < a.M ? par(a.l[l].sw, m) : 0.f;
+                cols[(2 * l + 1) * a.MT * 32 + m] = m < a.M && a.l[l].bias ? par(a.l[l].bias, m) : 0.f;
+            }
+    }
+    __syncthreads();
+    // a wave works for one layer; the sum of its x of row c
+    const int per_layer = waves / a.layers, l = wave / per_layer, wl = wave - l * per_layer, lx = SRC == ROWS_SRC_PACKED ? 0 : l;
+    int ones = 0;
+#pragma unroll 1
+    for (int t = 0; t < KT; t++) ones += popc4(raw_bits[(lx * KT + t) * TILE_U4 + lane]);
+    ones += __shfl_xor(ones, 32);
+    const float xsum = (float)(a.K - 2 * ones);
+    for (int i = wave; i < tiles_x; i += waves) {
+        const uint4 x = raw_bits[i * TILE_U4 + lane];
+#pragma unroll
+        for (int s = 0; s < 4; s++) operands[(i * 4 + s) * TILE_U4 + lane] = make_uint4(rows_x(~x.x, s), rows_x(~x.y, s), rows_x(~x.z, s), rows_x(~x.w, s));
+    }
+    __syncthreads();
+
+    // ---- the products --------------------------------------------------------------------------------------------------------------
+    const RowsLayer& L = a.l[l];
+    const int stride = a.splits * per_layer;
+    int gg = part * per_layer + wl, kt = 0, rg = gg, rkt = 0;         // the group that is multiplied, and the one whose weights are requested next
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(L.W), 0, a.MT * KT * 1024, 0x00020000);
+    const float sa = par(L.sa, 0), next = BITS && L.next_zp ? par(L.next_zp, 0) : 0.f;
+    const bool has_bias = L.bias != nullptr, has_next = L.next_zp != nullptr;
+    // which weight row a lane multiplies: bits: MFMA row 8 q + 4 half + i is column 16 half + 4 q + i, so that a lane ends up with 16
+    // neighbouring columns of its row; fp16: the even rows of a pair of tiles, then the odd ones; else the lane's own
+    const int own = BITS ? 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3) : c;
+    auto request = [&](v4i (&w)[CT]) {
+        const int mt0 = rg * CT;
+#pragma unroll
+        for (int j = 0; j < CT; j++) {
+            if constexpr (KIND == ROWS_F16) {
+                const int r = 2 * c + (j & 1), mt = min(mt0 + (j & ~1) + (r >> 5), a.MT - 1);
+                w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, mt * KT * 1024 + h * 512 + (r & 31) * 16, rkt * 1024, 0);
+            } else
+                w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, h * 512 + own * 16, (min(mt0 + j, a.MT - 1) * KT + rkt) * 1024, 0);
+        }
+        if (++rkt == KT) {
+            rkt = 0;
+            rg += stride;                                             // (past the last one: the last tile again, nobody multiplies it)
+        }
+    };
+    // the sums of x that the accumulators start from: BITS: the lane's row's, else those of its sixteen rows
+    v16f acc[CT], start;
+    if constexpr (BITS) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) start[v] = xsum;
+    } else {
+        xsums[c] = xsum;                        // (both halves the same; the wave's own, LDS keeps its order)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 s = *reinterpret_cast<const float4*>(xsums + 8 * q + 4 * h);
+            start[4 * q] = s.x; start[4 * q + 1] = s.y; start[4 * q + 2] = s.z; start[4 * q + 3] = s.w;
+        }
+    }
+    // numbers leave, and a residual comes, through buffers that end with the last row: what lies past it is dropped (and read as 0)
+    constexpr int ESZ = F32P ? 4 : 2;
+    const int row_b = a.M * ESZ, rows_b = min(a.N - rt * 32, 32) * row_b;
+    auto rows_of = [&](const void* p) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p)) + (int64_t)rt * 32 * row_b, 0, rows_b, 0x00020000);
+    };
+    auto store_group = [&] {
+        const int mt0 = gg * CT;
+        if constexpr (BITS) {
+            const int n = rt * 32 + c;
+#pragma unroll
+            for (int j = 0; j < CT; j++) {
+                const int mt = mt0 + j;
+                if (mt >= a.MT) break;
+                const float* const ps = cols + (2 * l) * a.MT * 32 + mt * 32 + 16 * h;
+                const float* const pb = ps + a.MT * 32;
+                unsigned bits = 0;
+                auto collect = [&](auto bias_c, auto next_c) {
+                    constexpr bool BIAS = decltype(bias_c)::value, NEXT = decltype(next_c)::value;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const float4 s4 = *reinterpret_cast<const float4*>(ps + 4 * q), b4 = BIAS ? *reinterpret_cast<const float4*>(pb + 4 * q) : float4{};
+                        const float s[4] = {s4.x, s4.y, s4.z, s4.w}, b[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+#pragma clang fp contract(off)      // every step rounds by itself, as torch's separate kernels do
+                            float y;
+                            if constexpr (F32P) {
+                                y = acc[j][4 * q + e] * s[e];
+                                y = y * sa;
+                                if (BIAS) y = y + b[e];
+                            } else {
+                                _Float16 r = (_Float16)acc[j][4 * q + e] * (_Float16)s[e];
+                                r = r * (_Float16)sa;
+                                if (BIAS) r = r + (_Float16)b[e];
+                                y = (float)r;
+                            }
+                            bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(NEXT ? y - next : y), 31);
+                        }
+                    }
+                };
+                if (!has_bias) collect(std::false_type{}, std::true_type{});
+                else if (has_next) collect(std::true_type{}, std::true_type{});
+                else collect(std::true_type{}, std::false_type{});
+                const unsigned other = __shfl_xor(bits, 32);
+                unsigned word = bits << 16 | other;
+                if ((mt + 1) * 32 > a.M) word &= 0xffffffffu << ((mt + 1) * 32 - a.M);
+                if (a.gather) {
+                    if (h == 0) words[(l * a.gather + mt) * 32 + c] = word;
+                } else if (h == 0 && n < a.N) reinterpret_cast<uint32_t*>(L.out)[tiled_word_offset(n, mt, k_tiles(a.M))] = word;
+            }
+        } else if constexpr (KIND == ROWS_F32) {
+            const __amdgpu_buffer_rsrc_t ro = rows_of(L.out), rr = rows_of(a.residual);
+#pragma unroll
+            for (int j = 0; j < CT; j++) {
+                const int mt = mt0 + j, m = mt * 32 + c;
+                if (mt >= a.MT) break;
+                const int mc = m < a.M ? m : a.M - 1, voff = m < a.M ? 4 * h * row_b + m * 4 : 0x7ffffff0;
+                const float s = par(L.sw, mc), b = has_bias ? par(L.bias, mc) : 0.f;
+                float y[16], res[16];
+                if (a.residual)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) res[v] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rr, voff, (8 * (v >> 2) + (v & 3)) * row_b, 0));
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+#pragma clang fp contract(off)      // every step rounds by itself, as torch's separate kernels do
+                    y[v] = acc[j][v] * s;
+                    y[v] = y[v] * sa;
+                }
+                if (has_bias)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) y[v] = __fadd_rn(y[v], b);
+                if (a.residual)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) y[v] = __fadd_rn(y[v], res[v]);
+                if (a.nt) {
+#pragma unroll
+                    for (int v = 0; v < 16; v++) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[v]), ro, voff, (8 * (v >> 2) + (v & 3)) * row_b, 2);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 16; v++) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[v]), ro, voff, (8 * (v >> 2) + (v & 3)) * row_b, 0);
+                }
+            }
+        } else {
+            const __amdgpu_buffer_rsrc_t ro = rows_of(L.out), rr = rows_of(a.residual);
+            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+            for (int p = 0; p < CT / 2; p++) {
+                const int mt = mt0 + 2 * p, m = mt * 32 + 2 * c;
+                if (mt >= a.MT) break;
+                // (the last column of an odd number stands alone)
+                const bool pair = m + 1 < a.M, single = m + 1 == a.M;
+                const int voff = pair ? 4 * h * row_b + m * 2 : 0x7ffffff0, voff1 = single ? 4 * h * row_b + m * 2 : 0x7ffffff0;
+                h2 s = {(_Float16)0.f, (_Float16)0.f}, b = s;
+                if (pair || single) {
+                    s[0] = reinterpret_cast<const _Float16*>(L.sw)[m];
+                    s[1] = reinterpret_cast<const _Float16*>(L.sw)[pair ? m + 1 : m];
+                    if (has_bias) {
+                        b[0] = reinterpret_cast<const _Float16*>(L.bias)[m];
+                        b[1] = reinterpret_cast<const _Float16*>(L.bias)[pair ? m + 1 : m];
+                    }
+                }
+                const h2 sah = {(_Float16)sa, (_Float16)sa};
+                h2 y[16];
+                unsigned res[16];
+                if (a.residual)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+                        const int o = (8 * (v >> 2) + (v & 3)) * row_b;
+                        res[v] = __builtin_amdgcn_raw_buffer_load_b32(rr, voff, o, 0);
+                        if (a.M & 1) res[v] |= __builtin_amdgcn_raw_buffer_load_b16(rr, voff1, o, 0);
+                    }
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+#pragma clang fp contract(off)
+                    y[v][0] = (_Float16)acc[2 * p][v];
+                    y[v][1] = (_Float16)acc[2 * p + 1][v];
+                    y[v] = y[v] * s;
+                    y[v] = y[v] * sah;
+                }
+                if (has_bias)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+#pragma clang fp contract(off)
+                        y[v] = y[v] + b;
+                    }
+                if (a.residual)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+#pragma clang fp contract(off)
+                        y[v] = y[v] + __builtin_bit_cast(h2, res[v]);
+                    }
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const int o = (8 * (v >> 2) + (v & 3)) * row_b;
+                    const unsigned u = __builtin_bit_cast(unsigned, y[v]);
+                    __builtin_amdgcn_raw_buffer_store_b32(u, ro, voff, o, 0);
+                    if (a.M & 1) __builtin_amdgcn_raw_buffer_store_b16((unsigned short)u, ro, voff1, o, 0);
+                }
+            }
+        }
+    };
+    auto step = [&](const v4i (&w)[CT]) {
+        const uint4* const op = operands + (lx * KT + kt) * 4 * TILE_U4 + lane;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const uint4 x = op[s * TILE_U4];
+            const unsigned fx[4] = {x.x, x.y, x.z, x.w};
+            unsigned fw[CT][4];
+#pragma unroll
+            for (int j = 0; j < CT; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) fw[j][q] = rows_w((unsigned)w[j][q], s);
+            auto multiply = [&](auto first_c) {
+#pragma unroll
+                for (int j = 0; j < CT; j++) {
+                    const v16f& from = decltype(first_c)::value ? start : acc[j];
+                    if constexpr (BITS) acc[j] = EngF4::mma(EngF4::make(fw[j]), EngF4::make(fx), from);
+                    else acc[j] = EngF4::mma(EngF4::make(fx), EngF4::make(fw[j]), from);
+                }
+            };
+            if (s == 0 && kt == 0) multiply(std::true_type{});
+            else multiply(std::false_type{});
+        }
+        if (++kt == KT) {
+            store_group();
+            kt = 0;
+            gg += stride;
+        }
+    };
+    if (gg < a.groups) {
+        v4i w0[CT], w1[CT], w2[CT];
+        request(w0);
+        request(w1);
+        for (;;) {
+            request(w2);
+            step(w0);
+            if (gg >= a.groups) break;
+            request(w0);
+            step(w1);
+            if (gg >= a.groups) break;
+            request(w1);
+            step(w2);
+            if (gg >= a.groups) break;
+        }
+    }
+    if (BITS && a.gather) {
+        // whole tiles of the output, their padding of zeros included
+        for (int i = threadIdx.x; i < a.layers * (a.gather - a.MT) * 32; i += waves * 64) words[(i / ((a.gather - a.MT) * 32) * a.gather + a.MT) * 32 + i % ((a.gather - a.MT) * 32)] = 0u;
+        __syncthreads();
+        for (int i = threadIdx.x; i < a.layers * a.gather * 8; i += waves * 64) {
+            const int l = i / (a.gather * 8), j = i - l * a.gather * 8, r = j & 31, q4 = j >> 5;      // words 4 q4 .. of row r
+            const uint32_t* const from = words + (l * a.gather + 4 * q4) * 32 + r;
+            if (rt * 32 + r < a.N)
+                *reinterpret_cast<uint4*>(reinterpret_cast<uint32_t*>(a.l[l].out) + ((int64_t)rt * (a.gather / 8) * TILE_U4 + j) * 4) = make_uint4(from[0], from[32], from[64], from[96]);
+        }
+    }
+}
+
+// What a block keeps in LDS: the rows' bits, later those of the output, and operands for every layer, and where bits leave the columns' parameters.
+static int64_t rows_first_lds(int64_t M, int64_t K, int planes, int layers, bool bits)
+{
+    const int64_t in = planes * k_tiles(K) * 1024, out = bits ? layers * k_tiles(M) * 1024 : 0;
+    return in > out ? in : out;
+}
+static int64_t rows_lds(int64_t M, int64_t K, int planes, int layers, bool bits)
+{
+    return rows_first_lds(M, K, planes, layers, bits) + planes * k_tiles(K) * 4096 + (bits ? layers * row_tiles(M) * 32 * 8 : ROWS_MAX_WAVES * 128);
+}
+
+}  // namespace bgemm
+
+using namespace bgemm;
+
+extern "C" int bgemm_linear_rows_supported(int64_t N, int64_t M, int64_t K, int layers, int out_dtype)
+{
+    const bool bits = out_dtype == BGEMM_OUT_BITS_F32 || out_dtype == BGEMM_OUT_BITS_F16;
+    if (!bits && out_dtype != BGEMM_OUT_F32_SCALED && out_dtype != BGEMM_OUT_F16_SCALED) return 0;
+    return N >= 1 && N <= (1 << 24) && M >= 1 && M <= (1 << 16) && K >= 8 && K <= ROWS_MAX_K && layers >= 1 && layers <= 3 &&
+           rows_lds(M, K, layers, layers, bits) <= (64 << 10);
+}
+
+extern "C" int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx, int64_t N, int64_t M, int64_t K, int layers,
+                                         const bgemm_rows_layer* layer, int out_dtype, const void* residual, int shape, void* stream)
+{
+    const char* who = "bgemm_linear_rows_forward";
+    const bool bits = out_dtype == BGEMM_OUT_BITS_F32 || out_dtype == BGEMM_OUT_BITS_F16;
+    const bool f32 = out_dtype == BGEMM_OUT_BITS_F32 || out_dtype == BGEMM_OUT_F32_SCALED, packed = x_dtype == BGEMM_SRC_BITS;
+    if (!bgemm_linear_rows_supported(N, M, K, layers, out_dtype))
+        return fail(BGEMM_EINVAL, "%s: N=%lld M=%lld K=%lld, %d layers, output %d", who, (long long)N, (long long)M, (long long)K, layers, out_dtype);
+    if (!packed && x_dtype != (f32 ? BGEMM_SRC_F32 : BGEMM_SRC_F16)) return fail(BGEMM_EINVAL, "%s: activations of type %d for that output", who, x_dtype);
+    if (!packed && ldx < K) return fail(BGEMM_EINVAL, "%s: row stride %lld < K", who, (long long)ldx);
+    if (residual && bits) return fail(BGEMM_EINVAL, "%s: a residual is added to numbers", who);
+    if (shape && (shape < 0 || (shape & 15) < 1 || (shape & 15) > 2 || (shape >> 4 & 31) < 1 || (shape >> 4 & 31) * layers > ROWS_MAX_WAVES || shape >> 22))
+        return fail(BGEMM_EINVAL, "%s: launch shape %d", who, shape);
+    if (!x || !layer) return fail(BGEMM_ENULL, "%s: null pointer", who);
+    const unsigned odd = f32 ? 3 : 1;
+    if (((uintptr_t)x & (packed ? 15 : odd)) || ((uintptr_t)residual & odd)) return fail(BGEMM_EALIGN, "%s: an operand is not aligned", who);
+    RowsArgs a = {};
+    for (int l = 0; l < layers; l++) {
+        const bgemm_rows_layer& s = layer[l];
+        if (!s.W_tiled || !s.sw || !s.sa || !s.out) return fail(BGEMM_ENULL, "%s: layer %d: null pointer", who, l);
+        if (((uintptr_t)s.W_tiled & 15) || ((uintptr_t)s.out & (bits ? 15 : odd)) || (((uintptr_t)s.sw | (uintptr_t)s.sa | (uintptr_t)s.bias | (uintptr_t)s.zero_point | (uintptr_t)s.next_zero_point) & odd))
+            return fail(BGEMM_EALIGN, "%s: layer %d: an operand is not aligned", who, l);
+        a.l[l] = {(const uint32_t*)s.W_tiled, packed ? nullptr : s.zero_point, s.sw, s.sa, s.bias, bits ? s.next_zero_point : nullptr, s.out};
+    }
+    a.x = x; a.ld = ldx; a.residual = residual;
+    a.N = (int)N; a.M = (int)M; a.K = (int)K; a.KT = (int)k_tiles(K); a.MT = (int)row_tiles(M); a.layers = layers;
+    const int64_t rt = row_tiles(N);
+    // How many column tiles a wave multiplies at once, how many waves a layer has in a block, how many blocks share a row tile: one block
+    // a compute unit at most, since each of those that share makes the rows' bits again (8192 x 768 x (3 x 768) bits: 20 us with two a
+    // unit, 14 with one), and as many waves as give each a tile or two (us, 4 / 8 / 16 waves: fp32 8192 x 768 x 3072 35.3 / 26.9 / 24.4,
+    // 2048 x 1024 x 1024 7.3 / 6.2 / 7.2, 128 x 768 x 3072 5.3 / 5.5 / 6.6).  Two tiles at once share an operand's reads from LDS: bits from
+    // sixteen tiles a compute unit on (8192 x 768 x (3 x 768) 15.3 -> 14.4, but 100 rows 7.2 -> 8.1); fp16 numbers leave in pairs of them.
+    const int64_t tiles = rt * a.MT;
+    const bool f16_numbers = out_dtype == BGEMM_OUT_F16_SCALED;
+    const int ct = f16_numbers ? 2 : shape ? shape & 15 : bits && layers * tiles >= 4096 ? 2 : 1;
+    a.groups = (int)cdiv(a.MT, ct);
+    int64_t per_layer = cdiv(cdiv(rt * a.groups, 256), 4) * 4;
+    const int64_t most = layers == 3 ? 4 : ROWS_MAX_WAVES / layers, least = f16_numbers && layers == 1 ? 8 : 4;
+    per_layer = shape ? shape >> 4 & 31 : per_layer < least ? least : per_layer > most ? most : per_layer;
+    int64_t splits = cdiv(a.groups, per_layer);
+    while (splits > 1 && rt * splits > 256) splits--;
+    if (shape >> 12) splits = shape >> 12;
+    const int64_t waves = layers * per_layer;
+    a.splits = (int)splits;
+    a.first_lds = (int)rows_first_lds(M, K, packed ? 1 : layers, layers, bits);
+    a.gather = bits && splits == 1 ? (int)k_tiles(M) * 8 : 0;
+    a.nt = N * M * 4 <= (32LL << 20);
+    const size_t lds = (size_t)rows_lds(M, K, packed ? 1 : layers, layers, bits);
+    const dim3 grid((unsigned)(rt * splits)), block((unsigned)(waves * 64));
+    const hipStream_t st = (hipStream_t)stream;
+    auto go = [&](auto src, auto kind) {
+        constexpr int SRC = decltype(src)::value, KIND = decltype(kind)::value;
+        if constexpr (KIND != ROWS_F16) {
+            if (ct == 1) hipLaunchKernelGGL((linear_rows_kernel<SRC, KIND, 1>), grid, block, lds, st, a);
+        }
+        if (ct == 2) hipLaunchKernelGGL((linear_rows_kernel<SRC, KIND, 2>), grid, block, lds, st, a);
+    };
+    auto kinds = [&](auto src32, auto src16) {
+        if (out_dtype == BGEMM_OUT_BITS_F32) go(src32, std::integral_constant<int, ROWS_BITS_F32>{});
+        else if (out_dtype == BGEMM_OUT_BITS_F16) go(src16, std::integral_constant<int, ROWS_BITS_F16>{});
+        else if (out_dtype == BGEMM_OUT_F32_SCALED) go(src32, std::integral_constant<int, ROWS_F32>{});
+        else go(src16, std::integral_constant<int, ROWS_F16>{});
+    };
+    typedef std::integral_constant<int, ROWS_SRC_PACKED> P;
+    if (packed) kinds(P{}, P{});
+    else kinds(std::integral_constant<int, ROWS_SRC_F32>{}, std::integral_constant<int, ROWS_SRC_F16>{});
+    return check_launch(who);
+}

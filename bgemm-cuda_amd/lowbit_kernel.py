@@ -19,7 +19,7 @@ import torch
 
 import _lib as _b
 from _lib import (MODE_AND, MODE_XOR, MODE_ATTN, MODE_BWTA, MODE_ATTN_X, OUT_I32, OUT_F16, OUT_F32_SCALED,
-                  OUT_F16_SCALED, OUT_BITS_F32, OUT_BITS_F16, SRC_F16, SRC_F32, VARIANT_AUTO, VARIANT_VALU, VARIANT_MFMA, VARIANT_MFMA_F4)
+                  OUT_F16_SCALED, OUT_BITS_F32, OUT_BITS_F16, SRC_F16, SRC_F32, SRC_BITS, VARIANT_AUTO, VARIANT_VALU, VARIANT_MFMA, VARIANT_MFMA_F4)
 
 AND_POP, XOR_POP, ATTN_MM = 0, 1, 2   # lowbit_kernel/csrc/include/configs.h:70-72
 
@@ -382,11 +382,12 @@ def attention_supported(batch, seq, heads, head_size):
     return bool(_b.lib().bgemm_attention_supported(batch, seq, heads, head_size))
 
 
-def attention_forward(q, k, v, batch, heads, dtype):
+def attention_forward(q, k, v, batch, heads, dtype, zero_point=None):
     """Binary self-attention on packed operands (bert.py:245-259), one launch.  ``q``, ``k``, ``v``: sign bits of ``batch * seq`` rows
     and ``heads * head_size`` columns.  Returns the scores ``half(q . k) / sqrt(head_size)``, fp16 ``[batch, heads, seq, seq]``, and
     the context in ``dtype``, ``[batch, seq, heads * head_size]``: the sum of sign(v) over the keys whose probability (softmax in
-    fp16 storage) is at least ``1 / seq``."""
+    fp16 storage) is at least ``1 / seq``.  With ``zero_point`` (a one-element tensor of ``dtype``) the context is not stored: its sign
+    bits after centring are returned, the operand of the binary layer behind it."""
     rows, hidden = q.rows, q.K
     for name, p in (("q", q), ("k", k), ("v", v)):
         if p.ternary or p.batch != 1 or (p.rows, p.K) != (rows, hidden):
@@ -399,13 +400,90 @@ def attention_forward(q, k, v, batch, heads, dtype):
     if dtype not in (torch.float32, torch.half):
         raise TypeError("dtype must be torch.float32 or torch.half")
     seq, dev = rows // batch, q.data.device
+    src = SRC_F32 if dtype == torch.float32 else SRC_F16
     scores = torch.empty((batch, heads, seq, seq), dtype=torch.half, device=dev)
+    if zero_point is not None:
+        _check_scalar(zero_point, "zero_point", dtype, dev)
+        bits = empty_packed(rows, hidden, dev)
+        with _on(dev):
+            _b.check(_b.lib().bgemm_attention_forward_bits(q.data.data_ptr(), k.data.data_ptr(), v.data.data_ptr(), batch, seq, heads, hidden // heads,
+                                                           scores.data_ptr(), bits.data.data_ptr(), zero_point.data_ptr(), src, _stream()))
+        return scores, bits
     context = torch.empty((batch, seq, hidden), dtype=dtype, device=dev)
     with _on(dev):
         _b.check(_b.lib().bgemm_attention_forward(q.data.data_ptr(), k.data.data_ptr(), v.data.data_ptr(), batch, seq, heads, hidden // heads,
-                                                  scores.data_ptr(), context.data_ptr(), SRC_F32 if dtype == torch.float32 else SRC_F16,
-                                                  _stream()))
+                                                  scores.data_ptr(), context.data_ptr(), src, _stream()))
     return scores, context
+
+
+def _check_scalar(t, name, dtype, device):
+    if not isinstance(t, torch.Tensor) or t.numel() != 1 or t.dtype != dtype or t.device != device:
+        raise ValueError("%s must be a one-element %s tensor on %s" % (name, dtype, device))
+
+
+_rows_shapes = {}         # (N, M, K, layers, output kind) -> does bgemm_linear_rows_forward take it
+
+
+def linear_rows_supported(N, M, K, layers, kind):
+    ok = _rows_shapes.get((N, M, K, layers, kind))
+    if ok is None:
+        if len(_rows_shapes) > 4096:
+            _rows_shapes.clear()
+        ok = _rows_shapes[(N, M, K, layers, kind)] = bool(_b.lib().bgemm_linear_rows_supported(N, M, K, layers, kind))
+    return ok
+
+
+def linear_rows_forward(x, layers, bits=False, residual=None, shape=0):
+    """Up to three scaled binary layers of one input and one size in ONE launch, packing included (bgemm_linear.py:479-484 without a
+    gradient).  ``x``: fp16 or fp32 ``[N, K]`` with dense rows, or a binary PackedBits that is centred already; ``layers``: a list of
+    ``(w, zero_point, sw, sa, bias)``, ``w`` a binary PackedBits of M x K bits, the others tensors of one type (``x``'s where that is a
+    tensor), ``zero_point`` and ``bias`` or None.  Returns a list: each layer's ``half(acc) * sw * sa (+ bias)``, ``[N, M]``, plus
+    ``residual`` if there is one, or with ``bits`` those outputs' sign bits, as ``bgemm_packed_forward(bits_out=)`` leaves them."""
+    packed = isinstance(x, PackedBits)
+    w0, dt = layers[0][0], layers[0][2].dtype
+    M, K, dev = w0.rows, w0.K, w0.data.device
+    if dt not in (torch.float32, torch.half):
+        raise TypeError("scales must be fp32 or fp16")
+    if packed:
+        _check_packed(x, "x")
+        if x.ternary or x.batch != 1 or x.K != K or x.data.device != dev:
+            raise ValueError("x must be one binary operand of K = %d on %s" % (K, dev))
+        N = x.rows
+    else:
+        _need_cuda(x, "x")
+        if x.dim() != 2 or x.shape[1] != K or x.dtype != dt or x.device != dev:
+            raise ValueError("x must be a %s tensor [N, %d] on %s" % (dt, K, dev))
+        N = x.shape[0]
+        if x.stride(1) != 1 or x.stride(0) < K:
+            x = x.contiguous()
+    f32 = dt == torch.float32
+    kind = (OUT_BITS_F32 if f32 else OUT_BITS_F16) if bits else OUT_F32_SCALED if f32 else OUT_F16_SCALED
+    if residual is not None and (bits or residual.dtype != dt or tuple(residual.shape) != (N, M) or not residual.is_contiguous() or residual.device != dev):
+        raise ValueError("residual must be a contiguous %s tensor [%d, %d] on %s, beside outputs that are numbers" % (dt, N, M, dev))
+    arr, outs = (_b.RowsLayer * len(layers))(), []
+    for a, (w, zp, sw, sa, bias) in zip(arr, layers):
+        if w.ternary or w.batch != 1 or (w.rows, w.K) != (M, K):
+            raise ValueError("every weight must be one binary matrix of %d x %d" % (M, K))
+        _check_packed(w, "w")
+        for name, t, n in (("sw", sw, M), ("sa", sa, 1), ("bias", bias, M), ("zero_point", zp, 1)):
+            if t is None and name in ("bias", "zero_point"):
+                continue
+            if t.dtype != dt or t.numel() != n or not t.is_contiguous() or t.device != dev:
+                raise ValueError("%s must be a contiguous %s tensor of %d elements on %s" % (name, dt, n, dev))
+        if w.data.device != dev:
+            raise ValueError("every weight must be on %s" % dev)
+        out = empty_packed(N, M, dev) if bits else torch.empty((N, M), dtype=dt, device=dev)
+        outs.append(out)
+        a.W_tiled, a.sw, a.sa, a.out = w.data.data_ptr(), sw.data_ptr(), sa.data_ptr(), (out.data if bits else out).data_ptr()
+        if zp is not None:
+            a.zero_point = zp.data_ptr()
+        if bias is not None:
+            a.bias = bias.data_ptr()
+    with _on(dev):
+        _b.check(_b.lib().bgemm_linear_rows_forward((x.data if packed else x).data_ptr(), SRC_BITS if packed else SRC_F32 if f32 else SRC_F16,
+                                                    0 if packed else max(x.stride(0), K), N, M, K, len(layers), arr, kind,
+                                                    None if residual is None else residual.data_ptr(), shape, _stream()))
+    return outs
 
 
 def _head_view(t):

@@ -43,7 +43,7 @@ enum { BGEMM_OUT_I32 = 0, BGEMM_OUT_F16 = 1, BGEMM_OUT_F32_SCALED = 2, BGEMM_OUT
         * (see bgemm_packed_forward_bits); parameters fp32 resp. fp16 */
        BGEMM_OUT_BITS_F32 = 4, BGEMM_OUT_BITS_F16 = 5 };
 /* Element type of a floating-point source operand. */
-enum { BGEMM_SRC_F16 = 0, BGEMM_SRC_F32 = 1 };
+enum { BGEMM_SRC_F16 = 0, BGEMM_SRC_F32 = 1, BGEMM_SRC_BITS = 2 /* sign bits, tiled: bgemm_linear_rows_forward only */ };
 /* Kernel family: AUTO picks per shape; VALU = and + popcount on the vector ALU;
  * MFMA = bit planes expanded to int8 in registers feeding v_mfma_i32_32x32x32_i8;
  * MFMA_F4 = bit planes expanded to E2M1 nibbles feeding v_mfma_f32_32x32x64_f8f6f4
@@ -320,6 +320,28 @@ int bgemm_elastic_backward(const void* x_sign, const void* x_nonzero, const void
                            const void* xs, const void* ws, float grad_scale, int64_t N, int64_t M, int64_t K, void* grad_x, void* grad_w,
                            void* grad_bias, void* grad_sw, void* grad_sa, void* work, size_t work_bytes, void* stream);
 
+/* ---- scaled binary Linear layers on activations as they come, one launch ---------------------------
+ * (tests/python/bgemm_linear.py:479-484 without a gradient.)  Up to three layers of one input and of one size: x [N][K] rows ldx elements
+ * apart in the parameters' type (BGEMM_SRC_F32 with BGEMM_OUT_F32_SCALED / BGEMM_OUT_BITS_F32, BGEMM_SRC_F16 with the fp16 kinds), centred
+ * by each layer's own zero point (NULL: 0), or BGEMM_SRC_BITS: one tiled operand of centred sign bits, the padding of K zero.
+ *   y = half(acc) * sw * sa (+ bias), every step rounded as bgemm_packed_forward_scaled does it
+ *   scaled kinds: out [N][M] = y, or y + residual (residual [N][M] of the output's type)
+ *   bits kinds:   out = the sign bits of half(y - *next_zero_point) (NULL: 0), tiled; its padding is not written
+ * Supported: 8 <= K <= 2048, M <= 65536, N <= 2^24, the rows' bits (and with bits out the parameters) within 64 KiB of LDS.
+ * tiles: column tiles a wave multiplies at once, 0 = chosen by size (1 to 3: tests). */
+typedef struct bgemm_rows_layer {
+    const void* W_tiled;
+    const void* zero_point;
+    const void* sw;
+    const void* sa;
+    const void* bias;
+    const void* next_zero_point;
+    void* out;
+} bgemm_rows_layer;
+int bgemm_linear_rows_supported(int64_t N, int64_t M, int64_t K, int layers, int out_dtype);
+int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx, int64_t N, int64_t M, int64_t K, int layers,
+                              const bgemm_rows_layer* layer, int out_dtype, const void* residual, int shape, void* stream);
+
 /* ---- binary self-attention without a gradient, one launch -----------------------------------------
  * (tests/python/bert/bert.py:245-259 on sign bits.)  q, k, v: sign bits [batch * seq][heads * head_size], tiled, 16-byte aligned.
  *   scores  [batch][heads][seq][seq] fp16 = half(half(sign(q) . sign(k)) / sqrt(head_size))
@@ -329,6 +351,10 @@ int bgemm_elastic_backward(const void* x_sign, const void* x_nonzero, const void
 int bgemm_attention_supported(int64_t batch, int64_t seq, int64_t heads, int64_t head_size);
 int bgemm_attention_forward(const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
                             void* scores, void* context, int context_type, void* stream);
+/* The same with the context as the next binary layer's operand: the sign bits of context - *zero_point (of context_type; NULL: 0),
+ * [batch * seq][heads * head_size], tiled, 16-byte aligned, the padding of its columns zero. */
+int bgemm_attention_forward_bits(const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
+                                 void* scores, void* context_bits, const void* zero_point, int context_type, void* stream);
 
 /* ---- gradients of both attention products, one launch each ----------------------------------------
  * (tests/python/bgemm_linear.py:28-42, 64-86 on `batch` matrices, `inner` to an outer one.)  fp16 throughout, sums in fp32; sign(0) = 0.
