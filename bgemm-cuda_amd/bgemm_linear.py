@@ -485,7 +485,7 @@ class BGEMMChain(nn.Sequential):
     """BGEMMLinear layers applied back to back (the binarisation is the only nonlinearity between them).
     When no gradient is recorded the activations between layers exist only as bits: every GEMM but the last
     writes the next layer's centred, sign-packed operand straight from its accumulators, so a chain of L
-    layers is L + 1 launches and never stores a hidden activation.  Same results as calling the layers one
+    layers is L launches (L + 1 on a long input) and never stores a hidden activation.  Same results as calling the layers one
     after the other, bit for bit.  Not in the reference, which has no layer container."""
 
     def _fusable(self, x):
@@ -499,7 +499,10 @@ class BGEMMChain(nn.Sequential):
             return super().forward(x)          # also the first call, which initialises the layers' scales
         layers = list(self)
         lead = x.shape[:-1]
-        xp = lowbit_kernel.pack_sign(x.reshape(-1, x.shape[-1]), zero_point=layers[0].zpa)
+        x2 = x.reshape(-1, x.shape[-1])
+        kind = lowbit_kernel.OUT_BITS_F32 if x.dtype == torch.float32 else lowbit_kernel.OUT_BITS_F16
+        one_launch = len(layers) > 1 and lowbit_kernel.linear_rows_supported(x2.shape[0], *layers[0].weight.shape, 1, kind) == 2
+        xp = None if one_launch else lowbit_kernel.pack_sign(x2, zero_point=layers[0].zpa)
         if not hasattr(self, "_bits"):
             self._bits = {}
         for i, layer in enumerate(layers):
@@ -507,12 +510,16 @@ class BGEMMChain(nn.Sequential):
             if i + 1 == len(layers):
                 out = lowbit_kernel.bgemm_packed_forward(layer._packed_weight(), xp, lowbit_kernel.MODE_XOR, splitK=8, scale=scale)
                 return out.reshape(*lead, layer.weight.shape[0])
-            key = (i, xp.rows, x.device)
+            key = (i, x2.shape[0], x.device)
             if key not in self._bits:      # zero-filled once: the GEMM writes real bits only, the padding stays zero
-                self._bits[key] = lowbit_kernel.zeros_packed(xp.rows, layer.weight.shape[0], 1, x.device)
-            xp = lowbit_kernel.bgemm_packed_forward(layer._packed_weight(), xp, lowbit_kernel.MODE_XOR, splitK=8, scale=scale,
-                                                    bits_out=self._bits[key],
-                                                    next_zero_point=layers[i + 1].zpa.detach().reshape(1))
+                self._bits[key] = lowbit_kernel.zeros_packed(x2.shape[0], layer.weight.shape[0], 1, x.device)
+            next_zero_point = layers[i + 1].zpa.detach().reshape(1)
+            if xp is None:                 # the first layer packs its input itself
+                xp, = lowbit_kernel.linear_rows_forward(x2, [(layer._packed_weight(), layer.zpa.detach().to(x.dtype).reshape(1), *scale)], bits=True,
+                                                        next_zero_point=next_zero_point, bits_out=[self._bits[key]])
+            else:
+                xp = lowbit_kernel.bgemm_packed_forward(layer._packed_weight(), xp, lowbit_kernel.MODE_XOR, splitK=8, scale=scale,
+                                                        bits_out=self._bits[key], next_zero_point=next_zero_point)
 
 
 class GraphedInference:

@@ -308,7 +308,8 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
                 for (int v = 0; v < 16; v++) {
                     const int o = (8 * (v >> 2) + (v & 3)) * row_b;
                     const unsigned u = __builtin_bit_cast(unsigned, y[v]);
-                    __builtin_amdgcn_raw_buffer_store_b32(u, ro, voff, o, 0);
+                    if (a.nt) __builtin_amdgcn_raw_buffer_store_b32(u, ro, voff, o, 2);
+                    else __builtin_amdgcn_raw_buffer_store_b32(u, ro, voff, o, 0);
                     if (a.M & 1) __builtin_amdgcn_raw_buffer_store_b16((unsigned short)u, ro, voff1, o, 0);
                 }
             }
@@ -390,8 +391,16 @@ extern "C" int bgemm_linear_rows_supported(int64_t N, int64_t M, int64_t K, int 
 {
     const bool bits = out_dtype == BGEMM_OUT_BITS_F32 || out_dtype == BGEMM_OUT_BITS_F16;
     if (!bits && out_dtype != BGEMM_OUT_F32_SCALED && out_dtype != BGEMM_OUT_F16_SCALED) return 0;
-    return N >= 1 && N <= (1 << 24) && M >= 1 && M <= (1 << 16) && K >= 8 && K <= ROWS_MAX_K && layers >= 1 && layers <= 3 &&
-           rows_lds(M, K, layers, layers, bits) <= (64 << 10);
+    if (N < 1 || N > (1 << 24) || M < 1 || M > (1 << 16) || K < 8 || K > ROWS_MAX_K || layers < 1 || layers > 3 ||
+        rows_lds(M, K, layers, layers, bits) > (64 << 10))
+        return 0;
+    // Against a pack and a GEMM (one layer, N = 5 .. 8192, M = 256 .. 22016, both types).  On few rows its time is that of one wave's walk
+    // over K, which the decode kernels split among their waves: us, two launches / this one, fp32 32 x 512 x 4096 7.3 / 4.5, 32 x 1000 x
+    // 4096 6.5 / 5.8 but 16 x 1000 x 1000 5.9 / 6.0, 128 x 1536 x 4096 7.4 / 7.7 and 512 x 1536 x 4096 10.1 / 7.8, 512 x 2048 x 1000 7.8 / 9.0
+    // and 2048 x 2048 x 1000 12.4 / 10.9.  Beyond 16384 columns a few hundred rows are too few for a block a row tile to share them
+    // (512 x 2048 x 22016 22.2 / 26.7, fp16 512 x 1000 x 22016 15.1 / 16.1).
+    const int64_t KT = k_tiles(K), rows = KT <= 2 ? 1 : KT <= 4 ? 33 : KT <= 6 ? 512 : 2048;
+    return N >= rows && (M <= 16384 || N < 256) ? 2 : 1;
 }
 
 extern "C" int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx, int64_t N, int64_t M, int64_t K, int layers,
@@ -421,26 +430,35 @@ extern "C" int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx
     a.x = x; a.ld = ldx; a.residual = residual;
     a.N = (int)N; a.M = (int)M; a.K = (int)K; a.KT = (int)k_tiles(K); a.MT = (int)row_tiles(M); a.layers = layers;
     const int64_t rt = row_tiles(N);
-    // How many column tiles a wave multiplies at once, how many waves a layer has in a block, how many blocks share a row tile: one block
-    // a compute unit at most, since each of those that share makes the rows' bits again (8192 x 768 x (3 x 768) bits: 20 us with two a
-    // unit, 14 with one), and as many waves as give each a tile or two (us, 4 / 8 / 16 waves: fp32 8192 x 768 x 3072 35.3 / 26.9 / 24.4,
-    // 2048 x 1024 x 1024 7.3 / 6.2 / 7.2, 128 x 768 x 3072 5.3 / 5.5 / 6.6).  Two tiles at once share an operand's reads from LDS: bits from
-    // sixteen tiles a compute unit on (8192 x 768 x (3 x 768) 15.3 -> 14.4, but 100 rows 7.2 -> 8.1); fp16 numbers leave in pairs of them.
+    // How many column tiles a wave multiplies at once, how many waves a layer has in a block, how many blocks share a row tile.
+    // Numbers, one tile (fp16: a pair), eight waves, as many blocks as there are groups for up to two a compute unit, one storing while the
+    // other makes its bits (us, 16 waves and one block / 8 and two, from and to memory: fp32 8192 x 768 x 3072 29.0 / 28.9, x 1008 16.0 /
+    // 14.9; fp16 20.3 / 19.3; 512 x 512 x 2048 7.1 / 5.7).  Beyond K = 1024 making them again costs more than that, fp32 rows of 16 KiB meet
+    // on the same memory channels when more blocks store at a time (8192 x 256 x 4096 30.7 / 37.1), and bits have nothing to store: one
+    // block a compute unit, of as many waves as give each a tile or two (2048 x 2048 x 2048 10.8, in two blocks of eight 13.7; 8192 x
+    // 768 x (3 x 768) bits 14 and 20).  Two tiles at once share an operand's reads from LDS: bits from sixteen tiles a
+    // compute unit on (8192 x 768 x (3 x 768) 15.3 -> 14.4, but 100 rows 7.2 -> 8.1).
     const int64_t tiles = rt * a.MT;
-    const bool f16_numbers = out_dtype == BGEMM_OUT_F16_SCALED;
+    const bool f16_numbers = out_dtype == BGEMM_OUT_F16_SCALED, one_a_unit = bits || K > 1024 || (f32 && M >= 4096);
     const int ct = f16_numbers ? 2 : shape ? shape & 15 : bits && layers * tiles >= 4096 ? 2 : 1;
     a.groups = (int)cdiv(a.MT, ct);
-    int64_t per_layer = cdiv(cdiv(rt * a.groups, 256), 4) * 4;
-    const int64_t most = layers == 3 ? 4 : ROWS_MAX_WAVES / layers, least = f16_numbers && layers == 1 ? 8 : 4;
-    per_layer = shape ? shape >> 4 & 31 : per_layer < least ? least : per_layer > most ? most : per_layer;
+    int64_t per_layer = 8 / layers;
+    if (one_a_unit) {
+        const int64_t want = cdiv(cdiv(rt * a.groups, 256), 4) * 4, most = layers == 3 ? 4 : ROWS_MAX_WAVES / layers;
+        per_layer = want < 4 ? 4 : want > most ? most : want;
+        if (f16_numbers && layers == 1 && per_layer < 8) per_layer = 8;
+    }
+    if (shape) per_layer = shape >> 4 & 31;
     int64_t splits = cdiv(a.groups, per_layer);
-    while (splits > 1 && rt * splits > 256) splits--;
+    while (splits > 1 && rt * splits > (one_a_unit ? 256 : 512)) splits--;
     if (shape >> 12) splits = shape >> 12;
     const int64_t waves = layers * per_layer;
     a.splits = (int)splits;
     a.first_lds = (int)rows_first_lds(M, K, packed ? 1 : layers, layers, bits);
     a.gather = bits && splits == 1 ? (int)k_tiles(M) * 8 : 0;
-    a.nt = N * M * 4 <= (32LL << 20);
+    // Past the caches where no two blocks share a 64-byte piece of a row (fp32 8192 x 768 x 3072 34.3 -> 28.9, 4096 x 1024 x 4096 26.6 ->
+    // 19.7, fp16 8192 x 768 x 768 12.9 -> 11.0; rows of 4000 bytes 19.0 -> 20.3, of fp16 6176 26.5 -> 28.6).
+    a.nt = M * (f32 ? 4 : 2) % 64 == 0;
     const size_t lds = (size_t)rows_lds(M, K, packed ? 1 : layers, layers, bits);
     const dim3 grid((unsigned)(rt * splits)), block((unsigned)(waves * 64));
     const hipStream_t st = (hipStream_t)stream;

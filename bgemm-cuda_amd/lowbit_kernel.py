@@ -421,7 +421,7 @@ def _check_scalar(t, name, dtype, device):
         raise ValueError("%s must be a one-element %s tensor on %s" % (name, dtype, device))
 
 
-_rows_shapes = {}         # (N, M, K, layers, output kind) -> does bgemm_linear_rows_forward take it
+_rows_shapes = {}         # (N, M, K, layers, output kind) -> 0, or 1: bgemm_linear_rows_forward takes it, 2: and is ahead of a pack and a GEMM
 
 
 def linear_rows_supported(N, M, K, layers, kind):
@@ -429,16 +429,17 @@ def linear_rows_supported(N, M, K, layers, kind):
     if ok is None:
         if len(_rows_shapes) > 4096:
             _rows_shapes.clear()
-        ok = _rows_shapes[(N, M, K, layers, kind)] = bool(_b.lib().bgemm_linear_rows_supported(N, M, K, layers, kind))
+        ok = _rows_shapes[(N, M, K, layers, kind)] = _b.lib().bgemm_linear_rows_supported(N, M, K, layers, kind)
     return ok
 
 
-def linear_rows_forward(x, layers, bits=False, residual=None, shape=0):
+def linear_rows_forward(x, layers, bits=False, residual=None, next_zero_point=None, bits_out=None, shape=0):
     """Up to three scaled binary layers of one input and one size in ONE launch, packing included (bgemm_linear.py:479-484 without a
     gradient).  ``x``: fp16 or fp32 ``[N, K]`` with dense rows, or a binary PackedBits that is centred already; ``layers``: a list of
     ``(w, zero_point, sw, sa, bias)``, ``w`` a binary PackedBits of M x K bits, the others tensors of one type (``x``'s where that is a
     tensor), ``zero_point`` and ``bias`` or None.  Returns a list: each layer's ``half(acc) * sw * sa (+ bias)``, ``[N, M]``, plus
-    ``residual`` if there is one, or with ``bits`` those outputs' sign bits, as ``bgemm_packed_forward(bits_out=)`` leaves them."""
+    ``residual`` if there is one, or with ``bits`` those outputs' sign bits after centring by ``next_zero_point`` (one element, or None
+    for 0), as ``bgemm_packed_forward(bits_out=)`` leaves them: in ``bits_out`` (a list), or in new operands whose padding is undefined."""
     packed = isinstance(x, PackedBits)
     w0, dt = layers[0][0], layers[0][2].dtype
     M, K, dev = w0.rows, w0.K, w0.data.device
@@ -460,8 +461,10 @@ def linear_rows_forward(x, layers, bits=False, residual=None, shape=0):
     kind = (OUT_BITS_F32 if f32 else OUT_BITS_F16) if bits else OUT_F32_SCALED if f32 else OUT_F16_SCALED
     if residual is not None and (bits or residual.dtype != dt or tuple(residual.shape) != (N, M) or not residual.is_contiguous() or residual.device != dev):
         raise ValueError("residual must be a contiguous %s tensor [%d, %d] on %s, beside outputs that are numbers" % (dt, N, M, dev))
+    if next_zero_point is not None:
+        _check_scalar(next_zero_point, "next_zero_point", dt, dev)
     arr, outs = (_b.RowsLayer * len(layers))(), []
-    for a, (w, zp, sw, sa, bias) in zip(arr, layers):
+    for i, (a, (w, zp, sw, sa, bias)) in enumerate(zip(arr, layers)):
         if w.ternary or w.batch != 1 or (w.rows, w.K) != (M, K):
             raise ValueError("every weight must be one binary matrix of %d x %d" % (M, K))
         _check_packed(w, "w")
@@ -472,13 +475,22 @@ def linear_rows_forward(x, layers, bits=False, residual=None, shape=0):
                 raise ValueError("%s must be a contiguous %s tensor of %d elements on %s" % (name, dt, n, dev))
         if w.data.device != dev:
             raise ValueError("every weight must be on %s" % dev)
-        out = empty_packed(N, M, dev) if bits else torch.empty((N, M), dtype=dt, device=dev)
+        if bits and bits_out is not None:
+            out = bits_out[i]
+            _check_packed(out, "bits_out")
+            if out.ternary or (out.batch, out.rows, out.K) != (1, N, M) or out.data.device != dev:
+                raise ValueError("bits_out must be binary operands of %d x %d rows x bits on %s" % (N, M, dev))
+            out.counts = None         # row popcounts taken of the old contents no longer describe it
+        else:
+            out = empty_packed(N, M, dev) if bits else torch.empty((N, M), dtype=dt, device=dev)
         outs.append(out)
         a.W_tiled, a.sw, a.sa, a.out = w.data.data_ptr(), sw.data_ptr(), sa.data_ptr(), (out.data if bits else out).data_ptr()
         if zp is not None:
             a.zero_point = zp.data_ptr()
         if bias is not None:
             a.bias = bias.data_ptr()
+        if next_zero_point is not None:
+            a.next_zero_point = next_zero_point.data_ptr()
     with _on(dev):
         _b.check(_b.lib().bgemm_linear_rows_forward((x.data if packed else x).data_ptr(), SRC_BITS if packed else SRC_F32 if f32 else SRC_F16,
                                                     0 if packed else max(x.stride(0), K), N, M, K, len(layers), arr, kind,
@@ -730,6 +742,9 @@ def bgemm_packed_weight_forward(w, x, mode=MODE_XOR, out_dtype=torch.int32, scal
     N, K, M = x.shape[0], w.K, w.rows
     L = _b.lib()
     if not decode_shape_supported(mode, M, N, K) or variant == VARIANT_VALU:
+        if (mode == MODE_XOR and variant == VARIANT_AUTO and scale is not None and scale[0].dtype == x.dtype
+                and linear_rows_supported(N, M, K, 1, OUT_F32_SCALED if x.dtype == torch.float32 else OUT_F16_SCALED) == 2):
+            return linear_rows_forward(x, [(w, x_zero_point, *scale)])[0]
         xp = pack_ternary(x) if ternary else pack_sign(x, zero_point=x_zero_point)
         return bgemm_packed_forward(w, xp, mode, out_dtype, 8, variant, scale=scale)[0]
     if x.stride(1) != 1 or x.stride(0) < K:

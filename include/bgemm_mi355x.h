@@ -327,7 +327,8 @@ int bgemm_elastic_backward(const void* x_sign, const void* x_nonzero, const void
  *   y = half(acc) * sw * sa (+ bias), every step rounded as bgemm_packed_forward_scaled does it
  *   scaled kinds: out [N][M] = y, or y + residual (residual [N][M] of the output's type)
  *   bits kinds:   out = the sign bits of half(y - *next_zero_point) (NULL: 0), tiled; its padding is not written
- * Supported: 8 <= K <= 2048, M <= 65536, N <= 2^24, the rows' bits (and with bits out the parameters) within 64 KiB of LDS.
+ * Supported (else 0): 8 <= K <= 2048, M <= 65536, N <= 2^24, the rows' bits (and with bits out the parameters) within 64 KiB of LDS;
+ * 2 where one layer is also ahead of a pack and a GEMM, else 1.
  * tiles: column tiles a wave multiplies at once, 0 = chosen by size (1 to 3: tests). */
 typedef struct bgemm_rows_layer {
     const void* W_tiled;
