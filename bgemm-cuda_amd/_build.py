@@ -27,7 +27,7 @@ def native_command():
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     return [os.environ.get("CXX", "g++"), "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
             "-I" + os.path.join(torch_dir, "include"), "-I" + os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
-            "-I" + os.path.join(rocm, "include"), "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "torch_ops.cpp"), "-o", NATIVE_SO,
+            "-I" + os.path.join(rocm, "include"), "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "torch_ops.cpp"), os.path.join(CSRC, "torch_infer.cpp"), "-o", NATIVE_SO,
             "-L" + os.path.join(torch_dir, "lib"), "-lc10", "-ltorch_cpu", "-ltorch_python", "-lc10_hip", "-L" + HERE, "-l:" + os.path.basename(SO),
             "-Wl,-rpath,$ORIGIN"]
 

@@ -134,6 +134,19 @@ def native():
     return _native
 
 
+_native_looked_for = False
+
+
+def native_or_none():
+    """native() if it has been built, else None: for calls that have a form without it."""
+    global _native_looked_for
+    if _native is None and not _native_looked_for:
+        _native_looked_for = True
+        if os.path.exists(os.path.join(_HERE, "_bgemm_native.so")):
+            return native()
+    return _native
+
+
 def native_for(dtypes, *tensors):
     """native() for a call whose tensors (or Nones) are all of one of `dtypes`, else None: what cannot be a call for it does not
     need it to be there."""

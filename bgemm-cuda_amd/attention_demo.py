@@ -17,6 +17,7 @@ import time
 import torch
 import torch.nn as nn
 
+import _lib
 import lowbit_kernel
 from bgemm_linear import BGEMMLinear, GraphedInference, bgemm_attn_matmul, bgemm_matmul, fused_bits
 
@@ -24,6 +25,12 @@ from bgemm_linear import BGEMMLinear, GraphedInference, bgemm_attn_matmul, bgemm
 def _pm1(t):
     """{-1,+1} by the sign bit (what the kernels read: -0.0 counts as negative)."""
     return torch.where(torch.signbit(t), -1.0, 1.0).to(t.dtype)
+
+
+def _unheard(layer):
+    """Whether a module is a plain BGEMMLinear whose call nothing listens to."""
+    return (type(layer) is BGEMMLinear and layer.fuse_inference and not layer._forward_hooks and not layer._forward_pre_hooks
+            and "forward" not in layer.__dict__ and not nn.modules.module._has_any_global_hook())
 
 
 class BinarySelfAttention(nn.Module):
@@ -48,22 +55,23 @@ class BinarySelfAttention(nn.Module):
 
     def _fusable(self, x):
         """Whether bits may stand for the projections' outputs: three plain layers that split into these heads, nothing that looks in between."""
+        if (torch.is_grad_enabled() or torch.is_autocast_enabled() or lowbit_kernel.watched()
+                or getattr(self.transpose_for_scores, "__func__", None) is not BinarySelfAttention.transpose_for_scores):
+            return False
+        layers = [self._modules.get(name) for name in ("query", "key", "value")]
         hidden = self.num_attention_heads * self.attention_head_size
-
-        def splits(layer):
-            # (asked on every call, of which the host is a part: the parameter itself, not through the module's attribute lookup)
-            weight = layer._parameters.get("weight") if type(layer) is BGEMMLinear else None
-            return weight is not None and weight.shape[0] == hidden and layer._bits_fusable(x)
-
-        return (not torch.is_grad_enabled() and x.dim() == 3 and x.numel() > 0 and not torch.is_autocast_enabled()
-                and not lowbit_kernel.watched() and getattr(self.transpose_for_scores, "__func__", None) is BinarySelfAttention.transpose_for_scores
-                and splits(self.query) and splits(self.key) and splits(self.value)
+        if not all(_unheard(l) and l.out_features == hidden for l in layers):
+            return False
+        native = _lib.native_or_none()
+        if native is not None and native.block_ready([l.__dict__ for l in layers], x, self.num_attention_heads):
+            return True
+        return (x.dim() == 3 and x.numel() > 0 and all(l.weight.shape[0] == hidden and l._bits_fusable(x) for l in layers)
                 and lowbit_kernel.attention_supported(x.shape[0], x.shape[1], self.num_attention_heads, self.attention_head_size))
 
     def _dense_fusable(self, x, rows, hidden):
         """Whether the last projection may read the context's bits and add the residual: a plain layer of this block's size."""
-        layer = self.dense
-        return (type(layer) is BGEMMLinear and layer.weight.shape == (hidden, hidden) and x.shape[-1] == hidden and layer._bits_fusable(x)
+        layer = self._modules.get("dense")
+        return (_unheard(layer) and layer.out_features == hidden and layer.weight.shape == (hidden, hidden) and x.shape[-1] == hidden and layer._bits_fusable(x)
                 and lowbit_kernel.linear_rows_supported(rows, hidden, hidden, 1, lowbit_kernel.OUT_F32_SCALED if x.dtype == torch.float32
                                                         else lowbit_kernel.OUT_F16_SCALED))
 
@@ -75,10 +83,16 @@ class BinarySelfAttention(nn.Module):
             rows, hidden = batch * seq, bits[0].K
             if self._dense_fusable(hidden_states, rows, hidden):
                 # of the context, too, the last projection reads its signs only, and it adds the residual as it stores
-                dense = self.dense._rows_layer(hidden_states.dtype)
-                scores, context = lowbit_kernel.attention_forward(*bits, batch, self.num_attention_heads, hidden_states.dtype, dense[1])
-                out = lowbit_kernel.linear_rows_forward(context, [dense], residual=hidden_states.reshape(rows, hidden).contiguous())[0]
-                return self.LayerNorm(out.view(batch, seq, hidden)), scores
+                zero_point = self.dense.zpa
+                if zero_point.dtype != hidden_states.dtype:
+                    zero_point = zero_point.detach().to(hidden_states.dtype)
+                scores, context = lowbit_kernel.attention_forward(*bits, batch, self.num_attention_heads, hidden_states.dtype, zero_point)
+                native = _lib.native_or_none()
+                out = None if native is None else native.rows_residual(self.dense.__dict__, context.data, hidden_states)
+                if out is None:
+                    residual = hidden_states.reshape(rows, hidden).contiguous()
+                    out = lowbit_kernel.linear_rows_forward(context, [self.dense._rows_layer(hidden_states.dtype)], residual=residual)[0].view(batch, seq, hidden)
+                return self.LayerNorm(out), scores
             scores, context = lowbit_kernel.attention_forward(*bits, batch, self.num_attention_heads, hidden_states.dtype)
             return self.LayerNorm(self.dense(context) + hidden_states), scores
         q = self.transpose_for_scores(self.query(hidden_states))

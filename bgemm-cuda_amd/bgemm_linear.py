@@ -62,6 +62,11 @@ def _pack_right(mat):
 def _batched_packed(x_rows, right, mode):
     """x_rows [..., N, K] @ right [..., K, M] with equal leading dimensions -> fp16 [..., N, M]: one launch over
     all leading dimensions on the batched packed entry point (no per-matrix Python loop)."""
+    native = _lib.native_or_none()
+    if native is not None:
+        out = native.batched_product(x_rows, right, mode)
+        if out is not None:
+            return out
     lead = x_rows.shape[:-2]
     if right.shape[:-2] != lead:
         raise ValueError("leading dimensions differ: %s vs %s" % (tuple(x_rows.shape), tuple(right.shape)))
@@ -94,6 +99,9 @@ def _any_tangent(*tensors):
 def _one_launch_grads(matrix, a, b, longest):
     """Whether the batched products' gradients go to their one-launch kernels: operands those read where they lie, and nothing that
     has to see the torch operations (a graph of the gradients, forward-mode derivatives, vmap, a tensor subclass, a mode)."""
+    native = _lib.native_or_none()
+    if native is not None:
+        return native.one_launch_grads(matrix, a, b, longest)
     return (not torch.is_grad_enabled() and lowbit_kernel.attention_grads_supported(a, b, longest) and type(matrix) is torch.Tensor
             and matrix.dtype == torch.half and matrix.device == a.device and not lowbit_kernel._wrapped(matrix)
             and not lowbit_kernel.watched() and not _any_tangent(matrix, a, b))
@@ -457,6 +465,12 @@ class BGEMMLinear(_ScaledBinaryLinear):
     def forward(self, x):
         if not self.initialized:
             self._initialize(x, self.weight)
+        if not torch.is_grad_enabled() and type(self) in _PLAIN_LAYERS and self.fuse_inference:
+            native = _lib.native_or_none()
+            if native is not None:
+                out = native.linear_infer(self.__dict__, x)
+                if out is not None:
+                    return out
         if self._fusable(x):
             return self._fused_forward(x)
         if self.fuse_training and x.is_cuda and (self._fn is bgemm_linear or self._fn is bgemm_linear_bireal):
@@ -473,6 +487,11 @@ class BGEMMLinear(_ScaledBinaryLinear):
 def fused_bits(layers, x):
     """The sign bits of ``layer(x)`` for every layer of a list, each of which is ``_bits_fusable(x)``: one launch where they are of one
     size that ``lowbit_kernel.linear_rows_forward`` takes, else two a layer."""
+    native = _lib.native_or_none()
+    if native is not None:
+        planes = native.rows_bits([l.__dict__ for l in layers], x)
+        if planes is not None:
+            return [lowbit_kernel.PackedBits(p, None, 1, x.numel() // x.shape[-1], layers[0].out_features) for p in planes]
     w = layers[0].weight
     kind = lowbit_kernel.OUT_BITS_F32 if x.dtype == torch.float32 else lowbit_kernel.OUT_BITS_F16
     if (all(l.weight.shape == w.shape for l in layers)
@@ -494,7 +513,23 @@ class BGEMMChain(nn.Sequential):
                 and all(l._fusable(x) for l in layers)
                 and all(a.weight.shape[0] == b.weight.shape[1] for a, b in zip(layers, layers[1:])))
 
+    def _native_forward(self, x):
+        """The fused forward by the native host side, once the bit buffers of this number of rows are there; None where it has to be Python's."""
+        native = _lib.native_or_none()
+        bits = self.__dict__.get("_bits")
+        if native is None or bits is None or torch.is_grad_enabled() or type(x) is not torch.Tensor or not x.numel():
+            return None
+        buffers = bits.get((x.numel() // x.shape[-1], x.device))
+        layers = list(self._modules.values())
+        if buffers is None or not all(type(l) in _PLAIN_LAYERS and l.fuse_inference for l in layers):
+            return None
+        return native.chain_infer([l.__dict__ for l in layers], x, buffers)
+
     def forward(self, x):
+        if type(self) is BGEMMChain:
+            out = self._native_forward(x)
+            if out is not None:
+                return out
         if not self._fusable(x):
             return super().forward(x)          # also the first call, which initialises the layers' scales
         layers = list(self)
@@ -509,6 +544,7 @@ class BGEMMChain(nn.Sequential):
             scale = (layer.sw.detach(), layer.sa.detach().reshape(1), None if layer.bias is None else layer.bias.detach())
             if i + 1 == len(layers):
                 out = lowbit_kernel.bgemm_packed_forward(layer._packed_weight(), xp, lowbit_kernel.MODE_XOR, splitK=8, scale=scale)
+                self._bits[x2.shape[0], x.device] = [self._bits[j, x2.shape[0], x.device].data for j in range(i)]
                 return out.reshape(*lead, layer.weight.shape[0])
             key = (i, x2.shape[0], x.device)
             if key not in self._bits:      # zero-filled once: the GEMM writes real bits only, the padding stays zero
@@ -560,6 +596,9 @@ class GraphedInference:
 class BGEMMLinear_bireal(BGEMMLinear):
     """BGEMMLinear with the Bi-Real backward (bgemm_linear.py:489-516)."""
     _fn = bgemm_linear_bireal
+
+
+_PLAIN_LAYERS = frozenset((BGEMMLinear, BGEMMLinear_bireal))      # whose forward is the one above
 
 
 class BGEMMLinear_elastic_signed(_ScaledBinaryLinear):

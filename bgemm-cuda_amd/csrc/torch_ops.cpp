@@ -1,89 +1,22 @@
 // The host side of the layers, native: what bgemm_linear.py and lowbit_kernel.py would do on every call in Python (argument
 // checks, allocation, the stream, the calls into the C ABI, autograd bookkeeping).  A small layer's kernels take a few
 // microseconds, less than those steps cost in Python.  Host code only: plain CPython functions on torch's C++ API, linked against
-// libbgemm_mi355x.so beside it.  Functions that find a case they do not take return None, and the caller goes the Python way.
-#include <Python.h>
+// libbgemm_mi355x.so beside it.  This part: training; torch_infer.cpp: inference and attention.  Functions that find a case they do not
+// take return None, and the caller goes the Python way.
+#include "torch_common.h"
 
-#include <ATen/ATen.h>
-#include <ATen/PythonTorchFunctionTLS.h>
-#include <ATen/SavedTensorHooks.h>
-#include <c10/core/DeviceGuard.h>
-#include <c10/core/GradMode.h>
-#include <c10/core/impl/LocalDispatchKeySet.h>
-#include <c10/hip/HIPStream.h>
-#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
-#include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
-#include <torch/csrc/autograd/variable.h>
 
 #include <utility>
-
-#include "../../include/bgemm_mi355x.h"
+#include <vector>
 
 namespace {
 
-using at::Tensor;
+using namespace bgemm_native;
 using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
-
-// Turns a negative status into the exception _lib.check() raises.
-void check(const int rc)
-{
-    if (rc == BGEMM_OK) return;
-    const std::string msg = bgemm_last_error();
-    if (rc == BGEMM_EINVAL || rc == BGEMM_ENULL || rc == BGEMM_EALIGN || rc == BGEMM_EWORKSPACE) TORCH_CHECK_VALUE(false, msg);
-    TORCH_CHECK(false, msg);
-}
-
-void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
-bool is_param_type(const at::ScalarType t) { return t == at::kFloat || t == at::kHalf; }
-int src_type(const Tensor& t) { return t.scalar_type() == at::kFloat ? BGEMM_SRC_F32 : BGEMM_SRC_F16; }
-void* data_or_null(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
-const Tensor& tensor_at(PyObject* o) { return THPVariable_Unpack(o); }
-Tensor tensor_or_none(PyObject* o) { return o == Py_None ? Tensor() : THPVariable_Unpack(o); }
-
-// Whether a tensor is memory on the GPU and nothing else: no transform's wrapper, no subclass with a dispatch of its own (fake tensors
-// among them), no view that is negated or conjugated when read, no sparse or quantised layout.
-bool is_memory(const Tensor& t)
-{
-    using c10::DispatchKey;
-    static const uint64_t usual = c10::DispatchKeySet({DispatchKey::Dense, DispatchKey::AutogradFunctionality, DispatchKey::ADInplaceOrView,
-                                                       DispatchKey::AutocastCUDA}).raw_repr() | c10::full_backend_mask;
-    return (t.key_set().raw_repr() & ~usual) == 0;
-}
-
-// Whether something else has to see each torch operation: a mode, a trace, a function transform.
-bool is_watched()
-{
-    using c10::DispatchKey;
-    static const uint64_t usual = c10::DispatchKeySet({DispatchKey::BackendSelect, DispatchKey::ADInplaceOrView, DispatchKey::AutocastCUDA,
-                                                       DispatchKey::AutocastCPU}).raw_repr() | c10::full_backend_mask;
-    return (c10::impl::tls_local_dispatch_key_set().included_.raw_repr() & ~usual) != 0 || at::impl::torch_function_mode_enabled();
-}
-
-// Forward-mode derivatives are torch's business: the kernels know none.
-bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
-
-// Kernels are enqueued and memory is allocated without the interpreter's lock.
-struct WithoutGil {
-    PyThreadState* state = PyEval_SaveThread();
-    ~WithoutGil() { PyEval_RestoreThread(state); }
-};
-
-// [..., C] as rows [R, C] whose elements are dense, and their stride (C or more: a single row's own stride means nothing and may be
-// anything, also after contiguous()).
-struct Rows { Tensor t; int64_t ld; };
-
-Rows rows_2d(const Tensor& t)
-{
-    const int64_t C = t.size(-1);
-    Tensor r = t.dim() == 2 ? t : t.reshape({t.numel() / C, C});
-    if (r.size(0) == 1) return {r.stride(1) == 1 || C == 1 ? r : r.contiguous(), C};
-    if (r.stride(1) != 1 || r.stride(0) < C) r = r.contiguous();
-    return {r, r.stride(0)};
-}
 
 // The interpreter's pending exception as a C++ one that outlives the lock and the thread it was raised on.
 [[noreturn]] void throw_pending()
@@ -426,13 +359,28 @@ PyObject* elastic_train(PyObject*, PyObject* const* args, const Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef methods[] = {
+const PyMethodDef train_methods[] = {
     {"elastic_train", (PyCFunction)(void (*)(void))elastic_train, METH_FASTCALL, "forward of a learned-scale binary Linear, recorded as one autograd node"},
-    {"linear_train", (PyCFunction)(void (*)(void))linear_train, METH_FASTCALL, "forward of a scaled binary Linear, recorded as one autograd node"},
-    {nullptr, nullptr, 0, nullptr}};
+    {"linear_train", (PyCFunction)(void (*)(void))linear_train, METH_FASTCALL, "forward of a scaled binary Linear, recorded as one autograd node"}};
 
-PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_bgemm_native", "host side of the binary layers", -1, methods, nullptr, nullptr, nullptr, nullptr};
+// both parts' functions and the end mark
+PyMethodDef* all_methods()
+{
+    static std::vector<PyMethodDef> all;
+    if (all.empty()) {
+        for (const PyMethodDef& m : train_methods) all.push_back(m);
+        for (int i = 0; i < infer_method_count; i++) all.push_back(infer_methods[i]);
+        all.push_back({nullptr, nullptr, 0, nullptr});
+    }
+    return all.data();
+}
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_bgemm_native", "host side of the binary layers", -1, nullptr, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__bgemm_native(void) { return PyModule_Create(&module_def); }
+PyMODINIT_FUNC PyInit__bgemm_native(void)
+{
+    module_def.m_methods = all_methods();
+    return PyModule_Create(&module_def);
+}

@@ -289,6 +289,13 @@ def bgemm_packed_forward(w, x, mode=MODE_XOR, out_dtype=torch.int32, splitK=1, v
     activations at all: the scaled output is centred by ``next_zero_point`` (a one-element tensor of the
     parameters' type, or None for 0), cast to fp16 and sign-packed as the next binary layer would do it, and
     those bits are written into ``bits_out``, which is returned."""
+    if scale is None and out is None and bits_out is None and splitK == 1 and variant == VARIANT_AUTO and type(w) is type(x) is PackedBits and w.K == x.K:
+        if w.data2 is None and (w.counts is None or x.counts is None) and (out_dtype is torch.int32 or out_dtype is torch.half):
+            native = _b.native_or_none()
+            if native is not None:
+                got = native.packed_forward(w.data, w.batch, w.rows, w.K, x.data, x.data2, x.batch, x.rows, mode, OUT_F16 if out_dtype is torch.half else OUT_I32)
+                if got is not None:
+                    return got
     if w.K != x.K:
         raise ValueError("K mismatch: %d vs %d" % (w.K, x.K))
     if (mode == MODE_BWTA) != x.ternary:
@@ -389,6 +396,12 @@ def attention_forward(q, k, v, batch, heads, dtype, zero_point=None):
     fp16 storage) is at least ``1 / seq``.  With ``zero_point`` (a one-element tensor of ``dtype``) the context is not stored: its sign
     bits after centring are returned, the operand of the binary layer behind it."""
     rows, hidden = q.rows, q.K
+    native = _b.native_or_none()
+    if native is not None and k.rows == v.rows == rows and k.K == v.K == hidden and (dtype is torch.float32 or dtype is torch.half):
+        if q.data2 is k.data2 is v.data2 is None:
+            got = native.attention_forward(q.data, k.data, v.data, rows, hidden, batch, heads, dtype is torch.float32, zero_point)
+            if got is not None:
+                return got if zero_point is None else (got[0], PackedBits(got[1], None, 1, rows, hidden))
     for name, p in (("q", q), ("k", k), ("v", v)):
         if p.ternary or p.batch != 1 or (p.rows, p.K) != (rows, hidden):
             raise ValueError("%s must be a binary operand of %d x %d" % (name, rows, hidden))
@@ -545,6 +558,11 @@ def _attention_backward(fn, m, a, b, out_a, out_b, strides_of):
 def scores_backward(grad_scores, a, b, need=(True, True)):
     """Straight-through gradients of ``sign(a) @ sign(b).T`` (bgemm_linear.py:28-42) in one launch: ``a`` [.., N, D], ``b`` [.., M, D],
     ``grad_scores`` [.., N, M] fp16.  The gradients have their operands' strides; one not needed is None."""
+    native = _b.native_or_none()
+    if native is not None:
+        got = native.attention_backward(False, grad_scores, a, b, need[0], need[1])
+        if got is not None:
+            return got
     g = grad_scores.contiguous()
     ga, gb = (_grad_like(t) if wanted else None for t, wanted in zip((a, b), need))
     _attention_backward(_b.lib().bgemm_scores_backward, g, a, b, ga, gb, (a, b, ga, gb))
@@ -554,6 +572,11 @@ def scores_backward(grad_scores, a, b, need=(True, True)):
 def context_backward(probs, grad_context, value, need=(True, True)):
     """Gradients of the attention matmul (bgemm_linear.py:64-86) in one launch: ``probs`` [.., N, M], ``grad_context`` [.., N, D],
     ``value`` [.., M, D], fp16.  Returns (grad_probs, grad_value), None for one not needed."""
+    native = _b.native_or_none()
+    if native is not None:
+        got = native.attention_backward(True, probs, grad_context, value, need[0], need[1])
+        if got is not None:
+            return got
     gp = torch.empty(probs.shape, dtype=torch.half, device=probs.device) if need[0] else None
     gv = _grad_like(value) if need[1] else None
     _attention_backward(_b.lib().bgemm_context_backward, probs.contiguous() if need[1] else None, grad_context, value, gp, gv,
@@ -724,6 +747,18 @@ def bgemm_packed_weight_forward(w, x, mode=MODE_XOR, out_dtype=torch.int32, scal
     activation bits itself (``MODE_BWTA``: the ternary planes of sign(x); the other modes: sign bits of ``x``
     or, with ``x_zero_point``, of ``(x - x_zero_point).to(torch.half)``).  Larger batches go through the pack
     kernel and the packed entry point: same results either way.  ``scale`` as in bgemm_packed_forward."""
+    if variant == VARIANT_AUTO and type(w) is PackedBits and w.data2 is None and w.batch == 1:
+        native = _b.native_or_none()
+        if native is not None:
+            if scale is None:
+                kind = OUT_I32 if out_dtype is torch.int32 else OUT_F16 if out_dtype is torch.half else -1
+                got = native.packed_weight_forward(w.data, w.rows, w.K, x, mode, kind, None, None, None, x_zero_point)
+            else:
+                sw, sa, bias = scale
+                kind = OUT_F32_SCALED if getattr(sw, "dtype", None) is torch.float32 else OUT_F16_SCALED
+                got = native.packed_weight_forward(w.data, w.rows, w.K, x, mode, kind, sw, sa, bias, x_zero_point)
+            if got is not None:
+                return got
     _need_cuda(x, "x")
     if x.dim() != 2 or x.shape[1] != w.K:
         raise ValueError("x must be [N, %d], got %s" % (w.K, tuple(x.shape)))
@@ -782,6 +817,12 @@ def bgemm_linear_forward_cuda(in_feats, weights, splitK=1, INSTR=1):
     INSTR 0 = and.popc, 1 = K - 2*xor.popc, 2 = attention ({0,1} weights side by sign bit clear).
     Unlike the reference (fp6_linear.cu:288-290, 568-576) any N, M, K >= 1 is accepted, inputs need
     not be contiguous, and the launch goes to the current stream."""
+    if not _weight_cache_entries:
+        native = _b.native_or_none()
+        if native is not None:
+            got = native.f16_forward(in_feats, weights, splitK, INSTR)
+            if got is not None:
+                return got
     _need_cuda(in_feats, "in_feats")
     _need_cuda(weights, "weights")
     if in_feats.dim() != 2 or weights.dim() != 2:
