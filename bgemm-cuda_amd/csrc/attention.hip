@@ -29,7 +29,7 @@ struct AttnArgs {
     __half* scores; void* context;    // context: numbers, or the tiled operand of their signs after *zp is subtracted
     const void* zp;
     int64_t KT;                       // of the operands
-    int S, heads, groups, qblocks, f32;
+    int S, heads, groups, qblocks, f32, past;      // past: scores are stored past the caches
     float scale, level;               // 1 / sqrt(D), 1 / S
 };
 
@@ -141,7 +141,12 @@ __global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
             const uint4 x = *reinterpret_cast<const uint4*>(stage + (r8 + 8 * i) * ATTN_STAGE + c8 * 16);
             __half* const to = srow + (int64_t)(8 * i) * S + grp * 64;
             if (q0 + r8 + 8 * i < S) {
-                if (!TAIL || grp * 64 + c8 * 8 + 8 <= S) __builtin_memcpy(to, &x, 16);
+                if (!TAIL && a.past) {
+                    // (as an instruction: a builtin beside an ordinary store of the same value becomes one ordinary store.  The s_nop is the
+                    // hazard between a wide store and a write to its data registers.)
+                    const v4i v = {(int)x.x, (int)x.y, (int)x.z, (int)x.w};
+                    asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" : : "v"(to), "v"(v) : "memory");
+                } else if (!TAIL || grp * 64 + c8 * 8 + 8 <= S) __builtin_memcpy(to, &x, 16);
                 else {
                     const unsigned d[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
@@ -257,7 +262,7 @@ static int attention(const char* who, const void* q, const void* k, const void* 
         return fail(BGEMM_EALIGN, "%s: operands and context must be 16-byte aligned", who);
     const int W = (int)head_size / 32;
     AttnArgs a = {(const uint32_t*)q, (const uint32_t*)k, (const uint32_t*)v, (__half*)scores, context, zero_point, k_tiles(heads * head_size)};
-    a.S = (int)seq; a.heads = (int)heads; a.groups = (int)cdiv(seq, 64); a.f32 = context_type == BGEMM_SRC_F32;
+    a.S = (int)seq; a.heads = (int)heads; a.groups = (int)cdiv(seq, 64); a.f32 = context_type == BGEMM_SRC_F32; a.past = seq % 32 == 0 && ((uintptr_t)scores & 63) == 0;
     a.scale = 1.0f / (float)sqrt((double)head_size);
     a.level = (float)(1.0 / (double)seq);
     // four waves share a block's operands; fewer where that leaves the chip without two blocks a compute unit

@@ -18,7 +18,7 @@ struct RowsArgs {
     const void* x; int64_t ld;        // unpacked rows (element stride), or one tiled operand of sign bits
     const void* residual;             // [N][M], or null
     int N, M, K, KT, MT, layers;
-    int groups, splits;               // column groups of a layer, blocks a row tile
+    int groups, splits, own;          // column groups of a layer, blocks a row tile, groups of a block (neighbours)
     int nt;                           // stores past the caches
     int first_lds;                    // bytes of the first area
     int gather;                       // bits of a whole row tile leave together: column tiles of the output, to the end of its last K-tile; else 0
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
     uint4* const raw_bits = reinterpret_cast<uint4*>(smem);                 // [layer][K-tile][64]
     uint32_t* const words = reinterpret_cast<uint32_t*>(smem);              // BITS, in the same place later: [layer][column tile][row], tiles to the end of K-tiles
     uint4* const operands = reinterpret_cast<uint4*>(smem + a.first_lds);   // [layer][K-tile][step][64]
-    float* const cols = reinterpret_cast<float*>(operands + tiles_x * 4 * TILE_U4);      // BITS: the columns' parameters, [layer][sw | bias][MT * 32]
+    float* const cols = reinterpret_cast<float*>(operands + tiles_x * 4 * TILE_U4);      // BITS: the block's columns' parameters, [layer][sw | bias][own * CT * 32]
     [[maybe_unused]] float* const xsums = cols + wave * 32;                 // else: the wave's row sums
     auto par = [](const void* p, const int64_t i) {
         if constexpr (F32P) return reinterpret_cast<const float*>(p)[i];
@@ -109,11 +109,13 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
             }
         }
     }
+    const int g0 = part * a.own, g1 = min(a.groups, g0 + a.own), cols_n = a.own * CT * 32;
     if constexpr (BITS) {
         for (int l = 0; l < a.layers; l++)
-            for (int m = threadIdx.x; m < a.MT * 32; m += waves * 64) {
-                cols[(2 * l) * a.MT * 32 + m] = m < a.M ? par(a.l[l].sw, m) : 0.f;
-                cols[(2 * l + 1) * a.MT * 32 + m] = m < a.M && a.l[l].bias ? par(a.l[l].bias, m) : 0.f;
+            for (int i = threadIdx.x; i < cols_n; i += waves * 64) {
+                const int m = g0 * CT * 32 + i;
+                cols[2 * l * cols_n + i] = m < a.M ? par(a.l[l].sw, m) : 0.f;
+                cols[(2 * l + 1) * cols_n + i] = m < a.M && a.l[l].bias ? par(a.l[l].bias, m) : 0.f;
             }
     }
     __syncthreads();
@@ -133,8 +135,7 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
 
     // ---- the products --------------------------------------------------------------------------------------------------------------
     const RowsLayer& L = a.l[l];
-    const int stride = a.splits * per_layer;
-    int gg = part * per_layer + wl, kt = 0, rg = gg, rkt = 0;         // the group that is multiplied, and the one whose weights are requested next
+    int gg = g0 + wl, kt = 0, rg = gg, rkt = 0;                       // the group that is multiplied, and the one whose weights are requested next
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(L.W), 0, a.MT * KT * 1024, 0x00020000);
     const float sa = par(L.sa, 0), next = BITS && L.next_zp ? par(L.next_zp, 0) : 0.f;
     const bool has_bias = L.bias != nullptr, has_next = L.next_zp != nullptr;
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
         }
         if (++rkt == KT) {
             rkt = 0;
-            rg += stride;                                             // (past the last one: the last tile again, nobody multiplies it)
+            rg += per_layer;                                           // (past the last one: the last tile again, nobody multiplies it)
         }
     };
     // the sums of x that the accumulators start from: BITS: the lane's row's, else those of its sixteen rows
@@ -186,8 +187,8 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
             for (int j = 0; j < CT; j++) {
                 const int mt = mt0 + j;
                 if (mt >= a.MT) break;
-                const float* const ps = cols + (2 * l) * a.MT * 32 + mt * 32 + 16 * h;
-                const float* const pb = ps + a.MT * 32;
+                const float* const ps = cols + 2 * l * cols_n + (mt - g0 * CT) * 32 + 16 * h;
+                const float* const pb = ps + cols_n;
                 unsigned bits = 0;
                 auto collect = [&](auto bias_c, auto next_c) {
                     constexpr bool BIAS = decltype(bias_c)::value, NEXT = decltype(next_c)::value;
@@ -340,23 +341,23 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
         if (++kt == KT) {
             store_group();
             kt = 0;
-            gg += stride;
+            gg += per_layer;
         }
     };
-    if (gg < a.groups) {
+    if (gg < g1) {
         v4i w0[CT], w1[CT], w2[CT];
         request(w0);
         request(w1);
         for (;;) {
             request(w2);
             step(w0);
-            if (gg >= a.groups) break;
+            if (gg >= g1) break;
             request(w0);
             step(w1);
-            if (gg >= a.groups) break;
+            if (gg >= g1) break;
             request(w1);
             step(w2);
-            if (gg >= a.groups) break;
+            if (gg >= g1) break;
         }
     }
     if (BITS && a.gather) {
@@ -372,15 +373,44 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
     }
 }
 
-// What a block keeps in LDS: the rows' bits, later those of the output, and operands for every layer, and where bits leave the columns' parameters.
-static int64_t rows_first_lds(int64_t M, int64_t K, int planes, int layers, bool bits)
+// How a size is launched, and what a block keeps in LDS: the rows' bits, later those of the output, and operands for every layer, and where
+// bits leave the parameters of its columns.
+struct RowsPlan { int64_t ct, per_layer, splits, groups, own, first_lds, lds; };
+
+static RowsPlan rows_plan(int64_t N, int64_t M, int64_t K, int layers, bool packed, int out_dtype, int shape)
 {
-    const int64_t in = planes * k_tiles(K) * 1024, out = bits ? layers * k_tiles(M) * 1024 : 0;
-    return in > out ? in : out;
-}
-static int64_t rows_lds(int64_t M, int64_t K, int planes, int layers, bool bits)
-{
-    return rows_first_lds(M, K, planes, layers, bits) + planes * k_tiles(K) * 4096 + (bits ? layers * row_tiles(M) * 32 * 8 : ROWS_MAX_WAVES * 128);
+    RowsPlan p;
+    const bool bits = out_dtype == BGEMM_OUT_BITS_F32 || out_dtype == BGEMM_OUT_BITS_F16, f32 = out_dtype == BGEMM_OUT_BITS_F32 || out_dtype == BGEMM_OUT_F32_SCALED;
+    const int64_t rt = row_tiles(N);
+    // How many column tiles a wave multiplies at once, how many waves a layer has in a block, how many blocks share a row tile.
+    // Numbers, one tile (fp16: a pair), eight waves, as many blocks as there are groups for up to two a compute unit, one storing while the
+    // other makes its bits (us, 16 waves and one block / 8 and two, from and to memory: fp32 8192 x 768 x 3072 29.0 / 28.9, x 1008 16.0 /
+    // 14.9; fp16 20.3 / 19.3; 512 x 512 x 2048 7.1 / 5.7).  Beyond K = 1024 making them again costs more than that, fp32 rows of 16 KiB meet
+    // on the same memory channels when more blocks store at a time (8192 x 256 x 4096 30.7 / 37.1), and bits have nothing to store: one
+    // block a compute unit, of as many waves as give each a tile or two (2048 x 2048 x 2048 10.8, in two blocks of eight 13.7; 8192 x
+    // 768 x (3 x 768) bits 14 and 20).  Two tiles at once share an operand's reads from LDS: bits from sixteen tiles a
+    // compute unit on (8192 x 768 x (3 x 768) 15.3 -> 14.4, but 100 rows 7.2 -> 8.1).
+    const int64_t tiles = rt * row_tiles(M);
+    const bool f16_numbers = out_dtype == BGEMM_OUT_F16_SCALED, one_a_unit = bits || K > 1024 || (f32 && M >= 4096);
+    p.ct = f16_numbers ? 2 : shape ? shape & 15 : bits && layers * tiles >= 4096 ? 2 : 1;
+    p.groups = cdiv(row_tiles(M), p.ct);
+    p.per_layer = 8 / layers;
+    if (one_a_unit) {
+        const int64_t want = cdiv(cdiv(rt * p.groups, 256), 4) * 4, most = layers == 3 ? 4 : ROWS_MAX_WAVES / layers;
+        p.per_layer = want < 4 ? 4 : want > most ? most : want;
+        if (f16_numbers && layers == 1 && p.per_layer < 8) p.per_layer = 8;
+    }
+    if (shape) p.per_layer = shape >> 4 & 31;
+    p.splits = cdiv(p.groups, p.per_layer);
+    while (p.splits > 1 && rt * p.splits > (one_a_unit ? 256 : 512)) p.splits--;
+    if (shape >> 12) p.splits = shape >> 12;
+    p.own = cdiv(p.groups, p.splits);
+    p.splits = cdiv(p.groups, p.own);
+    const int planes = packed ? 1 : layers;
+    const int64_t in = planes * k_tiles(K) * 1024, out = bits && p.splits == 1 ? layers * k_tiles(M) * 1024 : 0;
+    p.first_lds = in > out ? in : out;
+    p.lds = p.first_lds + planes * k_tiles(K) * 4096 + (bits ? layers * p.own * p.ct * 32 * 8 : ROWS_MAX_WAVES * 128);
+    return p;
 }
 
 }  // namespace bgemm
@@ -389,10 +419,9 @@ using namespace bgemm;
 
 extern "C" int bgemm_linear_rows_supported(int64_t N, int64_t M, int64_t K, int layers, int out_dtype)
 {
-    const bool bits = out_dtype == BGEMM_OUT_BITS_F32 || out_dtype == BGEMM_OUT_BITS_F16;
-    if (!bits && out_dtype != BGEMM_OUT_F32_SCALED && out_dtype != BGEMM_OUT_F16_SCALED) return 0;
+    if (out_dtype != BGEMM_OUT_F32_SCALED && out_dtype != BGEMM_OUT_F16_SCALED && out_dtype != BGEMM_OUT_BITS_F32 && out_dtype != BGEMM_OUT_BITS_F16) return 0;
     if (N < 1 || N > (1 << 24) || M < 1 || M > (1 << 16) || K < 8 || K > ROWS_MAX_K || layers < 1 || layers > 3 ||
-        rows_lds(M, K, layers, layers, bits) > (64 << 10))
+        rows_plan(N, M, K, layers, false, out_dtype, 0).lds > (64 << 10))
         return 0;
     // Against a pack and a GEMM (one layer, N = 5 .. 8192, M = 256 .. 22016, both types).  On few rows its time is that of one wave's walk
     // over K, which the decode kernels split among their waves: us, two launches / this one, fp32 32 x 512 x 4096 7.3 / 4.5, 32 x 1000 x
@@ -429,38 +458,17 @@ extern "C" int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx
     }
     a.x = x; a.ld = ldx; a.residual = residual;
     a.N = (int)N; a.M = (int)M; a.K = (int)K; a.KT = (int)k_tiles(K); a.MT = (int)row_tiles(M); a.layers = layers;
-    const int64_t rt = row_tiles(N);
-    // How many column tiles a wave multiplies at once, how many waves a layer has in a block, how many blocks share a row tile.
-    // Numbers, one tile (fp16: a pair), eight waves, as many blocks as there are groups for up to two a compute unit, one storing while the
-    // other makes its bits (us, 16 waves and one block / 8 and two, from and to memory: fp32 8192 x 768 x 3072 29.0 / 28.9, x 1008 16.0 /
-    // 14.9; fp16 20.3 / 19.3; 512 x 512 x 2048 7.1 / 5.7).  Beyond K = 1024 making them again costs more than that, fp32 rows of 16 KiB meet
-    // on the same memory channels when more blocks store at a time (8192 x 256 x 4096 30.7 / 37.1), and bits have nothing to store: one
-    // block a compute unit, of as many waves as give each a tile or two (2048 x 2048 x 2048 10.8, in two blocks of eight 13.7; 8192 x
-    // 768 x (3 x 768) bits 14 and 20).  Two tiles at once share an operand's reads from LDS: bits from sixteen tiles a
-    // compute unit on (8192 x 768 x (3 x 768) 15.3 -> 14.4, but 100 rows 7.2 -> 8.1).
-    const int64_t tiles = rt * a.MT;
-    const bool f16_numbers = out_dtype == BGEMM_OUT_F16_SCALED, one_a_unit = bits || K > 1024 || (f32 && M >= 4096);
-    const int ct = f16_numbers ? 2 : shape ? shape & 15 : bits && layers * tiles >= 4096 ? 2 : 1;
-    a.groups = (int)cdiv(a.MT, ct);
-    int64_t per_layer = 8 / layers;
-    if (one_a_unit) {
-        const int64_t want = cdiv(cdiv(rt * a.groups, 256), 4) * 4, most = layers == 3 ? 4 : ROWS_MAX_WAVES / layers;
-        per_layer = want < 4 ? 4 : want > most ? most : want;
-        if (f16_numbers && layers == 1 && per_layer < 8) per_layer = 8;
-    }
-    if (shape) per_layer = shape >> 4 & 31;
-    int64_t splits = cdiv(a.groups, per_layer);
-    while (splits > 1 && rt * splits > (one_a_unit ? 256 : 512)) splits--;
-    if (shape >> 12) splits = shape >> 12;
-    const int64_t waves = layers * per_layer;
-    a.splits = (int)splits;
-    a.first_lds = (int)rows_first_lds(M, K, packed ? 1 : layers, layers, bits);
-    a.gather = bits && splits == 1 ? (int)k_tiles(M) * 8 : 0;
+    const RowsPlan p = rows_plan(N, M, K, layers, packed, out_dtype, shape);
+    if (p.lds > (64 << 10)) return fail(BGEMM_EINVAL, "%s: launch shape %d needs %lld bytes of LDS", who, shape, (long long)p.lds);
+    a.groups = (int)p.groups; a.splits = (int)p.splits; a.own = (int)p.own;
+    a.first_lds = (int)p.first_lds;
+    a.gather = bits && p.splits == 1 ? (int)k_tiles(M) * 8 : 0;
     // Past the caches where no two blocks share a 64-byte piece of a row (fp32 8192 x 768 x 3072 34.3 -> 28.9, 4096 x 1024 x 4096 26.6 ->
     // 19.7, fp16 8192 x 768 x 768 12.9 -> 11.0; rows of 4000 bytes 19.0 -> 20.3, of fp16 6176 26.5 -> 28.6).
     a.nt = M * (f32 ? 4 : 2) % 64 == 0;
-    const size_t lds = (size_t)rows_lds(M, K, packed ? 1 : layers, layers, bits);
-    const dim3 grid((unsigned)(rt * splits)), block((unsigned)(waves * 64));
+    const size_t lds = (size_t)p.lds;
+    const int ct = (int)p.ct;
+    const dim3 grid((unsigned)(row_tiles(N) * p.splits)), block((unsigned)(layers * p.per_layer * 64));
     const hipStream_t st = (hipStream_t)stream;
     auto go = [&](auto src, auto kind) {
         constexpr int SRC = decltype(src)::value, KIND = decltype(kind)::value;
