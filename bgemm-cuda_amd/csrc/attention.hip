@@ -15,7 +15,11 @@
 // stay in the lane, and the order of the keys in a fragment is chosen such that a lane holds 32 consecutive ones: its bits are a
 // word, and that word, four ways shifted, is the second product's operand as it stands.  The scores are multiplied twice, once for
 // the sums and once for the bits: one MFMA per 32 x 32 tile and 64 of D, cheaper than keeping S of them a lane.
-// That size takes 37 us: 126 MB of scores and context written, 14 MB read (3.8 TB/s), vector units 46 % and matrix cores 4 % busy.
+// 16 x 512 tokens, 12 heads of 64: 100 MB of scores written in 30.7 us (3.3 TB/s; three waves a SIMD, vector units half busy, the rest of a
+// wave's time its chain of MFMA, table, LDS and store).  37 us with the table's index in two instructions, sums that were set to their
+// start tile by tile, operands of +-1 on both sides (11 vector instructions a word of keys instead of 5), and every wave waiting for
+// each word that a block prepares; the last also where there are few waves: 4 x 512 tokens 36 -> 16.4, 8 x 256 20 -> 10.2.  With a whole
+// group's sums on their way (210 registers, two waves a SIMD) 36.9.
 #include "common.h"
 #include "mfma_engines.h"
 #include "pack_bits.h"
@@ -35,18 +39,26 @@ struct AttnArgs {
 
 constexpr int ATTN_STAGE = 144;       // bytes of a staged row of 64 scores (padded)
 
-// One word of signed fp4 operands at step s: +1.0, or -1.0 where the bit is set; the same with 1.0 where it is set and 0 elsewhere.
-__device__ __forceinline__ unsigned attn_pm1(const unsigned w, const int s) { return (s == 3 ? w & 0x88888888u : (w << (3 - s)) & 0x88888888u) | 0x22222222u; }
-__device__ __forceinline__ unsigned attn_01(const unsigned w, const int s) { return (s == 0 ? w << 1 : w >> (s - 1)) & 0x22222222u; }
+// fp4 operands of one word at step s.  A bit that counts stays where it is (0.5, 1, 2; at step 3 it moves to 1.0), five instructions a
+// word; the other side has the reciprocals of those values: of a sign x = +-1 (given inverted) as -2 x, so that a sum that starts from
+// the sum of x is that of x (1 - 2 b), or of a bit as 1.
+__device__ __forceinline__ unsigned attn_bit(const unsigned w, const int s) { return s == 3 ? (w >> 2) & 0x22222222u : w & (0x11111111u << s); }
+__device__ __forceinline__ unsigned attn_sign(const unsigned inverted, const int s)
+{
+    return ((inverted << (3 - s)) & 0x88888888u) | (s == 0 ? 0x66666666u : s == 2 ? 0x22222222u : 0x44444444u);
+}
+__device__ __forceinline__ unsigned attn_one(const unsigned w, const int s)
+{
+    return s == 0 ? (w << 2) & 0x44444444u : s == 1 ? w & 0x22222222u : (w >> 2) & (s == 2 ? 0x11111111u : 0x22222222u);
+}
 
 // W: words a head (D = 32 W).  BITS: the context leaves as the next binary layer's operand.
 template <int W, bool BITS>
-__global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
+__global__ __launch_bounds__(512) void attention_kernel(const AttnArgs a)
 {
-    constexpr int D = W * 32, CH = (W + 1) / 2, PAD = CH * 64 - D;       // chunks of 64 bits, the last half a one if W is odd
+    constexpr int D = W * 32, CH = (W + 1) / 2;       // chunks of 64 bits, the last half a one if W is odd
     // a sum comes out as 2^23 + 2 * (matching bits): its bit pattern is an index
     constexpr unsigned BASE = 0x4b000000u;
-    constexpr float C0 = 8388608.f + (D - PAD);
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int h = lane >> 5, c = lane & 31;
@@ -66,33 +78,65 @@ __global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
         const __half s = score16(i);
         tbl[i] = make_uint2(__float_as_uint(expf(__half2float(s) - __half2float(score16(D)))), __half_as_ushort(s));
     }
-    for (int key = threadIdx.x; key < S64; key += blockDim.x)
+    // (a stretch of loads before its first use: one trip to the caches for several words, where each of a few waves would wait for its own)
+    constexpr int AHEAD = 4;
+    for (int key0 = threadIdx.x; key0 < S64; key0 += AHEAD * blockDim.x) {
+        uint32_t x[AHEAD][W];
 #pragma unroll
-        for (int w = 0; w < W; w++) kb[w * S64 + key] = key < S ? word(a.k, key, w) : 0u;
-    for (int u0 = wave * 2; u0 < a.groups * 2 * W; u0 += waves * 2) {
-        const int u = u0 + h, kw = u / W, w = u % W, key = kw * 32 + c;
-        const unsigned t = transpose32(__brev(key < S ? word(a.v, key, w) : 0u), lane);       // bit r: key r of the lane's column
-        vt[kw * D + w * 32 + c] = __brev(t);
+        for (int i = 0; i < AHEAD; i++)
+#pragma unroll
+            for (int w = 0; w < W; w++) x[i][w] = word(a.k, min(key0 + i * (int)blockDim.x, S - 1), w);
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            const int key = key0 + i * blockDim.x;
+            if (key < S64)
+#pragma unroll
+                for (int w = 0; w < W; w++) kb[w * S64 + key] = key < S ? x[i][w] : 0u;
+        }
     }
-    __syncthreads();
-
+    for (int u0 = wave * 2; u0 < a.groups * 2 * W; u0 += waves * 2 * AHEAD) {
+        uint32_t x[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            const int u = min(u0 + i * waves * 2 + h, a.groups * 2 * W - 1), kw = u / W, key = kw * 32 + c;
+            x[i] = word(a.v, min(key, S - 1), u % W);
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            const int u = u0 + i * waves * 2 + h, kw = u / W, w = u % W;
+            if (u0 + i * waves * 2 >= a.groups * 2 * W) break;
+            const unsigned t = transpose32(__brev(kw * 32 + c < S ? x[i] : 0u), lane);       // bit r: key r of the lane's column
+            if (u < a.groups * 2 * W) vt[kw * D + w * 32 + c] = __brev(t);
+        }
+    }
     const int q0 = (qb * waves + wave) * 32;
-    if (q0 >= S) return;
-    unsigned qf[CH][4];
+    unsigned qw[CH];
 #pragma unroll
     for (int ch = 0; ch < CH; ch++) {
         const int w = 2 * ch + h;
-        const unsigned x = w < W ? word(a.q, min(q0 + c, S - 1), w < W ? w : 0) : 0u;
-#pragma unroll
-        for (int s = 0; s < 4; s++) qf[ch][s] = attn_pm1(x, s);
+        qw[ch] = word(a.q, min(q0 + c, S - 1), w < W ? w : 0);
     }
+    __syncthreads();
+    if (q0 >= S) return;
+    unsigned qf[CH][4];
+    int ones = 0;
+#pragma unroll
+    for (int ch = 0; ch < CH; ch++) {
+        if (2 * ch + h < W) ones += __popc(qw[ch]);
+#pragma unroll
+        for (int s = 0; s < 4; s++) qf[ch][s] = attn_sign(~qw[ch], s);
+    }
+    ones += __shfl_xor(ones, 32);
+    // 2 * (matching bits) = D + (sum over the query's x of x (1 - 2 b)): what the sums start from
+    const float both = (float)(2 * D - 2 * ones);
+    EngF4::Acc start;
+#pragma unroll
+    for (int v = 0; v < 16; v++) start[v] = 8388608.f + both;
     // MFMA row r = 8 g + 4 half + i of tile j is key 32 half + 16 j + 4 g + i of the group's 64: register v of a lane is then key
     // 32 h + 16 j + v.  (The second product's rows, columns of V, likewise: register v is column 16 h + v.)
     const int row_key = 32 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3), row_col = 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3);
     auto tile = [&](const int grp, const int j) {
         EngF4::Acc acc;
-#pragma unroll
-        for (int v = 0; v < 16; v++) acc[v] = C0;
 #pragma unroll
         for (int ch = 0; ch < CH; ch++) {
             const int w = 2 * ch + h;
@@ -100,8 +144,8 @@ __global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
             if (W % 2 && ch == CH - 1 && h) x = 0;
             unsigned kf[4];
 #pragma unroll
-            for (int s = 0; s < 4; s++) kf[s] = attn_pm1(x, s);
-            acc = EngF4::mma(EngF4::make(kf), EngF4::make(qf[ch]), acc);
+            for (int s = 0; s < 4; s++) kf[s] = attn_bit(x, s);
+            acc = EngF4::mma(EngF4::make(kf), EngF4::make(qf[ch]), ch == 0 ? start : acc);
         }
         return acc;
     };
@@ -114,18 +158,31 @@ __global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
     // ---- scores out, sums of the exponentials --------------------------------------------------------------------------------------
     float s0 = 0.f, s1 = 0.f;
     const int r8 = lane >> 3, c8 = lane & 7;
-    __half* const srow = a.scores + ((int64_t)bh * S + q0 + r8) * S + c8 * 8;
+    __half* const matrix = a.scores + (int64_t)bh * S * S;
+    __half* const srow = matrix + (int64_t)(q0 + r8) * S + c8 * 8;
+    // (whole groups leave through a buffer that ends with the matrix: rows past the last one are dropped)
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(matrix, 0, S * S * 2, 0x00020000);
+    int voff[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) voff[i] = ((q0 + r8 + 8 * i) * S + c8 * 8) * 2;
+    // (an entry's address in LDS straight from the sum's bits: one instruction)
+    typedef unsigned pair_of __attribute__((ext_vector_type(2)));
+    typedef const __attribute__((address_space(3))) pair_of* lds_pair;
+    const uint32_t entry0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)tbl - (BASE << 2);
+    auto entry = [&](const float sum) { return *(lds_pair)(uintptr_t)(entry0 + (__float_as_uint(sum) << 2)); };
+    // (a tile's sums are on their way while the one before it is looked up)
+    EngF4::Acc even = tile(0, 0), odd;
     auto group_scores = [&](const int grp, auto tail_c) {
         constexpr bool TAIL = decltype(tail_c)::value;       // some of the group's keys do not exist
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const EngF4::Acc acc = tile(grp, j);
+            if (j == 0) odd = tile(grp, 1);
+            else even = tile(min(grp + 1, a.groups - 1), 0);
+            const EngF4::Acc& acc = j == 0 ? even : odd;
             unsigned hs[8];
 #pragma unroll
             for (int p = 0; p < 8; p++) {
-                const unsigned o0 = (__float_as_uint(acc[2 * p]) - BASE) << 2, o1 = (__float_as_uint(acc[2 * p + 1]) - BASE) << 2;
-                const uint2 e0 = *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(tbl) + o0);
-                const uint2 e1 = *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(tbl) + o1);
+                const pair_of e0 = entry(acc[2 * p]), e1 = entry(acc[2 * p + 1]);
                 const int key = grp * 64 + 32 * h + 16 * j + 2 * p;
                 s0 += !TAIL || key < S ? __uint_as_float(e0.x) : 0.f;
                 s1 += !TAIL || key + 1 < S ? __uint_as_float(e1.x) : 0.f;
@@ -139,19 +196,20 @@ __global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const uint4 x = *reinterpret_cast<const uint4*>(stage + (r8 + 8 * i) * ATTN_STAGE + c8 * 16);
-            __half* const to = srow + (int64_t)(8 * i) * S + grp * 64;
-            if (q0 + r8 + 8 * i < S) {
-                if (!TAIL && a.past) {
-                    // (as an instruction: a builtin beside an ordinary store of the same value becomes one ordinary store.  The s_nop is the
-                    // hazard between a wide store and a write to its data registers.)
-                    const v4i v = {(int)x.x, (int)x.y, (int)x.z, (int)x.w};
-                    asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" : : "v"(to), "v"(v) : "memory");
-                } else if (!TAIL || grp * 64 + c8 * 8 + 8 <= S) __builtin_memcpy(to, &x, 16);
-                else {
-                    const unsigned d[4] = {x.x, x.y, x.z, x.w};
+            if constexpr (!TAIL) {
+                const v4i v = {(int)x.x, (int)x.y, (int)x.z, (int)x.w};
+                if (a.past) __builtin_amdgcn_raw_buffer_store_b128(v, rs, voff[i], grp * 128, 2);
+                else __builtin_amdgcn_raw_buffer_store_b128(v, rs, voff[i], grp * 128, 0);
+            } else {
+                __half* const to = srow + (int64_t)(8 * i) * S + grp * 64;
+                if (q0 + r8 + 8 * i < S) {
+                    if (grp * 64 + c8 * 8 + 8 <= S) __builtin_memcpy(to, &x, 16);
+                    else {
+                        const unsigned d[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
-                    for (int e = 0; e < 7; e++)
-                        if (grp * 64 + c8 * 8 + e < S) to[e] = __ushort_as_half((uint16_t)(d[e >> 1] >> (16 * (e & 1))));
+                        for (int e = 0; e < 7; e++)
+                            if (grp * 64 + c8 * 8 + e < S) to[e] = __ushort_as_half((uint16_t)(d[e >> 1] >> (16 * (e & 1))));
+                    }
                 }
             }
         }
@@ -171,37 +229,50 @@ __global__ __launch_bounds__(256) void attention_kernel(const AttnArgs a)
         if (__half2float(__float2half_rn(__fdiv_rn(__uint_as_float(tbl[mid].x), total))) >= a.level) hi = mid;
         else lo = mid + 1;
     }
-    const unsigned first = BASE + 2 * lo;
+    // the sums less that level: negative where a probability counts as 0
+#pragma unroll
+    for (int v = 0; v < 16; v++) start[v] = both - (float)(2 * lo);
 
     // ---- bits of the probabilities, context --------------------------------------------------------------------------------------
+    // ctx: keys that count and whose sign of V is negative
     EngF4::Acc ctx[W];
 #pragma unroll
     for (int t = 0; t < W; t++)
 #pragma unroll
         for (int v = 0; v < 16; v++) ctx[t][v] = 0.f;
+    int counted = 0;
+    even = tile(0, 0);
 #pragma unroll 1
     for (int grp = 0; grp < a.groups; grp++) {
         unsigned below = 0;               // key 32 h + r of the group at bit 31 - r: set where its probability counts as 0
+        odd = tile(grp, 1);
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const EngF4::Acc acc = tile(grp, j);
+        for (int v = 0; v < 16; v++) below = __builtin_amdgcn_alignbit(below, __float_as_uint(even[v]), 31);
+        even = tile(min(grp + 1, a.groups - 1), 0);
 #pragma unroll
-            for (int v = 0; v < 16; v++) below = __builtin_amdgcn_alignbit(below, __float_as_uint(acc[v]) - first, 31);
-        }
+        for (int v = 0; v < 16; v++) below = __builtin_amdgcn_alignbit(below, __float_as_uint(odd[v]), 31);
         const int left = S - (grp * 64 + 32 * h);
         if (left < 32) below |= left <= 0 ? 0xffffffffu : 0xffffffffu >> left;
+        const unsigned counts = ~below;
+        counted += __popc(counts);
         unsigned pf[4];
 #pragma unroll
-        for (int s = 0; s < 4; s++) pf[s] = attn_01(~below, s);
+        for (int s = 0; s < 4; s++) pf[s] = attn_one(counts, s);
 #pragma unroll
         for (int t = 0; t < W; t++) {
             const unsigned x = vt[(2 * grp + h) * D + t * 32 + row_col];
             unsigned vf[4];
 #pragma unroll
-            for (int s = 0; s < 4; s++) vf[s] = attn_pm1(x, s);
+            for (int s = 0; s < 4; s++) vf[s] = attn_bit(x, s);
             ctx[t] = EngF4::mma(EngF4::make(vf), EngF4::make(pf), ctx[t]);
         }
     }
+    counted += __shfl_xor(counted, 32);
+    // the sum of the signs
+#pragma unroll
+    for (int t = 0; t < W; t++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) ctx[t][v] = fmaf(-2.f, ctx[t][v], (float)counted);
     if constexpr (BITS) {
         // a lane's 16 columns of its query, joined with the other half's: a word a head and 32 columns
         const float zp = !a.zp ? 0.f : a.f32 ? *reinterpret_cast<const float*>(a.zp) : __half2float(*reinterpret_cast<const __half*>(a.zp));
@@ -265,11 +336,14 @@ static int attention(const char* who, const void* q, const void* k, const void* 
     a.S = (int)seq; a.heads = (int)heads; a.groups = (int)cdiv(seq, 64); a.f32 = context_type == BGEMM_SRC_F32; a.past = seq % 32 == 0 && ((uintptr_t)scores & 63) == 0;
     a.scale = 1.0f / (float)sqrt((double)head_size);
     a.level = (float)(1.0 / (double)seq);
-    // four waves share a block's operands; fewer where that leaves the chip without two blocks a compute unit
-    int waves = 4;
-    while (waves > 1 && batch * heads * cdiv(seq, 32 * waves) < 512) waves /= 2;
+    // Four waves share a block's operands, or eight where that needs no more rounds of waves a compute unit: what a block prepares is a
+    // chain of its own, as long as a few groups of keys (us, heads of 64, 1 / 2 / 4 / 8 waves: 12 heads 4 x 512 tokens 33.7 / 27.2 / 19.6 /
+    // 20.3, 8 x 512 39.5 / 28.7 / 24.2 / 20.8, 16 x 512 73.6 / 41.9 / 33.9 / 36.2, 4 heads 64 tokens 7.3 / 6.4 / 6.3 / 6.4).
+    auto rounds = [&](const int w) { return cdiv(batch * heads * cdiv(seq, 32 * w), 256) * w; };
+    auto lds_bytes = [&](const int w) { return (size_t)w * 32 * ATTN_STAGE + (head_size + 2) * 8 + (size_t)2 * W * a.groups * 64 * 4; };
+    const int waves = rounds(8) <= rounds(4) && lds_bytes(8) <= (64 << 10) ? 8 : 4;
     a.qblocks = (int)cdiv(seq, 32 * waves);
-    const size_t lds = (size_t)waves * 32 * ATTN_STAGE + (head_size + 2) * 8 + (size_t)2 * W * a.groups * 64 * 4;
+    const size_t lds = lds_bytes(waves);
     const dim3 grid((unsigned)(batch * heads * a.qblocks)), block(waves * 64);
     const hipStream_t st = (hipStream_t)stream;
     auto go = [&](auto numbers, auto as_bits) {
