@@ -10,7 +10,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 SO = os.path.join(HERE, "libbgemm_mi355x.so")
 NATIVE_SO = os.path.join(HERE, "_bgemm_native.so")
-SOURCES = ["api.hip", "pack.hip", "gemm_mfma.hip", "gemm_valu.hip", "gemm_skinny.hip", "gemm_chain.hip", "linear_rows.hip", "train.hip", "attention.hip", "attention_grad.hip"]
+SOURCES = ["api.hip", "pack.hip", "gemm_mfma.hip", "gemm_valu.hip", "gemm_skinny.hip", "gemm_chain.hip", "linear_rows.hip", "train.hip", "attention.hip", "attention_products.hip", "attention_grad.hip"]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
          # "#pragma unroll" on loops with run-time bounds is a request, not a requirement
          "-Wno-pass-failed",

@@ -75,6 +75,8 @@ SIGNATURES = {
     "bgemm_attention_supported": (_int, [_i64, _i64, _i64, _i64]),
     "bgemm_attention_forward": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p, _int, _p]),
     "bgemm_attention_forward_bits": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _int, _p]),
+    "bgemm_scores_forward": (_int, [_int, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p]),
+    "bgemm_context_forward": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p]),
     "bgemm_scores_backward": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p]),
     "bgemm_context_backward": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p]),
     "bgemm_chain_workspace_bytes": (_sz, [_int, _p, _int, _i64]),

@@ -21,8 +21,7 @@
 // each word that a block prepares; the last also where there are few waves: 4 x 512 tokens 36 -> 16.4, 8 x 256 20 -> 10.2.  With a whole
 // group's sums on their way (210 registers, two waves a SIMD) 36.9.
 #include "common.h"
-#include "mfma_engines.h"
-#include "pack_bits.h"
+#include "attention_bits.h"
 #include <math.h>
 #include <type_traits>
 
@@ -36,21 +35,6 @@ struct AttnArgs {
     int S, heads, groups, qblocks, f32, past;      // past: scores are stored past the caches
     float scale, level;               // 1 / sqrt(D), 1 / S
 };
-
-constexpr int ATTN_STAGE = 144;       // bytes of a staged row of 64 scores (padded)
-
-// fp4 operands of one word at step s.  A bit that counts stays where it is (0.5, 1, 2; at step 3 it moves to 1.0), five instructions a
-// word; the other side has the reciprocals of those values: of a sign x = +-1 (given inverted) as -2 x, so that a sum that starts from
-// the sum of x is that of x (1 - 2 b), or of a bit as 1.
-__device__ __forceinline__ unsigned attn_bit(const unsigned w, const int s) { return s == 3 ? (w >> 2) & 0x22222222u : w & (0x11111111u << s); }
-__device__ __forceinline__ unsigned attn_sign(const unsigned inverted, const int s)
-{
-    return ((inverted << (3 - s)) & 0x88888888u) | (s == 0 ? 0x66666666u : s == 2 ? 0x22222222u : 0x44444444u);
-}
-__device__ __forceinline__ unsigned attn_one(const unsigned w, const int s)
-{
-    return s == 0 ? (w << 2) & 0x44444444u : s == 1 ? w & 0x22222222u : (w >> 2) & (s == 2 ? 0x11111111u : 0x22222222u);
-}
 
 // W: words a head (D = 32 W).  BITS: the context leaves as the next binary layer's operand.
 template <int W, bool BITS>
@@ -149,12 +133,6 @@ __global__ __launch_bounds__(512) void attention_kernel(const AttnArgs a)
         }
         return acc;
     };
-    auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-
     // ---- scores out, sums of the exponentials --------------------------------------------------------------------------------------
     float s0 = 0.f, s1 = 0.f;
     const int r8 = lane >> 3, c8 = lane & 7;
@@ -192,7 +170,7 @@ __global__ __launch_bounds__(512) void attention_kernel(const AttnArgs a)
             to[0] = make_uint4(hs[0], hs[1], hs[2], hs[3]);
             to[1] = make_uint4(hs[4], hs[5], hs[6], hs[7]);
         }
-        wave_sync();
+        attn_wave_sync();
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const uint4 x = *reinterpret_cast<const uint4*>(stage + (r8 + 8 * i) * ATTN_STAGE + c8 * 16);
@@ -213,7 +191,7 @@ __global__ __launch_bounds__(512) void attention_kernel(const AttnArgs a)
                 }
             }
         }
-        wave_sync();
+        attn_wave_sync();
     };
     const int whole = S / 64;
 #pragma unroll 1

@@ -9,8 +9,8 @@
 // the halving, copies of the head-split gradients) 12 heads of 64, 4 x 512 tokens, took 20 launches and a dozen passes over 25 MB;
 // here each product pair is one launch that reads or writes an [N][M] matrix once a product, in its own order, and the gradients
 // leave in the operands' strides.  What is left is that traffic: the contraction is D = 32 .. 128 long on one side, far below what
-// the matrix cores could do in the time.  Both forward products and both backward ones of that size, a training step: 392 -> 258 us,
-// of which the host's part is now the larger: the kernels here take 31 (context) and 19 us (scores), neither bandwidth's (3.1 and 5.3
+// the matrix cores could do in the time.  A training step of both products is that of the host, 160 us in all; of its 68 us of kernels
+// those here take 31 (context) and 19 us (scores), neither bandwidth's (3.1 and 5.3
 // TB/s counted) nor the matrix cores' (5 % busy): waves wait for 47 and 44 % of their cycles, and LDS, where fragments that lie across
 // the rows are read two bytes a lane, is active for 18 and 33 % of the compute units' time.
 #include "common.h"

@@ -403,7 +403,24 @@ Batch batch_of(const Tensor& t)
     return t.dim() == 3 ? Batch{1, t.size(0), 0, t.stride(0)} : Batch{t.size(0), t.size(1), t.stride(0), t.stride(1)};
 }
 
-// batched_product(x [.., N, K], right [.., K, M], mode) -> fp16 [.., N, M]: both operands packed where they lie, one GEMM over the batch
+// Whether the one-launch kernels are ahead of two packs and a GEMM (us, batch x rows x columns, D).  The scores' is until what it writes
+// outgrows the caches, where the GEMM's own store order is as good: 48 x 512^2, 64 14.5 -> 7.0; 192 x 512^2, 128 37.6 -> 30.5;
+// 192 x 340^2, 96 31.9 -> 23.7; 2 x 32^2, 32 10.3 -> 3.4; but 128 x 1024^2, 128 67.9 -> 70.4, 16 x 4096^2, 32 96.4 -> 101.3.
+bool scores_in_one(const int64_t batch, const int64_t N, const int64_t M, const int64_t D)
+{
+    return (D == 32 || D == 64 || D == 96 || D == 128) && N <= 1 << 20 && M <= 1 << 20 && N * M < 1 << 27 && batch * N * M < 1 << 27;
+}
+
+// The context's packs a matrix' [M][D] values again in each block, which has to stay a small part of its work: 48 x 512^2, 64 20.5 -> 10.8;
+// 192 x 256^2, 128 24.7 -> 21.7; 192 x 1024^2, 32 98.6 -> 86.1; 12 x 1024^2, 64 22.2 -> 15.8; 2 x 2048^2, 32 17.3 -> 16.3; but one
+// 2048^2, 32 14.8 -> 16.3, 192 x 1024^2, 64 110.6 -> 112.8, 192 x 512^2, 128 40.9 -> 40.8, 64 x 1024^2, 128 44.1 -> 56.6.
+bool context_in_one(const int64_t batch, const int64_t N, const int64_t M, const int64_t D)
+{
+    return (D == 32 || D == 64 || D == 96 || D == 128) && N <= 1 << 20 && M >= 8 && (M * D <= 1 << 15 || (M * D <= 1 << 16 && D <= 64 && batch > 1 && batch * N * M < 1 << 27));
+}
+
+// batched_product(x [.., N, K], right [.., K, M], mode) -> fp16 [.., N, M]: one launch on fp16 operands of an attention product's form,
+// else both operands packed where they lie and one GEMM over the batch
 PyObject* batched_product(PyObject*, PyObject* const* args, const Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
@@ -427,22 +444,31 @@ PyObject* batched_product(PyObject*, PyObject* const* args, const Py_ssize_t n)
     {
         const WithoutGil no_gil;
         const c10::OptionalDeviceGuard guard(x.device());
-        const int64_t wx = bgemm_tiled_words(N, K), wr = bgemm_tiled_words(M, K);
         const auto options = x.options().requires_grad(false);
-        const Tensor planes = at::empty({batch * (wx + wr)}, options.dtype(at::kInt));
-        int32_t* const px = planes.data_ptr<int32_t>();
-        int32_t* const pr = px + batch * wx;
-        void* const st = stream_of(x);
         std::vector<int64_t> shape = x.sizes().vec();
         shape.back() = M;
         out = at::empty(shape, options.dtype(at::kHalf));
-        check(bgemm_pack_batched(x.data_ptr(), src_type(x), 0, nullptr, bx.outer, bx.inner, N, K, x.stride(-2), bx.so, bx.si, px, nullptr, st));
-        if (by_rows)
-            check(bgemm_pack_batched(right.data_ptr(), src_type(right), 0, nullptr, br.outer, br.inner, M, K, right.stride(-1), br.so, br.si, pr, nullptr, st));
-        else
-            check(bgemm_pack_transposed_batched(right.data_ptr(), src_type(right), br.outer, br.inner, M, K, right.stride(-2), br.so, br.si, pr, st));
-        check(bgemm_packed_forward(mode, pr, px, nullptr, out.data_ptr(), BGEMM_OUT_F16, batch, M, N, K, batch > 1 ? wr : 0, batch > 1 ? wx : 0, N * M, 1, BGEMM_VARIANT_AUTO,
-                                   nullptr, 0, nullptr, 0, st));
+        void* const st = stream_of(x);
+        const bool half = x.scalar_type() == at::kHalf && right.scalar_type() == at::kHalf;
+        const bool scores = half && (mode == BGEMM_MODE_XOR || mode == BGEMM_MODE_AND) && by_rows && scores_in_one(batch, N, M, K);
+        const bool context = half && mode == BGEMM_MODE_ATTN_X && by_columns && context_in_one(batch, N, K, M);
+        if (scores || context) {
+            const int64_t strides[6] = {bx.so, bx.si, x.stride(-2), br.so, br.si, scores ? right.stride(-1) : right.stride(-2)};
+            check(scores ? bgemm_scores_forward(mode, x.data_ptr(), right.data_ptr(), strides, batch, bx.inner, N, M, K, out.data_ptr(), st)
+                         : bgemm_context_forward(x.data_ptr(), right.data_ptr(), strides, batch, bx.inner, N, K, M, out.data_ptr(), st));
+        } else {
+            const int64_t wx = bgemm_tiled_words(N, K), wr = bgemm_tiled_words(M, K);
+            const Tensor planes = at::empty({batch * (wx + wr)}, options.dtype(at::kInt));
+            int32_t* const px = planes.data_ptr<int32_t>();
+            int32_t* const pr = px + batch * wx;
+            check(bgemm_pack_batched(x.data_ptr(), src_type(x), 0, nullptr, bx.outer, bx.inner, N, K, x.stride(-2), bx.so, bx.si, px, nullptr, st));
+            if (by_rows)
+                check(bgemm_pack_batched(right.data_ptr(), src_type(right), 0, nullptr, br.outer, br.inner, M, K, right.stride(-1), br.so, br.si, pr, nullptr, st));
+            else
+                check(bgemm_pack_transposed_batched(right.data_ptr(), src_type(right), br.outer, br.inner, M, K, right.stride(-2), br.so, br.si, pr, st));
+            check(bgemm_packed_forward(mode, pr, px, nullptr, out.data_ptr(), BGEMM_OUT_F16, batch, M, N, K, batch > 1 ? wr : 0, batch > 1 ? wx : 0, N * M, 1, BGEMM_VARIANT_AUTO,
+                                       nullptr, 0, nullptr, 0, st));
+        }
     }
     return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS

@@ -357,6 +357,17 @@ int bgemm_attention_forward(const void* q, const void* k, const void* v, int64_t
 int bgemm_attention_forward_bits(const void* q, const void* k, const void* v, int64_t batch, int64_t seq, int64_t heads, int64_t head_size,
                                  void* scores, void* context_bits, const void* zero_point, int context_type, void* stream);
 
+/* ---- both attention products on fp16 operands where they lie, one launch each ---------------------
+ * (tests/python/bgemm_linear.py:9-61 on `batch` matrices, `inner` to an outer one.)  out fp16, dense.
+ *   scores   a [N][D], b [M][D]: out [N][M] = sign(a[n]) . sign(b[m]) (BGEMM_MODE_XOR), or the columns where both are negative (_AND)
+ *   context  probs [N][M], value [M][D]: out [N][D] = sum over the m with the sign bit of probs[n][m] clear of sign(value[m])
+ * strides: 6 numbers, the outer, inner and row stride in elements of the two operands; the last dimension is dense.  D is 32, 64, 96 or
+ * 128; context: 8 <= M, M * D <= 2^17, out 16-byte aligned; EINVAL otherwise. */
+int bgemm_scores_forward(int mode, const void* a, const void* b, const int64_t* strides, int64_t batch, int64_t inner, int64_t N, int64_t M,
+                         int64_t D, void* out, void* stream);
+int bgemm_context_forward(const void* probs, const void* value, const int64_t* strides, int64_t batch, int64_t inner, int64_t N, int64_t M,
+                          int64_t D, void* out, void* stream);
+
 /* ---- gradients of both attention products, one launch each ----------------------------------------
  * (tests/python/bgemm_linear.py:28-42, 64-86 on `batch` matrices, `inner` to an outer one.)  fp16 throughout, sums in fp32; sign(0) = 0.
  *   scores   a [N][D], b [M][D], grad_scores [N][M] dense:
