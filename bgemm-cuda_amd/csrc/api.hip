@@ -229,7 +229,7 @@ static int packed_forward(int mode, const void* W_tiled, const void* X_tiled, co
         return v == BGEMM_VARIANT_VALU ? BGEMM_KERNEL_VALU
                : force >= 0            ? force
                : skinny                ? gemm_skinny_kernel_id(a, fp4)
-                                       : gemm_mfma_kernel_id(batch, M, N, a.KT, a.mc.planes, out_elem_shift(a.out_kind), fp4);
+                                       : gemm_mfma_kernel_id(batch, M, N, a.KT, a.mc.planes, a.out_kind, fp4);
     if (splitK > 1 && v == BGEMM_VARIANT_VALU) {
         size_t part, cnt;
         ws_needs(v, a.mc.planes, batch, M, N, K, splitK, &part, &cnt);

@@ -14,25 +14,84 @@
 
 namespace bgemm {
 
+// What is left of a product beside its whole 256 x 128 tiles, one 32 x 32 tile a block: the four waves take the K-tiles in turn and
+// their sums meet in LDS.  Four loads of each operand a wave are in flight: a block is a few trips to L2 long.
+template <typename Eng>
+__device__ __forceinline__ void edge_tile(const GemmArgs& a, const int rt, const int ct, int* const sums)
+{
+    constexpr int AHEAD = 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint4* xp = a.X + (int64_t)rt * a.KT * TILE_U4 + lane;
+    const uint4* wp = a.W + (int64_t)ct * a.KT * TILE_U4 + lane;
+    typename Eng::Acc acc;
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = 0;
+    int px = 0, pw = 0;
+    for (int kt0 = wave; kt0 < a.KT; kt0 += 4 * AHEAD) {
+        uint4 x[AHEAD], w[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            const int kt = min(kt0 + 4 * i, a.KT - 1);
+            x[i] = xp[(int64_t)kt * TILE_U4];
+            w[i] = wp[(int64_t)kt * TILE_U4];
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            if (kt0 + 4 * i >= a.KT) break;
+            px += popc4(x[i]);
+            pw += popc4(w[i]);
+#pragma unroll
+            for (int s = 0; s < Eng::STEPS; s++) acc = Eng::mma(Eng::expand_x(x[i], s), Eng::expand_w(w[i], s), acc);
+        }
+    }
+    // [wave][16 values, activation bits, weight bits][lane]
+    int* const mine = sums + wave * 18 * 64 + lane;
+#pragma unroll
+    for (int v = 0; v < 16; v++) mine[v * 64] = Eng::to_int(acc, v);
+    mine[16 * 64] = px;
+    mine[17 * 64] = pw;
+    __syncthreads();
+    auto total = [&](const int k, const int l) {
+        int t = 0;
+#pragma unroll
+        for (int w = 0; w < 4; w++) t += sums[(w * 18 + k) * 64 + l];
+        return t;
+    };
+    const int col = lane & 31, half = lane >> 5;
+    const int64_t m = (int64_t)ct * 32 + col;
+    const int colterm = a.mc.c0 * (int)a.K + a.mc.ca * (total(17, col) + total(17, col + 32));
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int r = 8 * wave + 4 * half + i;
+        const int64_t n = (int64_t)rt * 32 + r;
+        if (n >= a.N || m >= a.M) continue;
+        store_out(a, n * a.M, m, colterm + a.mc.cb * (total(16, r) + total(16, r + 32)) + dot_term(a.mc, total(4 * wave + i, lane)));
+    }
+}
+
 // Block = WGN x WGM waves, each wave owns WN x WM tiles of 32x32 outputs, PL activation planes.
 // COUNTED (pipelined tiles only): the operands' row popcounts come with the call (GemmArgs::cntW / cntX) and the main
 // loop counts nothing: a sixth of its vector instructions on the 256 x 128 tile.
 // TERN (pipelined, fp4 engine, PL = 1): binary weights x ternary activations with signed operands (EngF4::tern_x / tern_w):
 // a slot of the activation side is made of both planes' raw words, one MFMA does what takes the AND-dot two, and the
 // accumulators hold the output itself: no popcounts, no rank-one terms.
-template <typename Eng, int WGN, int WGM, int WN, int WM, int PL, bool PIPE, bool COUNTED = false, bool TERN = false>
+// EDGES (pipelined tiles, one product, values out): the grid's tiles_n x tiles_m are whole tiles, and `edges` blocks, a multiple of eight,
+// the 32 x 32 tiles below and beside them (edge_tile).  They come first; behind a tile a compute unit at most, last: a unit's second place
+// is theirs then, and none gets two tiles while another has none (1030 x 8200 x 6200 -> fp16: 32.5 -> 22.4 us).
+template <typename Eng, int WGN, int WGM, int WN, int WM, int PL, bool PIPE, bool COUNTED = false, bool TERN = false, bool EDGES = false>
 // (Second launch bound: from two waves a SIMD on, a wave's register budget is the 256 architected registers, and the
 // compiler then keeps the accumulators there instead of in the accumulation registers, which the epilogue could
 // only reach through one copy per value.)
 __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void gemm_mfma_kernel(const GemmArgs a, const int tiles_n,
-                                                                   const int tiles_m)
+                                                                   const int tiles_m, const int edges)
 {
     // the wave index as a scalar: tile coordinates and operand bases stay on the scalar unit
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave / WGM, wm = wave % WGM;
 
     // logical block id: XCD-contiguous (see xcd_contiguous_id)
-    const unsigned bid = xcd_contiguous_id(blockIdx.x, gridDim.x);
+    const unsigned blocks = EDGES ? tiles_n * tiles_m : gridDim.x, ahead = EDGES && blocks > 256 ? edges : 0, block_id = blockIdx.x - ahead;
+    const unsigned bid = xcd_contiguous_id(block_id, blocks);
     const int per_gemm = tiles_n * tiles_m;
     const int tile_id = bid % per_gemm, b = bid / per_gemm;
     // Tiles are walked in bands along n, so that the blocks in flight share their weight panels: eight tile rows, or two
@@ -45,11 +104,11 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
     // (the other way round where only that divides, below 32 K-tiles)
     if (a.KT < 32 && (tiles_n % sn != 0 || tiles_m % (8 / sn) != 0)) sn = 8 / sn;
     const int sm = 8 / sn;
-    if (WGN * WN * 32 >= 128 && gridDim.x == (unsigned)per_gemm && tiles_n % sn == 0 && tiles_m % sm == 0) {
+    if (WGN * WN * 32 >= 128 && blocks == (unsigned)per_gemm && tiles_n % sn == 0 && tiles_m % sm == 0) {
         // One GEMM on the tall tiles whose tile grid splits evenly: XCD x (the hardware's block id modulo 8) takes a
         // sub-rectangle of the grid, 1/2 x 1/4 of it (1/4 x 1/2 on a short K), and walks that in bands: its L2 then
         // needs a half and a quarter of the operands instead of an eighth of one and all of the other.
-        const int x = blockIdx.x % 8, y = blockIdx.x / 8, sub_n = tiles_n / sn, sub_m = tiles_m / sm;
+        const int x = block_id % 8, y = block_id / 8, sub_n = tiles_n / sn, sub_m = tiles_m / sm;
         const int bd = y / (band * sub_m), ib = y % (band * sub_m);
         const int n0 = bd * band, bh = min(band, sub_n - n0);
         tn_block = (x / sm) * sub_n + n0 + ib % bh;
@@ -74,6 +133,16 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
                                              // different LDS banks)
     __shared__ __align__(16) int rowp[WGN * WGM * WN * 32];
     __shared__ __align__(16) int stage[WGN * WGM * 32 * ROW_I];
+    if constexpr (EDGES) {
+        static_assert(WGN * WGM == 4 && 4 * 32 * ROW_I >= 4 * 18 * 64, "edge_tile's sums take the staging area");
+        if (block_id >= blocks) {
+            // the rows below the whole tiles, over all columns; then what is beside them
+            const int e = ahead ? blockIdx.x : blockIdx.x - blocks, n0 = tiles_n * WGN * WN, m0 = tiles_m * WGM * WM, below = (a.NT - n0) * a.MT, right = a.MT - m0;
+            if (e < below) edge_tile<Eng>(a, n0 + e / a.MT, e % a.MT, stage);
+            else if (e < below + n0 * right) edge_tile<Eng>(a, (e - below) / right, m0 + (e - below) % right, stage);
+            return;
+        }
+    }
     // The tile's work is a function object of its own: written straight into the kernel body the same code came
     // out with 10 to 25 % more registers (113 against 89 for the 64 x 128 tile: three waves a SIMD instead of four).
   auto do_tile = [&](const int tn) {
@@ -447,7 +516,10 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
         // block's neighbours still need would otherwise leave the L2 for the output lines (weights rotating through HBM:
         // 16384 x 8192 x 4096 198.1 -> 184.4 us, 8192^2 x 2048 63.5 -> 61.0, 11008 x 2048 x 4096 40.8 -> 39.5; on four K-tiles
         // ordinary stores are 7 % ahead, 8192^2 x 1024 49.0 against 52.4, from 32 on there is no difference)
-        if (a.nt_store || (a.KT >= 8 && a.KT < 32)) rows_out(std::true_type{});
+        // Not on rows that share lines, unless they are few: the L2 puts those together (8195^2 x 2048 152.0 -> 81.8 us, 4096 x 4104 x 2048
+        // 37.5 -> 24.9, 2000 x 3001 x 2048 (24 MB) 14.4 -> 13.0; but 8192 x 515 x 2048 (17 MB) 11.7 against 12.7), edge tiles' with them.
+        const bool share = (row_b & 63) != 0 && (EDGES || a.batch * a.N * row_b > (20 << 20));
+        if ((a.nt_store || (a.KT >= 8 && a.KT < 32)) && !share) rows_out(std::true_type{});
         else rows_out(std::false_type{});
         return;
     }
@@ -532,7 +604,7 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
     // fp16: 121 -> 99 us, fp32 scaled 148 -> 130; 4096 x 768 x 3080 fp16 scaled (25 MB) 18.0 -> 15.7; but 2048 x 4096 x 4104
     // (17 MB) 21.7 past the caches against 22.8).  Stored element by element, ragged rows took
     // 64 us instead of 43 (2053 x 4345 x 8195 -> fp16), scaled 98 instead of 44, 8192 x 768 x 3075 37 instead of 20.
-    const bool past = a.row_aligned && ((row_bytes & 63) == 0 || a.batch * a.N * row_bytes <= (20 << 20));
+    const bool past = a.row_aligned && ((row_bytes & 63) == 0 || (!EDGES && a.batch * a.N * row_bytes <= (20 << 20)));
     // Plain fp16: the integers are rounded once, staged as halves, and a
     // lane reads back the eight it stores with one 16-byte LDS read (no conversion behind the staging).
     if (a.out_kind == BGEMM_OUT_F16) {
@@ -790,6 +862,38 @@ static MfmaCfg pick_cfg(int64_t batch, int64_t M, int64_t N, int64_t KT, int pla
     return {BGEMM_KERNEL_MFMA_32x128, 32, 128};
 }
 
+// Whether a product runs its whole 256 x 128 tiles and leaves the rest to edge_tile: where the tiles that are not whole take a round of
+// blocks more (512 tiles at once, or the first 256 alone on their units at 0.87 of the rate; us, int32 / fp16 out): 2053 x 8195 x 4345
+// (585 tiles, 512 whole, 321 edge blocks) 53.9 -> 35.5 / 41.3 -> 35.8, 4100 x 4100 x 16384 100.1 -> 83.7, 1030 x 8200 x 6200 (325, 256, 289)
+// 29.8 -> 24.0 / 27.7 -> 22.8, 8195^2 x 8192 182 -> 174; where none is saved there is no gain (4099 x 6145 x 4000, 833 tiles, 768 whole:
+// 45.2 -> 45.9 fp16).  Few edge blocks beside the tiles: 2150 x 8200 x 4096 (1092) 34.8 -> 35.7 fp16, x 12288 79.1 -> 75.1;
+// 1100 x 8200 x 16384 (803 on 256 tiles) 57.7 -> 52.8, 1150 x 8292 x 8192 (1168) 33.2 -> 34.7.
+static int64_t edge_blocks(const int64_t M, const int64_t N) { return row_tiles(N) * row_tiles(M) - N / 256 * 8 * (M / 128 * 4); }
+
+static bool edges_ahead(int64_t batch, int64_t M, int64_t N, int64_t KT, int planes, int out_kind, bool fp4)
+{
+    if (!fp4 || batch != 1 || planes != 1 || out_kind == BGEMM_OUT_BITS_F32 || out_kind == BGEMM_OUT_BITS_F16 || N < 256 || M < 128) return false;
+    const int64_t whole = (N / 256) * (M / 128), all = cdiv(N, 256) * cdiv(M, 128);
+    if (all > (1 << 20) || edge_blocks(M, N) > (KT < 32 ? 640 : whole <= 256 ? 800 : 1100)) return false;
+    auto half_rounds = [](const int64_t tiles) { return tiles / 512 * 2 + (tiles % 512 > 256 ? 2 : tiles % 512 > 0 ? 1 : 0); };
+    const int64_t saved = half_rounds(all) - half_rounds(whole);
+    if (saved < 1 || (all > 512 && half_rounds(whole) % 2 != 0)) return false;
+    return pick_cfg(1, M / 128 * 128, N / 256 * 256, KT, 1, out_elem_shift(out_kind), true).id == BGEMM_KERNEL_MFMA_256x128;
+}
+
+// 256 x 128 tiles and the edges beside them in one launch
+static int launch_edges(const GemmArgs& a, hipStream_t st)
+{
+    const int tiles_n = (int)(a.N / 256), tiles_m = (int)(a.M / 128), edges = (int)(cdiv(edge_blocks(a.M, a.N), 8) * 8);
+    const int64_t grid = (int64_t)tiles_n * tiles_m + edges;
+    if (grid > 0x7fffffffLL) return fail(BGEMM_EINVAL, "gemm_mfma: grid of %lld blocks", (long long)grid);
+    if (a.cntW && a.cntX)
+        hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 4, 2, 1, true, true, false, true>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, edges);
+    else
+        hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 4, 2, 1, true, false, false, true>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, edges);
+    return check_launch("gemm_mfma");
+}
+
 template <typename Eng, int WGN, int WGM, int WN, int WM>
 static int launch_cfg(const GemmArgs& a, hipStream_t st)
 {
@@ -808,12 +912,12 @@ static int launch_cfg(const GemmArgs& a, hipStream_t st)
                 const bool pairs2 = a.out_kind == BGEMM_OUT_F16 && a.row_aligned;
                 if (a.KT >= 8 && (!pairs2 || a.KT >= 16)) {
                     hipLaunchKernelGGL((gemm_mfma_kernel<Eng, WGN, WGM, WN, WM, 2, true>), dim3((unsigned)grid),
-                                       dim3(WGN * WGM * 64), 0, st, a, tiles_n, tiles_m);
+                                       dim3(WGN * WGM * 64), 0, st, a, tiles_n, tiles_m, 0);
                     return check_launch("gemm_mfma");
                 }
             }
             hipLaunchKernelGGL((gemm_mfma_kernel<Eng, WGN, WGM, WN, WM, 2, false>), dim3((unsigned)grid),
-                               dim3(WGN * WGM * 64), 0, st, a, tiles_n, tiles_m);
+                               dim3(WGN * WGM * 64), 0, st, a, tiles_n, tiles_m, 0);
         } else
             return fail(BGEMM_EINVAL, "gemm_mfma: tile not built for two planes");
     } else {
@@ -827,14 +931,14 @@ static int launch_cfg(const GemmArgs& a, hipStream_t st)
         if constexpr (CAN_PIPE) {
             if (MUST_PIPE || (a.KT >= 8 && (!pairs || a.KT >= 16))) {
                 if (a.cntW && a.cntX)
-                    hipLaunchKernelGGL((gemm_mfma_kernel<Eng, WGN, WGM, WN, WM, 1, true, true>), g, blk, 0, st, a, tiles_n, tiles_m);
+                    hipLaunchKernelGGL((gemm_mfma_kernel<Eng, WGN, WGM, WN, WM, 1, true, true>), g, blk, 0, st, a, tiles_n, tiles_m, 0);
                 else
-                    hipLaunchKernelGGL((gemm_mfma_kernel<Eng, WGN, WGM, WN, WM, 1, true>), g, blk, 0, st, a, tiles_n, tiles_m);
+                    hipLaunchKernelGGL((gemm_mfma_kernel<Eng, WGN, WGM, WN, WM, 1, true>), g, blk, 0, st, a, tiles_n, tiles_m, 0);
                 return check_launch("gemm_mfma");
             }
         }
         if constexpr (!MUST_PIPE)
-            hipLaunchKernelGGL((gemm_mfma_kernel<Eng, WGN, WGM, WN, WM, 1, false>), g, blk, 0, st, a, tiles_n, tiles_m);
+            hipLaunchKernelGGL((gemm_mfma_kernel<Eng, WGN, WGM, WN, WM, 1, false>), g, blk, 0, st, a, tiles_n, tiles_m, 0);
     }
     return check_launch("gemm_mfma");
 }
@@ -849,20 +953,23 @@ static int launch_tern(const GemmArgs& a, hipStream_t st)
         const int tiles_n = (int)cdiv(a.N, 128), tiles_m = (int)cdiv(a.M, 256);
         const int64_t grid = (int64_t)a.batch * tiles_n * tiles_m;
         if (grid <= 0 || grid > 0x7fffffffLL) return fail(BGEMM_EINVAL, "gemm_mfma: grid of %lld blocks", (long long)grid);
-        hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 2, 4, 1, true, false, true>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m);
+        hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 2, 4, 1, true, false, true>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, 0);
         return check_launch("gemm_mfma");
     } else
         return fail(BGEMM_EINVAL, "gemm_mfma: the signed ternary tile runs on the fp4 engine");
 }
 
-int gemm_mfma_kernel_id(int64_t batch, int64_t M, int64_t N, int64_t KT, int planes, int out_shift, bool fp4)
+int gemm_mfma_kernel_id(int64_t batch, int64_t M, int64_t N, int64_t KT, int planes, int out_kind, bool fp4)
 {
-    return pick_cfg(batch, M, N, KT, planes, out_shift, fp4).id;
+    if (edges_ahead(batch, M, N, KT, planes, out_kind, fp4)) return BGEMM_KERNEL_MFMA_256x128;
+    return pick_cfg(batch, M, N, KT, planes, out_elem_shift(out_kind), fp4).id;
 }
 
 template <typename Eng>
 static int launch_eng(const GemmArgs& a, hipStream_t st)
 {
+    if constexpr (std::is_same<Eng, EngF4>::value)
+        if (a.force < 0 && edges_ahead(a.batch, a.M, a.N, a.KT, a.mc.planes, a.out_kind, true)) return launch_edges(a, st);
     const int id = a.force >= 0 ? a.force : pick_cfg(a.batch, a.M, a.N, a.KT, a.mc.planes, out_elem_shift(a.out_kind), std::is_same<Eng, EngF4>::value).id;
     switch (id) {
     case BGEMM_KERNEL_MFMA_256x256: return launch_cfg<Eng, 2, 2, 4, 4>(a, st);
