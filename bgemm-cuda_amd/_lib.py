@@ -72,6 +72,8 @@ SIGNATURES = {
     "bgemm_elastic_backward": (_int, [_p, _p, _p, _p, _p, _p, _p, ctypes.c_float, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "bgemm_linear_rows_supported": (_int, [_i64, _i64, _i64, _int, _int]),
     "bgemm_linear_rows_forward": (_int, [_p, _int, _i64, _i64, _i64, _i64, _int, _p, _int, _p, _int, _p]),
+    "bgemm_linear_rows_norm_supported": (_int, [_i64, _i64, _i64]),
+    "bgemm_linear_rows_norm_forward": (_int, [_p, _i64, _i64, _i64, _p, _p, _p, _p, ctypes.c_double, _p]),
     "bgemm_attention_supported": (_int, [_i64, _i64, _i64, _i64]),
     "bgemm_attention_forward": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p, _int, _p]),
     "bgemm_attention_forward_bits": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _int, _p]),

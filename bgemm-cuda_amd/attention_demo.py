@@ -75,6 +75,18 @@ class BinarySelfAttention(nn.Module):
                 and lowbit_kernel.linear_rows_supported(rows, hidden, hidden, 1, lowbit_kernel.OUT_F32_SCALED if x.dtype == torch.float32
                                                         else lowbit_kernel.OUT_F16_SCALED))
 
+    def _norm(self, x, rows, hidden):
+        """The layer norm as ``linear_rows_forward`` takes it; None where it is not a plain fp32 one over these features whose call nothing listens to."""
+        norm = self._modules.get("LayerNorm")
+        if (type(norm) is not nn.LayerNorm or norm.normalized_shape != (hidden,) or norm._forward_hooks or norm._forward_pre_hooks
+                or "forward" in norm.__dict__ or x.dtype != torch.float32):
+            return None
+        parameters = norm._parameters.get("weight"), norm._parameters.get("bias")
+        for t in parameters:
+            if t is not None and (type(t) is not nn.Parameter or t.dtype != torch.float32 or t.device != x.device or t.shape != (hidden,) or not t.is_contiguous()):
+                return None
+        return (*parameters, norm.eps) if lowbit_kernel.linear_rows_norm_supported(rows, hidden, hidden) == 2 else None
+
     def forward(self, hidden_states, attention_mask=None):
         if self.kernels and attention_mask is None and self._fusable(hidden_states):
             # nothing but the projections' signs is read: they leave their GEMMs as bits, and one kernel does the rest
@@ -87,12 +99,12 @@ class BinarySelfAttention(nn.Module):
                 if zero_point.dtype != hidden_states.dtype:
                     zero_point = zero_point.detach().to(hidden_states.dtype)
                 scores, context = lowbit_kernel.attention_forward(*bits, batch, self.num_attention_heads, hidden_states.dtype, zero_point)
-                native = _lib.native_or_none()
-                out = None if native is None else native.rows_residual(self.dense.__dict__, context.data, hidden_states)
+                native, norm = _lib.native_or_none(), self._norm(hidden_states, rows, hidden)
+                out = None if native is None else native.rows_residual(self.dense.__dict__, context.data, hidden_states, norm)
                 if out is None:
                     residual = hidden_states.reshape(rows, hidden).contiguous()
-                    out = lowbit_kernel.linear_rows_forward(context, [self.dense._rows_layer(hidden_states.dtype)], residual=residual)[0].view(batch, seq, hidden)
-                return self.LayerNorm(out), scores
+                    out = lowbit_kernel.linear_rows_forward(context, [self.dense._rows_layer(hidden_states.dtype)], residual=residual, norm=norm)[0].view(batch, seq, hidden)
+                return out if norm is not None else self.LayerNorm(out), scores
             scores, context = lowbit_kernel.attention_forward(*bits, batch, self.num_attention_heads, hidden_states.dtype)
             return self.LayerNorm(self.dense(context) + hidden_states), scores
         q = self.transpose_for_scores(self.query(hidden_states))

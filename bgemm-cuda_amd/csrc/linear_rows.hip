@@ -373,6 +373,172 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
     }
 }
 
+// A layer of packed rows whose fp32 outputs, plus a residual, go through a layer norm: as the numbers kernel above, but a block keeps all
+// columns of its rows in registers, a wave CT column tiles, until their mean and deviation are known, so that they are stored once.
+struct RowsNorm { const float* gamma; const float* beta; double eps, share; };      // (either pointer may be null; share: 1 / M)
+constexpr int NORM_MAX_KT = 4, NORM_MAX_M = ROWS_MAX_WAVES * 64;
+
+// Rows' mean, then the mean square of what is left (two passes over registers: nothing cancels), each a sum over 32 lanes and the waves.
+// What bounds it: reading the residual and storing, one block a compute unit; the residual and all weights are requested before the
+// bits are there.  8192 x 768 x 768 27.0 us with the layer norm as a launch of its own (25 MB written and read again), 11.9 here (50 MB
+// of residual and stores, 4.2 TB/s); its relative error to 64 bits 4.0e-8 where that of the separate one is 4.6e-8.
+template <int CT>
+__global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void rows_norm_kernel(const RowsArgs a, const RowsNorm norm)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int h = lane >> 5, c = lane & 31;
+    const int rt = xcd_contiguous_id(blockIdx.x, gridDim.x), KT = a.KT, mt0 = wave * CT;
+    uint4* const raw_bits = reinterpret_cast<uint4*>(smem);                 // [K-tile][64]
+    uint4* const operands = raw_bits + KT * TILE_U4;                        // [K-tile][step][64]
+    float* const shares = reinterpret_cast<float*>(operands + KT * 4 * TILE_U4);      // [2][wave][row]: the waves' shares of the sums
+    float* const mine = shares + (2 * waves + wave) * 32;                   // a value a row, for the wave's lanes
+    const RowsLayer& L = a.l[0];
+    const uint4* const x = reinterpret_cast<const uint4*>(a.x) + (int64_t)rt * KT * TILE_U4;
+    for (int i = threadIdx.x; i < KT * TILE_U4; i += waves * 64) raw_bits[i] = x[i];
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(L.W), 0, a.MT * KT * 1024, 0x00020000);
+    v4i w[NORM_MAX_KT][CT];
+#pragma unroll
+    for (int kt = 0; kt < NORM_MAX_KT; kt++)
+#pragma unroll
+        for (int j = 0; j < CT; j++)
+            w[kt][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, h * 512 + c * 16, (min(mt0 + j, a.MT - 1) * KT + min(kt, KT - 1)) * 1024, 0);
+    const int row_b = a.M * 4, rows_b = min(a.N - rt * 32, 32) * row_b;
+    auto rows_of = [&](const void* p) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p)) + (int64_t)rt * 32 * row_b, 0, rows_b, 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t ro = rows_of(L.out), rr = rows_of(a.residual);
+    int voff[CT];                                                           // (columns past the last one: past the buffer's end)
+    float y[CT][16];
+#pragma unroll
+    for (int j = 0; j < CT; j++) {
+        const int m = (mt0 + j) * 32 + c;
+        voff[j] = m < a.M ? 4 * h * row_b + m * 4 : 0x7ffffff0;
+#pragma unroll
+        for (int v = 0; v < 16; v++) y[j][v] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rr, voff[j], (8 * (v >> 2) + (v & 3)) * row_b, 0));
+    }
+    __syncthreads();
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    // the wave's values a row, as the lane's sixteen rows have them
+    auto of_rows = [&](const float value, float (&to)[16]) {
+        wave_sync();
+        mine[c] = value;                        // (both halves the same)
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 s = *reinterpret_cast<const float4*>(mine + 8 * q + 4 * h);
+            to[4 * q] = s.x; to[4 * q + 1] = s.y; to[4 * q + 2] = s.z; to[4 * q + 3] = s.w;
+        }
+    };
+    int ones = 0;
+    for (int t = 0; t < KT; t++) ones += popc4(raw_bits[t * TILE_U4 + lane]);
+    ones += __shfl_xor(ones, 32);
+    for (int i = wave; i < KT; i += waves) {
+        const uint4 b = raw_bits[i * TILE_U4 + lane];
+#pragma unroll
+        for (int s = 0; s < 4; s++) operands[(i * 4 + s) * TILE_U4 + lane] = make_uint4(rows_x(~b.x, s), rows_x(~b.y, s), rows_x(~b.z, s), rows_x(~b.w, s));
+    }
+    float start[16];
+    of_rows((float)(a.K - 2 * ones), start);
+    v16f acc[CT];
+#pragma unroll
+    for (int j = 0; j < CT; j++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[j][v] = start[v];
+    __syncthreads();
+#pragma unroll
+    for (int kt = 0; kt < NORM_MAX_KT; kt++) {
+        if (kt >= KT) break;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const uint4 b = operands[(kt * 4 + s) * TILE_U4 + lane];
+            const unsigned fx[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int j = 0; j < CT; j++) {
+                unsigned fw[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) fw[q] = rows_w((unsigned)w[kt][j][q], s);
+                acc[j] = EngF4::mma(EngF4::make(fx), EngF4::make(fw), acc[j]);
+            }
+        }
+    }
+    const float sa = *reinterpret_cast<const float*>(L.sa);
+#pragma unroll
+    for (int j = 0; j < CT; j++) {
+        const int m = min((mt0 + j) * 32 + c, a.M - 1);
+        const float s = reinterpret_cast<const float*>(L.sw)[m], b = L.bias ? reinterpret_cast<const float*>(L.bias)[m] : 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+#pragma clang fp contract(off)      // every step rounds by itself, as torch's separate kernels do
+            float t = acc[j][v] * s;
+            t = t * sa;
+            if (L.bias) t = t + b;
+            y[j][v] = t + y[j][v];
+        }
+    }
+    // the sum of a lane's sixteen values over the block's columns, of row c
+    auto over_columns = [&](float (&s)[16], float* const area) {
+        // lanes d apart share the work: each keeps one half of the values (v = c >> 1 in the end)
+        auto halve = [&](auto d_c) {
+            constexpr int d = decltype(d_c)::value;
+            const bool upper = c & d;
+#pragma unroll
+            for (int i = 0; i < d / 2; i++) {
+                const float keep = upper ? s[i + d / 2] : s[i], give = upper ? s[i] : s[i + d / 2];
+                s[i] = keep + __shfl_xor(give, d);
+            }
+        };
+        halve(std::integral_constant<int, 16>{});
+        halve(std::integral_constant<int, 8>{});
+        halve(std::integral_constant<int, 4>{});
+        halve(std::integral_constant<int, 2>{});
+        s[0] += __shfl_xor(s[0], 1);
+        const int v = c >> 1;
+        if (!(c & 1)) area[wave * 32 + 8 * (v >> 2) + 4 * h + (v & 3)] = s[0];
+        __syncthreads();
+        double t = 0.;                          // (a value a lane: in 64 bits, as what follows from it, for nothing)
+#pragma unroll 4
+        for (int i = 0; i < waves; i++) t += (double)area[i * 32 + c];
+        return t;
+    };
+    float sum[16], of[16];
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        sum[v] = 0.f;
+#pragma unroll
+        for (int j = 0; j < CT; j++) sum[v] += voff[j] == 0x7ffffff0 ? 0.f : y[j][v];
+    }
+    of_rows((float)(over_columns(sum, shares) * norm.share), of);
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        sum[v] = 0.f;
+#pragma unroll
+        for (int j = 0; j < CT; j++) {
+            y[j][v] -= of[v];
+            sum[v] += voff[j] == 0x7ffffff0 ? 0.f : y[j][v] * y[j][v];
+        }
+    }
+    of_rows((float)rsqrt(over_columns(sum, shares + waves * 32) * norm.share + norm.eps), of);
+#pragma unroll
+    for (int j = 0; j < CT; j++) {
+        const int m = min((mt0 + j) * 32 + c, a.M - 1);
+        const float g = norm.gamma ? norm.gamma[m] : 1.f, b = norm.beta ? norm.beta[m] : 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; v++) y[j][v] = y[j][v] * of[v] * g + b;
+        if (a.nt) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[j][v]), ro, voff[j], (8 * (v >> 2) + (v & 3)) * row_b, 2);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 16; v++) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[j][v]), ro, voff[j], (8 * (v >> 2) + (v & 3)) * row_b, 0);
+        }
+    }
+}
+
 // How a size is launched, and what a block keeps in LDS: the rows' bits, later those of the output, and operands for every layer, and where
 // bits leave the parameters of its columns.
 struct RowsPlan { int64_t ct, per_layer, splits, groups, own, first_lds, lds; };
@@ -486,5 +652,40 @@ extern "C" int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx
     typedef std::integral_constant<int, ROWS_SRC_PACKED> P;
     if (packed) kinds(P{}, P{});
     else kinds(std::integral_constant<int, ROWS_SRC_F32>{}, std::integral_constant<int, ROWS_SRC_F16>{});
+    return check_launch(who);
+}
+
+extern "C" int bgemm_linear_rows_norm_supported(int64_t N, int64_t M, int64_t K)
+{
+    if (N < 1 || N > (1 << 24) || M < 1 || M > NORM_MAX_M || K < 1 || K > NORM_MAX_KT * TILE_KBITS) return 0;
+    // Against the layer with its residual and the layer norm as a launch of its own (us, N x M x M, two launches / this one): 8192 x
+    // 768 27.0 / 11.9, 2048 x 768 11.6 / 9.8, 1024 x 768 9.7 / 9.8, 512 x 768 8.4 / 9.7, 2048 x 1024 13.5 / 12.3, 1024 x 1024 10.6 / 12.3; 1024 x
+    // 512 8.3 / 7.7, 512 x 512 7.8 / 7.6.  (512 x 64 6.6 / 4.0, but the call around so few rows is the host's time either way, and its sums
+    // are in the separate one's order.)
+    return N >= (M <= 512 ? 1024 : 2048) ? 2 : 1;
+}
+
+extern "C" int bgemm_linear_rows_norm_forward(const void* x_tiled, int64_t N, int64_t M, int64_t K, const bgemm_rows_layer* layer, const void* residual,
+                                              const void* gamma, const void* beta, double eps, void* stream)
+{
+    const char* who = "bgemm_linear_rows_norm_forward";
+    if (!bgemm_linear_rows_norm_supported(N, M, K)) return fail(BGEMM_EINVAL, "%s: N=%lld M=%lld K=%lld", who, (long long)N, (long long)M, (long long)K);
+    if (!x_tiled || !layer || !residual) return fail(BGEMM_ENULL, "%s: null pointer", who);
+    if (!layer->W_tiled || !layer->sw || !layer->sa || !layer->out) return fail(BGEMM_ENULL, "%s: the layer: null pointer", who);
+    if ((((uintptr_t)x_tiled | (uintptr_t)layer->W_tiled) & 15) ||
+        (((uintptr_t)residual | (uintptr_t)layer->sw | (uintptr_t)layer->sa | (uintptr_t)layer->bias | (uintptr_t)layer->out | (uintptr_t)gamma | (uintptr_t)beta) & 3))
+        return fail(BGEMM_EALIGN, "%s: an operand is not aligned", who);
+    RowsArgs a = {};
+    a.l[0] = {(const uint32_t*)layer->W_tiled, nullptr, layer->sw, layer->sa, layer->bias, nullptr, layer->out};
+    a.x = x_tiled; a.residual = residual;
+    a.N = (int)N; a.M = (int)M; a.K = (int)K; a.KT = (int)k_tiles(K); a.MT = (int)row_tiles(M); a.layers = 1;
+    a.nt = M % 16 == 0;                     // (as above)
+    // one column tile a wave while sixteen waves are enough
+    const int ct = a.MT <= ROWS_MAX_WAVES ? 1 : 2, waves = (a.MT + ct - 1) / ct;
+    const size_t lds = (size_t)a.KT * 5 * 1024 + (size_t)3 * waves * 128;
+    const RowsNorm norm = {(const float*)gamma, (const float*)beta, eps, 1. / (double)M};
+    const dim3 grid((unsigned)row_tiles(N)), block(waves * 64);
+    if (ct == 1) hipLaunchKernelGGL(rows_norm_kernel<1>, grid, block, lds, (hipStream_t)stream, a, norm);
+    else hipLaunchKernelGGL(rows_norm_kernel<2>, grid, block, lds, (hipStream_t)stream, a, norm);
     return check_launch(who);
 }

@@ -255,25 +255,43 @@ PyObject* rows_bits(PyObject*, PyObject* const* args, const Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
-// rows_residual(module.__dict__, plane of centred sign bits, residual) -> the layer's output plus the residual, in the residual's shape
+// rows_residual(module.__dict__, plane of centred sign bits, residual, norm) -> the layer's output plus the residual, in the residual's
+// shape; norm: None, or (gamma | None, beta | None, eps) of a layer norm over that
 PyObject* rows_residual(PyObject*, PyObject* const* args, const Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    TORCH_CHECK_TYPE(n == 3, "rows_residual takes 3 arguments");
+    TORCH_CHECK_TYPE(n == 4, "rows_residual takes 4 arguments");
     if (!quiet_call(args[2]) || !plain_gpu(args[1])) Py_RETURN_NONE;
     const Tensor &bits = tensor_at(args[1]), &res = tensor_at(args[2]);
     Layer l;
     if (res.dim() < 1 || res.numel() == 0 || !res.is_contiguous() || !l.read(args[0], res) || res.size(-1) != l.M) Py_RETURN_NONE;
     const int64_t N = res.numel() / l.M;
     const int kind = scaled_kind(res.scalar_type() == at::kFloat);
-    if (!is_plane(bits, res.device(), 1, N, l.K) || !bgemm_linear_rows_supported(N, l.M, l.K, 1, kind)) Py_RETURN_NONE;
+    if (!is_plane(bits, res.device(), 1, N, l.K)) Py_RETURN_NONE;
+    const bool norm = args[3] != Py_None;
+    Tensor gamma, beta;
+    double eps = 0;
+    if (norm) {
+        if (!PyTuple_CheckExact(args[3]) || PyTuple_GET_SIZE(args[3]) != 3 || kind != BGEMM_OUT_F32_SCALED || !bgemm_linear_rows_norm_supported(N, l.M, l.K)) Py_RETURN_NONE;
+        Tensor* const to[2] = {&gamma, &beta};
+        for (int i = 0; i < 2; i++) {
+            PyObject* const o = PyTuple_GET_ITEM(args[3], i);
+            if (o == Py_None) continue;
+            if (!exact(o) || !fits(tensor_at(o), at::kFloat, res.device()) || tensor_at(o).dim() != 1 || tensor_at(o).size(0) != l.M || !tensor_at(o).is_contiguous()) Py_RETURN_NONE;
+            *to[i] = tensor_at(o);
+        }
+        eps = PyFloat_AsDouble(PyTuple_GET_ITEM(args[3], 2));
+        if (PyErr_Occurred()) throw python_error();
+    } else if (!bgemm_linear_rows_supported(N, l.M, l.K, 1, kind))
+        Py_RETURN_NONE;
     Tensor out;
     {
         const WithoutGil no_gil;
         const c10::OptionalDeviceGuard guard(res.device());
         out = at::empty(res.sizes(), res.options().requires_grad(false));
         const bgemm_rows_layer layer = l.rows_layer(out.data_ptr());
-        check(bgemm_linear_rows_forward(bits.data_ptr(), BGEMM_SRC_BITS, 0, N, l.M, l.K, 1, &layer, kind, res.data_ptr(), 0, stream_of(res)));
+        check(norm ? bgemm_linear_rows_norm_forward(bits.data_ptr(), N, l.M, l.K, &layer, res.data_ptr(), data_or_null(gamma), data_or_null(beta), eps, stream_of(res))
+                   : bgemm_linear_rows_forward(bits.data_ptr(), BGEMM_SRC_BITS, 0, N, l.M, l.K, 1, &layer, kind, res.data_ptr(), 0, stream_of(res)));
     }
     return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS

@@ -446,13 +446,20 @@ def linear_rows_supported(N, M, K, layers, kind):
     return ok
 
 
-def linear_rows_forward(x, layers, bits=False, residual=None, next_zero_point=None, bits_out=None, shape=0):
+def linear_rows_norm_supported(N, M, K):
+    """0, or 1: ``linear_rows_forward(norm=)`` takes it, 2: and is worth it."""
+    return _b.lib().bgemm_linear_rows_norm_supported(N, M, K)
+
+
+def linear_rows_forward(x, layers, bits=False, residual=None, next_zero_point=None, bits_out=None, shape=0, norm=None):
     """Up to three scaled binary layers of one input and one size in ONE launch, packing included (bgemm_linear.py:479-484 without a
     gradient).  ``x``: fp16 or fp32 ``[N, K]`` with dense rows, or a binary PackedBits that is centred already; ``layers``: a list of
     ``(w, zero_point, sw, sa, bias)``, ``w`` a binary PackedBits of M x K bits, the others tensors of one type (``x``'s where that is a
     tensor), ``zero_point`` and ``bias`` or None.  Returns a list: each layer's ``half(acc) * sw * sa (+ bias)``, ``[N, M]``, plus
     ``residual`` if there is one, or with ``bits`` those outputs' sign bits after centring by ``next_zero_point`` (one element, or None
-    for 0), as ``bgemm_packed_forward(bits_out=)`` leaves them: in ``bits_out`` (a list), or in new operands whose padding is undefined."""
+    for 0), as ``bgemm_packed_forward(bits_out=)`` leaves them: in ``bits_out`` (a list), or in new operands whose padding is undefined.
+    ``norm``: ``(gamma, beta, eps)`` of a layer norm over the rows of output plus residual, ``gamma`` and ``beta`` fp32 ``[M]`` or None; for
+    one layer of packed rows, fp32 parameters and a size that ``linear_rows_norm_supported`` takes."""
     packed = isinstance(x, PackedBits)
     w0, dt = layers[0][0], layers[0][2].dtype
     M, K, dev = w0.rows, w0.K, w0.data.device
@@ -504,6 +511,17 @@ def linear_rows_forward(x, layers, bits=False, residual=None, next_zero_point=No
             a.bias = bias.data_ptr()
         if next_zero_point is not None:
             a.next_zero_point = next_zero_point.data_ptr()
+    if norm is not None:
+        gamma, beta, eps = norm
+        if not packed or not f32 or bits or residual is None or len(layers) != 1:
+            raise ValueError("norm needs one layer of packed rows, fp32 parameters and a residual")
+        for name, t in (("gamma", gamma), ("beta", beta)):
+            if t is not None and (t.dtype != dt or tuple(t.shape) != (M,) or not t.is_contiguous() or t.device != dev):
+                raise ValueError("%s must be a contiguous %s tensor of %d elements on %s" % (name, dt, M, dev))
+        with _on(dev):
+            _b.check(_b.lib().bgemm_linear_rows_norm_forward(x.data.data_ptr(), N, M, K, arr, residual.data_ptr(), None if gamma is None else gamma.data_ptr(),
+                                                             None if beta is None else beta.data_ptr(), eps, _stream()))
+        return outs
     with _on(dev):
         _b.check(_b.lib().bgemm_linear_rows_forward((x.data if packed else x).data_ptr(), SRC_BITS if packed else SRC_F32 if f32 else SRC_F16,
                                                     0 if packed else max(x.stride(0), K), N, M, K, len(layers), arr, kind,

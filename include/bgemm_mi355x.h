@@ -342,6 +342,13 @@ typedef struct bgemm_rows_layer {
 int bgemm_linear_rows_supported(int64_t N, int64_t M, int64_t K, int layers, int out_dtype);
 int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx, int64_t N, int64_t M, int64_t K, int layers,
                               const bgemm_rows_layer* layer, int out_dtype, const void* residual, int shape, void* stream);
+/* One layer of packed rows (sign bits, tiled, 16-byte aligned, the padding of their columns zero), fp32 parameters, with a residual and a
+ * layer norm behind it: out [N][M] = (z - mean(z)) / sqrt(var(z) + eps) * gamma + beta over each row of
+ * z = y + residual, y as above; gamma, beta [M] or NULL (1, 0); zero_point and next_zero_point are not looked at.  Supported (else 0): M, K
+ * <= 1024, N <= 2^24; 2: and worth a layer norm with another order of sums than the separate one's. */
+int bgemm_linear_rows_norm_supported(int64_t N, int64_t M, int64_t K);
+int bgemm_linear_rows_norm_forward(const void* x_tiled, int64_t N, int64_t M, int64_t K, const bgemm_rows_layer* layer, const void* residual,
+                                   const void* gamma, const void* beta, double eps, void* stream);
 
 /* ---- binary self-attention without a gradient, one launch -----------------------------------------
  * (tests/python/bert/bert.py:245-259 on sign bits.)  q, k, v: sign bits [batch * seq][heads * head_size], tiled, 16-byte aligned.

@@ -96,3 +96,34 @@ def test_block_with_other_parts_takes_its_general_path(other, monkeypatch):
         want, want_scores = block(x)
     assert torch.equal(out, want) and torch.equal(scores, want_scores)
     assert other != "heads" or calls.count("heads") == 6
+
+
+@pytest.mark.parametrize("change", ["none", "plain", "hook", "half", "other"])
+def test_block_of_many_rows_with_its_layer_norm_in_the_last_projection(change, monkeypatch):
+    """From a thousand rows on the block's layer norm is part of its last launch, unless it is another module or somebody listens to it."""
+    torch.manual_seed(5)
+    block = attention_demo.BinarySelfAttention(96, 3).to(DEV)
+    with torch.no_grad():
+        block.LayerNorm.weight.uniform_(0.5, 1.5)
+        block.LayerNorm.bias.normal_()
+    x, seen = torch.randn(9, 130, 96, device=DEV), []
+    if change == "plain":
+        block.LayerNorm = torch.nn.LayerNorm(96, elementwise_affine=False)
+    if change == "hook":
+        block.LayerNorm.register_forward_hook(lambda m, i, o: seen.append(1))
+    if change == "half":
+        block, x = block.half(), x.half()
+    if change == "other":
+        block.LayerNorm = torch.nn.Identity()
+    with torch.no_grad():
+        block(x)
+        del seen[:]
+        calls = []
+        monkeypatch.setattr(torch.nn.functional, "layer_norm", lambda *a, f=torch.nn.functional.layer_norm: calls.append(1) or f(*a))
+        out, scores = block(x)
+        assert len(calls) == (1 if change in ("hook", "half") else 0) and len(seen) == (change == "hook")
+        monkeypatch.setattr(lk, "linear_rows_norm_supported", lambda *a: 1)
+        want, want_scores = block(x)
+    assert torch.equal(scores, want_scores) and out.dtype == want.dtype
+    # two orders of a sum of 96 values of about one: some 2^-24 each
+    torch.testing.assert_close(out, want, rtol=0, atol=0 if change in ("hook", "half", "other") else 2e-5)

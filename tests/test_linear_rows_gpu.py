@@ -118,3 +118,26 @@ def test_context_as_bits(B, S, H, d, dt):
         assert torch.equal(lk.logical_from_tiled(bits), lk.logical_from_tiled(want))
         real = (B * S) // 32 * bits.words // -(-B * S // 32)                   # whole row tiles, their padding of columns included
         assert torch.equal(bits.data[:, :real], want.data[:, :real])
+
+
+# column tiles and waves (32, 16 x 32, 1024), rows (32), K-tiles (256), one column; a row far from zero against its deviation, equal outputs
+@pytest.mark.parametrize("N, M, K", [(1, 1, 1), (31, 33, 40), (33, 512, 256), (64, 513, 257), (65, 768, 768), (100, 1001, 1000), (32, 1024, 1024)])
+def test_layer_norm_of_rows_and_residual(N, M, K):
+    for offset, bias, gamma, beta in ((0.0, True, True, True), (50.0, False, True, False), (0.0, True, False, True)):
+        x, ls = made(N, M, max(K, 8), 1, torch.float32, bias, seed=int(offset))
+        x, ls[0] = x[:, :K], (ls[0][0][:, :K].contiguous(),) + ls[0][1:]
+        residual = torch.randn(N, M, device=DEV) + offset
+        g, b = (torch.randn(M, device=DEV) if wanted else None for wanted in (gamma, beta))
+        w, zp, sw, sa, bi = ls[0]
+        if offset:
+            sw, residual[N // 2] = sw * 0.0, offset                            # a row of equal values
+        xp = lk.pack_sign(x.contiguous(), zp)
+        got, = lk.linear_rows_forward(xp, [(lk.pack_sign(w), zp, sw, sa, bi)], residual=residual, norm=(g, b, 1e-12))
+        z = (formula(x, w, zp, sw, sa, bi) + residual).double()
+        mean, var = z.mean(1, keepdim=True), z.var(1, unbiased=False, keepdim=True)
+        gd, bd = 1.0 if g is None else g.double(), 0.0 if b is None else b.double()
+        want = (z - mean) / (var + 1e-12).sqrt() * gd + bd
+        # a mean of at most 64 fp32 roundings of 2^-24 on values of that size, over a deviation whose relative error is no larger
+        far = z.abs().amax(1, keepdim=True)
+        bound = 64 * 2.0 ** -24 * ((1 + far / (var + 1e-12).sqrt()) * (torch.ones_like(z) * gd).abs() + (want - bd).abs() + abs(bd))
+        assert bool(((got.double() - want).abs() <= bound).all())
