@@ -69,6 +69,40 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
         else return __half2float(reinterpret_cast<const __half*>(p)[i]);
     };
 
+    // ---- a wave's weights ----------------------------------------------------------------------------------------------------------
+    const int g0 = part * a.own, g1 = min(a.groups, g0 + a.own), cols_n = a.own * CT * 32;
+    // a wave works for one layer
+    const int per_layer = waves / a.layers, l = wave / per_layer, wl = wave - l * per_layer, lx = SRC == ROWS_SRC_PACKED ? 0 : l;
+    const RowsLayer& L = a.l[l];
+    int gg = g0 + wl, kt = 0, rg = gg, rkt = 0;                       // the group that is multiplied, and the one whose weights are requested next
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(L.W), 0, a.MT * KT * 1024, 0x00020000);
+    // which weight row a lane multiplies: bits: MFMA row 8 q + 4 half + i is column 16 half + 4 q + i, so that a lane ends up with 16
+    // neighbouring columns of its row; fp16: the even rows of a pair of tiles, then the odd ones; else the lane's own
+    const int own = BITS ? 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3) : c;
+    auto request = [&](v4i (&w)[CT]) {
+        const int mt0 = rg * CT;
+#pragma unroll
+        for (int j = 0; j < CT; j++) {
+            if constexpr (KIND == ROWS_F16) {
+                const int r = 2 * c + (j & 1), mt = min(mt0 + (j & ~1) + (r >> 5), a.MT - 1);
+                w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, mt * KT * 1024 + h * 512 + (r & 31) * 16, rkt * 1024, 0);
+            } else
+                w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, h * 512 + own * 16, (min(mt0 + j, a.MT - 1) * KT + rkt) * 1024, 0);
+        }
+        if (++rkt == KT) {
+            rkt = 0;
+            rg += per_layer;                                           // (past the last one: the last tile again, nobody multiplies it)
+        }
+    };
+    // Those of the first two K-tiles are on their way while the bits are made, where bits leave and little else fills that time (us:
+    // 8192 x 768 x (3 x 768) 15.9 -> 15.4, 2048 x 768 x (3 x 768) 8.4 -> 8.0, 128 x 784 x 4096 7.2 -> 7.1; numbers, which have stores to
+    // wait for: 8192 x 768 x 3072 packed 23.3 -> 23.7, fp16 4096 x 1024 x 1024 8.2 -> 8.3).
+    v4i w0[CT], w1[CT], w2[CT];
+    if constexpr (BITS) {
+        request(w0);
+        request(w1);
+    }
+
     // ---- the rows' bits ----------------------------------------------------------------------------------------------------------
     if constexpr (SRC == ROWS_SRC_PACKED) {
         const uint4* const x = reinterpret_cast<const uint4*>(a.x) + (int64_t)rt * KT * TILE_U4;
@@ -109,7 +143,6 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
             }
         }
     }
-    const int g0 = part * a.own, g1 = min(a.groups, g0 + a.own), cols_n = a.own * CT * 32;
     if constexpr (BITS) {
         for (int l = 0; l < a.layers; l++)
             for (int i = threadIdx.x; i < cols_n; i += waves * 64) {
@@ -119,8 +152,7 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
             }
     }
     __syncthreads();
-    // a wave works for one layer; the sum of its x of row c
-    const int per_layer = waves / a.layers, l = wave / per_layer, wl = wave - l * per_layer, lx = SRC == ROWS_SRC_PACKED ? 0 : l;
+    // the sum of the wave's x of row c
     int ones = 0;
 #pragma unroll 1
     for (int t = 0; t < KT; t++) ones += popc4(raw_bits[(lx * KT + t) * TILE_U4 + lane]);
@@ -134,29 +166,8 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
     __syncthreads();
 
     // ---- the products --------------------------------------------------------------------------------------------------------------
-    const RowsLayer& L = a.l[l];
-    int gg = g0 + wl, kt = 0, rg = gg, rkt = 0;                       // the group that is multiplied, and the one whose weights are requested next
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(L.W), 0, a.MT * KT * 1024, 0x00020000);
     const float sa = par(L.sa, 0), next = BITS && L.next_zp ? par(L.next_zp, 0) : 0.f;
     const bool has_bias = L.bias != nullptr, has_next = L.next_zp != nullptr;
-    // which weight row a lane multiplies: bits: MFMA row 8 q + 4 half + i is column 16 half + 4 q + i, so that a lane ends up with 16
-    // neighbouring columns of its row; fp16: the even rows of a pair of tiles, then the odd ones; else the lane's own
-    const int own = BITS ? 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3) : c;
-    auto request = [&](v4i (&w)[CT]) {
-        const int mt0 = rg * CT;
-#pragma unroll
-        for (int j = 0; j < CT; j++) {
-            if constexpr (KIND == ROWS_F16) {
-                const int r = 2 * c + (j & 1), mt = min(mt0 + (j & ~1) + (r >> 5), a.MT - 1);
-                w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, mt * KT * 1024 + h * 512 + (r & 31) * 16, rkt * 1024, 0);
-            } else
-                w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, h * 512 + own * 16, (min(mt0 + j, a.MT - 1) * KT + rkt) * 1024, 0);
-        }
-        if (++rkt == KT) {
-            rkt = 0;
-            rg += per_layer;                                           // (past the last one: the last tile again, nobody multiplies it)
-        }
-    };
     // the sums of x that the accumulators start from: BITS: the lane's row's, else those of its sixteen rows
     v16f acc[CT], start;
     if constexpr (BITS) {
@@ -345,9 +356,10 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
         }
     };
     if (gg < g1) {
-        v4i w0[CT], w1[CT], w2[CT];
-        request(w0);
-        request(w1);
+        if constexpr (!BITS) {
+            request(w0);
+            request(w1);
+        }
         for (;;) {
             request(w2);
             step(w0);
