@@ -575,8 +575,11 @@ static RowsPlan rows_plan(int64_t N, int64_t M, int64_t K, int layers, bool pack
     p.per_layer = 8 / layers;
     if (one_a_unit) {
         const int64_t want = cdiv(cdiv(rt * p.groups, 256), 4) * 4, most = layers == 3 ? 4 : ROWS_MAX_WAVES / layers;
-        p.per_layer = want < 4 ? 4 : want > most ? most : want;
-        if (f16_numbers && layers == 1 && p.per_layer < 8) p.per_layer = 8;
+        // (one layer at least eight: the waves make the bits of 32 rows together, on few rows four of them in as many trips to memory as
+        // their products take: bits 128 x 784 x 4096 fp16 7.0 -> 5.7, fp32 5.9 -> 5.2; 512 x 1000 x 2048 6.1 -> 5.2; 40 x 1024 x 4096 7.0 ->
+        // 5.6; 64 x 512 x 1024 4.4 -> 4.0; sixteen 5.8, 5.3, 5.6, 5.7, 4.1; three layers have twelve)
+        const int64_t least = layers == 1 ? 8 : 4;
+        p.per_layer = want < least ? least : want > most ? most : want;
     }
     if (shape) p.per_layer = shape >> 4 & 31;
     p.splits = cdiv(p.groups, p.per_layer);
