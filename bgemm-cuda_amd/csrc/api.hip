@@ -121,8 +121,11 @@ __global__ void fill_empty_bits_kernel(const GemmArgs a)
     unsigned w = 0;
     for (int c = 0; c < 32; c++)
         if (jw * 32 + c < a.M) w |= next_sign_bit(a, jw * 32 + c, 0) << (31 - c);
-    for (int64_t b = blockIdx.y; b < a.batch; b += gridDim.y)
-        reinterpret_cast<uint32_t*>(a.out)[b * a.strideC + tiled_word_offset(n, jw, k_tiles(a.M))] = w;
+    for (int64_t b = blockIdx.y; b < a.batch; b += gridDim.y) {
+        uint32_t* const out = reinterpret_cast<uint32_t*>(a.out) + b * a.strideC;
+        out[tiled_word_offset(n, jw, k_tiles(a.M))] = w;
+        if (jw == Mw - 1) end_bits_row(out, n, a.M);
+    }
 }
 
 // Unpacked activations for the decode kernel that packs them itself (null = X_tiled / X2_tiled are used).

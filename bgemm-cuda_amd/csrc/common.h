@@ -282,6 +282,13 @@ __device__ __forceinline__ unsigned next_sign_bit(const GemmArgs& a, const int64
         d = __half2float(scaled_f16(a, m, v)) - (a.ep_zp ? __half2float(*reinterpret_cast<const __half*>(a.ep_zp)) : 0.f);
     return __float_as_uint(d) >> 31;
 }
+// The words of row n of an operand of M bits that lie behind its last one, to the end of that K-tile, as zeros: a product counts the bits
+// of whole K-tiles, so whoever stores a row's last word stores these too, and it does not matter what the buffer held before.
+__device__ __forceinline__ void end_bits_row(uint32_t* out, const int64_t n, const int64_t M)
+{
+    const int64_t KT = k_tiles(M);
+    for (int64_t jw = (M + 31) >> 5; jw < KT * 8; jw++) out[tiled_word_offset(n, jw, KT)] = 0u;
+}
 // One word of the tiled output: the 32 lanes of a half-wave hold the bits of columns m32 .. m32 + 31
 // (m32 a multiple of 32) of output row n, bit = 0 where the column does not exist.  Every lane of the
 // wave calls this; column i lands at bit 31 - i.
@@ -291,8 +298,11 @@ __device__ __forceinline__ void store_bits_word(const GemmArgs& a, const int b, 
     const int lane = threadIdx.x & 63;
     const unsigned long long bal = __ballot(bit != 0);
     const unsigned w = __brev((unsigned)(lane < 32 ? bal : bal >> 32));
-    if ((lane & 31) == 0 && n < a.N && m32 < a.M)
-        reinterpret_cast<uint32_t*>(a.out)[(int64_t)b * a.strideC + tiled_word_offset(n, m32 >> 5, k_tiles(a.M))] = w;
+    if ((lane & 31) == 0 && n < a.N && m32 < a.M) {
+        uint32_t* const out = reinterpret_cast<uint32_t*>(a.out) + (int64_t)b * a.strideC;
+        out[tiled_word_offset(n, m32 >> 5, k_tiles(a.M))] = w;
+        if (m32 + 32 >= a.M) end_bits_row(out, n, a.M);
+    }
 }
 
 // Final store of one output element (column m of a row whose first element has index row0).

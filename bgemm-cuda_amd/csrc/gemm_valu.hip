@@ -152,9 +152,11 @@ __global__ __launch_bounds__(256) void gemm_valu_kernel(const GemmArgs a, const 
                     field[q] = (unsigned)(bal >> (16 * g)) & 0xffffu;
                 }
                 const int64_t m32 = (int64_t)tm * 64 + 32 * jj;
-                if (tx == 0 && n < a.N && m32 < a.M)
-                    reinterpret_cast<uint32_t*>(a.out)[out_off + tiled_word_offset(n, m32 >> 5, k_tiles(a.M))] =
-                        __brev(field[0] | (field[1] << 16));
+                if (tx == 0 && n < a.N && m32 < a.M) {
+                    uint32_t* const out = reinterpret_cast<uint32_t*>(a.out) + out_off;
+                    out[tiled_word_offset(n, m32 >> 5, k_tiles(a.M))] = __brev(field[0] | (field[1] << 16));
+                    if (m32 + 32 >= a.M) end_bits_row(out, n, a.M);
+                }
             }
         }
         return;

@@ -233,7 +233,11 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
                 if ((mt + 1) * 32 > a.M) word &= 0xffffffffu << ((mt + 1) * 32 - a.M);
                 if (a.gather) {
                     if (h == 0) words[(l * a.gather + mt) * 32 + c] = word;
-                } else if (h == 0 && n < a.N) reinterpret_cast<uint32_t*>(L.out)[tiled_word_offset(n, mt, k_tiles(a.M))] = word;
+                } else if (h == 0 && n < a.N) {
+                    uint32_t* const out = reinterpret_cast<uint32_t*>(L.out);
+                    out[tiled_word_offset(n, mt, k_tiles(a.M))] = word;
+                    if (mt == a.MT - 1) end_bits_row(out, n, a.M);
+                }
             }
         } else if constexpr (KIND == ROWS_F32) {
             const __amdgpu_buffer_rsrc_t ro = rows_of(L.out), rr = rows_of(a.residual);

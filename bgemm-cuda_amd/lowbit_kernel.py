@@ -152,14 +152,13 @@ def packed_kernel_id(w, x, mode=MODE_XOR, splitK=1, variant=VARIANT_AUTO, out_dt
 
 
 def zeros_packed(rows, K, batch=1, device="cuda"):
-    """An all-zero binary operand of `rows` x `K` bits: the buffer a GEMM with ``bits_out=`` writes the next
-    layer's operand into (its padding must be zero, which later calls of the same shape preserve)."""
+    """An all-zero binary operand of `rows` x `K` bits."""
     words = _b.lib().bgemm_tiled_words(rows, K)
     return PackedBits(torch.zeros((batch, words), dtype=torch.int32, device=device), None, batch, rows, K)
 
 
 def empty_packed(rows, K, device="cuda"):
-    """The same without the zeros, for a reader that looks at real bits only."""
+    """The same without the zeros: the buffer a GEMM with ``bits_out=`` writes the next layer's operand into."""
     return PackedBits(torch.empty((1, _b.lib().bgemm_tiled_words(rows, K)), dtype=torch.int32, device=device), None, 1, rows, K)
 
 
@@ -285,7 +284,7 @@ def bgemm_packed_forward(w, x, mode=MODE_XOR, out_dtype=torch.int32, splitK=1, v
     (bgemm_linear.py:482-484) into the store: ``sw`` [M], ``sa`` one element, ``bias`` [M] or None,
     all fp32 (fp32 output) or all fp16 (fp16 output), rounded step by step as torch does.
 
-    ``bits_out=`` (a PackedBits of N rows x M bits from ``zeros_packed``, with ``scale``) stores no
+    ``bits_out=`` (a PackedBits of N rows x M bits, whatever it held before; with ``scale``) stores no
     activations at all: the scaled output is centred by ``next_zero_point`` (a one-element tensor of the
     parameters' type, or None for 0), cast to fp16 and sign-packed as the next binary layer would do it, and
     those bits are written into ``bits_out``, which is returned."""
@@ -457,7 +456,7 @@ def linear_rows_forward(x, layers, bits=False, residual=None, next_zero_point=No
     ``(w, zero_point, sw, sa, bias)``, ``w`` a binary PackedBits of M x K bits, the others tensors of one type (``x``'s where that is a
     tensor), ``zero_point`` and ``bias`` or None.  Returns a list: each layer's ``half(acc) * sw * sa (+ bias)``, ``[N, M]``, plus
     ``residual`` if there is one, or with ``bits`` those outputs' sign bits after centring by ``next_zero_point`` (one element, or None
-    for 0), as ``bgemm_packed_forward(bits_out=)`` leaves them: in ``bits_out`` (a list), or in new operands whose padding is undefined.
+    for 0), as ``bgemm_packed_forward(bits_out=)`` leaves them: in ``bits_out`` (a list), or in new operands.
     ``norm``: ``(gamma, beta, eps)`` of a layer norm over the rows of output plus residual, ``gamma`` and ``beta`` fp32 ``[M]`` or None; for
     one layer of packed rows, fp32 parameters and a size that ``linear_rows_norm_supported`` takes."""
     packed = isinstance(x, PackedBits)

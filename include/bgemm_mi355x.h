@@ -220,8 +220,8 @@ int bgemm_packed_forward_scaled(int mode, const void* W_tiled, const void* X_til
  * then centred and sign-packed as the next layer would do it (tests/python/bgemm_linear.py:479-482
  * followed by :140-141 and the pack of ptx_mma.cuh:341-380): bit = sign bit of half_rn(y - *zero_point).
  * out_tiled receives the tiled operand of N rows x M bits (bgemm_tiled_words(N, M) words per batch
- * entry, strideOut words apart).  Only real bits are written: the padding of the last row tile and
- * K-tile must already be zero (zero-fill the buffer once; calls of the same shape keep it valid).
+ * entry, strideOut words apart).  The padding of a row's last
+ * K-tile is written as zeros, rows past the last one are left as they are: the buffer may have held anything before.
  * out_dtype: BGEMM_OUT_BITS_F32 (fp32 sw, sa, bias, zero_point) or BGEMM_OUT_BITS_F16 (fp16); all
  * are DEVICE pointers, bias may be NULL, zero_point NULL means 0.  No counterpart in the reference,
  * which materialises the fp16 activations between layers. */
@@ -326,7 +326,7 @@ int bgemm_elastic_backward(const void* x_sign, const void* x_nonzero, const void
  * by each layer's own zero point (NULL: 0), or BGEMM_SRC_BITS: one tiled operand of centred sign bits, the padding of K zero.
  *   y = half(acc) * sw * sa (+ bias), every step rounded as bgemm_packed_forward_scaled does it
  *   scaled kinds: out [N][M] = y, or y + residual (residual [N][M] of the output's type)
- *   bits kinds:   out = the sign bits of half(y - *next_zero_point) (NULL: 0), tiled; its padding is not written
+ *   bits kinds:   out = the sign bits of half(y - *next_zero_point) (NULL: 0), tiled; padding as bgemm_packed_forward_bits leaves it
  * Supported (else 0): 8 <= K <= 2048, M <= 65536, N <= 2^24, the rows' bits (and with bits out the parameters) within 64 KiB of LDS;
  * 2 where one layer is also ahead of a pack and a GEMM, else 1.
  * tiles: column tiles a wave multiplies at once, 0 = chosen by size (1 to 3: tests). */

@@ -1,5 +1,7 @@
 """The layer mirror on the GPU: same numbers as the reference CPU path (torch matmul on +-1
 tensors) fed identical operands, compared bit for bit (tolerance 0)."""
+import functools
+
 import numpy as np
 import pytest
 import torch
@@ -178,6 +180,24 @@ def test_chain_keeps_only_bits_between_layers(dtype):
             h = layer(h)
         assert torch.equal(chain(x2), h)
     assert chain(x).requires_grad                          # with gradients: the ordinary path
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.half])
+@pytest.mark.parametrize("N", [3, 32, 128, 600])
+def test_chain_whose_layers_are_replaced_by_narrower_ones(N, dtype):
+    """The new hidden width ends in the same K-tile as the old one: the next layer must not count bits of the old columns."""
+    torch.manual_seed(12)
+    made = lambda *sizes: [bl.BGEMMLinear(k, m, bias=True).to(DEV).to(dtype) for k, m in zip(sizes, sizes[1:])]
+    layer_by_layer = lambda layers: functools.reduce(lambda h, l: l(h), layers, x)
+    chain, others = bl.BGEMMChain(*made(300, 500, 500, 10)), made(300, 470, 450, 10)
+    x = torch.randn(N, 300, device=DEV).to(dtype)
+    with torch.no_grad():
+        for _ in range(2):
+            chain(x)
+        want = [layer_by_layer(others) for _ in range(2)][1]       # (the new layers have their scales and packed weights)
+        for i, layer in enumerate(others):
+            chain[i] = layer
+        assert torch.equal(chain(x), want) and torch.equal(chain(x), want)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.half])

@@ -66,6 +66,12 @@ def test_numbers_residuals_and_bits(N, M, K, layers, dt):
                     bits = lk.logical_from_tiled(got)
                     expected = lk.logical_from_tiled(lk.pack_sign(y))
                     assert torch.equal(bits, expected)
+                into = [lk.zeros_packed(N, M, 1, DEV) for _ in ls]             # of ones: the padding of the columns is written, too
+                for p in into:
+                    p.data.fill_(-1)
+                for got, y in zip(lk.linear_rows_forward(x, packed(ls), bits=True, shape=shape, bits_out=into), want):
+                    whole = N // 32 * -(-M // 256) * 256
+                    assert torch.equal(got.data[:, :whole], lk.pack_sign(y).data[:, :whole])
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.half])

@@ -770,6 +770,24 @@ def test_bits_output_is_next_layers_operand(oracle, variant, dtype, M, N, K, spl
         assert int(np.unpackbits(words.view(np.uint8)).sum()) == logical_bits
 
 
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("M,N,K,batch", [(96, 64, 784, 1), (300, 128, 4096, 1), (4100, 32, 300, 3), (513, 256, 512, 2), (225, 1024, 2048, 1), (10, 128, 4096, 1), (800, 32, 40, 1),
+                                         (70, 32, 0, 1)])
+def test_bits_output_writes_the_padding_of_its_columns(variant, M, N, K, batch):
+    """Into a buffer of ones, on whole row tiles: every word is that of the packed numbers, zeros behind the last column."""
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    empty = lambda b, r: lk.PackedBits(torch.empty((b, 0), dtype=torch.int32, device=DEV), None, b, r, 0)
+    wp, xp = (lk.pack_sign(rnd(batch, M, K)), lk.pack_sign(rnd(batch, N, K))) if K else (empty(batch, M), empty(batch, N))
+    for dtype in (torch.float32, torch.half):
+        scale, zp = (rnd(M).to(dtype), torch.ones(1, dtype=dtype, device=DEV), rnd(M).to(dtype)), torch.full((1,), 0.25, dtype=dtype, device=DEV)
+        want = lk.pack_sign(lk.bgemm_packed_forward(wp, xp, MODE_XOR, variant=variant, scale=scale), zero_point=zp)
+        out = lk.zeros_packed(N, M, batch, DEV)
+        out.data.fill_(-1)
+        lk.bgemm_packed_forward(wp, xp, MODE_XOR, variant=variant, bits_out=out, scale=scale, next_zero_point=zp)
+        assert torch.equal(out.data, want.data)
+
+
 def test_bits_output_chains_two_layers_and_empty_k(oracle):
     """Two binary layers with nothing but bits in between equal the op-by-op chain; K = 0 gives the bits of the bias."""
     rng = np.random.default_rng(99)
