@@ -514,16 +514,12 @@ class BGEMMChain(nn.Sequential):
                 and all(a.weight.shape[0] == b.weight.shape[1] for a, b in zip(layers, layers[1:])))
 
     def _native_forward(self, x):
-        """The fused forward by the native host side, once the bit buffers of this number of rows are there; None where it has to be Python's."""
+        """The fused forward by the native host side; None where it has to be Python's."""
         native = _lib.native_or_none()
-        bits = self.__dict__.get("_bits")
-        if native is None or bits is None or torch.is_grad_enabled() or type(x) is not torch.Tensor or not x.numel():
+        layers = self._modules.values()
+        if native is None or torch.is_grad_enabled() or not all(type(l) in _PLAIN_LAYERS and l.fuse_inference for l in layers):
             return None
-        buffers = bits.get((x.numel() // x.shape[-1], x.device))
-        layers = list(self._modules.values())
-        if buffers is None or not all(type(l) in _PLAIN_LAYERS and l.fuse_inference for l in layers):
-            return None
-        return native.chain_infer([l.__dict__ for l in layers], x, buffers)
+        return native.chain_infer([l.__dict__ for l in layers], x)
 
     def forward(self, x):
         if type(self) is BGEMMChain:
@@ -538,24 +534,19 @@ class BGEMMChain(nn.Sequential):
         kind = lowbit_kernel.OUT_BITS_F32 if x.dtype == torch.float32 else lowbit_kernel.OUT_BITS_F16
         one_launch = len(layers) > 1 and lowbit_kernel.linear_rows_supported(x2.shape[0], *layers[0].weight.shape, 1, kind) == 2
         xp = None if one_launch else lowbit_kernel.pack_sign(x2, zero_point=layers[0].zpa)
-        if not hasattr(self, "_bits"):
-            self._bits = {}
         for i, layer in enumerate(layers):
             scale = (layer.sw.detach(), layer.sa.detach().reshape(1), None if layer.bias is None else layer.bias.detach())
             if i + 1 == len(layers):
                 out = lowbit_kernel.bgemm_packed_forward(layer._packed_weight(), xp, lowbit_kernel.MODE_XOR, splitK=8, scale=scale)
-                self._bits[x2.shape[0], x.device] = [self._bits[j, x2.shape[0], x.device].data for j in range(i)]
                 return out.reshape(*lead, layer.weight.shape[0])
-            key = (i, x2.shape[0], x.device)
-            if key not in self._bits:      # zero-filled once: the GEMM writes real bits only, the padding stays zero
-                self._bits[key] = lowbit_kernel.zeros_packed(x2.shape[0], layer.weight.shape[0], 1, x.device)
             next_zero_point = layers[i + 1].zpa.detach().reshape(1)
             if xp is None:                 # the first layer packs its input itself
                 xp, = lowbit_kernel.linear_rows_forward(x2, [(layer._packed_weight(), layer.zpa.detach().to(x.dtype).reshape(1), *scale)], bits=True,
-                                                        next_zero_point=next_zero_point, bits_out=[self._bits[key]])
+                                                        next_zero_point=next_zero_point)
             else:
                 xp = lowbit_kernel.bgemm_packed_forward(layer._packed_weight(), xp, lowbit_kernel.MODE_XOR, splitK=8, scale=scale,
-                                                        bits_out=self._bits[key], next_zero_point=next_zero_point)
+                                                        bits_out=lowbit_kernel.empty_packed(x2.shape[0], layer.weight.shape[0], x.device),
+                                                        next_zero_point=next_zero_point)
 
 
 class GraphedInference:

@@ -5,6 +5,7 @@
 
 #include <torch/csrc/DynamicTypes.h>
 
+#include <algorithm>
 #include <vector>
 
 namespace bgemm_native {
@@ -144,26 +145,22 @@ PyObject* linear_infer(PyObject*, PyObject* const* args, const Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
-// chain_infer([module.__dict__, ..], x, [bit buffer of every layer but the last]) -> y: only bits between the layers
+// chain_infer([module.__dict__, ..], x) -> y: only bits between the layers
 PyObject* chain_infer(PyObject*, PyObject* const* args, const Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    TORCH_CHECK_TYPE(n == 3 && PyList_CheckExact(args[0]) && PyList_CheckExact(args[2]), "chain_infer takes a list, a tensor and a list");
+    TORCH_CHECK_TYPE(n == 2 && PyList_CheckExact(args[0]), "chain_infer takes a list and a tensor");
     const Py_ssize_t layers = PyList_GET_SIZE(args[0]);
-    if (layers < 2 || PyList_GET_SIZE(args[2]) != layers - 1 || !quiet_call(args[1])) Py_RETURN_NONE;
+    if (layers < 2 || !quiet_call(args[1])) Py_RETURN_NONE;
     const Tensor& x = tensor_at(args[1]);
     if (x.dim() < 1 || x.numel() == 0) Py_RETURN_NONE;
     const int64_t K0 = x.size(-1), N = x.numel() / K0;
     std::vector<Layer> l(layers);
-    std::vector<Tensor> bits(layers - 1);
-    int64_t K = K0;
+    int64_t K = K0, most = 0;                 // words of the largest operand between two layers
     for (Py_ssize_t i = 0; i < layers; i++) {
         if (!l[i].read(PyList_GET_ITEM(args[0], i), x) || l[i].K != K || l[i].M == 0) Py_RETURN_NONE;
         K = l[i].M;
-        if (i + 1 == layers) break;
-        PyObject* const b = PyList_GET_ITEM(args[2], i);
-        if (!exact(b) || !is_plane(tensor_at(b), x.device(), 1, N, K)) Py_RETURN_NONE;
-        bits[i] = tensor_at(b);
+        if (i + 1 < layers) most = std::max(most, bgemm_tiled_words(N, K));
     }
     Tensor out;
     {
@@ -172,27 +169,33 @@ PyObject* chain_infer(PyObject*, PyObject* const* args, const Py_ssize_t n)
         const Rows r = rows_2d(x);
         const bool f32 = x.scalar_type() == at::kFloat;
         void* const st = stream_of(x);
-        Tensor in;                            // the operand of the layer at hand; undefined: x itself
+        // The call's own bits, so that other streams and threads may be in the same modules: a layer reads one half and writes the other.
+        const Tensor planes = at::empty({layers > 2 ? 2 : 1, most}, x.options().dtype(at::kInt).requires_grad(false));
+        int32_t* const half[2] = {planes.data_ptr<int32_t>(), planes.data_ptr<int32_t>() + (layers > 2 ? most : 0)};
+        const void* in = nullptr;             // the operand of the layer at hand; null: x itself
+        Tensor first;
         if (bgemm_linear_rows_supported(N, l[0].M, K0, 1, bits_kind(f32)) != 2) {
-            in = new_plane(x, 1, N, K0);
-            check(bgemm_pack_batched(r.t.data_ptr(), src_type(x), 0, l[0].zpa.data_ptr(), 1, 1, N, K0, r.ld, 0, 0, in.data_ptr(), nullptr, st));
+            first = new_plane(x, 1, N, K0);
+            in = first.data_ptr();
+            check(bgemm_pack_batched(r.t.data_ptr(), src_type(x), 0, l[0].zpa.data_ptr(), 1, 1, N, K0, r.ld, 0, 0, first.data_ptr(), nullptr, st));
         }
         out = at::empty(with_last(x, l.back().M), x.options().requires_grad(false));
         for (Py_ssize_t i = 0; i < layers; i++) {
             const Layer& a = l[i];
             if (i + 1 == layers)
-                check(bgemm_packed_forward_scaled(BGEMM_MODE_XOR, a.packed.data_ptr(), in.data_ptr(), nullptr, out.data_ptr(), scaled_kind(f32), 1, a.M, N, a.K, 0, 0, N * a.M,
+                check(bgemm_packed_forward_scaled(BGEMM_MODE_XOR, a.packed.data_ptr(), in, nullptr, out.data_ptr(), scaled_kind(f32), 1, a.M, N, a.K, 0, 0, N * a.M,
                                                   8, BGEMM_VARIANT_AUTO, nullptr, 0, nullptr, 0, a.sw.data_ptr(), a.sa.data_ptr(), data_or_null(a.bias), st));
             else {
                 const void* const next = l[i + 1].zpa.data_ptr();
-                if (!in.defined()) {
-                    const bgemm_rows_layer layer = a.rows_layer(bits[i].data_ptr(), next);
+                int32_t* const bits = half[i & 1];
+                if (!in) {
+                    const bgemm_rows_layer layer = a.rows_layer(bits, next);
                     check(bgemm_linear_rows_forward(r.t.data_ptr(), src_type(x), r.ld, N, a.M, a.K, 1, &layer, bits_kind(f32), nullptr, 0, st));
                 } else
-                    check(bgemm_packed_forward_bits(BGEMM_MODE_XOR, a.packed.data_ptr(), in.data_ptr(), nullptr, bits[i].data_ptr(), bits_kind(f32), 1, a.M, N, a.K, 0, 0,
-                                                    bits[i].numel(), 8, BGEMM_VARIANT_AUTO, nullptr, 0, nullptr, 0, a.sw.data_ptr(), a.sa.data_ptr(),
+                    check(bgemm_packed_forward_bits(BGEMM_MODE_XOR, a.packed.data_ptr(), in, nullptr, bits, bits_kind(f32), 1, a.M, N, a.K, 0, 0,
+                                                    bgemm_tiled_words(N, a.M), 8, BGEMM_VARIANT_AUTO, nullptr, 0, nullptr, 0, a.sw.data_ptr(), a.sa.data_ptr(),
                                                     data_or_null(a.bias), next, st));
-                in = bits[i];
+                in = bits;
             }
         }
     }

@@ -8,6 +8,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
+import _lib
 import bgemm_linear as bl
 import lowbit_kernel as lk
 
@@ -180,6 +181,34 @@ def test_chain_keeps_only_bits_between_layers(dtype):
             h = layer(h)
         assert torch.equal(chain(x2), h)
     assert chain(x).requires_grad                          # with gradients: the ordinary path
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_chain_on_two_streams_beside_its_own_graph(native, monkeypatch):
+    """The bits between the layers are the call's own: calls on other streams and replays of a capture may run at the same time."""
+    if not native:
+        monkeypatch.setattr(_lib, "_native", None)
+        monkeypatch.setattr(_lib, "_native_looked_for", True)
+    torch.manual_seed(13)
+    chain = bl.BGEMMChain(*(bl.BGEMMLinear(k, m).to(DEV) for k, m in ((512, 2000), (2000, 2000), (2000, 2000), (2000, 100))))
+    xs = [torch.randn(256, 512, device=DEV) for _ in range(3)]
+    with torch.no_grad():
+        chain(xs[0])
+        kept = set(chain.__dict__)
+        want = [chain(x) for x in xs]
+        assert set(chain.__dict__) == kept                          # nothing of a call is left in the module
+        graph = bl.GraphedInference(chain, xs[2])
+        streams = [torch.cuda.Stream() for _ in xs]
+        torch.cuda.synchronize()
+        got = [[] for _ in xs]
+        for _ in range(20):
+            for i, (x, s) in enumerate(zip(xs, streams)):
+                with torch.cuda.stream(s):
+                    got[i].append(graph(x).clone() if i == 2 else chain(x))
+        torch.cuda.synchronize()
+    for outs, y in zip(got, want):
+        for out in outs:
+            assert torch.equal(out, y)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.half])
