@@ -63,7 +63,7 @@ class BinarySelfAttention(nn.Module):
         if not all(_unheard(l) and l.out_features == hidden for l in layers):
             return False
         native = _lib.native_or_none()
-        if native is not None and native.block_ready([l.__dict__ for l in layers], x, self.num_attention_heads):
+        if native is not None and native.block_ready([l.__dict__ for l in layers], x, self.num_attention_heads, self.attention_head_size):
             return True
         return (x.dim() == 3 and x.numel() > 0 and all(l.weight.shape[0] == hidden and l._bits_fusable(x) for l in layers)
                 and lowbit_kernel.attention_supported(x.shape[0], x.shape[1], self.num_attention_heads, self.attention_head_size))

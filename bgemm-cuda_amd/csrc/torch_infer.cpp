@@ -203,24 +203,20 @@ PyObject* chain_infer(PyObject*, PyObject* const* args, const Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
-// block_ready([module.__dict__, ..], x [batch, seq, hidden], heads) -> whether these layers are projections of x into that many heads that the
-// attention kernel takes, one after the other of hidden features and in x's type
+// block_ready([module.__dict__, ..], x [batch, seq, features], heads, head size) -> whether these layers are projections of x into such heads, in
+// x's type, and the attention kernel takes those
 PyObject* block_ready(PyObject*, PyObject* const* args, const Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    TORCH_CHECK_TYPE(n == 3 && PyList_CheckExact(args[0]), "block_ready takes a list, a tensor and a number");
+    TORCH_CHECK_TYPE(n == 4 && PyList_CheckExact(args[0]), "block_ready takes a list, a tensor and two numbers");
     if (!quiet_call(args[1])) Py_RETURN_FALSE;
     const Tensor& x = tensor_at(args[1]);
-    const int64_t heads = PyLong_AsLongLong(args[2]);
+    const int64_t heads = PyLong_AsLongLong(args[2]), size = PyLong_AsLongLong(args[3]);
     if (PyErr_Occurred()) throw python_error();
-    if (x.dim() != 3 || x.numel() == 0 || heads < 1) Py_RETURN_FALSE;
+    if (x.dim() != 3 || x.numel() == 0 || !bgemm_attention_supported(x.size(0), x.size(1), heads, size)) Py_RETURN_FALSE;
     Layer l;
-    int64_t hidden = 0;
-    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[0]); i++) {
-        if (!l.read(PyList_GET_ITEM(args[0], i), x, false) || l.K != x.size(-1) || l.M % heads || (i && l.M != hidden)) Py_RETURN_FALSE;
-        hidden = l.M;
-    }
-    if (!PyList_GET_SIZE(args[0]) || !bgemm_attention_supported(x.size(0), x.size(1), heads, l.M / heads)) Py_RETURN_FALSE;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[0]); i++)
+        if (!l.read(PyList_GET_ITEM(args[0], i), x, false) || l.K != x.size(-1) || l.M != heads * size) Py_RETURN_FALSE;
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }

@@ -7,6 +7,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
+import _lib
 import attention_demo
 import bgemm_linear as bl
 import lowbit_kernel as lk
@@ -127,3 +128,23 @@ def test_block_of_many_rows_with_its_layer_norm_in_the_last_projection(change, m
     assert torch.equal(scores, want_scores) and out.dtype == want.dtype
     # two orders of a sum of 96 values of about one: some 2^-24 each
     torch.testing.assert_close(out, want, rtol=0, atol=0 if change in ("hook", "half", "other") else 2e-5)
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("width", [128, 512])
+def test_block_refuses_projections_of_another_width(width, native, monkeypatch):
+    """Parameters of another width than heads x head size, the modules' own sizes left as they were: refused as by the general path, also where
+    the width splits into heads that the kernel takes."""
+    if not native:
+        monkeypatch.setattr(_lib, "_native", None)
+        monkeypatch.setattr(_lib, "_native_looked_for", True)
+    block = attention_demo.BinarySelfAttention(256, 4).to(DEV)
+    x = torch.randn(2, 40, 256, device=DEV)
+    with torch.no_grad():
+        block(x)
+        for layer in (block.query, block.key, block.value):
+            for name, t in (("weight", torch.randn(width, 256)), ("sw", torch.rand(width)), ("bias", torch.randn(width))):
+                setattr(layer, name, torch.nn.Parameter(t.to(DEV)))
+        for _ in range(2):
+            with pytest.raises(RuntimeError, match="invalid for input of size"):
+                block(x)
