@@ -79,9 +79,9 @@ class BinarySelfAttention(nn.Module):
         """The layer norm as ``linear_rows_forward`` takes it; None where it is not a plain fp32 one over these features whose call nothing listens to."""
         norm = self._modules.get("LayerNorm")
         if (type(norm) is not nn.LayerNorm or norm.normalized_shape != (hidden,) or norm._forward_hooks or norm._forward_pre_hooks
-                or "forward" in norm.__dict__ or x.dtype != torch.float32):
-            return None
-        parameters = norm._parameters.get("weight"), norm._parameters.get("bias")
+                or "forward" in norm.__dict__ or x.dtype != torch.float32 or "weight" not in norm._parameters or "bias" not in norm._parameters):
+            return None          # (one that is not registered, not even as None, has been replaced by something else)
+        parameters = norm._parameters["weight"], norm._parameters["bias"]
         for t in parameters:
             if t is not None and (type(t) is not nn.Parameter or t.dtype != torch.float32 or t.device != x.device or t.shape != (hidden,) or not t.is_contiguous()):
                 return None

@@ -99,7 +99,7 @@ def test_block_with_other_parts_takes_its_general_path(other, monkeypatch):
     assert other != "heads" or calls.count("heads") == 6
 
 
-@pytest.mark.parametrize("change", ["none", "plain", "hook", "half", "other"])
+@pytest.mark.parametrize("change", ["none", "plain", "hook", "half", "other", "tensor"])
 def test_block_of_many_rows_with_its_layer_norm_in_the_last_projection(change, monkeypatch):
     """From a thousand rows on the block's layer norm is part of its last launch, unless it is another module or somebody listens to it."""
     torch.manual_seed(5)
@@ -116,18 +116,22 @@ def test_block_of_many_rows_with_its_layer_norm_in_the_last_projection(change, m
         block, x = block.half(), x.half()
     if change == "other":
         block.LayerNorm = torch.nn.Identity()
+    if change == "tensor":                                                     # as some reparametrisations leave it: no parameter, an attribute
+        weight = block.LayerNorm.weight.detach().clone()
+        del block.LayerNorm.weight
+        block.LayerNorm.weight = weight
     with torch.no_grad():
         block(x)
         del seen[:]
         calls = []
         monkeypatch.setattr(torch.nn.functional, "layer_norm", lambda *a, f=torch.nn.functional.layer_norm: calls.append(1) or f(*a))
         out, scores = block(x)
-        assert len(calls) == (1 if change in ("hook", "half") else 0) and len(seen) == (change == "hook")
+        assert len(calls) == (1 if change in ("hook", "half", "tensor") else 0) and len(seen) == (change == "hook")
         monkeypatch.setattr(lk, "linear_rows_norm_supported", lambda *a: 1)
         want, want_scores = block(x)
     assert torch.equal(scores, want_scores) and out.dtype == want.dtype
     # two orders of a sum of 96 values of about one: some 2^-24 each
-    torch.testing.assert_close(out, want, rtol=0, atol=0 if change in ("hook", "half", "other") else 2e-5)
+    torch.testing.assert_close(out, want, rtol=0, atol=0 if change in ("hook", "half", "other", "tensor") else 2e-5)
 
 
 @pytest.mark.parametrize("native", [True, False])
