@@ -10,12 +10,13 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 SO_PATH = os.path.join(_HERE, "libbgemm_mi355x.so")
+NATIVE_PATH = os.path.join(_HERE, "_bgemm_native.so")
 
 OK, EINVAL, ENULL, EWORKSPACE, ELAUNCH, EALIGN, ETIMEOUT = 0, -1, -2, -3, -4, -5, -6
 MODE_AND, MODE_XOR, MODE_ATTN, MODE_BWTA, MODE_ATTN_X = 0, 1, 2, 3, 4
 OUT_I32, OUT_F16, OUT_F32_SCALED, OUT_F16_SCALED, OUT_BITS_F32, OUT_BITS_F16 = 0, 1, 2, 3, 4, 5
 SRC_F16, SRC_F32, SRC_BITS = 0, 1, 2
-ABI_VERSION = 11
+ABI_VERSION = 12
 LAYOUT_VERSION = 6     # of the tiled operand layout, written into packed files; changes only when the layout does
 STATIC_SCRATCH_BYTES = 32 << 20      # BGEMM_STATIC_SCRATCH_BYTES
 VARIANT_AUTO, VARIANT_VALU, VARIANT_MFMA, VARIANT_MFMA_F4 = 0, 1, 2, 3
@@ -126,14 +127,16 @@ def native():
     global _native
     if _native is None:
         lib()                                  # the same library, with its version checked
-        path = os.path.join(_HERE, "_bgemm_native.so")
-        if not os.path.exists(path):
-            raise ImportError("%s is missing: build it with `python %s`" % (path, os.path.join(_HERE, "_build.py")))
+        if not os.path.exists(NATIVE_PATH):
+            raise ImportError("%s is missing: build it with `python %s`" % (NATIVE_PATH, os.path.join(_HERE, "_build.py")))
         import torch                           # noqa: F401  (its libraries must be loaded first)
-        loader = importlib.machinery.ExtensionFileLoader("_bgemm_native", path)
-        spec = importlib.util.spec_from_file_location("_bgemm_native", path, loader=loader)
+        loader = importlib.machinery.ExtensionFileLoader("_bgemm_native", NATIVE_PATH)
+        spec = importlib.util.spec_from_file_location("_bgemm_native", NATIVE_PATH, loader=loader)
         module = importlib.util.module_from_spec(spec)
         loader.exec_module(module)
+        version = getattr(module, "abi_version", None)
+        if version != ABI_VERSION:
+            raise ImportError("%s is of version %s, this binding needs %d: rebuild it" % (NATIVE_PATH, version, ABI_VERSION))
         _native = module
     return _native
 
@@ -146,7 +149,7 @@ def native_or_none():
     global _native_looked_for
     if _native is None and not _native_looked_for:
         _native_looked_for = True
-        if os.path.exists(os.path.join(_HERE, "_bgemm_native.so")):
+        if os.path.exists(NATIVE_PATH):
             return native()
     return _native
 

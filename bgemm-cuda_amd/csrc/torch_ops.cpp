@@ -382,5 +382,11 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_bgemm_native", "host side of 
 PyMODINIT_FUNC PyInit__bgemm_native(void)
 {
     module_def.m_methods = all_methods();
-    return PyModule_Create(&module_def);
+    PyObject* const module = PyModule_Create(&module_def);
+    // what it was built for: an older one lacks functions that the Python side calls
+    if (module && PyModule_AddIntConstant(module, "abi_version", BGEMM_ABI_VERSION) != 0) {
+        Py_DECREF(module);
+        return nullptr;
+    }
+    return module;
 }

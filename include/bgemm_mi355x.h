@@ -78,8 +78,9 @@ enum {
 
 /* Message for the last error returned on the calling thread ("" if none). */
 const char* bgemm_last_error(void);
-/* ABI version; bumped when a signature or the tiled layout changes. */
-int bgemm_abi_version(void);
+/* ABI version; bumped when an entry point is added or its signature or behaviour changes, or the tiled layout does. */
+#define BGEMM_ABI_VERSION 12
+int bgemm_abi_version(void);          /* of the library */
 
 /* ---- packed operand layout -------------------------------------------------------
  * "Logical" format = the reference's (weight_prepacking.h:181-230): uint32 [rows][ceil(K/32)],

@@ -6,6 +6,7 @@ import re
 import shutil
 import struct
 import subprocess
+import sysconfig
 
 import pytest
 
@@ -52,7 +53,7 @@ def test_header_is_plain_c_and_a_c_program_links(tmp_path):
 
 def test_layout_sizes():
     L = _lib.lib()
-    assert L.bgemm_abi_version() == _lib.ABI_VERSION == 11
+    assert L.bgemm_abi_version() == _lib.ABI_VERSION == 12
     assert L.bgemm_tiled_words(1, 1) == 256
     assert L.bgemm_tiled_words(32, 256) == 256
     assert L.bgemm_tiled_words(33, 257) == 4 * 256
@@ -406,6 +407,26 @@ def test_a_library_of_another_version_says_so(tmp_path, monkeypatch):
     monkeypatch.setattr(_lib, "SO_PATH", str(so))
     with pytest.raises(ImportError, match="rebuild it"):
         _lib.lib()
+
+
+def test_a_native_host_side_of_another_version_says_so(tmp_path, monkeypatch):
+    """One from before it stated its version, and one of the version before this."""
+    gcc = shutil.which("gcc")
+    if not gcc:
+        pytest.skip("no gcc")
+    state = 'PyObject* m = PyModule_Create(&def); PyModule_AddIntConstant(m, "abi_version", %d); return m;' % (_lib.ABI_VERSION - 1)
+    for i, body in enumerate(("return PyModule_Create(&def);", state)):
+        src, so = tmp_path / ("old%d.c" % i), tmp_path / ("old%d.so" % i)
+        src.write_text('#include <Python.h>\nstatic struct PyModuleDef def = {PyModuleDef_HEAD_INIT, "_bgemm_native", 0, -1, 0};\n'
+                       'PyMODINIT_FUNC PyInit__bgemm_native(void) { %s }\n' % body)
+        subprocess.check_call([gcc, "-shared", "-fPIC", "-I", sysconfig.get_paths()["include"], str(src), "-o", str(so)])
+        monkeypatch.setattr(_lib, "_native", None)
+        monkeypatch.setattr(_lib, "NATIVE_PATH", str(so))
+        with pytest.raises(ImportError, match="rebuild it"):
+            _lib.native()
+    monkeypatch.undo()
+    monkeypatch.setattr(_lib, "_native", None)
+    assert _lib.native().abi_version == _lib.ABI_VERSION
 
 
 def test_the_native_host_side_is_loaded_for_calls_that_can_take_it(monkeypatch):
