@@ -145,12 +145,13 @@ _native_looked_for = False
 
 
 def native_or_none():
-    """native() if it has been built, else None: for calls that have a form without it."""
+    """native() if it has been built, else None: for calls that have a form without it.  One that is there and does not load says so on
+    every call."""
     global _native_looked_for
     if _native is None and not _native_looked_for:
-        _native_looked_for = True
         if os.path.exists(NATIVE_PATH):
             return native()
+        _native_looked_for = True
     return _native
 
 

@@ -429,6 +429,19 @@ def test_a_native_host_side_of_another_version_says_so(tmp_path, monkeypatch):
     assert _lib.native().abi_version == _lib.ABI_VERSION
 
 
+def test_a_native_host_side_that_does_not_load_says_so_on_every_call(tmp_path, monkeypatch):
+    broken = tmp_path / "broken.so"
+    broken.write_bytes(b"no library")
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(_lib, "_native_looked_for", False)
+    monkeypatch.setattr(_lib, "NATIVE_PATH", str(broken))
+    for _ in range(3):
+        with pytest.raises(ImportError):
+            _lib.native_or_none()
+    monkeypatch.setattr(_lib, "NATIVE_PATH", str(tmp_path / "missing.so"))
+    assert _lib.native_or_none() is None and _lib.native_or_none() is None
+
+
 def test_the_native_host_side_is_loaded_for_calls_that_can_take_it(monkeypatch):
     import torch
 
