@@ -348,6 +348,9 @@ struct LinearPack {
 };
 int pack_linear_pair(const LinearPack& a, hipStream_t st, const char* who);
 
+// Outputs that the one-launch rows kernel (linear_rows.hip) stores later than a GEMM.
+bool linear_rows_past_caches(int64_t N, int64_t M, int64_t K, int out_dtype);
+
 // Kernel families (each in its own translation unit).
 int launch_gemm_mfma(const GemmArgs& a, hipStream_t st, bool fp4);
 int gemm_mfma_kernel_id(int64_t batch, int64_t M, int64_t N, int64_t KT, int planes, int out_kind, bool fp4);     // BGEMM_KERNEL_MFMA_* by shape

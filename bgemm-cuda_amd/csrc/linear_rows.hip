@@ -598,6 +598,15 @@ static RowsPlan rows_plan(int64_t N, int64_t M, int64_t K, int layers, bool pack
     return p;
 }
 
+// fp32 numbers of which there are more than the caches take, on rows that share lines of 128 bytes and on a K so short that little but their
+// stores is left: a GEMM's tiles finish such lines sooner than blocks that share a row tile (us, pack and GEMM / here: 16384 x 128 x 3000 51 / 65, x
+// 768 64 / 73, but x 1024 69 / 71 and 16384 x 1024 x 4100 135 / 106; rows that share no 64 bytes 16384 x 128 x 6000 84 / 103, x 512 99 / 105, but x
+// 768 112 / 104; half as many numbers 8192 x 128 x 4100 36.7 / 31.0).
+bool linear_rows_past_caches(int64_t N, int64_t M, int64_t K, int out_dtype)
+{
+    return out_dtype == BGEMM_OUT_F32_SCALED && N * M > (40 << 20) && M % 32 && k_tiles(K) <= (M % 16 ? 3 : 2);
+}
+
 }  // namespace bgemm
 
 using namespace bgemm;
@@ -612,9 +621,14 @@ extern "C" int bgemm_linear_rows_supported(int64_t N, int64_t M, int64_t K, int 
     // over K, which the decode kernels split among their waves: us, two launches / this one, fp32 32 x 512 x 4096 7.3 / 4.5, 32 x 1000 x
     // 4096 6.5 / 5.8 but 16 x 1000 x 1000 5.9 / 6.0, 128 x 1536 x 4096 7.4 / 7.7 and 512 x 1536 x 4096 10.1 / 7.8, 512 x 2048 x 1000 7.8 / 9.0
     // and 2048 x 2048 x 1000 12.4 / 10.9.  Beyond 16384 columns a few hundred rows are too few for a block a row tile to share them
-    // (512 x 2048 x 22016 22.2 / 26.7, fp16 512 x 1000 x 22016 15.1 / 16.1).
+    // (512 x 2048 x 22016 22.2 / 26.7, fp16 512 x 1000 x 22016 15.1 / 16.1).  Bits (one layer, fp32 32 x 512 x 4096 8.6 / 4.4, 1 x 512 x 512 5.2 /
+    // 4.1, 512 x 1500 x 4096 10.0 / 7.2, 2048 x 2048 x 512 11.5 / 7.9) are ahead on fewer rows than that, already on 8 at three or four K-tiles and on 32 at six
+    // (32 x 1024 x 512 7.2 / 5.3, 128 x 1500 x 512 7.5 / 6.6; 1 x 1500 x 512 5.3 / 6.3, 128 x 2048 x 512 6.8 / 7.7), never behind where this says 2.
+    // Three layers' bits are ahead wherever they are taken (1 x 1024 x (3 x 1024) six launches 15.3, one 7.6), and a residual on a packed operand
+    // beside a pack, a GEMM and the addition from two rows on (4 x 2048 x 2048 fp32 5.9 / 5.3, 256 rows 10.0 / 5.6; one row 4.9 / 5.3, four fp16 5.8 /
+    // 7.0: no more than the launches that fall away cost the host).
     const int64_t KT = k_tiles(K), rows = KT <= 2 ? 1 : KT <= 4 ? 33 : KT <= 6 ? 512 : 2048;
-    return N >= rows && (M <= 16384 || N < 256) ? 2 : 1;
+    return N >= rows && (M <= 16384 || N < 256) && !linear_rows_past_caches(N, M, K, out_dtype) ? 2 : 1;
 }
 
 extern "C" int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx, int64_t N, int64_t M, int64_t K, int layers,
