@@ -145,12 +145,13 @@ __global__ __launch_bounds__(WAVES * 64) void scores_kernel(const AttnProductArg
     }
 }
 
-// A wave takes 32 rows of P and one of `splits` equal parts of its columns, 64 at a time and two groups requested ahead; a lane's eight
+// A wave takes 32 rows of P and all of its columns or one half of them, 64 at a time and two groups requested ahead; a lane's eight
 // elements become a byte, and the bytes of a row, through LDS, the word that is the product's operand.  A block's rows are CTX_ROWS.
 constexpr int CTX_ROWS = 128;
 
+// (blocks of at most 512 threads; the registers of four waves a SIMD are enough up to D = 96, which takes 124)
 template <int W>
-__global__ __launch_bounds__(W == 4 ? 512 : 1024) void context_kernel(const AttnProductArgs a)
+__global__ __launch_bounds__(512, W == 4 ? 2 : 4) void context_kernel(const AttnProductArgs a)
 {
     constexpr int D = W * 32;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -248,11 +249,11 @@ __global__ __launch_bounds__(W == 4 ? 512 : 1024) void context_kernel(const Attn
         ++grp;
     }
     counted += __shfl_xor(counted, 32);
-    // The parts' sums, whole numbers of at most M <= 4096, meet in 16 bits where V's words were.
-    for (int n = parts >> 1; n; n >>= 1) {
-        uint32_t* const to = reinterpret_cast<uint32_t*>(smem) + ((part & (n - 1)) * 4 + (wave & 3)) * (W * 8 + 1) * 64 + lane;
+    // The halves' sums, whole numbers of at most M <= 4096, meet in 16 bits where V's words were.
+    if (parts == 2) {
+        uint32_t* const to = reinterpret_cast<uint32_t*>(smem) + (wave & 3) * (W * 8 + 1) * 64 + lane;
         __syncthreads();
-        if (part >= n && part < 2 * n) {
+        if (part) {
 #pragma unroll
             for (int t = 0; t < W; t++)
 #pragma unroll
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(W == 4 ? 512 : 1024) void context_kernel(const Attn
             to[W * 8 * 64] = (uint32_t)counted;
         }
         __syncthreads();
-        if (part < n) {
+        if (!part) {
 #pragma unroll
             for (int t = 0; t < W; t++)
 #pragma unroll
@@ -351,7 +352,7 @@ extern "C" int bgemm_context_forward(const void* probs, const void* value, const
     // Two waves to a row fill the chip (48 x 512^2, D = 64: 13.5 -> 10.8 us; 2 x 512^2: 11.9 -> 9.1) unless the blocks already do
     // (192 x 512^2: 28.6 -> 31.6) or a row is short (16 x 128^2: 5.4 -> 5.9).  Four were never ahead of two by more than 2 us.
     const int parts = M < 256 || blocks > 512 ? 1 : 2;
-    const size_t words = (size_t)2 * (D / 32) * cdiv(M, 64) * 64 * 4 + (size_t)parts * 4 * 256, sums = (size_t)(parts / 2) * 4 * (D / 32 * 8 + 1) * 256;
+    const size_t words = (size_t)2 * (D / 32) * cdiv(M, 64) * 64 * 4 + (size_t)parts * 4 * 256, sums = (size_t)(parts - 1) * 4 * (D / 32 * 8 + 1) * 256;
     const size_t lds = words > sums ? words : sums;
     const dim3 grid((unsigned)blocks), block(parts * 256);
     const hipStream_t st = (hipStream_t)stream;
