@@ -111,6 +111,24 @@ def test_scales_that_are_not_ordinary(scale, dt):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.half])
+@pytest.mark.parametrize("scale", [0.0, -0.0, -1.0, float("inf"), -float("inf"), 2.0 ** -24, 60000.0])
+def test_bits_of_scales_that_are_not_ordinary(scale, dt):
+    """Wherever the centred number is one (the sign of a NaN is not defined)."""
+    for shape in (0, 1 | 5 << 4 | 1 << 12, 2 | 2 << 4 | 2 << 12):
+        x, ls = made(40, 70, 96, 1, dt, True)
+        w, zp, sw, sa, bias = ls[0]
+        sw[::3] = scale
+        sw[1::7] = float("nan")
+        bias[::5] = -scale
+        following = torch.full((1,), 0.25, dtype=dt, device=DEV)
+        got, = lk.linear_rows_forward(x, packed(ls), bits=True, next_zero_point=following, shape=shape)
+        words = lk.logical_from_tiled(got)
+        bits = (words[:, torch.arange(70, device=DEV) // 32] >> (31 - torch.arange(70, device=DEV) % 32)) & 1
+        want = formula(x, *ls[0]) - following
+        assert torch.equal(bits[~want.isnan()] != 0, torch.signbit(want[~want.isnan()])) and bool((~want.isnan()).any())
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.half])
 @pytest.mark.parametrize("B, S, H, d", [(1, 1, 1, 32), (2, 33, 5, 64), (3, 70, 3, 96), (1, 130, 7, 128), (2, 64, 8, 32)])
 def test_context_as_bits(B, S, H, d, dt):
     g = torch.Generator(device=DEV).manual_seed(S + d)
@@ -147,3 +165,30 @@ def test_layer_norm_of_rows_and_residual(N, M, K):
         far = z.abs().amax(1, keepdim=True)
         bound = 64 * 2.0 ** -24 * ((1 + far / (var + 1e-12).sqrt()) * (torch.ones_like(z) * gd).abs() + (want - bd).abs() + abs(bd))
         assert bool(((got.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("N, M", [(1, 33), (33, 64), (40, 97), (95, 31), (65, 513), (31, 1001)])
+def test_the_layer_norm_writes_nothing_past_the_output_and_keeps_rows_apart(N, M):
+    """The last row tile and column tile end where the output does; infinities and NaNs of one row stay in it."""
+    K = 100
+    x, ls = made(N, M, K, 1, torch.float32, True)
+    (w, zp, sw, sa, bias), = packed(ls)
+    xp, residual = lk.pack_sign(x.contiguous(), zp), torch.randn(N, M, device=DEV)
+    lost = torch.arange(N, device=DEV) % 4 == 1
+    for row, value in zip(lost.nonzero()[:, 0].tolist(), [float("inf"), -float("inf"), float("nan")] * N):
+        residual[row, row % M] = value
+    gamma, beta = torch.randn(M, device=DEV), torch.randn(M, device=DEV)
+    room = torch.full(((N + 64) * M + 2048,), 7.0, device=DEV)                 # a further row tile would fit
+    out = room[1024:1024 + N * M]
+    layer = (_lib.RowsLayer * 1)()
+    layer[0].W_tiled, layer[0].sw, layer[0].sa, layer[0].bias, layer[0].out = w.data.data_ptr(), sw.data_ptr(), sa.data_ptr(), bias.data_ptr(), out.data_ptr()
+    _lib.check(_lib.lib().bgemm_linear_rows_norm_forward(xp.data.data_ptr(), N, M, K, layer, residual.data_ptr(), gamma.data_ptr(), beta.data_ptr(), 1e-12, None))
+    assert bool((room[:1024] == 7).all()) and bool((room[1024 + N * M:] == 7).all())
+    got = out.view(N, M)
+    assert bool(got[lost].isnan().all())                                       # a mean that is not finite leaves nothing of its row
+    z = (formula(x, *ls[0]) + residual)[~lost].double()
+    want = torch.nn.functional.layer_norm(z, (M,), gamma.double(), beta.double(), 1e-12)
+    # (as above: at most 64 roundings of 2^-24 on values of the mean's size and deviation)
+    far, dev = z.abs().amax(1, keepdim=True), (z.var(1, unbiased=False, keepdim=True) + 1e-12).sqrt()
+    bound = 64 * 2.0 ** -24 * ((1 + far / dev) * gamma.double().abs() + (want - beta.double()).abs() + beta.double().abs())
+    assert bool(((got[~lost].double() - want).abs() <= bound).all())
