@@ -580,8 +580,10 @@ def bench_c2(steps=200, warmup=20):
     """3-layer binarised MLP forward 784->4096->4096->10, batch 128, fp16 activations and per-output-channel
     fp16 scales.  Timed op by op through the fp16 drop-in call (weights packed on every call, scaling as
     separate torch kernels, as the reference layer does), fused (weights prepacked once, activations
-    sign-packed in one pass, scaling applied in the GEMM's store), and with nothing but bits between the layers."""
+    sign-packed in one pass, scaling applied in the GEMM's store), and with nothing but bits between the layers: a pack and three
+    GEMMs from a graph, and as users call it, three launches of ``BGEMMChain`` from Python."""
     import torch
+    import bgemm_linear as bl
     import lowbit_kernel as lk
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(2001)
@@ -611,22 +613,33 @@ def bench_c2(steps=200, warmup=20):
         for l in range(2):
             hp = lk.bgemm_packed_forward(Wps[l], hp, lk.MODE_XOR, splitK=8, scale=(sws[l], sa, None), bits_out=hidden[l])
         return lk.bgemm_packed_forward(Wps[2], hp, lk.MODE_XOR, splitK=8, scale=(sws[2], sa, None))[0]
+    chain = bl.BGEMMChain(*(bl.BGEMMLinear(k, m) for k, m in zip(dims, dims[1:]))).half().to(dev)
+    with torch.no_grad():
+        chain(x)                                # sets the layers' scales and zero points
+        for layer, W, sw in zip(chain, Ws, sws):
+            for t, value in ((layer.weight, W), (layer.sw, sw), (layer.sa, sa[0]), (layer.zpa, 0), (layer.zpw, 0)):
+                t.copy_(value) if isinstance(value, torch.Tensor) else t.fill_(value)
+
+    def fwd_chain(i):
+        with torch.no_grad():
+            return chain(x)
     # the fp16 reference: torch matmul on the de-binarised tensors, scaled op by op
     h = x
     for W, sw in zip(Ws, sws):
         sx = torch.where(h.view(torch.int16) < 0, -1.0, 1.0)
         sw_ = torch.where(W.view(torch.int16) < 0, -1.0, 1.0)
         h = (sx @ sw_.T).half() * sw * sa
-    same = bool(torch.equal(fwd_ops(0), h)) and bool(torch.equal(fwd_fused(0), h)) and bool(torch.equal(fwd_bits(0), h))
+    same = bool(torch.equal(fwd_ops(0), h)) and bool(torch.equal(fwd_fused(0), h)) and bool(torch.equal(fwd_bits(0), h)) and bool(torch.equal(fwd_chain(0), h))
     ms_ops = time_gpu(fwd_ops, warmup, steps)
     ms_fused = time_gpu(fwd_fused, warmup, steps)
     ms_graph = time_gpu_graph(fwd_fused, 4, 2, max(2, steps // 4))
     ms_bits = time_gpu_graph(fwd_bits, 4, 2, max(2, steps // 4))
+    ms_chain = time_gpu(fwd_chain, warmup, steps)
     ops = 2.0 * 128 * (784 * 4096 + 4096 * 4096 + 4096 * 10)
     bytes_alg = sum(W.numel() for W in Ws) / 8 + 2.0 * 128 * (784 + 10)
     return row("C2 MLP 784-4096-4096-10 b128, bits between layers, 4 launches (graph)", ms_bits, ops,
                bytes_alg, same, "pack+3 gemm", "mfma", us_6_launches=round(ms_graph * 1e3, 2),
-               us_from_python=round(ms_fused * 1e3, 2), us_op_by_op=round(ms_ops * 1e3, 2))
+               us_chain_from_python=round(ms_chain * 1e3, 2), us_from_python=round(ms_fused * 1e3, 2), us_op_by_op=round(ms_ops * 1e3, 2))
 
 
 # ---------------------------------------------------------------- thresholds behind the dispatch

@@ -504,7 +504,8 @@ class BGEMMChain(nn.Sequential):
     """BGEMMLinear layers applied back to back (the binarisation is the only nonlinearity between them).
     When no gradient is recorded the activations between layers exist only as bits: every GEMM but the last
     writes the next layer's centred, sign-packed operand straight from its accumulators, so a chain of L
-    layers is L launches (L + 1 on a long input) and never stores a hidden activation.  Same results as calling the layers one
+    layers is L launches (L + 1 where the first layer's rows are packed by themselves: more than 2048 features, or
+    few rows of more than 512) and never stores a hidden activation.  Same results as calling the layers one
     after the other, bit for bit.  Not in the reference, which has no layer container."""
 
     def _fusable(self, x):

@@ -43,11 +43,11 @@ __device__ __forceinline__ unsigned rows_x(const unsigned inverted, const int s)
 // whose weights come straight from the caches into registers, two K-tiles ahead.  The accumulators leave without a detour: a lane holds a
 // column of sixteen rows (numbers: a half-wave stores a whole line; fp16 in pairs of columns), or with the operands exchanged sixteen
 // columns of a row (bits: one instruction collects a sign, and whole 16-byte pieces of the output's tiles leave behind a barrier).
-// What bounds it: numbers on many rows the stores, 8192 x 768 x 3072 fp32 24.3 us in place of 34 in two launches (101 MB of stores and
-// 25 of reads, 5.2 TB/s; fp16 18.7 for 23.5); bits the vector units, half of them the scaling: three layers 8192 x 768 x 768 14 us
-// where three packs and three GEMMs took 46.7, each reading x and passing its outputs through LDS and a ballot a row; with a residual
-// and a packed operand 8192 x 768 x 768 8.4 for 24.3 with the addition as its own pass.  Few rows: the chain of one row tile, 64 x 512
-// x 512 4.5 for 7.6.
+// What bounds it: numbers on many rows the stores, 8192 x 768 x 3072 fp32 25.3 us in place of 34.1 in two launches (101 MB of stores and
+// 25 of reads, 5.0 TB/s; from and to memory, sets of buffers in turn, 26.5 for 37.8; fp16 17.7 for 26.7); bits the vector units, half of
+// them the scaling: three layers 8192 x 768 x 768 14 us where three packs and three GEMMs took 46.7, each reading x and passing its outputs
+// through LDS and a ballot a row; with a residual and a packed operand 8192 x 768 x 768 8.4 for 24.3 with the addition as its own pass.
+// Few rows: the chain of one row tile, 64 x 512 x 512 4.5 for 7.6.
 template <int SRC, int KIND, int CT>
 __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const RowsArgs a)
 {
@@ -96,7 +96,7 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
     };
     // Those of the first two K-tiles are on their way while the bits are made, where bits leave and little else fills that time (us:
     // 8192 x 768 x (3 x 768) 15.9 -> 15.4, 2048 x 768 x (3 x 768) 8.4 -> 8.0, 128 x 784 x 4096 7.2 -> 7.1; numbers, which have stores to
-    // wait for: 8192 x 768 x 3072 packed 23.3 -> 23.7, fp16 4096 x 1024 x 1024 8.2 -> 8.3).
+    // wait for: on packed rows 8192 x 768 x 3072 23.3 -> 23.7, fp16 4096 x 1024 x 1024 8.2 -> 8.3).
     v4i w0[CT], w1[CT], w2[CT];
     if constexpr (BITS) {
         request(w0);
@@ -566,7 +566,7 @@ static RowsPlan rows_plan(int64_t N, int64_t M, int64_t K, int layers, bool pack
     const int64_t rt = row_tiles(N);
     // How many column tiles a wave multiplies at once, how many waves a layer has in a block, how many blocks share a row tile.
     // Numbers, one tile (fp16: a pair), eight waves, as many blocks as there are groups for up to two a compute unit, one storing while the
-    // other makes its bits (us, 16 waves and one block / 8 and two, from and to memory: fp32 8192 x 768 x 3072 29.0 / 28.9, x 1008 16.0 /
+    // other makes its bits (us, 16 waves and one block / 8 and two, from and to memory, on a kernel that is 10 % faster now: fp32 8192 x 768 x 3072 29.0 / 28.9, x 1008 16.0 /
     // 14.9; fp16 20.3 / 19.3; 512 x 512 x 2048 7.1 / 5.7).  Beyond K = 1024 making them again costs more than that, fp32 rows of 16 KiB meet
     // on the same memory channels when more blocks store at a time (8192 x 256 x 4096 30.7 / 37.1), and bits have nothing to store: one
     // block a compute unit, of as many waves as give each a tile or two (2048 x 2048 x 2048 10.8, in two blocks of eight 13.7; 8192 x
@@ -662,7 +662,7 @@ extern "C" int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx
     a.groups = (int)p.groups; a.splits = (int)p.splits; a.own = (int)p.own;
     a.first_lds = (int)p.first_lds;
     a.gather = bits && p.splits == 1 ? (int)k_tiles(M) * 8 : 0;
-    // Past the caches where no two blocks share a 64-byte piece of a row (fp32 8192 x 768 x 3072 34.3 -> 28.9, 4096 x 1024 x 4096 26.6 ->
+    // Past the caches where no two blocks share a 64-byte piece of a row (from and to memory, on a kernel that is 10 % faster now: fp32 8192 x 768 x 3072 34.3 -> 28.9, 4096 x 1024 x 4096 26.6 ->
     // 19.7, fp16 8192 x 768 x 768 12.9 -> 11.0; rows of 4000 bytes 19.0 -> 20.3, of fp16 6176 26.5 -> 28.6).
     a.nt = M * (f32 ? 4 : 2) % 64 == 0;
     const size_t lds = (size_t)p.lds;

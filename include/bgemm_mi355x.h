@@ -330,7 +330,8 @@ int bgemm_elastic_backward(const void* x_sign, const void* x_nonzero, const void
  *   bits kinds:   out = the sign bits of half(y - *next_zero_point) (NULL: 0), tiled; padding as bgemm_packed_forward_bits leaves it
  * Supported (else 0): 8 <= K <= 2048, M <= 65536, N <= 2^24, the rows' bits (and with bits out the parameters) within 64 KiB of LDS;
  * 2 where one layer is also ahead of a pack and a GEMM, else 1.
- * tiles: column tiles a wave multiplies at once, 0 = chosen by size (1 to 3: tests). */
+ * shape: 0 = chosen by size; else (tests) column tiles a wave multiplies at once, 1 or 2 | waves a layer << 4 | blocks a row tile << 12, the
+ * last 0 = chosen by size.  Results do not depend on it. */
 typedef struct bgemm_rows_layer {
     const void* W_tiled;
     const void* zero_point;
@@ -346,7 +347,8 @@ int bgemm_linear_rows_forward(const void* x, int x_dtype, int64_t ldx, int64_t N
 /* One layer of packed rows (sign bits, tiled, 16-byte aligned, the padding of their columns zero), fp32 parameters, with a residual and a
  * layer norm behind it: out [N][M] = (z - mean(z)) / sqrt(var(z) + eps) * gamma + beta over each row of
  * z = y + residual, y as above; gamma, beta [M] or NULL (1, 0); zero_point and next_zero_point are not looked at.  Supported (else 0): M, K
- * <= 1024, N <= 2^24; 2: and worth a layer norm with another order of sums than the separate one's. */
+ * <= 1024, N <= 2^24; 2: and worth a layer norm with another order of sums than the separate one's.  z, its sums over a wave's columns and what
+ * is stored are in 32 bits; the sums over the waves, the mean (rounded to 32 before it is subtracted) and the deviation in 64. */
 int bgemm_linear_rows_norm_supported(int64_t N, int64_t M, int64_t K);
 int bgemm_linear_rows_norm_forward(const void* x_tiled, int64_t N, int64_t M, int64_t K, const bgemm_rows_layer* layer, const void* residual,
                                    const void* gamma, const void* beta, double eps, void* stream);
