@@ -800,7 +800,7 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
                 if ((lane & 31) == 0 && row_ok && word_ok[k]) obase[wbase[k] + row * 4] = w;
             }
             // (the strip with the rows' last words)
-            if (mcol0 < a.M && mcol0 + 32 * WM >= a.M && lane < 32 && nrow0 + lane < a.N) end_bits_row(obase, nrow0 + lane, a.M);
+            if (a.MT % 8 && mcol0 < a.M && mcol0 + 32 * WM >= a.M && lane < 32 && nrow0 + lane < a.N) end_bits_row(obase, nrow0 + lane, a.M);
         }
         wave_sync();                                 // the next strip overwrites the staging area
     }

@@ -233,11 +233,7 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
                 if ((mt + 1) * 32 > a.M) word &= 0xffffffffu << ((mt + 1) * 32 - a.M);
                 if (a.gather) {
                     if (h == 0) words[(l * a.gather + mt) * 32 + c] = word;
-                } else if (h == 0 && n < a.N) {
-                    uint32_t* const out = reinterpret_cast<uint32_t*>(L.out);
-                    out[tiled_word_offset(n, mt, k_tiles(a.M))] = word;
-                    if (mt == a.MT - 1) end_bits_row(out, n, a.M);
-                }
+                } else if (h == 0 && n < a.N) reinterpret_cast<uint32_t*>(L.out)[tiled_word_offset(n, mt, k_tiles(a.M))] = word;
             }
         } else if constexpr (KIND == ROWS_F32) {
             const __amdgpu_buffer_rsrc_t ro = rows_of(L.out), rr = rows_of(a.residual);
@@ -375,6 +371,11 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void linear_rows_kernel(const 
             step(w2);
             if (gg >= g1) break;
         }
+    }
+    if (BITS && !a.gather && a.MT % 8 && g1 == a.groups) {
+        // the block with the rows' last words ends them
+        for (int i = threadIdx.x; i < a.layers * 32; i += waves * 64)
+            if (rt * 32 + i % 32 < a.N) end_bits_row(reinterpret_cast<uint32_t*>(a.l[i / 32].out), rt * 32 + i % 32, a.M);
     }
     if (BITS && a.gather) {
         // whole tiles of the output, their padding of zeros included

@@ -788,6 +788,22 @@ def test_bits_output_writes_the_padding_of_its_columns(variant, M, N, K, batch):
         assert torch.equal(out.data, want.data)
 
 
+@pytest.mark.parametrize("kernel, N", [(k, 32) for k in (0, 1, 2, 3, 4, 5, 6, 7, 16, 17, 18)] + [(16, 5), (19, 2)])
+@pytest.mark.parametrize("M", [32, 33, 224, 225, 290])
+def test_every_kernel_writes_the_padding_of_its_columns(kernel, N, M):
+    """As above, by each tile of the general product and each decode kernel; from one word of columns in a K-tile to all eight."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    wp, xp = lk.pack_sign(rnd(M, 2048)), lk.pack_sign(rnd(N, 2048))
+    scale = (rnd(M), torch.ones(1, device=DEV), rnd(M))
+    want = lk.pack_sign(lk.bgemm_packed_forward(wp, xp, MODE_XOR, scale=scale))
+    out = lk.zeros_packed(N, M, 1, DEV)
+    out.data.fill_(-1)
+    lk.bgemm_packed_forward(wp, xp, MODE_XOR, variant=(kernel + 1) << 8 | VARIANT_MFMA_F4, bits_out=out, scale=scale)
+    rows = lambda p: p.data.view(-1, 2, 32, 4)[:, :, :N]
+    assert torch.equal(rows(out), rows(want)) and bool((out.data.view(-1, 2, 32, 4)[:, :, N:] == -1).all())
+
+
 def test_bits_output_chains_two_layers_and_empty_k(oracle):
     """Two binary layers with nothing but bits in between equal the op-by-op chain; K = 0 gives the bits of the bias."""
     rng = np.random.default_rng(99)
