@@ -517,10 +517,14 @@ class BGEMMChain(nn.Sequential):
     def _native_forward(self, x):
         """The fused forward by the native host side; None where it has to be Python's."""
         native = _lib.native_or_none()
-        layers = self._modules.values()
-        if native is None or torch.is_grad_enabled() or not all(type(l) in _PLAIN_LAYERS and l.fuse_inference for l in layers):
+        if native is None or torch.is_grad_enabled():
             return None
-        return native.chain_infer([l.__dict__ for l in layers], x)
+        layers = []
+        for l in self._modules.values():
+            if type(l) not in _PLAIN_LAYERS or not l.fuse_inference:
+                return None
+            layers.append(l.__dict__)
+        return native.chain_infer(layers, x)
 
     def forward(self, x):
         if type(self) is BGEMMChain:

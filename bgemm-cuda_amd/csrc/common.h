@@ -286,8 +286,10 @@ __device__ __forceinline__ unsigned next_sign_bit(const GemmArgs& a, const int64
 // of whole K-tiles, so whoever stores a row's last word stores these too, and it does not matter what the buffer held before.
 __device__ __forceinline__ void end_bits_row(uint32_t* out, const int64_t n, const int64_t M)
 {
-    const int64_t KT = k_tiles(M);
-    for (int64_t jw = (M + 31) >> 5; jw < KT * 8; jw++) out[tiled_word_offset(n, jw, KT)] = 0u;
+    const int MT = (int)((M + 31) >> 5), KT = (MT + 7) >> 3;
+    uint32_t* const last = out + ((n >> 5) * KT + KT - 1) * TILE_WORDS + (n & 31) * 4;      // of the row in its last K-tile
+#pragma unroll 1
+    for (int j = MT & 7; j != 0 && j < 8; j++) last[(j >> 2) * 128 + (j & 3)] = 0u;
 }
 // One word of the tiled output: the 32 lanes of a half-wave hold the bits of columns m32 .. m32 + 31
 // (m32 a multiple of 32) of output row n, bit = 0 where the column does not exist.  Every lane of the
@@ -301,11 +303,12 @@ __device__ __forceinline__ void store_bits_word(const GemmArgs& a, const int b, 
     if ((lane & 31) == 0 && n < a.N && m32 < a.M)
         reinterpret_cast<uint32_t*>(a.out)[(int64_t)b * a.strideC + tiled_word_offset(n, m32 >> 5, k_tiles(a.M))] = w;
 }
-// end_bits_row for rows n0 .. n0 + rows - 1, by whoever stores their last words that way, thread by thread: once behind the stores, since a test at
-// every word costs 1 % of a chain of layers (128 x 784 - 4096 - 4096 - 10 14.5 -> 14.65 us).
+// end_bits_row for rows n0 .. n0 + rows - 1, by whoever stores their last words that way, thread by thread: once behind the stores, and from
+// arguments that the kernel has in registers anyway: outside a graph, where arguments come from host memory, one more load of them or a
+// test at every word cost a chain of three layers 2 % (128 x 784 - 4096 - 4096 - 10 14.8 -> 15.1 us).
 __device__ __forceinline__ void end_bits_rows(const GemmArgs& a, const int b, const int64_t n0, const int rows, const int thread, const int threads)
 {
-    if (a.MT % 8 == 0) return;
+    if ((((int)a.M + 31) >> 5) % 8 == 0) return;
     uint32_t* const out = reinterpret_cast<uint32_t*>(a.out) + (int64_t)b * a.strideC;
     for (int i = thread; i < rows; i += threads) end_bits_row(out, n0 + i, a.M);
 }

@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256, 2) void gemm_skinny_stream_kernel(const GemmAr
                 store_out(a, out_row0 + (int64_t)n * a.M, m, val);
         }
     }
-    if (bits_kind(a.out_kind) && (int64_t)grp * RT + RT >= a.MT) end_bits_rows(a, b, 0, (int)a.N, lane, 64);
+    if (bits_kind(a.out_kind) && ((int64_t)grp * RT + RT) * 32 >= a.M) end_bits_rows(a, b, 0, (int)a.N, lane, 64);
 }
 
 // ---- split-K kernel ----------------------------------------------------------------------------
@@ -450,7 +450,7 @@ __global__ __launch_bounds__(KW * 64, FUSEX && KW <= 8 ? 4 : 2) void gemm_skinny
         outputs([&](const int n, const int m, const int val) {
             store_bits_word(a, b, n, (int64_t)rt * 32, m < M ? next_sign_bit(a, m, val) : 0u);
         });
-        if (rt == a.MT - 1) end_bits_rows(a, b, nbase, nout >> 5, threadIdx.x, NT);
+        if (rt * 32 + 32 >= M) end_bits_rows(a, b, nbase, nout >> 5, threadIdx.x, NT);
     }
 }
 
@@ -625,7 +625,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_popc_kernel(const GemmArg
         outputs([&](const int n, const int m, const int val) {
             store_bits_word(a, b, n, (int64_t)rt * 32, m < M ? next_sign_bit(a, m, val) : 0u);
         });
-        if (rt == a.MT - 1) end_bits_rows(a, b, 0, (int)a.N, threadIdx.x, NT);
+        if (rt * 32 + 32 >= M) end_bits_rows(a, b, 0, (int)a.N, threadIdx.x, NT);
     }
 }
 
@@ -787,7 +787,7 @@ __global__ __launch_bounds__(KW * 64, 2) void gemm_skinny_splitk_quad_kernel(con
         outputs([&](const int n, const int m, const int i, const int val) {
             store_bits_word(a, b, n, (int64_t)(rt0 + i) * 32, m < M ? next_sign_bit(a, m, val) : 0u);
         });
-        if (rt0 + 2 >= a.MT) end_bits_rows(a, b, (int64_t)nt0 * 32, nrows_out, threadIdx.x, KW * 64);
+        if (rt0 * 32 + 64 >= M) end_bits_rows(a, b, (int64_t)nt0 * 32, nrows_out, threadIdx.x, KW * 64);
     }
 }
 

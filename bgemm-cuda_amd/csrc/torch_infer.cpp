@@ -170,8 +170,8 @@ PyObject* chain_infer(PyObject*, PyObject* const* args, const Py_ssize_t n)
         const bool f32 = x.scalar_type() == at::kFloat;
         void* const st = stream_of(x);
         // The call's own bits, so that other streams and threads may be in the same modules: a layer reads one half and writes the other.
-        const Tensor planes = at::empty({layers > 2 ? 2 : 1, most}, x.options().dtype(at::kInt).requires_grad(false));
-        int32_t* const half[2] = {planes.data_ptr<int32_t>(), planes.data_ptr<int32_t>() + (layers > 2 ? most : 0)};
+        const c10::DataPtr planes = c10::GetAllocator(x.device().type())->allocate((layers > 2 ? 2 : 1) * most * sizeof(int32_t));
+        int32_t* const half[2] = {static_cast<int32_t*>(planes.get()), static_cast<int32_t*>(planes.get()) + (layers > 2 ? most : 0)};
         const void* in = nullptr;             // the operand of the layer at hand; null: x itself
         Tensor first;
         if (bgemm_linear_rows_supported(N, l[0].M, K0, 1, bits_kind(f32)) != 2) {
