@@ -61,6 +61,8 @@ SIGNATURES = {
     "bgemm_pack_transposed_batched": (_int, [_p, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p, _p]),
     "bgemm_packed_weight_forward_supported": (_int, [_int, _i64, _i64, _i64]),
     "bgemm_packed_weight_forward": (_int, [_int, _p, _p, _int, _i64, _p, _p, _int, _i64, _i64, _i64, _int, _p, _p, _p, _p, _p]),
+    "bgemm_unpacked_workspace_bytes": (_sz, [_int, _i64, _i64, _i64]),
+    "bgemm_unpacked_forward": (_int, [_int, _p, _p, _int, _i64, _p, _p, _int, _i64, _i64, _i64, _p, _p, _p, _p, _sz, _p]),
     "bgemm_f16_workspace_bytes": (_sz, [_i64, _i64, _i64, _int]),
     "bgemm_f16_forward": (_int, [_p, _p, _p, _i64, _i64, _i64, _p, _sz, _int, _int, _p]),
     "bgemm_f16_forward_static": (_int, [_p, _p, _p, _i64, _i64, _i64, _int, _int, _p]),
@@ -113,7 +115,9 @@ def lib():
         if version != ABI_VERSION:
             raise ImportError("%s is ABI version %d, this binding needs %d: rebuild it" % (SO_PATH, version, ABI_VERSION))
         for name, (res, args) in SIGNATURES.items():
-            fn = getattr(L, name)
+            fn = getattr(L, name, None)
+            if fn is None:
+                raise ImportError("%s has no %s: rebuild it" % (SO_PATH, name))
             fn.restype, fn.argtypes = res, args
         _lib = L
     return _lib

@@ -140,7 +140,7 @@ static int packed_forward(int mode, const void* W_tiled, const void* X_tiled, co
                           void* counters, size_t counter_bytes,
                           const void* sw, const void* sa, const void* bias, const void* zp, void* stream,
                           const RawActivations* raw = nullptr, const bool kernel_id_only = false,
-                          const RowCounts* counts = nullptr)
+                          const RowCounts* counts = nullptr, const bool codes = false)
 {
     g_err[0] = 0;
     GemmArgs a;
@@ -211,6 +211,7 @@ static int packed_forward(int mode, const void* W_tiled, const void* X_tiled, co
         a.cntW = (const int32_t*)counts->w; a.cntX = (const int32_t*)counts->x;
     }
     a.W = (const uint4*)W_tiled; a.X = (const uint4*)X_tiled; a.X2 = (const uint4*)X2_tiled;
+    a.codes = codes;
     a.MT = (int)row_tiles(M); a.NT = (int)row_tiles(N); a.KT = (int)k_tiles(K);
     a.strideW = strideW / 4; a.strideX = strideX / 4;
     a.splitK = splitK;
@@ -352,6 +353,55 @@ extern "C" int bgemm_packed_weight_forward(int mode, const void* W_tiled, const 
     const RawActivations raw = {x, x_dtype == BGEMM_SRC_F32, ldx, x_zero_point};
     return packed_forward(mode, W_tiled, nullptr, nullptr, out, out_dtype, 1, M, N, K, 0, 0, 0, 1, variant, nullptr, 0,
                           nullptr, 0, sw, sa, bias, next_zero_point, stream, &raw);
+}
+
+// ---- prepacked weights x activations as they are, any number of rows -------------------------------------------------------------
+// Workspace layout: [plane] [second plane], each rounded to 256 bytes.
+// A ternary operand goes as codes to the tile that multiplies signed operands, where there is enough of that loop to make up for the pack's
+// few instructions more (tiles x K-tiles; us a call, planes / codes, N x K x M): 11008: 2048 x 4096 x 11008 int32 52.8 / 50.0, fp16 scaled 47.3 / 46.0,
+// 2048 x 11008 x 4096 48.0 / 46.9; 12288: 1500 x 8192 x 8192 54.7 / 52.6; 8192: 2048 x 4096 x 8192 40.0 / 37.5; but 2752: 400 x 4096 x 11008
+// 19.1 / 19.3, 1376: 2048 x 512 x 11008 21.6 / 21.9; 1088: 1024 x 2048 x 4352 15.1 / 15.1.
+static bool ternary_as_codes(int mode, int out_dtype, int64_t M, int64_t N, int64_t K)
+{
+    return mode == BGEMM_MODE_BWTA && cdiv(N, 128) * cdiv(M, 256) * k_tiles(K) >= 4096 && pick_variant(mode, 1, M, N, K) == BGEMM_VARIANT_MFMA_F4 && !gemm_skinny_shape(2, 1, M, N, K) &&
+           gemm_mfma_kernel_id(1, M, N, k_tiles(K), 2, out_dtype, true) == BGEMM_KERNEL_MFMA_128x256T;
+}
+
+extern "C" size_t bgemm_unpacked_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K)
+{
+    ModeCoef mc;
+    if (!mode_coef(mode, &mc) || M <= 0 || N <= 0 || K <= 0 || K >= (1LL << 24)) return 0;
+    return mc.planes * round256((size_t)bgemm_tiled_words(N, K) * 4);
+}
+
+extern "C" int bgemm_unpacked_forward(int mode, const void* W_tiled, const void* x, int x_dtype, int64_t ldx, const void* x_zero_point,
+                                      void* out, int out_dtype, int64_t M, int64_t N, int64_t K, const void* sw, const void* sa,
+                                      const void* bias, void* ws, size_t ws_bytes, void* stream)
+{
+    const char* who = "bgemm_unpacked_forward";
+    g_err[0] = 0;
+    ModeCoef mc;
+    if (!mode_coef(mode, &mc)) return fail(BGEMM_EINVAL, "%s: unknown mode %d", who, mode);
+    if (x_dtype != BGEMM_SRC_F16 && x_dtype != BGEMM_SRC_F32) return fail(BGEMM_EINVAL, "%s: unknown activation type %d", who, x_dtype);
+    if (out_dtype != BGEMM_OUT_I32 && out_dtype != BGEMM_OUT_F16 && out_dtype != BGEMM_OUT_F32_SCALED && out_dtype != BGEMM_OUT_F16_SCALED)
+        return fail(BGEMM_EINVAL, "%s: unknown output dtype %d", who, out_dtype);
+    if (mode == BGEMM_MODE_BWTA && x_zero_point) return fail(BGEMM_EINVAL, "%s: a zero point goes with the sign modes only", who);
+    if (M < 1 || N < 1 || K < 1 || K >= (1LL << 24) || M > 0x7fffffff || N > 0x7fffffff || ldx < K)
+        return fail(BGEMM_EINVAL, "%s: bad shape M=%lld N=%lld K=%lld, row stride %lld", who, (long long)M, (long long)N, (long long)K, (long long)ldx);
+    if (!W_tiled || !x || !out || !ws) return fail(BGEMM_ENULL, "%s: null pointer", who);
+    const bool f32 = x_dtype == BGEMM_SRC_F32, scaled = out_dtype == BGEMM_OUT_F32_SCALED || out_dtype == BGEMM_OUT_F16_SCALED;
+    if (scaled && (!sw || !sa)) return fail(BGEMM_ENULL, "%s: sw or sa is NULL", who);
+    if (((uintptr_t)x & (f32 ? 3 : 1)) || ((uintptr_t)ws & 255) || ((uintptr_t)W_tiled & 15) || ((uintptr_t)out & ((1u << out_elem_shift(out_dtype)) - 1)))
+        return fail(BGEMM_EALIGN, "%s: an operand is not aligned", who);
+    const size_t need = bgemm_unpacked_workspace_bytes(mode, M, N, K);
+    if (ws_bytes < need) return fail(BGEMM_EWORKSPACE, "%s: workspace %zu < %zu bytes", who, ws_bytes, need);
+    char* const p0 = (char*)ws;
+    char* const p1 = mode == BGEMM_MODE_BWTA ? p0 + need / 2 : nullptr;
+    const bool codes = ternary_as_codes(mode, out_dtype, M, N, K);
+    const int rc = pack_activations(x, f32, p1 != nullptr, codes, x_zero_point, N, K, ldx, p0, p1, (hipStream_t)stream, who);
+    if (rc) return rc;
+    return packed_forward(mode, W_tiled, p0, p1, out, out_dtype, 1, M, N, K, 0, 0, N * M, 8, BGEMM_VARIANT_AUTO, nullptr, 0, nullptr, 0,
+                          scaled ? sw : nullptr, scaled ? sa : nullptr, scaled ? bias : nullptr, nullptr, stream, nullptr, false, nullptr, codes);
 }
 
 // ---- fp16-operand call: pack both operands into the workspace, then the packed GEMM ----

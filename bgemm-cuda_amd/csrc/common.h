@@ -88,6 +88,7 @@ struct GemmArgs {
     int force;            // BGEMM_KERNEL_* the caller insists on (BGEMM_FORCE_KERNEL), or -1: chosen by shape
     const int32_t* cntW; const int32_t* cntX;   // row popcounts of W and X ([batch][rows], a shared operand once), or null:
                                                 // the pipelined tiles then count nothing themselves
+    int codes;            // a ternary operand's planes are codes (ternary_codes)
     ModeCoef mc;
     // activations not packed yet (the decode kernel packs them itself): X/X2 are null and these describe
     // the [N][K] source; with two planes the ternary planes of sign(x) are formed
@@ -313,6 +314,15 @@ __device__ __forceinline__ void end_bits_rows(const GemmArgs& a, const int b, co
     for (int i = thread; i < rows; i += threads) end_bits_row(out, n0 + i, a.M);
 }
 
+// The two planes of a ternary operand (z: nonzero, zs: negative) as the fp4 engine likes them best (EngF4::code_x), a word at a time.  Bit
+// 4 c + s of a word is the element that nibble c holds at step s; of a code nibble's bits,
+//   first plane:   3 sign, 0 value of step 2;  2 sign, 1 value of step 0         second:   3 sign, 1 value of step 1;  2 sign, 0 value of step 3
+__device__ __forceinline__ void ternary_codes(const unsigned z, const unsigned zs, unsigned& a, unsigned& b)
+{
+    a = ((zs << 1) & 0x88888888u) | ((zs << 2) & 0x44444444u) | ((z << 1) & 0x22222222u) | ((z >> 2) & 0x11111111u);
+    b = ((zs << 2) & 0x88888888u) | ((zs >> 1) & 0x44444444u) | (z & 0x22222222u) | ((z >> 3) & 0x11111111u);
+}
+
 // Final store of one output element (column m of a row whose first element has index row0).
 template <int KIND>
 __device__ __forceinline__ void store_out_as(const GemmArgs& a, const int64_t row0, const int64_t m, const int v)
@@ -337,6 +347,10 @@ __device__ __forceinline__ void store_out(const GemmArgs& a, const int64_t row0,
 // Sign-packs two fp16 [rows][K] operands (row stride K) into tiled buffers with one launch.
 int pack_sign_pair(const void* srcA, int64_t rowsA, void* dstA, const void* srcB, int64_t rowsB, void* dstB,
                    int64_t K, hipStream_t st, const char* who);
+
+// One operand as the layers have it, rows of fp16 or fp32, into its plane or two planes, those as codes or not.
+int pack_activations(const void* src, bool f32, bool ternary, bool codes, const void* zero_point, int64_t rows, int64_t K, int64_t ld, void* d0, void* d1,
+                     hipStream_t st, const char* who);
 
 // bgemm_packed_forward with the kind OUT_F32_ELASTIC on one bit plane a side.
 int packed_forward_elastic(const void* W_tiled, const void* X_tiled, float* out, int64_t M, int64_t N, int64_t K, const float* sw, const float* sa,

@@ -74,11 +74,13 @@ __device__ __forceinline__ void edge_tile(const GemmArgs& a, const int rt, const
 // loop counts nothing: a sixth of its vector instructions on the 256 x 128 tile.
 // TERN (pipelined, fp4 engine, PL = 1): binary weights x ternary activations with signed operands (EngF4::tern_x / tern_w):
 // a slot of the activation side is made of both planes' raw words, one MFMA does what takes the AND-dot two, and the
-// accumulators hold the output itself: no popcounts, no rank-one terms.
+// accumulators hold the output itself: no popcounts, no rank-one terms.  TERN 2: the planes are codes (EngF4::code_x): 5 vector
+// instructions a MFMA instead of 6.5.  (Four, with weights of 0 and 1 and the rows' sums from the pack, are slower: the matrix cores then
+// run at a lower rate, 8192^3 218 us against 200 here.)
 // EDGES (pipelined tiles, one product, values out): the grid's tiles_n x tiles_m are whole tiles, and `edges` blocks, a multiple of eight,
 // the 32 x 32 tiles below and beside them (edge_tile).  They come first; behind a tile a compute unit at most, last: a unit's second place
 // is theirs then, and none gets two tiles while another has none (1030 x 8200 x 6200 -> fp16: 32.5 -> 22.4 us).
-template <typename Eng, int WGN, int WGM, int WN, int WM, int PL, bool PIPE, bool COUNTED = false, bool TERN = false, bool EDGES = false>
+template <typename Eng, int WGN, int WGM, int WN, int WM, int PL, bool PIPE, bool COUNTED = false, int TERN = 0, bool EDGES = false>
 // (Second launch bound: from two waves a SIMD on, a wave's register budget is the 256 architected registers, and the
 // compiler then keeps the accumulators there instead of in the accumulation registers, which the epilogue could
 // only reach through one copy per value.)
@@ -252,7 +254,8 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
         if constexpr (TERN) tern_c1 = Eng::tern_const();
         // register d of fragment f at step s, from the raw words of the K-tile it belongs to
         auto expand_reg = [&](const unsigned (&R)[NF][4], const unsigned (&R2)[XN2][4], const int f, const int c, const int s) -> unsigned {
-            if constexpr (TERN) return f < XN ? Eng::tern_x(R[f][c], R2[f < XN2 ? f : 0][c], s) : Eng::tern_w(R[f][c], s, tern_c1);
+            if constexpr (TERN == 2) return f < XN ? Eng::code_x(R[f][c], R2[f < XN2 ? f : 0][c], s) : Eng::tern_w(R[f][c], s, tern_c1, true);
+            else if constexpr (TERN == 1) return f < XN ? Eng::tern_x(R[f][c], R2[f < XN2 ? f : 0][c], s) : Eng::tern_w(R[f][c], s, tern_c1);
             else return (f < XN) == XS_FIRST ? Eng::expand1_x(R[f][c], s) : Eng::expand1_w(R[f][c], s);
         };
         auto k_tile = [&](unsigned (&A)[NF][4], unsigned (&B)[NF][4], unsigned (&A2)[XN2][4], unsigned (&B2)[XN2][4], const int kt) {
@@ -311,7 +314,7 @@ __global__ __launch_bounds__(WGN* WGM * 64, (WN * WM * PL <= 8 ? 2 : 1)) void ge
                 }
             }
         }
-        if constexpr (TERN) {          // nothing was counted and nothing is needed
+        if constexpr (TERN) {          // nothing was counted
 #pragma unroll
             for (int i = 0; i < WN; i++) pb[0][i] = 0;
 #pragma unroll
@@ -890,9 +893,9 @@ static int launch_edges(const GemmArgs& a, hipStream_t st)
     const int64_t grid = (int64_t)tiles_n * tiles_m + edges;
     if (grid > 0x7fffffffLL) return fail(BGEMM_EINVAL, "gemm_mfma: grid of %lld blocks", (long long)grid);
     if (a.cntW && a.cntX)
-        hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 4, 2, 1, true, true, false, true>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, edges);
+        hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 4, 2, 1, true, true, 0, true>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, edges);
     else
-        hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 4, 2, 1, true, false, false, true>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, edges);
+        hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 4, 2, 1, true, false, 0, true>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, edges);
     return check_launch("gemm_mfma");
 }
 
@@ -955,7 +958,8 @@ static int launch_tern(const GemmArgs& a, hipStream_t st)
         const int tiles_n = (int)cdiv(a.N, 128), tiles_m = (int)cdiv(a.M, 256);
         const int64_t grid = (int64_t)a.batch * tiles_n * tiles_m;
         if (grid <= 0 || grid > 0x7fffffffLL) return fail(BGEMM_EINVAL, "gemm_mfma: grid of %lld blocks", (long long)grid);
-        hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 2, 4, 1, true, false, true>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, 0);
+        if (a.codes) hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 2, 4, 1, true, false, 2>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, 0);
+        else hipLaunchKernelGGL((gemm_mfma_kernel<EngF4, 2, 2, 2, 4, 1, true, false, 1>), dim3((unsigned)grid), dim3(256), 0, st, a, tiles_n, tiles_m, 0);
         return check_launch("gemm_mfma");
     } else
         return fail(BGEMM_EINVAL, "gemm_mfma: the signed ternary tile runs on the fp4 engine");

@@ -115,18 +115,25 @@ struct EngF4 {
         asm volatile("" : "+v"(c));          // kept in a register: as a literal it would be a second constant operand
         return c;
     }
-    __device__ static __forceinline__ unsigned tern_w(const unsigned w, const int s, const unsigned c1)
+    __device__ static __forceinline__ unsigned tern_w(const unsigned w, const int s, const unsigned c1, const bool coded = false)
     {
         unsigned r;
         if (s == 3) {
             asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(w), "s"(0x88888888u), "v"(c1));
             return r;
         }
-        const unsigned m = w & (0x11111111u << s), c = 0x44444444u >> s;
+        const unsigned m = w & (0x11111111u << s), c = coded ? 0x11111111u << s : 0x44444444u >> s;
         if (s == 0) asm("v_lshl_or_b32 %0, %1, 3, %2" : "=v"(r) : "v"(m), "s"(c));
         else if (s == 1) asm("v_lshl_or_b32 %0, %1, 2, %2" : "=v"(r) : "v"(m), "s"(c));
         else asm("v_lshl_or_b32 %0, %1, 1, %2" : "=v"(r) : "v"(m), "s"(c));
         return r;
+    }
+    // A ternary operand as two planes of codes (ternary_codes): two of an element's nibble bits are together in one word already, so a
+    // step's operand is a mask, or a shift and a mask, where tern_x takes three to four instructions that read two planes.  Its
+    // values are tern_x's reciprocals (2, 1, 0.5, 1), the weights' tern_w's (`coded`: 0.5, 1, 2, 1).
+    __device__ static __forceinline__ unsigned code_x(const unsigned a, const unsigned b, const int s)
+    {
+        return s == 0 ? (a << 1) & 0xccccccccu : s == 1 ? b & 0xaaaaaaaau : s == 2 ? a & 0x99999999u : (b << 1) & 0xaaaaaaaau;
     }
     // a = activation-side fragment, b = weight-side fragment
     __device__ static __forceinline__ Acc mma(const Frag a, const Frag b, const Acc c)
@@ -136,6 +143,7 @@ struct EngF4 {
     __device__ static __forceinline__ int to_int(const Acc& c, const int v) { return (int)c[v]; }
     __device__ static __forceinline__ float to_float(const Acc& c, const int v) { return c[v]; }
 };
+
 
 __device__ __forceinline__ int popc4(const uint4 w)
 {

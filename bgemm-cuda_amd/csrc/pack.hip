@@ -13,7 +13,8 @@ namespace bgemm {
 // One operand to pack.  mode bit3: tiled output written by the row-segment waves (small operands:
 // many short waves); bit5 / bit6: by waves of 8 / 16 rows of a tile instead of all 32.  mode bit0: also write the (sign & nonzero) plane and make plane 0 the
 // nonzero plane; mode bit4: plane 0 = sign, plane 1 = nonzero.  mode bit1: write the logical layout instead of the tiled one.  mode bit2: the
-// source is fp32 (rounded to fp16 first, as the layers' `.to(torch.half)` does).
+// source is fp32 (rounded to fp16 first, as the layers' `.to(torch.half)` does).  mode bit7 (with bit 0): the two planes are written as
+// codes (ternary_codes); always by waves of whole tile rows.
 // zp: device scalar of the source type subtracted before that rounding, or null.
 // A job may hold nmat = outer x inner matrices of `rows` rows each (tiled output only): matrix (o, i) starts
 // so * o + si * i elements into src and fills its own mtiles row tiles of the output, one matrix after the other.
@@ -245,6 +246,17 @@ __device__ __forceinline__ void pack_tile(const PackJob& j, const int64_t gw, co
     __builtin_amdgcn_wave_barrier();       // the slots were written by this wave alone: LDS keeps its order
     if (lane < 2 * RW) {
         const int64_t at = (int64_t)tile * TILE_U4 + (lane / RW) * 32 + row0 + lane % RW;
+        if constexpr (!TRAIN) {
+            if (j.mode & 128) {
+                const uint4 z = reinterpret_cast<const uint4*>(lds)[lane], zs = reinterpret_cast<const uint4*>(lds + PLANE)[lane];
+                uint4 a, b;
+                ternary_codes(z.x, zs.x, a.x, b.x); ternary_codes(z.y, zs.y, a.y, b.y);
+                ternary_codes(z.z, zs.z, a.z, b.z); ternary_codes(z.w, zs.w, a.w, b.w);
+                reinterpret_cast<uint4*>(j.dst0)[at] = a;
+                reinterpret_cast<uint4*>(j.dst1)[at] = b;
+                return;
+            }
+        }
         reinterpret_cast<uint4*>(j.dst0)[at] = reinterpret_cast<const uint4*>(lds)[lane];
         if (ternary) reinterpret_cast<uint4*>(j.dst1)[at] = reinterpret_cast<const uint4*>(lds + PLANE)[lane];
     }
@@ -340,7 +352,7 @@ static int make_job(PackJob* j, const void* src, int64_t rows, int64_t K, int64_
     const int64_t tiles = j->nmat * j->mtiles * j->KT;
     int rows_per_wave = 8;
     if (tiles >= 2048) rows_per_wave = K <= 64 ? 32 : K <= 128 || !(mode & 4) ? 16 : 8;
-    if (!(mode & 2)) j->mode |= tiles < 160 ? 8 : rows_per_wave == 8 ? 32 : rows_per_wave == 16 ? 64 : 0;
+    if (!(mode & 2)) j->mode |= tiles < 160 && !(mode & 128) ? 8 : rows_per_wave == 8 ? 32 : rows_per_wave == 16 ? 64 : 0;
     j->waves = (j->mode & (2 | 8)) ? j->rows_out * j->nseg : tiles * (TILE_ROWS / rows_per_wave);
     return BGEMM_OK;
 }
@@ -369,6 +381,15 @@ static int pack_common(const void* src, int64_t rows, int64_t K, int64_t ld, voi
     PackJob j0, j1;
     memset(&j1, 0, sizeof j1);
     const int rc = make_job(&j0, src, rows, K, ld, d0, d1, mode, zp, who, outer, inner, so, si);
+    return rc ? rc : launch_jobs(j0, j1, st, who);
+}
+
+int pack_activations(const void* src, bool f32, bool ternary, bool codes, const void* zero_point, int64_t rows, int64_t K, int64_t ld, void* d0, void* d1,
+                     hipStream_t st, const char* who)
+{
+    PackJob j0, j1;
+    memset(&j1, 0, sizeof j1);
+    const int rc = make_job(&j0, src, rows, K, ld, d0, d1, (ternary ? 1 : 0) | (codes ? 128 : 0) | (f32 ? 4 : 0), zero_point, who);
     return rc ? rc : launch_jobs(j0, j1, st, who);
 }
 

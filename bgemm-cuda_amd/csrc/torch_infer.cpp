@@ -342,15 +342,10 @@ PyObject* packed_weight_forward(PyObject*, PyObject* const* args, const Py_ssize
             const bgemm_rows_layer layer = {w.data_ptr(), data_or_null(zp), sw.data_ptr(), sa.data_ptr(), data_or_null(bias), nullptr, out.data_ptr()};
             check(bgemm_linear_rows_forward(r.t.data_ptr(), src_type(x), r.ld, N, M, K, 1, &layer, kind, nullptr, 0, st));
         } else {
-            const Tensor planes = new_plane(x, ternary ? 2 : 1, N, K);
-            int32_t* const p = planes.data_ptr<int32_t>();
-            int32_t* const p2 = ternary ? p + planes.size(1) : nullptr;
-            check(bgemm_pack_batched(r.t.data_ptr(), src_type(x), ternary, data_or_null(zp), 1, 1, N, K, r.ld, 0, 0, p, p2, st));
-            if (scaled)
-                check(bgemm_packed_forward_scaled(mode, w.data_ptr(), p, p2, out.data_ptr(), kind, 1, M, N, K, 0, 0, N * M, 8, BGEMM_VARIANT_AUTO, nullptr, 0, nullptr, 0,
-                                                  sw.data_ptr(), sa.data_ptr(), data_or_null(bias), st));
-            else
-                check(bgemm_packed_forward(mode, w.data_ptr(), p, p2, out.data_ptr(), kind, 1, M, N, K, 0, 0, N * M, 8, BGEMM_VARIANT_AUTO, nullptr, 0, nullptr, 0, st));
+            const size_t bytes = bgemm_unpacked_workspace_bytes(mode, M, N, K);
+            const Tensor ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte).requires_grad(false));
+            check(bgemm_unpacked_forward(mode, w.data_ptr(), r.t.data_ptr(), src_type(x), r.ld, data_or_null(zp), out.data_ptr(), kind, M, N, K, data_or_null(sw),
+                                         data_or_null(sa), data_or_null(bias), ws.data_ptr(), bytes, st));
         }
     }
     return THPVariable_Wrap(out);

@@ -1,0 +1,61 @@
+"""Prepacked weights x activations as they are (bgemm_unpacked_forward) against the pack and the packed entry point, whole numbers: equal."""
+import pytest
+import torch
+
+import _lib
+import lowbit_kernel as lk
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def tern(g, n, k, dtype, special):
+    x = torch.randint(-1, 2, (n, k), generator=g, device=DEV).to(dtype)
+    if special:           # what the ternary pack calls zero, negative and nonzero
+        v = torch.tensor([0.0, -0.0, float("inf"), -float("inf"), float("nan"), 6e-8, -6e-8, 65504.0], device=DEV).to(dtype)
+        at = torch.randint(0, 8, (n, k), generator=g, device=DEV)
+        x = torch.where(torch.rand(n, k, generator=g, device=DEV) < 0.3, v[at], x)
+    return x
+
+
+def planes_product(w, x, out, scale):
+    return lk.bgemm_packed_forward(w, lk.pack_ternary(x), lk.MODE_BWTA, out, scale=scale)[0]
+
+
+# (rows, columns, K): the two-plane kernels; the signed tile on planes; the same as codes, from where those are taken on: whole tiles and
+# ragged ones, an even and an odd number of K-tiles, the last one of a bit, half and whole
+@pytest.mark.parametrize("N,M,K", [(64, 1024, 768), (1024, 4352, 512), (2048, 4096, 4096), (1000, 4321, 7937), (1025, 5000, 8000), (2048, 16000, 2047), (2049, 11008, 2177)])
+@pytest.mark.parametrize("dtype", [torch.half, torch.float32])
+def test_ternary_rows_as_codes_are_the_two_planes(N, M, K, dtype):
+    g = torch.Generator(device=DEV).manual_seed(N * 7 + M + K)
+    signed = _lib.lib().bgemm_packed_kernel_id(lk.MODE_BWTA, lk.OUT_I32, 1, M, N, K, 8, lk.VARIANT_AUTO) == 8
+    assert signed == (N > 64)
+    w = lk.pack_sign(torch.randn(M, K, generator=g, device=DEV).half())
+    sw, bias, sa = (torch.randn(M, generator=g, device=DEV).half(), torch.randn(M, generator=g, device=DEV).half(), torch.full((1,), 0.37, device=DEV).half())
+    for special in (False, True):
+        x = tern(g, N, K, dtype, special)
+        for out, scale in ((torch.int32, None), (torch.half, None), (None, (sw, sa, bias)), (None, (sw.float(), sa.float(), None))):
+            kw = {"scale": scale} if scale else {}
+            got = lk.bgemm_packed_weight_forward(w, x, lk.MODE_BWTA, **({"out_dtype": out} if out else {}), **kw)
+            want = planes_product(w, x, out or torch.int32, scale)
+            assert got.dtype == want.dtype and torch.equal(got, want), (special, out, scale is not None)
+    # every product one sign over all of K, rows at odd addresses
+    wide = torch.ones(N, K + 3, dtype=dtype, device=DEV)
+    wide[::2] = -1
+    ones = lk.pack_sign(-torch.ones(M, K, dtype=torch.half, device=DEV))
+    assert torch.equal(lk.bgemm_packed_weight_forward(ones, wide[:, 3:], lk.MODE_BWTA), -K * wide[:, :1].int().expand(N, M))
+
+
+def test_sign_rows_and_refusals():
+    g = torch.Generator(device=DEV).manual_seed(3)
+    w, x = lk.pack_sign(torch.randn(4100, 700, generator=g, device=DEV).half()), torch.randn(1030, 700, generator=g, device=DEV)
+    zp = torch.full((1,), 0.1, device=DEV)
+    for mode in (lk.MODE_AND, lk.MODE_XOR, lk.MODE_ATTN):
+        assert torch.equal(lk.bgemm_packed_weight_forward(w, x, mode, x_zero_point=zp), lk.bgemm_packed_forward(w, lk.pack_sign(x, zero_point=zp), mode)[0])
+    with pytest.raises(ValueError):
+        lk.bgemm_packed_weight_forward(w, x, lk.MODE_BWTA, x_zero_point=zp)
+    L, out, ws = _lib.lib(), torch.empty(1030, 4100, dtype=torch.int32, device=DEV), torch.empty(1 << 20, dtype=torch.uint8, device=DEV)
+    call = lambda **k: L.bgemm_unpacked_forward(*{**dict(mode=3, w=w.data.data_ptr(), x=x.data_ptr(), t=lk.SRC_F32, ld=700, zp=None, out=out.data_ptr(), kind=lk.OUT_I32,
+                                                         M=4100, N=1030, K=700, sw=None, sa=None, bias=None, ws=ws.data_ptr(), bytes=ws.numel(), stream=None), **k}.values())
+    assert call(bytes=1000) == _lib.EWORKSPACE and call(ld=699) == _lib.EINVAL and call(ws=None) == _lib.ENULL and call(kind=lk.OUT_F16_SCALED) == _lib.ENULL
+    assert call(x=x.data_ptr() + 1) == _lib.EALIGN and call(mode=9) == _lib.EINVAL and call(zp=zp.data_ptr()) == _lib.EINVAL and call(t=7) == _lib.EINVAL
