@@ -129,7 +129,7 @@ __global__ void fill_empty_bits_kernel(const GemmArgs a)
 }
 
 // Unpacked activations for the decode kernel that packs them itself (null = X_tiled / X2_tiled are used).
-struct RawActivations { const void* src; int f32; int64_t ld; const void* zero_point; };
+struct RawActivations { const void* src; int f32; int64_t ld; const void* zero_point; bool rows; };      // rows: the kernel for more than four
 // Row popcounts the caller brings for both operands (one bit plane), or null.
 struct RowCounts { const void* w; const void* x; };
 
@@ -192,7 +192,7 @@ static int packed_forward(int mode, const void* W_tiled, const void* X_tiled, co
     if (raw) {
         if (!W_tiled || !raw->src) return fail(BGEMM_ENULL, "bgemm_packed_weight_forward: operand pointer is NULL");
         if (raw->ld < K) return fail(BGEMM_EINVAL, "bgemm_packed_weight_forward: row stride %lld < K", (long long)raw->ld);
-        if (batch != 1 || !gemm_skinny_fusex_shape(a.mc.planes, M, N) || family == BGEMM_VARIANT_VALU)
+        if (batch != 1 || (!raw->rows && !gemm_skinny_fusex_shape(a.mc.planes, M, N)) || family == BGEMM_VARIANT_VALU)
             return fail(BGEMM_EINVAL, "bgemm_packed_weight_forward: shape M=%lld N=%lld not taken by the decode kernel "
                                       "(see bgemm_packed_weight_forward_supported)", (long long)M, (long long)N);
         if ((uintptr_t)raw->src & (raw->f32 ? 3 : 1))
@@ -220,6 +220,7 @@ static int packed_forward(int mode, const void* W_tiled, const void* X_tiled, co
     a.nt_store = batch * N * M * 4 <= (32LL << 20);
     const int v = family == BGEMM_VARIANT_AUTO ? pick_variant(mode, batch, M, N, K) : family;
     const bool fp4 = v == BGEMM_VARIANT_MFMA_F4;
+    if (raw && raw->rows) return launch_gemm_skinny_rows(a, (hipStream_t)stream);
     if (raw) {
         if (force >= 0 && force < BGEMM_KERNEL_SKINNY_STREAM)
             return fail(BGEMM_EINVAL, "bgemm_packed_weight_forward: kernel %d does not pack activations", force);
@@ -350,7 +351,7 @@ extern "C" int bgemm_packed_weight_forward(int mode, const void* W_tiled, const 
     if (K == 0 || M == 0 || N == 0)      // nothing to pack: the packed entry point's empty cases
         return packed_forward(mode, W_tiled, nullptr, nullptr, out, out_dtype, 1, M, N, K, 0, 0, 0, 1, variant, nullptr, 0,
                               nullptr, 0, sw, sa, bias, next_zero_point, stream);
-    const RawActivations raw = {x, x_dtype == BGEMM_SRC_F32, ldx, x_zero_point};
+    const RawActivations raw = {x, x_dtype == BGEMM_SRC_F32, ldx, x_zero_point, false};
     return packed_forward(mode, W_tiled, nullptr, nullptr, out, out_dtype, 1, M, N, K, 0, 0, 0, 1, variant, nullptr, 0,
                           nullptr, 0, sw, sa, bias, next_zero_point, stream, &raw);
 }
@@ -367,10 +368,10 @@ static bool ternary_as_codes(int mode, int out_dtype, int64_t M, int64_t N, int6
            gemm_mfma_kernel_id(1, M, N, k_tiles(K), 2, out_dtype, true) == BGEMM_KERNEL_MFMA_128x256T;
 }
 
-extern "C" size_t bgemm_unpacked_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K)
+extern "C" size_t bgemm_unpacked_workspace_bytes(int mode, const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_t K)
 {
     ModeCoef mc;
-    if (!mode_coef(mode, &mc) || M <= 0 || N <= 0 || K <= 0 || K >= (1LL << 24)) return 0;
+    if (!mode_coef(mode, &mc) || M <= 0 || N <= 0 || K <= 0 || K >= (1LL << 24) || gemm_skinny_rows_shape(mc.planes, x_dtype == BGEMM_SRC_F32, x, ldx, M, N, K)) return 0;
     return mc.planes * round256((size_t)bgemm_tiled_words(N, K) * 4);
 }
 
@@ -388,12 +389,18 @@ extern "C" int bgemm_unpacked_forward(int mode, const void* W_tiled, const void*
     if (mode == BGEMM_MODE_BWTA && x_zero_point) return fail(BGEMM_EINVAL, "%s: a zero point goes with the sign modes only", who);
     if (M < 1 || N < 1 || K < 1 || K >= (1LL << 24) || M > 0x7fffffff || N > 0x7fffffff || ldx < K)
         return fail(BGEMM_EINVAL, "%s: bad shape M=%lld N=%lld K=%lld, row stride %lld", who, (long long)M, (long long)N, (long long)K, (long long)ldx);
-    if (!W_tiled || !x || !out || !ws) return fail(BGEMM_ENULL, "%s: null pointer", who);
+    if (!W_tiled || !x || !out) return fail(BGEMM_ENULL, "%s: null pointer", who);
     const bool f32 = x_dtype == BGEMM_SRC_F32, scaled = out_dtype == BGEMM_OUT_F32_SCALED || out_dtype == BGEMM_OUT_F16_SCALED;
     if (scaled && (!sw || !sa)) return fail(BGEMM_ENULL, "%s: sw or sa is NULL", who);
     if (((uintptr_t)x & (f32 ? 3 : 1)) || ((uintptr_t)ws & 255) || ((uintptr_t)W_tiled & 15) || ((uintptr_t)out & ((1u << out_elem_shift(out_dtype)) - 1)))
         return fail(BGEMM_EALIGN, "%s: an operand is not aligned", who);
-    const size_t need = bgemm_unpacked_workspace_bytes(mode, M, N, K);
+    if (gemm_skinny_rows_shape(mc.planes, f32, x, ldx, M, N, K)) {
+        const RawActivations raw = {x, f32, ldx, x_zero_point, true};
+        return packed_forward(mode, W_tiled, nullptr, nullptr, out, out_dtype, 1, M, N, K, 0, 0, N * M, 1, BGEMM_VARIANT_AUTO, nullptr, 0, nullptr, 0,
+                              scaled ? sw : nullptr, scaled ? sa : nullptr, scaled ? bias : nullptr, nullptr, stream, &raw);
+    }
+    const size_t need = bgemm_unpacked_workspace_bytes(mode, x, x_dtype, ldx, M, N, K);
+    if (!ws) return fail(BGEMM_ENULL, "%s: null pointer", who);
     if (ws_bytes < need) return fail(BGEMM_EWORKSPACE, "%s: workspace %zu < %zu bytes", who, ws_bytes, need);
     char* const p0 = (char*)ws;
     char* const p1 = mode == BGEMM_MODE_BWTA ? p0 + need / 2 : nullptr;

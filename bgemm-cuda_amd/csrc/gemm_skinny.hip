@@ -454,6 +454,198 @@ __global__ __launch_bounds__(KW * 64, FUSEX && KW <= 8 ? 4 : 2) void gemm_skinny
     }
 }
 
+// ---- split-K kernel that packs more rows than four itself ---------------------------------------
+// 5 to 32 rows (two planes: 16) of no more than a block packs about as quickly as its weights arrive: RT weight row tiles a block, a K-tile a
+// wave, and the waves meet in LDS as above.  A lane turns eight elements of a row into a byte of signs (and one of
+// nonzeros) by gathering the elements' high bytes and a dot product with the bits' weights, 6 vector instructions (12 for the
+// nonzeros); the bytes of four rows of four lanes, transposed among those lanes, are a word a lane, which goes to its place in the
+// wave's operand tile in LDS: one write in place of four.  (Whole words a lane need no transposition, but its loads then touch four times
+// the lines: 16 x 4096 ternary rows x 11008 9.3 us for 8.2.)  Rows that do not exist are neither loaded nor cleared: a row of the
+// operand meets no other, and their outputs are not stored.
+// What bounds it: latency, launch, rows and weights, and from there on the packing, 0.4 to 0.7 us for eight rows of 4096 (ternary 1.8).  Eight
+// waves with two K-tiles each, both requested at once, take 0.3 to 1.5 us more (16 x 4096 x 11008 6.8 / 6.2, 32 x 4096 x 4096 7.4 / 6.4); waves that
+// walk over further ones of a longer K are as slow as two launches.
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// Sign bits of eight fp16 (element e at bit 14 - e), whose high bytes hold them.
+__device__ __forceinline__ unsigned signs8(const v4i v)
+{
+    const unsigned p0 = __builtin_amdgcn_perm(v.y, v.x, 0x07050301u) & 0x80808080u, p1 = __builtin_amdgcn_perm(v.w, v.z, 0x07050301u) & 0x80808080u;
+    return __builtin_amdgcn_udot4(p0, 0x10204080u, __builtin_amdgcn_udot4(p1, 0x01020408u, 0u, false), false);
+}
+// Which of eight fp16 are not zero (element e at bit 7 - e).
+__device__ __forceinline__ unsigned nonzeros8(const v4i v)
+{
+    auto ones = [](const int d) { return __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_bit_cast(u16x2, d & 0x7fff7fff), u16x2{1, 1})); };
+    const unsigned p0 = __builtin_amdgcn_perm(ones(v.y), ones(v.x), 0x06040200u), p1 = __builtin_amdgcn_perm(ones(v.w), ones(v.z), 0x06040200u);
+    return __builtin_amdgcn_udot4(p0, 0x10204080u, __builtin_amdgcn_udot4(p1, 0x01020408u, 0u, false), false);
+}
+
+constexpr int ROWS_KT = 16;            // K-tiles: waves of a block
+
+template <int RT, bool F32, bool TWO>
+__global__ __launch_bounds__(ROWS_KT * 64) void gemm_skinny_rows_kernel(const GemmArgs a)
+{
+    static_assert(!(F32 && TWO), "ternary rows are taken as fp16");
+    constexpr int ESZ = F32 ? 4 : 2, LOADS = F32 ? 2 : 1, GROUPS = TWO ? 2 : 4, NT = ROWS_KT * 64;
+    __shared__ int sAcc[RT][16][64];
+    __shared__ int sPa[RT][32], sPb[32];
+    __shared__ __align__(16) uint32_t sX[ROWS_KT][TILE_WORDS];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rt0 = blockIdx.x * RT, N = (int)a.N, KT = a.KT, kt = wave;
+    // a lane loads eight elements, chunk c of a K-tile, of rows 8 g + 2 i + h, i = 0 .. 3, and ends up with word c >> 2 of row 8 g + 2 (c & 3) + h
+    const int c = lane & 31, h = lane >> 5, j = c >> 2;
+    const __amdgpu_buffer_rsrc_t rsX = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.xsrc), 0, (int)((N - 1) * a.xld + a.K) * ESZ, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsW = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(a.W + (int64_t)rt0 * KT * TILE_U4), 0,
+                                                                         min(RT, a.MT - rt0) * KT * (TILE_U4 * 16), 0x00020000);
+    constexpr int PAST = 0x7ffffff0;
+    const int groups = min(GROUPS, (N + 7) >> 3), row_b = (int)a.xld * ESZ;
+    // (K is a multiple of eight: a load lies before its end or behind it, and comes back as zeros)
+    v4i x[8][LOADS], w[RT];
+    auto request_x = [&](const int g0) {
+        const int k = kt * TILE_KBITS + 8 * c;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int n = 8 * g0 + 2 * i + h, at = n < N && k < (int)a.K ? n * row_b + k * ESZ : PAST;
+#pragma unroll
+            for (int q = 0; q < LOADS; q++) x[i][q] = __builtin_amdgcn_raw_buffer_load_b128(rsX, at, 16 * q, 0);
+        }
+    };
+    if (kt < KT) {
+        request_x(0);
+#pragma unroll
+        for (int t = 0; t < RT; t++) w[t] = __builtin_amdgcn_raw_buffer_load_b128(rsW, lane * 16 + (t * KT + kt) * (TILE_U4 * 16), 0, 2);
+    }
+    float zf = 0.f;
+    if (a.xzp) zf = F32 ? *reinterpret_cast<const float*>(a.xzp) : __half2float(*reinterpret_cast<const __half*>(a.xzp));
+    const f16x2 z = {(_Float16)zf, (_Float16)zf};
+    const bool centred = a.xzp != nullptr;
+
+    EngF4::Acc acc[RT];
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
+    uint32_t* const tile = sX[wave] + ((j >> 2) * 32 + 2 * (c & 3) + h) * 4 + (j & 3);
+    // byte i of lane p of four neighbours <-> byte 3 - p of lane i
+    const unsigned sel1 = c & 1 ? 0x03070105u : 0x06020400u, sel2 = c & 2 ? 0x06070203u : 0x00010405u;
+    auto transpose4 = [&](unsigned w) {
+        w = __builtin_amdgcn_perm((unsigned)__builtin_amdgcn_mov_dpp((int)w, 0xb1, 0xf, 0xf, true), w, sel1);
+        return __builtin_amdgcn_perm((unsigned)__builtin_amdgcn_mov_dpp((int)w, 0x4e, 0xf, 0xf, true), w, sel2);
+    };
+    auto put = [&](const int g0) {
+        // (what lies past K is zero, but not less a zero point)
+        const int left = (int)a.K - (kt * TILE_KBITS + 32 * j);
+        const unsigned keep = left >= 32 ? 0xffffffffu : left > 0 ? 0xffffffffu << (32 - left) : 0u;
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            if (g0 + g >= groups) break;
+            unsigned sg = 0, nz = 0;
+            // (fp32: byte by byte from the last row's: each goes in at the bottom)
+            if constexpr (F32) {
+#pragma unroll
+                for (int i = 31; i >= 0; i--) {
+                    const float f = __uint_as_float((unsigned)x[4 * g + (i >> 3)][(7 - i & 7) >> 2][(7 - i & 7) & 3]);
+                    sg = __builtin_amdgcn_alignbit(sg, __float_as_uint(centred ? __fsub_rn(f, zf) : f), 31);
+                }
+            } else
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                v4i v = x[4 * g + i][0];
+                if (!TWO && centred) {
+                    // (in fp16: a difference of two numbers has the sign of its rounding)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int two = v[e];
+                        v[e] = __builtin_bit_cast(int, __builtin_bit_cast(f16x2, two) - z);
+                    }
+                }
+                const unsigned s = signs8(v);
+                sg |= i == 0 ? s >> 7 : s << (8 * i - 7);
+                if (TWO) nz |= nonzeros8(v) << (8 * i);
+            }
+            const int at = (g0 + g) * 32;
+            sg = transpose4(sg);
+            if (TWO) {
+                nz = transpose4(nz);
+                tile[at] = nz;
+                tile[at + 64] = sg & nz;
+            } else
+                tile[at] = centred ? sg & keep : sg;
+        }
+    };
+    // (cleared while the loads are in flight)
+    for (int i = threadIdx.x; i < RT * 16 * 64; i += NT) (&sAcc[0][0][0])[i] = 0;
+    if (threadIdx.x < 32) {
+        sPb[threadIdx.x] = 0;
+#pragma unroll
+        for (int t = 0; t < RT; t++) sPa[t][threadIdx.x] = 0;
+    }
+    __syncthreads();
+    if (kt < KT) {
+        put(0);
+        if (!TWO && groups > 2) {
+            request_x(2);
+            put(2);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");      // the wave's own tile: LDS keeps its order
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const uint4 bits = reinterpret_cast<const uint4*>(sX[wave])[lane];
+        int pa[RT], pb = popc4(bits);
+        uint4 wt[RT];
+#pragma unroll
+        for (int t = 0; t < RT; t++) {
+            wt[t] = make_uint4(w[t].x, w[t].y, w[t].z, w[t].w);
+            pa[t] = popc4(wt[t]);
+        }
+#pragma unroll
+        for (int s = 0; s < EngF4::STEPS; s++) {
+            const EngF4::Frag f = EngF4::expand_x(bits, s);
+#pragma unroll
+            for (int t = 0; t < RT; t++) acc[t] = EngF4::mma(f, EngF4::expand_w(wt[t], s), acc[t]);
+        }
+
+        // ---- meet in LDS ----
+        pb += __shfl_xor(pb, 32);
+#pragma unroll
+        for (int t = 0; t < RT; t++) pa[t] += __shfl_xor(pa[t], 32);
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            if (8 * (TWO ? (g & 1) : g) >= N) continue;
+#pragma unroll
+            for (int v = 4 * g; v < 4 * g + 4; v++)
+#pragma unroll
+                for (int t = 0; t < RT; t++) atomicAdd(&sAcc[t][v][lane], EngF4::to_int(acc[t], v));
+        }
+        if (lane < 32) {
+            atomicAdd(&sPb[lane], pb);
+#pragma unroll
+            for (int t = 0; t < RT; t++) atomicAdd(&sPa[t][lane], pa[t]);
+        }
+    }
+    __syncthreads();
+    const ModeCoef mc = a.mc;
+    const int M = (int)a.M, kbits = (int)a.K;
+    auto elements = [&](auto kind) {
+        for (int o = threadIdx.x; o < N * RT * 32; o += NT) {
+            const int nl = o / (RT * 32), cc = o % (RT * 32), t = cc >> 5, c = cc & 31;
+            const int v = 4 * (nl >> 3) + (nl & 3), hh = (nl >> 2) & 1, m = rt0 * 32 + cc;
+            const int d = sAcc[t][v][hh * 32 + c], d2 = TWO ? sAcc[t][v + 8][hh * 32 + c] : 0;
+            if (m < M) store_out_as<decltype(kind)::value>(a, (int64_t)nl * M, m, skinny_value(mc, TWO, kbits, sPa[t][c], sPb[nl], TWO ? sPb[nl + 16] : 0, d, d2));
+        }
+    };
+    switch (a.out_kind) {
+    case BGEMM_OUT_I32: elements(std::integral_constant<int, BGEMM_OUT_I32>{}); break;
+    case BGEMM_OUT_F16: elements(std::integral_constant<int, BGEMM_OUT_F16>{}); break;
+    case BGEMM_OUT_F32_SCALED: elements(std::integral_constant<int, BGEMM_OUT_F32_SCALED>{}); break;
+    default: elements(std::integral_constant<int, BGEMM_OUT_F16_SCALED>{}); break;
+    }
+}
+
 // ---- split-K kernel on the vector ALU: one or two activation vectors ------------------------------
 // With one or two rows the matrix cores have nothing to amortise the bit expansion over (13 vector-ALU
 // instructions per MFMA, of whose 32 output rows a few are used).  Here a lane keeps the weight words of
@@ -954,6 +1146,29 @@ bool gemm_skinny_fusex_shape(int planes, int64_t M, int64_t N)
 {
     (void)planes;
     return N >= 1 && N <= 4 && row_tiles(M) < 4096;
+}
+
+// Whether a product of 5 to 32 unpacked rows goes to the kernel that packs them itself: rows of whole aligned 16-byte pieces, a K-tile a
+// wave and one round of blocks.  GPU time from a graph, us, two launches / one, N x K x M: fp16 signs 5 x 4096 x 11008 7.2 / 5.1, 32 x 4096 x 11008
+// 8.1 / 7.8, 32 x 4096 x 4096 6.7 / 6.4, 16 x 2048 x 2048 5.9 / 4.1, 32 x 768 x 11008 8.5 / 6.0; ternary 8 x 4096 x 11008 6.8 / 5.8, 16 x 2048 x 16384 6.5 / 5.8, 16 x
+// 3000 x 3000 6.4 / 5.7, 16 x 4096 x 11008 7.3 / 7.7; fp32 8 x 4096 x 11008 7.2 / 6.7, 16 x 4096 x 11008 7.4 / 7.7, 32 x 1024 x 8192 7.0 / 6.0, 32 x 2048 x 2048
+// 6.2 / 6.6 but 24 x 4096 x 4096 6.6 / 7.6.  A call without a graph is the host's time, a launch and an allocation less: 10.2 / 6.4 us a layer, also
+// where the GPU takes some percent longer.  Two rounds of blocks are behind (16 x 2048 x 22016 7.6 / 9.6).
+bool gemm_skinny_rows_shape(int planes, int x_f32, const void* x, int64_t ldx, int64_t M, int64_t N, int64_t K)
+{
+    return N >= 5 && N <= (planes == 2 ? 16 : 32) && !(planes == 2 && x_f32) && (!x_f32 || N * K <= 65536) && k_tiles(K) <= ROWS_KT && M <= 16384 && K % 8 == 0 &&
+           (uintptr_t)x % 16 == 0 && ldx * (x_f32 ? 4 : 2) % 16 == 0 && ldx <= (1 << 20);
+}
+
+// Two row tiles a block, which share the packing, where one would be more than a block a compute unit.
+int launch_gemm_skinny_rows(const GemmArgs& a, hipStream_t st)
+{
+    const int rt = a.MT > 256 ? 2 : 1;
+    auto go = [&](auto one, auto two) { hipLaunchKernelGGL(rt == 1 ? one : two, dim3((unsigned)cdiv(a.MT, rt)), dim3(ROWS_KT * 64), 0, st, a); };
+    if (a.mc.planes == 2) go(gemm_skinny_rows_kernel<1, false, true>, gemm_skinny_rows_kernel<2, false, true>);
+    else if (a.xsrc_f32) go(gemm_skinny_rows_kernel<1, true, false>, gemm_skinny_rows_kernel<2, true, false>);
+    else go(gemm_skinny_rows_kernel<1, false, false>, gemm_skinny_rows_kernel<2, false, false>);
+    return check_launch("gemm_skinny");
 }
 
 // Which of the kernels above a shape gets (BGEMM_KERNEL_* ids).

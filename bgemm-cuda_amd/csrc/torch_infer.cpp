@@ -109,6 +109,17 @@ struct Layer {
 // Whether a call without a gradient may go past torch's operations at all.
 bool quiet_call(PyObject* x) { return !c10::GradMode::is_enabled() && plain_gpu(x) && !is_watched(); }
 
+// Packed weights x rows as they are, with the scratch that the size needs.
+void unpacked(const int mode, const Tensor& w, const Rows& x, const Tensor& zp, const Tensor& out, const int kind, const int64_t M, const int64_t N, const int64_t K,
+              const Tensor& sw, const Tensor& sa, const Tensor& bias)
+{
+    const size_t bytes = bgemm_unpacked_workspace_bytes(mode, x.t.data_ptr(), src_type(x.t), x.ld, M, N, K);
+    Tensor ws;
+    if (bytes) ws = at::empty({(int64_t)bytes}, x.t.options().dtype(at::kByte).requires_grad(false));
+    check(bgemm_unpacked_forward(mode, w.data_ptr(), x.t.data_ptr(), src_type(x.t), x.ld, data_or_null(zp), out.data_ptr(), kind, M, N, K, data_or_null(sw),
+                                 data_or_null(sa), data_or_null(bias), data_or_null(ws), bytes, stream_of(out)));
+}
+
 // linear_infer(module.__dict__, x) -> y
 PyObject* linear_infer(PyObject*, PyObject* const* args, const Py_ssize_t n)
 {
@@ -135,10 +146,7 @@ PyObject* linear_infer(PyObject*, PyObject* const* args, const Py_ssize_t n)
             const bgemm_rows_layer layer = l.rows_layer(out.data_ptr());
             check(bgemm_linear_rows_forward(r.t.data_ptr(), src_type(x), r.ld, N, l.M, l.K, 1, &layer, kind, nullptr, 0, st));
         } else {
-            const Tensor bits = new_plane(x, 1, N, l.K);
-            check(bgemm_pack_batched(r.t.data_ptr(), src_type(x), 0, l.zpa.data_ptr(), 1, 1, N, l.K, r.ld, 0, 0, bits.data_ptr(), nullptr, st));
-            check(bgemm_packed_forward_scaled(BGEMM_MODE_XOR, l.packed.data_ptr(), bits.data_ptr(), nullptr, out.data_ptr(), kind, 1, l.M, N, l.K, 0, 0, N * l.M, 8,
-                                              BGEMM_VARIANT_AUTO, nullptr, 0, nullptr, 0, l.sw.data_ptr(), l.sa.data_ptr(), data_or_null(l.bias), st));
+            unpacked(BGEMM_MODE_XOR, l.packed, r, l.zpa, out, kind, l.M, N, l.K, l.sw, l.sa, l.bias);
         }
     }
     return THPVariable_Wrap(out);
@@ -342,10 +350,7 @@ PyObject* packed_weight_forward(PyObject*, PyObject* const* args, const Py_ssize
             const bgemm_rows_layer layer = {w.data_ptr(), data_or_null(zp), sw.data_ptr(), sa.data_ptr(), data_or_null(bias), nullptr, out.data_ptr()};
             check(bgemm_linear_rows_forward(r.t.data_ptr(), src_type(x), r.ld, N, M, K, 1, &layer, kind, nullptr, 0, st));
         } else {
-            const size_t bytes = bgemm_unpacked_workspace_bytes(mode, M, N, K);
-            const Tensor ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte).requires_grad(false));
-            check(bgemm_unpacked_forward(mode, w.data_ptr(), r.t.data_ptr(), src_type(x), r.ld, data_or_null(zp), out.data_ptr(), kind, M, N, K, data_or_null(sw),
-                                         data_or_null(sa), data_or_null(bias), ws.data_ptr(), bytes, st));
+            unpacked(mode, w, r, zp, out, kind, M, N, K, sw, sa, bias);
         }
     }
     return THPVariable_Wrap(out);

@@ -760,7 +760,8 @@ def bgemm_packed_weight_forward(w, x, mode=MODE_XOR, out_dtype=torch.int32, scal
                                 variant=VARIANT_AUTO):
     """Prepacked weights ``w`` (M rows) x activations ``x`` as they are, fp16 or fp32 ``[N,K]`` -> ``[N,M]``.
 
-    For the few rows of a decode step (N <= 4) this is ONE launch: the kernel forms the
+    For the few rows of a decode step (N <= 4; up to 32, ternary 16, where K is at most 4096 and rows are aligned) this is ONE
+    launch: the kernel forms the
     activation bits itself (``MODE_BWTA``: the ternary planes of sign(x); the other modes: sign bits of ``x``
     or, with ``x_zero_point``, of ``(x - x_zero_point).to(torch.half)``).  Larger batches go through the pack
     kernel and the packed entry point: same results either way.  ``scale`` as in bgemm_packed_forward."""

@@ -253,8 +253,8 @@ int bgemm_packed_weight_forward(int mode, const void* W_tiled, const void* x, in
 /* Prepacked weights x activations as they are, any number of rows: the pack of the activations (bgemm_pack_sign_centered /
  * bgemm_pack_ternary_f16) and the packed entry point in one call, in whatever form between them suits the size.  out_dtype: BGEMM_OUT_I32,
  * F16 or the scaled kinds (sw, sa; bias optional, as bgemm_packed_forward_scaled).  ws: 256-byte aligned scratch of
- * bgemm_unpacked_workspace_bytes, which need not be initialised. */
-size_t bgemm_unpacked_workspace_bytes(int mode, int64_t M, int64_t N, int64_t K);
+ * bgemm_unpacked_workspace_bytes, which need not be initialised (0: a few rows, which one launch packs and multiplies; ws may be NULL). */
+size_t bgemm_unpacked_workspace_bytes(int mode, const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_t K);
 int bgemm_unpacked_forward(int mode, const void* W_tiled, const void* x, int x_dtype, int64_t ldx, const void* x_zero_point,
                            void* out, int out_dtype, int64_t M, int64_t N, int64_t K, const void* sw, const void* sa,
                            const void* bias, void* ws, size_t ws_bytes, void* stream);

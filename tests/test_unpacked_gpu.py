@@ -59,3 +59,26 @@ def test_sign_rows_and_refusals():
                                                          M=4100, N=1030, K=700, sw=None, sa=None, bias=None, ws=ws.data_ptr(), bytes=ws.numel(), stream=None), **k}.values())
     assert call(bytes=1000) == _lib.EWORKSPACE and call(ld=699) == _lib.EINVAL and call(ws=None) == _lib.ENULL and call(kind=lk.OUT_F16_SCALED) == _lib.ENULL
     assert call(x=x.data_ptr() + 1) == _lib.EALIGN and call(mode=9) == _lib.EINVAL and call(zp=zp.data_ptr()) == _lib.EINVAL and call(t=7) == _lib.EINVAL
+
+
+# rows that one launch packs and multiplies: both ends of N, one and two row tiles a block with and without a rest, K of one chunk, a word and
+# a half, one K-tile to sixteen, rows of a wider matrix; and, beside them, rows that launch does not take
+@pytest.mark.parametrize("N,M,K,ld", [(5, 64, 256, 256), (8, 33, 264, 272), (16, 100, 2048, 2048), (7, 1000, 1000, 1008), (16, 11008, 2048, 2048), (5, 11008, 4096, 4096), (16, 16384, 4096, 4096),
+                                      (32, 500, 2048, 2056), (25, 8225, 512, 520), (17, 77, 8, 8), (31, 16384, 2000, 2000), (9, 300, 8, 16), (10, 4096, 4104, 4104), (32, 2050, 4096, 4096), (16, 700, 4080, 4088),
+                                      (16, 200, 2052, 2056), (8, 100, 256, 257), (33, 64, 512, 512), (4, 64, 512, 512)])
+@pytest.mark.parametrize("dtype", [torch.half, torch.float32])
+def test_few_rows_in_one_launch(N, M, K, ld, dtype):
+    g = torch.Generator(device=DEV).manual_seed(N + M + K)
+    w = lk.pack_sign(torch.randn(M, K, generator=g, device=DEV).half())
+    sw, sa = torch.randn(M, generator=g, device=DEV).to(dtype), torch.full((1,), 0.3, device=DEV).to(dtype)
+    special = torch.tensor([0.0, -0.0, float("inf"), -float("inf"), float("nan"), -float("nan"), 6e-8, -6e-8, 0.05], device=DEV).to(dtype)
+    for mode in (lk.MODE_AND, lk.MODE_XOR, lk.MODE_ATTN, lk.MODE_BWTA):
+        ternary = mode == lk.MODE_BWTA
+        x = (torch.randint(-1, 2, (N, ld), generator=g, device=DEV) if ternary else torch.randn(N, ld, generator=g, device=DEV)).to(dtype)
+        x = torch.where(torch.rand(N, ld, generator=g, device=DEV) < 0.3, special[torch.randint(0, 9, (N, ld), generator=g, device=DEV)], x)[:, :K]
+        for zp in (None,) if ternary else (None, special[8:], special[2:3]):
+            xp = lk.pack_ternary(x) if ternary else lk.pack_sign(x, zero_point=zp)
+            for out, scale in ((torch.int32, None), (torch.half, None), (None, (sw, sa, sw)), (None, (sw, sa, None))):
+                got = lk.bgemm_packed_weight_forward(w, x, mode, x_zero_point=zp, scale=scale, **({"out_dtype": out} if out else {}))
+                want = lk.bgemm_packed_forward(w, xp, mode, out or torch.int32, scale=scale)[0]
+                assert got.dtype == want.dtype and torch.equal(got, want), (mode, None if zp is None else zp.item(), out, scale is not None)
