@@ -80,6 +80,7 @@ def _batched_packed(x_rows, right, mode):
 # twice, which is ahead while the caches hold one (16 x 3072^2, D = 64: 153 -> 146) and not when each reading comes from memory
 # (16 x 4096^2: 217 -> 260).
 SCORES_GRAD_ROWS, CONTEXT_GRAD_ROWS = 2048, 4096
+SCORES_GRAD_PRODUCT = 6 << 30          # multiplications above D = 64: see _scores_grad_ahead
 
 
 def _scores_grad_ahead(batch, N, M, D):
@@ -88,7 +89,7 @@ def _scores_grad_ahead(batch, N, M, D):
     8 * 2^30 multiplications a product (D = 96: 64 x 1024^2 = 6 * 2^30 104 -> 88 us, 64 x 1536^2 183 -> 194, 64 x 2048^2 288 -> 324;
     D = 128: 16 x 1536^2 = 4.5 * 2^30 103 -> 72, 64 x 1024^2 = 8 * 2^30 102 -> 115, 16 x 2048^2 101 -> 115, 64 x 2048^2 306 -> 416); up to
     64 the kernel is ahead at every such size (D = 64: 64 x 1024^2 104 -> 75, 64 x 1536^2 158 -> 145, 64 x 2048^2 265 -> 253)."""
-    return max(N, M) <= SCORES_GRAD_ROWS and (D <= 64 or batch * N * M * D < 6 << 30)
+    return max(N, M) <= SCORES_GRAD_ROWS and (D <= 64 or batch * N * M * D < SCORES_GRAD_PRODUCT)
 
 
 def _any_tangent(*tensors):
@@ -107,9 +108,48 @@ def _one_launch_grads(matrix, a, b, longest):
             and not lowbit_kernel.watched() and not _any_tangent(matrix, a, b))
 
 
+def _scores_grads(need, x, right, grad_out):
+    """Gradients of ``sign(x) @ sign(right)`` on batches of fp16 matrices."""
+    g = grad_out.to(x.dtype)
+    rows = right.transpose(-1, -2)
+    N, M = g.shape[-2:]
+    if _one_launch_grads(g, x, rows, SCORES_GRAD_ROWS) and _scores_grad_ahead(g.numel() // (N * M), N, M, x.shape[-1]):
+        grad_x, grad_rows = lowbit_kernel.scores_backward(g, x, rows, need)
+        return grad_x, None if grad_rows is None else grad_rows.transpose(-1, -2)
+    return g @ right.sign().transpose(-1, -2), x.sign().transpose(-1, -2) @ g
+
+
+def _context_grads(need, attn, value, grad_out):
+    """Gradients of the attention matmul (bgemm_linear.py:64-86)."""
+    g = grad_out.to(value.dtype)
+    if attn.dim() > 2 and _one_launch_grads(attn, g, value, CONTEXT_GRAD_ROWS):
+        return lowbit_kernel.context_backward(attn, g, value, need)
+    a01 = (attn.sign() + 1) / 2
+    a01 = torch.where(a01 == 0, torch.ones_like(a01), a01)     # as the reference does (:70-71)
+    v = value.sign()
+    return (g @ v.transpose(-1, -2)) / 2, a01.transpose(-1, -2) @ g
+
+
+_SCORES_BACKWARD, _CONTEXT_BACKWARD = lowbit_kernel.scores_backward, lowbit_kernel.context_backward
+
+
 class bgemm_matmul(torch.autograd.Function):
     """matA [.., N, K] @ matB [K, M] with both operands binarised by sign (bgemm_linear.py:9-42).
     A matB with leading dimensions ([B, H, K, M], as K^T in attention) is a batched matmul."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        # Recorded products of fp16 batches are one native node; everything else is this Function, also where a program has put
+        # something else in the place of the gradients' launch, which the Function calls by its name.
+        if (cls is bgemm_matmul and not kwargs and 2 <= len(args) <= 3 and torch.is_grad_enabled()
+                and lowbit_kernel.scores_backward is _SCORES_BACKWARD):
+            native = _lib.native_or_none()
+            if native is not None:
+                mode = lowbit_kernel.MODE_AND if len(args) == 3 and args[2] == 'and' else lowbit_kernel.MODE_XOR
+                out = native.product_train(args[0], args[1], mode, SCORES_GRAD_ROWS, SCORES_GRAD_PRODUCT)
+                if out is not None:
+                    return out
+        return super().apply(*args, **kwargs)
 
     @staticmethod
     def forward(ctx, matA, matB, instruction='xor'):
@@ -129,13 +169,7 @@ class bgemm_matmul(torch.autograd.Function):
     def backward(ctx, grad_output):
         matA, matB = ctx.saved_tensors
         if matB.dim() > 2:
-            g = grad_output.to(matA.dtype)
-            right = matB.transpose(-1, -2)
-            N, M = g.shape[-2:]
-            if _one_launch_grads(g, matA, right, SCORES_GRAD_ROWS) and _scores_grad_ahead(g.numel() // (N * M), N, M, matA.shape[-1]):
-                grad_a, grad_bt = lowbit_kernel.scores_backward(g, matA, right, ctx.needs_input_grad[:2])
-                return grad_a, None if grad_bt is None else grad_bt.transpose(-1, -2), None
-            return g @ matB.sign().transpose(-1, -2), matA.sign().transpose(-1, -2) @ g, None
+            return (*_scores_grads(ctx.needs_input_grad[:2], matA, matB, grad_output), None)
         grad_a, grad_bt = _linear_grads(grad_output, matA.sign(), matB.sign().transpose(-1, -2))
         return grad_a, grad_bt.transpose(-1, -2), None
 
@@ -143,6 +177,17 @@ class bgemm_matmul(torch.autograd.Function):
 class bgemm_attn_matmul(torch.autograd.Function):
     """attn [S_q, S_k] ({0,1}: 1 where the sign bit is clear) @ value [S_k, d] ({-1,1})
     (bgemm_linear.py:45-86).  The kernel sees attn as the weight-side operand with INSTR=2."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        if (cls is bgemm_attn_matmul and not kwargs and 2 <= len(args) <= 3 and torch.is_grad_enabled()
+                and lowbit_kernel.context_backward is _CONTEXT_BACKWARD):
+            native = _lib.native_or_none()
+            if native is not None:
+                out = native.product_train(args[0], args[1], lowbit_kernel.MODE_ATTN_X, CONTEXT_GRAD_ROWS, 1 << 62)
+                if out is not None:
+                    return out
+        return super().apply(*args, **kwargs)
 
     @staticmethod
     def forward(ctx, input1, input2, instruction="attn_mm"):
@@ -159,16 +204,7 @@ class bgemm_attn_matmul(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        attn, value = ctx.saved_tensors
-        if attn.dim() > 2:
-            g = grad_output.to(value.dtype)
-            if _one_launch_grads(attn, g, value, CONTEXT_GRAD_ROWS):
-                return (*lowbit_kernel.context_backward(attn, g, value, ctx.needs_input_grad[:2]), None)
-        a01 = (attn.sign() + 1) / 2
-        a01 = torch.where(a01 == 0, torch.ones_like(a01), a01)     # as the reference does (:70-71)
-        v = value.sign()
-        g = grad_output.to(v.dtype)
-        return (g @ v.transpose(-1, -2)) / 2, a01.transpose(-1, -2) @ g, None
+        return (*_context_grads(ctx.needs_input_grad[:2], *ctx.saved_tensors, grad_output), None)
 
 
 class bgemm_linear(torch.autograd.Function):

@@ -76,6 +76,13 @@ inline Rows rows_2d(const Tensor& t)
     return {r, r.stride(0)};
 }
 
+// x [.., N, K] @ right [.., K, M] of binarised operands, one launch over the batch -> fp16 [.., N, M]; undefined: a form it does not take.
+Tensor batched_product_of(const Tensor& x, const Tensor& right, int mode);
+// The gradients of such a product by their one-launch kernel (bgemm_linear._one_launch_grads, and `most` multiplications a product above 64
+// columns); false: a form it does not take.
+bool attention_grads(bool context, const Tensor& m, const Tensor& a, const Tensor& b, bool need0, bool need1, int64_t longest, int64_t most, Tensor& g0,
+                     Tensor& g1);
+
 // Functions of the inference and attention part, for the module's table.
 extern PyMethodDef infer_methods[];
 extern const int infer_method_count;

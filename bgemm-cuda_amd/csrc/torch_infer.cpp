@@ -436,57 +436,68 @@ bool context_in_one(const int64_t batch, const int64_t N, const int64_t M, const
     return (D == 32 || D == 64 || D == 96 || D == 128) && N <= 1 << 20 && M >= 8 && (M * D <= 1 << 15 || (M * D <= 1 << 16 && D <= 64 && batch > 1 && batch * N * M < 1 << 27));
 }
 
-// batched_product(x [.., N, K], right [.., K, M], mode) -> fp16 [.., N, M]: one launch on fp16 operands of an attention product's form,
-// else both operands packed where they lie and one GEMM over the batch
+}  // namespace
+
+// One launch on fp16 operands of an attention product's form, else both operands packed where they lie and one GEMM over the batch.
+Tensor batched_product_of(const Tensor& x, const Tensor& right, const int mode)
+{
+    const int64_t d = x.dim();
+    if ((d != 3 && d != 4) || right.dim() != d || !is_param_type(x.scalar_type()) || !is_param_type(right.scalar_type()) || right.device() != x.device() || x.numel() == 0 ||
+        right.numel() == 0 || x.size(-1) != right.size(-2) || x.size(0) != right.size(0) || (d == 4 && x.size(1) != right.size(1)))
+        return Tensor();
+    const int64_t N = x.size(-2), K = x.size(-1), M = right.size(-1);
+    // rows read where they lie; the right operand row by row of its transpose if that is dense, else column by column
+    const bool by_rows = right.stride(-2) == 1 && right.stride(-1) >= K, by_columns = right.stride(-1) == 1 && right.stride(-2) >= M;
+    if (x.stride(-1) != 1 || x.stride(-2) < K || !(by_rows || by_columns)) return Tensor();
+    const Batch bx = batch_of(x), br = batch_of(right);
+    if (bx.so < 0 || bx.si < 0 || br.so < 0 || br.si < 0) return Tensor();
+    const int64_t batch = bx.outer * bx.inner;
+    Tensor out;
+    const c10::OptionalDeviceGuard guard(x.device());
+    const auto options = x.options().requires_grad(false);
+    std::vector<int64_t> shape = x.sizes().vec();
+    shape.back() = M;
+    out = at::empty(shape, options.dtype(at::kHalf));
+    void* const st = stream_of(x);
+    const bool half = x.scalar_type() == at::kHalf && right.scalar_type() == at::kHalf;
+    const bool scores = half && (mode == BGEMM_MODE_XOR || mode == BGEMM_MODE_AND) && by_rows && scores_in_one(batch, N, M, K);
+    const bool context = half && mode == BGEMM_MODE_ATTN_X && by_columns && context_in_one(batch, N, K, M);
+    if (scores || context) {
+        const int64_t strides[6] = {bx.so, bx.si, x.stride(-2), br.so, br.si, scores ? right.stride(-1) : right.stride(-2)};
+        check(scores ? bgemm_scores_forward(mode, x.data_ptr(), right.data_ptr(), strides, batch, bx.inner, N, M, K, out.data_ptr(), st)
+                     : bgemm_context_forward(x.data_ptr(), right.data_ptr(), strides, batch, bx.inner, N, K, M, out.data_ptr(), st));
+    } else {
+        const int64_t wx = bgemm_tiled_words(N, K), wr = bgemm_tiled_words(M, K);
+        const Tensor planes = at::empty({batch * (wx + wr)}, options.dtype(at::kInt));
+        int32_t* const px = planes.data_ptr<int32_t>();
+        int32_t* const pr = px + batch * wx;
+        check(bgemm_pack_batched(x.data_ptr(), src_type(x), 0, nullptr, bx.outer, bx.inner, N, K, x.stride(-2), bx.so, bx.si, px, nullptr, st));
+        if (by_rows)
+            check(bgemm_pack_batched(right.data_ptr(), src_type(right), 0, nullptr, br.outer, br.inner, M, K, right.stride(-1), br.so, br.si, pr, nullptr, st));
+        else
+            check(bgemm_pack_transposed_batched(right.data_ptr(), src_type(right), br.outer, br.inner, M, K, right.stride(-2), br.so, br.si, pr, st));
+        check(bgemm_packed_forward(mode, pr, px, nullptr, out.data_ptr(), BGEMM_OUT_F16, batch, M, N, K, batch > 1 ? wr : 0, batch > 1 ? wx : 0, N * M, 1, BGEMM_VARIANT_AUTO,
+                                   nullptr, 0, nullptr, 0, st));
+    }
+    return out;
+}
+
+namespace {
+
+// batched_product(x [.., N, K], right [.., K, M], mode) -> fp16 [.., N, M]
 PyObject* batched_product(PyObject*, PyObject* const* args, const Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
     TORCH_CHECK_TYPE(n == 3, "batched_product takes 3 arguments");
     if (!plain_gpu(args[0]) || !plain_gpu(args[1]) || is_watched()) Py_RETURN_NONE;
-    const Tensor &x = tensor_at(args[0]), &right = tensor_at(args[1]);
     const int mode = (int)PyLong_AsLong(args[2]);
     if (PyErr_Occurred()) throw python_error();
-    const int64_t d = x.dim();
-    if ((d != 3 && d != 4) || right.dim() != d || !is_param_type(x.scalar_type()) || !is_param_type(right.scalar_type()) || right.device() != x.device() || x.numel() == 0 ||
-        right.numel() == 0 || x.size(-1) != right.size(-2) || x.size(0) != right.size(0) || (d == 4 && x.size(1) != right.size(1)))
-        Py_RETURN_NONE;
-    const int64_t N = x.size(-2), K = x.size(-1), M = right.size(-1);
-    // rows read where they lie; the right operand row by row of its transpose if that is dense, else column by column
-    const bool by_rows = right.stride(-2) == 1 && right.stride(-1) >= K, by_columns = right.stride(-1) == 1 && right.stride(-2) >= M;
-    if (x.stride(-1) != 1 || x.stride(-2) < K || !(by_rows || by_columns)) Py_RETURN_NONE;
-    const Batch bx = batch_of(x), br = batch_of(right);
-    if (bx.so < 0 || bx.si < 0 || br.so < 0 || br.si < 0) Py_RETURN_NONE;
-    const int64_t batch = bx.outer * bx.inner;
     Tensor out;
     {
         const WithoutGil no_gil;
-        const c10::OptionalDeviceGuard guard(x.device());
-        const auto options = x.options().requires_grad(false);
-        std::vector<int64_t> shape = x.sizes().vec();
-        shape.back() = M;
-        out = at::empty(shape, options.dtype(at::kHalf));
-        void* const st = stream_of(x);
-        const bool half = x.scalar_type() == at::kHalf && right.scalar_type() == at::kHalf;
-        const bool scores = half && (mode == BGEMM_MODE_XOR || mode == BGEMM_MODE_AND) && by_rows && scores_in_one(batch, N, M, K);
-        const bool context = half && mode == BGEMM_MODE_ATTN_X && by_columns && context_in_one(batch, N, K, M);
-        if (scores || context) {
-            const int64_t strides[6] = {bx.so, bx.si, x.stride(-2), br.so, br.si, scores ? right.stride(-1) : right.stride(-2)};
-            check(scores ? bgemm_scores_forward(mode, x.data_ptr(), right.data_ptr(), strides, batch, bx.inner, N, M, K, out.data_ptr(), st)
-                         : bgemm_context_forward(x.data_ptr(), right.data_ptr(), strides, batch, bx.inner, N, K, M, out.data_ptr(), st));
-        } else {
-            const int64_t wx = bgemm_tiled_words(N, K), wr = bgemm_tiled_words(M, K);
-            const Tensor planes = at::empty({batch * (wx + wr)}, options.dtype(at::kInt));
-            int32_t* const px = planes.data_ptr<int32_t>();
-            int32_t* const pr = px + batch * wx;
-            check(bgemm_pack_batched(x.data_ptr(), src_type(x), 0, nullptr, bx.outer, bx.inner, N, K, x.stride(-2), bx.so, bx.si, px, nullptr, st));
-            if (by_rows)
-                check(bgemm_pack_batched(right.data_ptr(), src_type(right), 0, nullptr, br.outer, br.inner, M, K, right.stride(-1), br.so, br.si, pr, nullptr, st));
-            else
-                check(bgemm_pack_transposed_batched(right.data_ptr(), src_type(right), br.outer, br.inner, M, K, right.stride(-2), br.so, br.si, pr, st));
-            check(bgemm_packed_forward(mode, pr, px, nullptr, out.data_ptr(), BGEMM_OUT_F16, batch, M, N, K, batch > 1 ? wr : 0, batch > 1 ? wx : 0, N * M, 1, BGEMM_VARIANT_AUTO,
-                                       nullptr, 0, nullptr, 0, st));
-        }
+        out = batched_product_of(tensor_at(args[0]), tensor_at(args[1]), mode);
     }
+    if (!out.defined()) Py_RETURN_NONE;
     return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS
 }
@@ -510,6 +521,14 @@ bool head_operand(const Tensor& t)
     return ((s[0] | s[1] | s[2]) & 7) == 0;
 }
 
+// Operands that the gradients' kernels read where they lie, and no more rows than `longest`.
+bool grads_in_one(const Tensor& a, const Tensor& b, const int64_t longest)
+{
+    if (a.device() != b.device() || !head_operand(a) || !head_operand(b)) return false;
+    const int64_t N = a.size(-2), M = b.size(-2), batch = a.numel() / (N * a.size(-1));
+    return N <= longest && M <= longest && batch * ((N + 63) / 64) * ((M + 63) / 64 + 1) < (int64_t)(1LL << 31) - (1 << 24);
+}
+
 // one_launch_grads(matrix, a, b, longest) -> whether the products' gradients go to their kernels (bgemm_linear._one_launch_grads)
 PyObject* one_launch_grads(PyObject*, PyObject* const* args, const Py_ssize_t n)
 {
@@ -521,9 +540,7 @@ PyObject* one_launch_grads(PyObject*, PyObject* const* args, const Py_ssize_t n)
     const Tensor &m = tensor_at(args[0]), &a = tensor_at(args[1]), &b = tensor_at(args[2]);
     const int64_t longest = PyLong_AsLongLong(args[3]);
     if (PyErr_Occurred()) throw python_error();
-    if (m.scalar_type() != at::kHalf || m.device() != a.device() || a.device() != b.device() || !head_operand(a) || !head_operand(b)) Py_RETURN_FALSE;
-    const int64_t N = a.size(-2), M = b.size(-2), batch = a.numel() / (N * a.size(-1));
-    if (N > longest || M > longest || batch * ((N + 63) / 64) * ((M + 63) / 64 + 1) >= (int64_t)(1LL << 31) - (1 << 24)) Py_RETURN_FALSE;
+    if (m.scalar_type() != at::kHalf || m.device() != a.device() || !grads_in_one(a, b, longest)) Py_RETURN_FALSE;
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }
@@ -535,6 +552,49 @@ Tensor grad_like(const Tensor& t)
     return g.stride(-1) == 1 ? g : at::empty_like(t, at::MemoryFormat::Contiguous);
 }
 
+// The matrix and the operands of one product, such as its kernel takes.
+bool grads_match(const Tensor& m, const Tensor& a, const Tensor& b)
+{
+    if (!head_operand(a) || !head_operand(b) || a.dim() != b.dim() || a.size(-1) != b.size(-1) || m.scalar_type() != at::kHalf || m.device() != a.device() ||
+        b.device() != a.device() || m.dim() != a.dim() || m.size(-2) != a.size(-2) || m.size(-1) != b.size(-2))
+        return false;
+    for (int64_t i = 0; i < a.dim() - 2; i++)
+        if (a.size(i) != b.size(i) || a.size(i) != m.size(i)) return false;
+    return true;
+}
+
+void launch_grads(const bool context, const Tensor& m0, const Tensor& a, const Tensor& b, const bool need0, const bool need1, Tensor& g0, Tensor& g1)
+{
+    const c10::OptionalDeviceGuard guard(a.device());
+    const Tensor m = context && !need1 ? Tensor() : m0.contiguous();
+    int64_t s[12] = {0};
+    head_view(a, s);
+    head_view(b, s + 3);
+    const int64_t inner = a.size(-3), batch = a.dim() == 4 ? a.size(0) * inner : inner, N = a.size(-2), M = b.size(-2), D = a.size(-1);
+    if (context) {
+        if (need0) g0 = at::empty(m0.sizes(), m0.options().requires_grad(false));
+        if (need1) { g1 = grad_like(b); head_view(g1, s + 9); }
+        check(bgemm_context_backward(data_or_null(m), a.data_ptr(), b.data_ptr(), s, batch, inner, N, M, D, data_or_null(g0), data_or_null(g1), stream_of(a)));
+    } else {
+        if (need0) { g0 = grad_like(a); head_view(g0, s + 6); }
+        if (need1) { g1 = grad_like(b); head_view(g1, s + 9); }
+        check(bgemm_scores_backward(m.data_ptr(), a.data_ptr(), b.data_ptr(), s, batch, inner, N, M, D, data_or_null(g0), data_or_null(g1), stream_of(a)));
+    }
+}
+
+}  // namespace
+
+bool attention_grads(const bool context, const Tensor& m, const Tensor& a, const Tensor& b, const bool need0, const bool need1, const int64_t longest,
+                     const int64_t most, Tensor& g0, Tensor& g1)
+{
+    if (!is_memory(m) || !is_memory(a) || !is_memory(b) || !grads_match(m, a, b) || !grads_in_one(a, b, longest)) return false;
+    if (a.size(-1) > 64 && a.numel() * b.size(-2) >= most) return false;
+    launch_grads(context, m, a, b, need0, need1, g0, g1);
+    return true;
+}
+
+namespace {
+
 // attention_backward(context, m | None, a, b, need a (context: the probabilities), need b) -> (gradient | None, gradient | None); operands
 // that one_launch_grads has looked at
 PyObject* attention_backward(PyObject*, PyObject* const* args, const Py_ssize_t n)
@@ -544,30 +604,12 @@ PyObject* attention_backward(PyObject*, PyObject* const* args, const Py_ssize_t 
     const bool context = args[0] == Py_True, need0 = PyObject_IsTrue(args[4]), need1 = PyObject_IsTrue(args[5]);
     for (int i = 1; i < 4; i++)
         if (!plain_gpu(args[i])) Py_RETURN_NONE;
-    const Tensor &m0 = tensor_at(args[1]), &a = tensor_at(args[2]), &b = tensor_at(args[3]);
-    if (c10::GradMode::is_enabled() || !head_operand(a) || !head_operand(b) || a.dim() != b.dim() || a.size(-1) != b.size(-1) || m0.scalar_type() != at::kHalf ||
-        m0.device() != a.device() || b.device() != a.device() || m0.dim() != a.dim() || m0.size(-2) != a.size(-2) || m0.size(-1) != b.size(-2))
-        Py_RETURN_NONE;
-    for (int64_t i = 0; i < a.dim() - 2; i++)
-        if (a.size(i) != b.size(i) || a.size(i) != m0.size(i)) Py_RETURN_NONE;
+    const Tensor &m = tensor_at(args[1]), &a = tensor_at(args[2]), &b = tensor_at(args[3]);
+    if (c10::GradMode::is_enabled() || !grads_match(m, a, b)) Py_RETURN_NONE;
     Tensor g0, g1;
     {
         const WithoutGil no_gil;
-        const c10::OptionalDeviceGuard guard(a.device());
-        const Tensor m = context && !need1 ? Tensor() : m0.contiguous();
-        int64_t s[12] = {0};
-        head_view(a, s);
-        head_view(b, s + 3);
-        const int64_t inner = a.size(-3), batch = a.dim() == 4 ? a.size(0) * inner : inner, N = a.size(-2), M = b.size(-2), D = a.size(-1);
-        if (context) {
-            if (need0) g0 = at::empty(m0.sizes(), m0.options());
-            if (need1) { g1 = grad_like(b); head_view(g1, s + 9); }
-            check(bgemm_context_backward(data_or_null(m), a.data_ptr(), b.data_ptr(), s, batch, inner, N, M, D, data_or_null(g0), data_or_null(g1), stream_of(a)));
-        } else {
-            if (need0) { g0 = grad_like(a); head_view(g0, s + 6); }
-            if (need1) { g1 = grad_like(b); head_view(g1, s + 9); }
-            check(bgemm_scores_backward(m.data_ptr(), a.data_ptr(), b.data_ptr(), s, batch, inner, N, M, D, data_or_null(g0), data_or_null(g1), stream_of(a)));
-        }
+        launch_grads(context, m, a, b, need0, need1, g0, g1);
     }
     PyObject* const t = PyTuple_New(2);
     PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(g0));

@@ -359,7 +359,97 @@ PyObject* elastic_train(PyObject*, PyObject* const* args, const Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
+// ---- attention's products as one autograd node each ----------------------------------------------------------------------------------
+// bgemm_matmul and bgemm_attn_matmul on batches of fp16 matrices (bgemm_linear.py).  Kept are the operands themselves, as the Functions
+// keep them: changed in place they are refused.  As Python Functions the two took 45 of the 155 us of a step of 4 x 512 tokens, 12 heads
+// of 64, half of that waiting for the interpreter's lock on the engine's thread.
+struct ProductNode : public torch::autograd::Node {
+    bool context;
+    int64_t longest, most;
+    SavedVariable x_, right_;
+
+    std::string name() const override { return context ? "BinaryContextBackward" : "BinaryScoresBackward"; }
+
+    void release_variables() override
+    {
+        std::lock_guard<std::mutex> lock(mutex_);
+        x_.reset_data();
+        right_.reset_data();
+    }
+
+    variable_list apply(variable_list&& grads) override
+    {
+        if (!grads[0].defined()) return variable_list(2);
+        const bool need0 = task_should_compute_output(0), need1 = task_should_compute_output(1);
+        std::unique_lock<std::mutex> lock(mutex_);
+        const Tensor x = x_.unpack(), right = right_.unpack();
+        lock.unlock();
+        const Tensor& g = grads[0];
+        if (!LayerNode::by_operations(g) && g.scalar_type() == at::kHalf && !has_tangent(x) && !has_tangent(right)) {
+            Tensor g0, g1;
+            const bool done = context ? attention_grads(true, x, g, right, need0, need1, longest, most, g0, g1)
+                                      : attention_grads(false, g, x, right.transpose(-1, -2), need0, need1, longest, most, g0, g1);
+            if (done) return {g0, !context && g1.defined() ? g1.transpose(-1, -2) : g1};
+        }
+        pybind11::gil_scoped_acquire gil;
+        PyObject* const module = PyImport_ImportModule("bgemm_linear");
+        if (!module) throw_pending();
+        PyObject* const f = PyObject_GetAttrString(module, context ? "_context_grads" : "_scores_grads");
+        Py_DECREF(module);
+        if (!f) throw_pending();
+        PyObject* const args = PyTuple_New(4), * const need = PyTuple_New(2);
+        PyTuple_SET_ITEM(need, 0, PyBool_FromLong(need0));
+        PyTuple_SET_ITEM(need, 1, PyBool_FromLong(need1));
+        PyTuple_SET_ITEM(args, 0, need);
+        PyTuple_SET_ITEM(args, 1, THPVariable_Wrap(x));
+        PyTuple_SET_ITEM(args, 2, THPVariable_Wrap(right));
+        PyTuple_SET_ITEM(args, 3, THPVariable_Wrap(g));
+        PyObject* const got = PyObject_CallObject(f, args);
+        Py_DECREF(f); Py_DECREF(args);
+        if (!got) throw_pending();
+        variable_list r = {tensor_or_none(PyTuple_GET_ITEM(got, 0)), tensor_or_none(PyTuple_GET_ITEM(got, 1))};
+        Py_DECREF(got);
+        return r;
+    }
+};
+
+// product_train(x [.., N, K], right [.., K, M], mode, longest, most) -> fp16 [.., N, M], or None where the Function has to run
+PyObject* product_train(PyObject*, PyObject* const* args, const Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    TORCH_CHECK_TYPE(n == 5, "product_train takes 5 arguments");
+    if (!c10::GradMode::is_enabled() || !plain_call(args, 2)) Py_RETURN_NONE;
+    const Tensor &x = tensor_at(args[0]), &right = tensor_at(args[1]);
+    const int mode = (int)PyLong_AsLong(args[2]);
+    const int64_t longest = PyLong_AsLongLong(args[3]), most = PyLong_AsLongLong(args[4]);
+    if (PyErr_Occurred()) throw python_error();
+    if (!x.requires_grad() && !right.requires_grad()) Py_RETURN_NONE;
+    for (const Tensor* t : {&x, &right})
+        if (!t->is_cuda() || !is_memory(*t) || has_tangent(*t) || t->scalar_type() != at::kHalf) Py_RETURN_NONE;
+    Tensor out;
+    {
+        const WithoutGil no_gil;
+        {
+            const c10::NoGradGuard no_grad;
+            out = batched_product_of(x, right, mode);
+        }
+        if (out.defined()) {
+            auto node = std::shared_ptr<ProductNode>(new ProductNode(), torch::autograd::deleteNode);
+            node->context = mode == BGEMM_MODE_ATTN_X;
+            node->longest = longest; node->most = most;
+            node->x_ = SavedVariable(x, false);
+            node->right_ = SavedVariable(right, false);
+            node->set_next_edges(torch::autograd::collect_next_edges(x, right));
+            torch::autograd::set_history(out, node);
+        }
+    }
+    if (!out.defined()) Py_RETURN_NONE;
+    return THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
 const PyMethodDef train_methods[] = {
+    {"product_train", (PyCFunction)(void (*)(void))product_train, METH_FASTCALL, "batched product of two binarised operands, recorded as one autograd node"},
     {"elastic_train", (PyCFunction)(void (*)(void))elastic_train, METH_FASTCALL, "forward of a learned-scale binary Linear, recorded as one autograd node"},
     {"linear_train", (PyCFunction)(void (*)(void))linear_train, METH_FASTCALL, "forward of a scaled binary Linear, recorded as one autograd node"}};
 
