@@ -9,11 +9,16 @@
 // the halving, copies of the head-split gradients) 12 heads of 64, 4 x 512 tokens, took 20 launches and a dozen passes over 25 MB;
 // here each product pair is one launch that reads or writes an [N][M] matrix once a product, in its own order, and the gradients
 // leave in the operands' strides.  What is left is that traffic: the contraction is D = 32 .. 128 long on one side, far below what
-// the matrix cores could do in the time.  A training step of both products is that of the host, 160 us in all; of its 68 us of kernels
-// those here take 31 (context) and 19 us (scores), neither bandwidth's (3.1 and 5.3
-// TB/s counted) nor the matrix cores' (5 % busy): waves wait for 47 and 44 % of their cycles, and LDS, where fragments that lie across
-// the rows are read two bytes a lane, is active for 18 and 33 % of the compute units' time.
+// the matrix cores could do in the time.  48 matrices of 512 x 512, D = 64: scores 19.6 -> 16.0 us, context 30.8 -> 18.2, the latter's two
+// halves 10.4 (25 MB written) and 12.8 (25 MB read) alone.  Blocks of a matrix on one XCD did most of it: dealt round robin, an XCD read the
+// same eighth of every row, from few of its L2's channels, and the scores' second reading came from beyond its L2 (a pass of one product
+// 15 -> 12 us).  Fragments that lie across the rows come out of LDS by transposing reads (two-byte ones: 96 for 24), and grad_P leaves
+// from registers, 128 bytes of a row a half-wave (through LDS in 64 x 64 tiles 18.1 -> 11.9).  A wave's life is then half waiting for memory and a
+// quarter vector instructions, at 1.5 blocks a unit.  Not ahead: stretches of 128 rows (15.0 and 17.6, but 64 x 64 3.9 -> 4.5),
+// two of them in flight (172 registers: 15.2 -> 19.8), eight waves a block with stretches of their own and no barrier before the sums meet (scores
+// 22.7, context 19.4; 64 x 64 5.4).
 #include "common.h"
+#include <type_traits>
 
 namespace bgemm {
 
@@ -29,72 +34,97 @@ struct AttnGradArgs {
     __half* gp;                       // context: grad_P, dense
     int N, M, inner, first;           // first: blocks a matrix of the first kind
     int per_batch;                    // blocks a matrix
+    int batch, chunks;                // 64 columns of grad_P each, a block
 };
-
-constexpr int AG_ROW = 72;            // staged row of 64 halves, padded by a 16-byte unit
 
 __device__ __forceinline__ __half* head_at(const HeadView& v, const int z, const int inner)
 {
     return const_cast<__half*>(v.p) + (z / inner) * v.so + (z % inner) * v.si;
 }
 
-// Two fp16 numbers -> their signs; zeros and NaN give 0.
+// Two fp16 numbers at a time: 1 where a number is neither zero nor NaN.
+typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ ushort2v is_signed(const unsigned x)
+{
+    const ushort2v one = {1, 1}, inf = {0x7c00, 0x7c00}, a = __builtin_bit_cast(ushort2v, x & 0x7fff7fffu);
+    return __builtin_elementwise_min(a, one) - __builtin_elementwise_min(__builtin_elementwise_sub_sat(a, inf), one);
+}
+// Their signs; zeros and NaN give 0.
 __device__ __forceinline__ unsigned sign_pair(const unsigned x)
 {
-    auto one = [](const unsigned b) { return ((b & 0x7fffu) - 1u < 0x7c00u ? 0x3c00u : 0u) | (b & 0x8000u); };
-    return one(x & 0xffffu) | one(x >> 16) << 16;
+    const ushort2v one = {0x3c00, 0x3c00};
+    return __builtin_bit_cast(unsigned, (ushort2v)(is_signed(x) * one)) | (x & 0x80008000u);
 }
 // Two entries of P -> their weights.
 __device__ __forceinline__ unsigned weight_pair(const unsigned x)
 {
-    auto one = [](const unsigned b) { return (b & 0x7fffu) - 1u < 0x7c00u ? 0x3c00u : 0x3800u; };
-    return one(x & 0xffffu) | one(x >> 16) << 16;
+    const ushort2v step = {0x400, 0x400}, half = {0x3800, 0x3800};
+    return __builtin_bit_cast(unsigned, (ushort2v)(is_signed(x) * step + half));
 }
 __device__ __forceinline__ uint4 sign8(const uint4 x) { return make_uint4(sign_pair(x.x), sign_pair(x.y), sign_pair(x.z), sign_pair(x.w)); }
+__device__ __forceinline__ uint4 weight8(const uint4 x) { return make_uint4(weight_pair(x.x), weight_pair(x.y), weight_pair(x.z), weight_pair(x.w)); }
+// Eight rows of a column each: lane (c, h) gets rows row0 + 8 h .. + 7 of column col0 + c of a staged matrix, by two reads that transpose 4 x 4
+// elements among sixteen lanes (lane i of sixteen names row i / 4 and the four columns from 4 (i % 4) on, and gets column i).
+typedef short short4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ half8 column8(const _Float16* const staged, const int stride, const int row0, const int col0, const int lane)
+{
+    typedef __attribute__((address_space(3))) short4v* lds4;
+    const int i = lane & 15, g = lane >> 4;
+    const _Float16* const at = staged + (row0 + 8 * (g >> 1) + (i >> 2)) * stride + col0 + 16 * (g & 1) + 4 * (i & 3);
+    union { short4v s[2]; half8 h; } u;
+#pragma unroll
+    for (int k = 0; k < 2; k++) u.s[k] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(__attribute__((address_space(3))) void*)(at + 4 * k * stride));
+    return u.h;
+}
 __device__ __forceinline__ float16v mma(const half8 a, const half8 b, const float16v c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
 
 // out[i,:] = sum_r X[i,r] Y[r,:] for the 64 rows i of a block: X is m, or its transpose (TRANS).  64 of r at a time go through LDS,
 // the next 64 on their way in registers; two waves share 32 rows and halve the contraction, so that a fragment of X serves all of
-// Y's column tiles.  Columns come out of LDS two bytes a lane.
+// Y's column tiles.  What lies across the rows comes out of LDS by reads that transpose.
+constexpr int AG_STEP = 64;
 template <int DT, bool TRANS, bool WEIGHTS>
 __device__ __forceinline__ void tall_product(const AttnGradArgs& a, const HeadView& yv, const HeadView& ov, const int z, const int i0, unsigned char* smem)
 {
     constexpr int D = DT * 32, YROW = D + 8, UNITS = D / 8;
+    constexpr int XW = TRANS ? 8 : AG_STEP / 8, XROW = XW * 8 + 8, XLOADS = AG_STEP * 64 / 8 / 256, YLOADS = AG_STEP * UNITS / 256;      // 16-byte units of a staged row of X
     __half* const xs = reinterpret_cast<__half*>(smem);
-    __half* const ys = xs + 64 * AG_ROW;
+    __half* const ys = xs + (TRANS ? AG_STEP : 64) * XROW;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c = lane & 31, it = wave & 1, part = wave >> 1;
     const int rows = TRANS ? a.M : a.N, len = TRANS ? a.N : a.M;
     const __half* const x = a.m + (int64_t)z * a.N * a.M;
     const __half* const y = head_at(yv, z, a.inner);
-    const int xr = tid >> 2, xc = (tid & 3) * 16;
 
-    uint4 xreg[2], yreg[DT];
+    uint4 xreg[XLOADS], yreg[YLOADS];
     auto load = [&](const int r0) {
-        const int row = (TRANS ? r0 : i0) + xr;
 #pragma unroll
-        for (int p = 0; p < 2; p++) {
-            const int col = (TRANS ? i0 : r0) + xc + 8 * p;
+        for (int p = 0; p < XLOADS; p++) {
+            const int u = tid + 256 * p, row = (TRANS ? r0 : i0) + u / XW, col = (TRANS ? i0 : r0) + u % XW * 8;
             uint4 v = make_uint4(0, 0, 0, 0);
-            if (row < a.N) {
+            if (row < a.N && col < a.M) {
                 const __half* const from = x + (int64_t)row * a.M + col;
-                if (col + 8 <= a.M) {
-                    __builtin_memcpy(&v, from, 16);
-                    if constexpr (WEIGHTS) v = make_uint4(weight_pair(v.x), weight_pair(v.y), weight_pair(v.z), weight_pair(v.w));
+                if (col + 8 <= a.M) __builtin_memcpy(&v, from, 16);
+                else if (a.M >= 8) {
+                    // a row's last elements: its last eight, those before them shifted out
+                    uint64_t d[2];
+                    __builtin_memcpy(d, from - (col + 8 - a.M), 16);
+                    const int bits = (col + 8 - a.M) * 16;
+                    d[0] = bits < 64 ? d[0] >> bits | d[1] << (64 - bits) : d[1] >> (bits - 64);
+                    d[1] = bits < 64 ? d[1] >> bits : 0;
+                    __builtin_memcpy(&v, d, 16);
                 } else {
                     unsigned d[4] = {0, 0, 0, 0};
 #pragma unroll
                     for (int e = 0; e < 7; e++)
-                        if (col + e < a.M) {
-                            const unsigned b = __half_as_ushort(from[e]);
-                            d[e >> 1] |= (WEIGHTS ? weight_pair(b) & 0xffffu : b) << (16 * (e & 1));
-                        }
+                        if (col + e < a.M) d[e >> 1] |= (unsigned)__half_as_ushort(from[e]) << (16 * (e & 1));
                     v = make_uint4(d[0], d[1], d[2], d[3]);
                 }
+                // (entries that do not exist then weigh something, in rows of the output that do not exist either)
+                if constexpr (WEIGHTS) v = weight8(v);
             }
             xreg[p] = v;
         }
 #pragma unroll
-        for (int j = 0; j < DT; j++) {
+        for (int j = 0; j < YLOADS; j++) {
             const int u = tid + 256 * j, r = r0 + u / UNITS;
             uint4 v = make_uint4(0, 0, 0, 0);
             if (r < len) v = *reinterpret_cast<const uint4*>(y + r * yv.row + u % UNITS * 8);
@@ -109,34 +139,28 @@ __device__ __forceinline__ void tall_product(const AttnGradArgs& a, const HeadVi
         for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
     load(0);
 #pragma unroll 1
-    for (int r0 = 0; r0 < len; r0 += 64) {
+    for (int r0 = 0; r0 < len; r0 += AG_STEP) {
         __syncthreads();
 #pragma unroll
-        for (int p = 0; p < 2; p++) *reinterpret_cast<uint4*>(xs + xr * AG_ROW + xc + 8 * p) = xreg[p];
+        for (int p = 0; p < XLOADS; p++) {
+            const int u = tid + 256 * p;
+            *reinterpret_cast<uint4*>(xs + u / XW * XROW + u % XW * 8) = xreg[p];
+        }
 #pragma unroll
-        for (int j = 0; j < DT; j++) {
+        for (int j = 0; j < YLOADS; j++) {
             const int u = tid + 256 * j;
             *reinterpret_cast<uint4*>(ys + u / UNITS * YROW + u % UNITS * 8) = WEIGHTS ? yreg[j] : sign8(yreg[j]);
         }
         __syncthreads();
-        if (r0 + 64 < len) load(r0 + 64);
+        if (r0 + AG_STEP < len) load(r0 + AG_STEP);
         const _Float16* const xf = reinterpret_cast<const _Float16*>(xs);
         const _Float16* const yf = reinterpret_cast<const _Float16*>(ys);
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const int r = part * 32 + s * 16 + 8 * h;
-            half8 xv;
-            if constexpr (TRANS) {
+        for (int s = 0; s < AG_STEP / 32; s++) {
+            const int r = 64 * (s >> 1) + part * 32 + (s & 1) * 16;
+            const half8 xv = TRANS ? column8(xf, XROW, r, it * 32, lane) : *reinterpret_cast<const half8*>(xf + (it * 32 + c) * XROW + r + 8 * h);
 #pragma unroll
-                for (int e = 0; e < 8; e++) xv[e] = xf[(r + e) * AG_ROW + it * 32 + c];
-            } else xv = *reinterpret_cast<const half8*>(xf + (it * 32 + c) * AG_ROW + r);
-#pragma unroll
-            for (int t = 0; t < DT; t++) {
-                half8 yv8;
-#pragma unroll
-                for (int e = 0; e < 8; e++) yv8[e] = yf[(r + e) * YROW + t * 32 + c];
-                acc[t] = mma(yv8, xv, acc[t]);
-            }
+            for (int t = 0; t < DT; t++) acc[t] = mma(column8(yf, YROW, r, t * 32, lane), xv, acc[t]);
         }
     }
     __syncthreads();
@@ -161,55 +185,88 @@ __device__ __forceinline__ void tall_product(const AttnGradArgs& a, const HeadVi
         }
 }
 
-// 64 x 64 of grad_P: the operands are fragments as they lie, the result goes through LDS so that it leaves in pieces of 16 bytes.
+// grad_P of 128 rows, a wave 32 of them, and `a.chunks` times 64 columns: the signs of V go through LDS, G's rows are operands as they lie.  The
+// columns are dealt to two operands as even and odd ones, so that a lane has pairs of neighbours: a half-wave stores a line.
 template <int DT>
-__device__ __forceinline__ void probs_tile(const AttnGradArgs& a, const int z, const int n0, const int m0, unsigned char* smem)
+__device__ __forceinline__ void probs_strip(const AttnGradArgs& a, const int z, const int n0, const int m0, unsigned char* smem)
 {
-    __half* const stage = reinterpret_cast<__half*>(smem);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c = lane & 31, nt = wave & 1, mt = wave >> 1;
-    const __half* const g = head_at(a.a, z, a.inner) + min(n0 + nt * 32 + c, a.N - 1) * a.a.row + 8 * h;
-    const __half* const v = head_at(a.b, z, a.inner) + min(m0 + mt * 32 + c, a.M - 1) * a.b.row + 8 * h;
-    float16v acc;
+    constexpr int D = DT * 32, VROW = D + 8, UNITS = D / 8, LOADS = 64 * UNITS / 256;
+    typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+    typedef float float2v __attribute__((ext_vector_type(2)));
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c = lane & 31, nw = n0 + wave * 32;
+    const __half* const g = head_at(a.a, z, a.inner) + min(nw + c, a.N - 1) * a.a.row + 8 * h;
+    const __half* const v = head_at(a.b, z, a.inner);
+    __half* const vs = reinterpret_cast<__half*>(smem);
+    uint4 vreg[LOADS];
+    auto load = [&](const int m) {
 #pragma unroll
-    for (int i = 0; i < 16; i++) acc[i] = 0.f;
+        for (int j = 0; j < LOADS; j++) {
+            const int u = tid + 256 * j;
+            vreg[j] = *reinterpret_cast<const uint4*>(v + min(m + u / UNITS, a.M - 1) * a.b.row + u % UNITS * 8);
+        }
+    };
+    load(m0);
+    half8 gf[2 * DT];
 #pragma unroll
-    for (int s = 0; s < 2 * DT; s++) {
-        const uint4 x = sign8(*reinterpret_cast<const uint4*>(v + 16 * s));
-        half8 vf;
-        __builtin_memcpy(&vf, &x, 16);
-        acc = mma(vf, *reinterpret_cast<const half8*>(g + 16 * s), acc);
-    }
+    for (int s = 0; s < 2 * DT; s++) gf[s] = *reinterpret_cast<const half8*>(g + 16 * s);
+    __half* const out = a.gp + ((int64_t)z * a.N + nw + 4 * h) * a.M;
+#pragma unroll 1
+    for (int k = 0; k < a.chunks; k++) {
+        const int m1 = m0 + 64 * k;
+        if (m1 >= a.M) break;
+        if (k) __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        union { __half x[4]; uint2 u; } pk;
+        for (int j = 0; j < LOADS; j++) {
+            const int u = tid + 256 * j;
+            *reinterpret_cast<uint4*>(vs + u / UNITS * VROW + u % UNITS * 8) = sign8(vreg[j]);
+        }
+        __syncthreads();
+        if (k + 1 < a.chunks) load(m1 + 64);
+        float16v acc[2];
 #pragma unroll
-        for (int e = 0; e < 4; e++) pk.x[e] = __float2half_rn(__half2float(__float2half_rn(acc[4 * q + e])) * 0.5f);
-        *reinterpret_cast<uint2*>(stage + (nt * 32 + c) * AG_ROW + mt * 32 + 8 * q + 4 * h) = pk.u;
-    }
-    __syncthreads();
-    const int n = n0 + (tid >> 2);
-    if (n >= a.N) return;
+        for (int j = 0; j < 2; j++)
 #pragma unroll
-    for (int p = 0; p < 2; p++) {
-        const int at = (tid & 3) * 16 + 8 * p, m = m0 + at;
-        __half* const to = a.gp + ((int64_t)z * a.N + n) * a.M + m;
-        const __half* const from = stage + (tid >> 2) * AG_ROW + at;
-        if (m + 8 <= a.M) __builtin_memcpy(to, from, 16);
-        else
+            for (int i = 0; i < 16; i++) acc[j][i] = 0.f;
 #pragma unroll
-            for (int e = 0; e < 7; e++)
-                if (m + e < a.M) to[e] = from[e];
+        for (int s = 0; s < 2 * DT; s++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                acc[j] = mma(gf[s], *reinterpret_cast<const half8*>(reinterpret_cast<const _Float16*>(vs) + (2 * c + j) * VROW + 16 * s + 8 * h), acc[j]);
+        const int m = m1 + 2 * c;
+        auto rows_out = [&](auto whole_c) {
+            constexpr bool WHOLE = decltype(whole_c)::value;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int r = 8 * (i >> 2) + (i & 3);
+                const half2v half = {(_Float16)0.5f, (_Float16)0.5f};
+                const float2v two = {acc[0][i], acc[1][i]};
+                const half2v p = __builtin_convertvector(two, half2v) * half;
+                __half* const to = out + (int64_t)r * a.M + m;
+                if (WHOLE) __builtin_memcpy(to, &p, 4);
+                else if (nw + 4 * h + r < a.N) {
+                    if (m < a.M) reinterpret_cast<_Float16*>(to)[0] = p[0];
+                    if (m + 1 < a.M) reinterpret_cast<_Float16*>(to)[1] = p[1];
+                }
+            }
+        };
+        if (nw + 32 <= a.N && m1 + 64 <= a.M) rows_out(std::true_type{});
+        else rows_out(std::false_type{});
     }
 }
 
-template <int DT> constexpr int ag_lds() { return (64 * AG_ROW + 64 * (DT * 32 + 8)) * 2 > DT * 8192 ? (64 * AG_ROW + 64 * (DT * 32 + 8)) * 2 : DT * 8192; }
+// (TRANS, or 64 rows of AG_STEP: about the same)
+template <int DT> constexpr int ag_lds()
+{
+    constexpr int x = (AG_STEP * 72 > 64 * (AG_STEP + 8) ? AG_STEP * 72 : 64 * (AG_STEP + 8)) * 2, y = AG_STEP * (DT * 32 + 8) * 2;
+    return x + y > DT * 8192 ? x + y : DT * 8192;
+}
 
 // A matrix's blocks are neighbours: its second reading finds it in the caches.
 template <int DT>
 __global__ __launch_bounds__(256) void scores_grad_kernel(const AttnGradArgs a)
 {
     __shared__ __align__(16) unsigned char smem[ag_lds<DT>()];
-    const int z = blockIdx.x / a.per_batch, t = blockIdx.x % a.per_batch;
+    const int id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), z = id / a.per_batch, t = id % a.per_batch;
     if (t < a.first) tall_product<DT, false, false>(a, a.b, a.ga, z, t * 64, smem);
     else tall_product<DT, true, false>(a, a.a, a.gb, z, (t - a.first) * 64, smem);
 }
@@ -218,10 +275,15 @@ template <int DT>
 __global__ __launch_bounds__(256) void context_grad_kernel(const AttnGradArgs a)
 {
     __shared__ __align__(16) unsigned char smem[ag_lds<DT>()];
-    const int z = blockIdx.x / a.per_batch, t = blockIdx.x % a.per_batch;
-    if (t < a.first) return tall_product<DT, true, true>(a, a.a, a.gb, z, t * 64, smem);
-    const int mb = (a.M + 63) / 64, u = t - a.first;
-    probs_tile<DT>(a, z, u / mb * 64, u % mb * 64, smem);
+    // (the longer blocks first)
+    const int tall = a.batch * a.first;
+    if ((int)blockIdx.x < tall) {
+        const int id = (int)xcd_contiguous_id(blockIdx.x, tall);
+        return tall_product<DT, true, true>(a, a.a, a.gb, id / a.first, id % a.first * 64, smem);
+    }
+    const int id = (int)xcd_contiguous_id(blockIdx.x - tall, gridDim.x - tall), strips = a.per_batch - a.first, u = id % strips;
+    const int mb = (a.M + 64 * a.chunks - 1) / (64 * a.chunks);
+    probs_strip<DT>(a, id / strips, u / mb * 128, u % mb * 64 * a.chunks, smem);
 }
 
 }  // namespace bgemm
@@ -241,14 +303,18 @@ static int attention_backward(const char* who, const bool context, const void* m
     for (int i = 0; i < 12; i++)
         if (strides[i] % 8) return fail(BGEMM_EALIGN, "%s: strides must be multiples of 8", who);
     const int64_t nb = cdiv(N, 64), mb = cdiv(M, 64);
+    // (enough blocks of grad_P for eight a compute unit)
+    int64_t chunks = 1;
+    while (chunks < 8 && batch * cdiv(N, 128) * cdiv(M, 128 * chunks) >= 2048) chunks *= 2;
+    const int64_t strips = cdiv(N, 128) * cdiv(M, 64 * chunks);
     AttnGradArgs g = {};
     auto view = [&](const void* p, const int i) { return HeadView{(const __half*)p, strides[3 * i], strides[3 * i + 1], strides[3 * i + 2]}; };
     g.m = (const __half*)m; g.a = view(a, 0); g.b = view(b, 1); g.ga = view(grad_a, 2); g.gb = view(grad_b, 3); g.gp = (__half*)grad_p;
     g.N = (int)N; g.M = (int)M; g.inner = (int)inner;
-    const int64_t first = context ? (grad_b ? mb : 0) : (grad_a ? nb : 0), second = context ? (grad_p ? nb * mb : 0) : (grad_b ? mb : 0);
+    const int64_t first = context ? (grad_b ? mb : 0) : (grad_a ? nb : 0), second = context ? (grad_p ? strips : 0) : (grad_b ? mb : 0);
     if (first + second == 0) return BGEMM_OK;
     if (batch > 0x7fffffffLL / (first + second)) return fail(BGEMM_EINVAL, "%s: too many blocks", who);
-    g.first = (int)first; g.per_batch = (int)(first + second);
+    g.first = (int)first; g.per_batch = (int)(first + second); g.batch = (int)batch; g.chunks = (int)chunks;
     const dim3 grid((unsigned)(batch * g.per_batch)), block(256);
     const hipStream_t st = (hipStream_t)stream;
     auto go = [&](auto scores, auto ctx) {
