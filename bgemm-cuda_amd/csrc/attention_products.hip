@@ -59,7 +59,9 @@ __global__ __launch_bounds__(WAVES * 64) void scores_kernel(const AttnProductArg
     __shared__ uint32_t qb[W * AP_ROWS], kb[W * AP_COLS];
     __shared__ __align__(16) unsigned char stages[WAVES][32 * ATTN_STAGE];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, c = lane & 31;
-    const int per = a.nblocks * a.mblocks, z = blockIdx.x / per, t = blockIdx.x % per, n0 = t / a.mblocks * AP_ROWS, m0 = t % a.mblocks * AP_COLS;
+    // (a matrix's blocks on one XCD, which reads its operands once: 48 of 512 x 512, D = 64, 8.1 -> 7.4 us under the profiler, the context 13.0 -> 11.9)
+    const int per = a.nblocks * a.mblocks, id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), z = id / per, t = id % per;
+    const int n0 = t / a.mblocks * AP_ROWS, m0 = t % a.mblocks * AP_COLS;
     {
         RowBits<W, AP_COLS, THREADS> kr;
         RowBits<W, AP_ROWS, THREADS> qr;
@@ -160,7 +162,7 @@ __global__ __launch_bounds__(512, W == 4 ? 2 : 4) void context_kernel(const Attn
     uint32_t* const vb = reinterpret_cast<uint32_t*>(smem);      // [W][S64]: words of a row of V
     uint32_t* const vt = vb + W * S64;                           // [2 groups][D]: words of 32 rows
     unsigned char* const stage = reinterpret_cast<unsigned char*>(vt + W * S64) + wave * 256;
-    const int z = blockIdx.x / a.nblocks, q0 = blockIdx.x % a.nblocks * CTX_ROWS + (wave & 3) * 32;
+    const int id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), z = id / a.nblocks, q0 = id % a.nblocks * CTX_ROWS + (wave & 3) * 32;
     const int first = groups * part / parts, end = q0 < a.N ? groups * (part + 1) / parts : first;
     const __half* v = view_at(a.b, z, a.inner);
     const __half* p = view_at(a.a, z, a.inner);
