@@ -78,7 +78,8 @@ enum {
 
 /* Message for the last error returned on the calling thread ("" if none). */
 const char* bgemm_last_error(void);
-/* ABI version; bumped when an entry point is added or its signature or behaviour changes, or the tiled layout does. */
+/* ABI version; bumped when an entry point's signature or behaviour changes, or the tiled layout does.  One that is new shows by its name: a
+ * binding that finds it missing has an older library. */
 #define BGEMM_ABI_VERSION 12
 int bgemm_abi_version(void);          /* of the library */
 
