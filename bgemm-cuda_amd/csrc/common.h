@@ -77,6 +77,7 @@ constexpr int OUT_F32_ELASTIC = 6;
 struct GemmArgs {
     const uint4* W; const uint4* X; const uint4* X2;
     void* out; int out_kind;       // BGEMM_OUT_*
+    int codes;            // a ternary operand's planes are codes (ternary_codes)
     const void* ep_sw; const void* ep_sa; const void* ep_bias;   // scaled output kinds: per-column scale, scalar, bias
     const void* ep_zp;    // bits kinds: the next layer's zero point (null = 0)
     int nt_store;         // general kernel: 4-byte outputs are stored past the caches (set for outputs of up to 32 MiB)
@@ -88,7 +89,6 @@ struct GemmArgs {
     int force;            // BGEMM_KERNEL_* the caller insists on (BGEMM_FORCE_KERNEL), or -1: chosen by shape
     const int32_t* cntW; const int32_t* cntX;   // row popcounts of W and X ([batch][rows], a shared operand once), or null:
                                                 // the pipelined tiles then count nothing themselves
-    int codes;            // a ternary operand's planes are codes (ternary_codes)
     ModeCoef mc;
     // activations not packed yet (the decode kernel packs them itself): X/X2 are null and these describe
     // the [N][K] source; with two planes the ternary planes of sign(x) are formed
