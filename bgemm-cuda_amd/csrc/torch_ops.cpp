@@ -379,7 +379,8 @@ struct ProductNode : public torch::autograd::Node {
 
     variable_list apply(variable_list&& grads) override
     {
-        if (!grads[0].defined()) return variable_list(2);
+        // (what has no gradient has zeros, as the Functions have it)
+        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
         const bool need0 = task_should_compute_output(0), need1 = task_should_compute_output(1);
         std::unique_lock<std::mutex> lock(mutex_);
         const Tensor x = x_.unpack(), right = right_.unpack();

@@ -86,3 +86,32 @@ def test_what_torch_has_to_see_goes_its_way(kind):
     for t in (out, ref):
         with pytest.raises(RuntimeError, match="inplace"):
             torch.autograd.grad(t, (a, b), g.detach())
+
+
+class Stops(torch.autograd.Function):
+    """Gives what it is given, and no gradient for it."""
+
+    @staticmethod
+    def forward(ctx, t):
+        return t.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+@pytest.mark.parametrize("kind", ["scores", "context"])
+def test_no_gradient_from_above_is_zeros(kind):
+    node, fn, _ = PAIRS[kind]
+    for wants in ((0, 1), (0,), (1,)):
+        got = []
+        for f in (node, fn):
+            (a, b), args = leaves(kind, 1, 2, 40, 56, 32)
+            for i, t in enumerate((a, b)):
+                t.requires_grad_(i in wants)
+            ins, out = [(a, b)[i] for i in wants], Stops.apply(f.apply(*args()))
+            got.append(torch.autograd.grad(out, ins, torch.ones_like(out), retain_graph=True))
+            out.backward(torch.ones_like(out))
+            assert all(torch.equal(t.grad, g) for t, g in zip(ins, got[-1]))
+        for x, y, t in zip(*got, ins):
+            assert x.dtype == y.dtype == t.dtype and x.stride() == y.stride() and torch.equal(x, y) and torch.equal(x, torch.zeros_like(t))
