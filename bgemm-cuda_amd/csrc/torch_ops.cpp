@@ -43,6 +43,15 @@ struct LayerNode : public torch::autograd::Node {
     // Whether release_variables() (under its lock) follows such a pass.
     bool nothing_to_release() { return std::exchange(released_by_bias, false); }
 
+    // No gradient from above: zeros for the inputs `which`, as the binary product's Function among the separate operations gives them.
+    variable_list zeros_for(std::initializer_list<size_t> which)
+    {
+        variable_list r(num_outputs());
+        for (const size_t i : which)
+            if (task_should_compute_output(i)) r[i] = next_edge(i).function->input_metadata(next_edge(i).input_nr).zeros_like();
+        return r;
+    }
+
     // Whether torch has to see the operations of this gradient: it will itself be differentiated (in either mode), or it is no plain
     // tensor (a batch of vmap's), or something listens.
     static bool by_operations(const Tensor& grad) { return c10::GradMode::is_enabled() || !is_memory(grad) || has_tangent(grad) || is_watched(); }
@@ -120,13 +129,12 @@ struct LinearNode : public LayerNode {
 
     variable_list apply(variable_list&& grads) override
     {
-        const size_t inputs = has_bias ? 5 : 4;
-        if (!grads[0].defined()) return variable_list(inputs);
         if (bias_alone()) return {Tensor(), Tensor(), Tensor(), Tensor(), grads[0]};
         const bool want_x = task_should_compute_output(0), want_w = task_should_compute_output(1), want_sw = task_should_compute_output(2),
                    want_sa = task_should_compute_output(3), want_b = has_bias && task_should_compute_output(4);
         std::unique_lock<std::mutex> lock(mutex_);
         TORCH_CHECK(planes.defined(), torch::autograd::ERR_BACKWARD_TWICE);
+        if (!grads[0].defined()) return zeros_for({0, 1});
         const c10::OptionalDeviceGuard guard(planes.device());
         const int32_t* const p = planes.data_ptr<int32_t>();
         const int32_t* const pw = p + 2 * words_x;
@@ -268,11 +276,10 @@ struct ElasticNode : public LayerNode {
 
     variable_list apply(variable_list&& grads) override
     {
-        const size_t inputs = has_bias ? 5 : 4;
-        if (!grads[0].defined()) return variable_list(inputs);
         if (bias_alone()) return {Tensor(), Tensor(), Tensor(), Tensor(), grads[0]};
         std::unique_lock<std::mutex> lock(mutex_);
         TORCH_CHECK(planes.defined(), torch::autograd::ERR_BACKWARD_TWICE);
+        if (!grads[0].defined()) return zeros_for({0, 1, 2, 3});
         if (by_operations(grads[0])) {
             const Tensor x = planes.narrow(0, xs_at(), N * K).view(at::kFloat).view(x_shape), w = planes.narrow(0, ws_at(), M * K).view(at::kFloat).view({M, K});
             lock.unlock();                          // (whoever waits for the lock may hold the interpreter's)
