@@ -9,14 +9,15 @@
 // the halving, copies of the head-split gradients) 12 heads of 64, 4 x 512 tokens, took 20 launches and a dozen passes over 25 MB;
 // here each product pair is one launch that reads or writes an [N][M] matrix once a product, in its own order, and the gradients
 // leave in the operands' strides.  What is left is that traffic: the contraction is D = 32 .. 128 long on one side, far below what
-// the matrix cores could do in the time.  48 matrices of 512 x 512, D = 64: scores 19.6 -> 16.0 us, context 30.8 -> 18.2, the latter's two
-// halves 10.4 (25 MB written) and 12.8 (25 MB read) alone.  Blocks of a matrix on one XCD did most of it: dealt round robin, an XCD read the
-// same eighth of every row, from few of its L2's channels, and the scores' second reading came from beyond its L2 (a pass of one product
-// 15 -> 12 us).  Fragments that lie across the rows come out of LDS by transposing reads (two-byte ones: 96 for 24), and grad_P leaves
-// from registers, 128 bytes of a row a half-wave (through LDS in 64 x 64 tiles 18.1 -> 11.9).  A wave's life is then half waiting for memory and a
-// quarter vector instructions, at 1.5 blocks a unit.  Not ahead: stretches of 128 rows (15.0 and 17.6, but 64 x 64 3.9 -> 4.5),
-// two of them in flight (172 registers: 15.2 -> 19.8), eight waves a block with stretches of their own and no barrier before the sums meet (scores
-// 22.7, context 19.4; 64 x 64 5.4).
+// the matrix cores could do in the time.  48 matrices of 512 x 512, D = 64, launches in turn: scores 18.9 -> 12.0 us, context 28.8 -> 13.8, the
+// latter's two halves 8.8 (25 MB written) and 8.6 (25 MB read) alone.  Blocks of a matrix on one XCD: dealt round robin, an XCD reads the
+// same eighth of every row, from few of its L2's channels, and the scores' second reading comes from beyond its L2 (192 matrices: 43 and 51
+// us for 63 and 59; a few long ones are the same).  Fragments that lie across the rows come out of LDS by transposing reads (two-byte ones: 96 for
+// 24), and grad_P leaves from registers, 128 bytes of a row a half-wave.  A block's steps are a chain: loads, signs or weights, LDS, products.  So
+// signs are seven instructions a word (is_signed; with packed minima, which the compiler takes apart into compares and selects, twice as
+// many: 4 x 2048^2, D = 64, scores 34.9 for 29.3), and weights are formed on the way into LDS, not where they are loaded (V's gradient alone
+// 45.9 for 32.5).  Not ahead: stretches of 128 rows, two of them in flight, eight waves a block with stretches of their own and no barrier
+// before the sums meet.
 #include "common.h"
 #include <type_traits>
 
@@ -42,25 +43,17 @@ __device__ __forceinline__ __half* head_at(const HeadView& v, const int z, const
     return const_cast<__half*>(v.p) + (z / inner) * v.so + (z % inner) * v.si;
 }
 
-// Two fp16 numbers at a time: 1 where a number is neither zero nor NaN.
-typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ ushort2v is_signed(const unsigned x)
+// Two fp16 numbers at a time: bit 15 of each where it is neither zero nor NaN.  (Sums that stay within their halves: 1 .. 0x7c00 are those
+// that 0x7fff carries into bit 15 and 0x3ff does not.)
+__device__ __forceinline__ unsigned is_signed(const unsigned x)
 {
-    const ushort2v one = {1, 1}, inf = {0x7c00, 0x7c00}, a = __builtin_bit_cast(ushort2v, x & 0x7fff7fffu);
-    return __builtin_elementwise_min(a, one) - __builtin_elementwise_min(__builtin_elementwise_sub_sat(a, inf), one);
+    const unsigned m = x & 0x7fff7fffu;
+    return (m + 0x7fff7fffu) & ~(m + 0x03ff03ffu) & 0x80008000u;
 }
 // Their signs; zeros and NaN give 0.
-__device__ __forceinline__ unsigned sign_pair(const unsigned x)
-{
-    const ushort2v one = {0x3c00, 0x3c00};
-    return __builtin_bit_cast(unsigned, (ushort2v)(is_signed(x) * one)) | (x & 0x80008000u);
-}
+__device__ __forceinline__ unsigned sign_pair(const unsigned x) { return (is_signed(x) >> 15) * 0x3c00u | (x & 0x80008000u); }
 // Two entries of P -> their weights.
-__device__ __forceinline__ unsigned weight_pair(const unsigned x)
-{
-    const ushort2v step = {0x400, 0x400}, half = {0x3800, 0x3800};
-    return __builtin_bit_cast(unsigned, (ushort2v)(is_signed(x) * step + half));
-}
+__device__ __forceinline__ unsigned weight_pair(const unsigned x) { return 0x38003800u + (is_signed(x) >> 5); }
 __device__ __forceinline__ uint4 sign8(const uint4 x) { return make_uint4(sign_pair(x.x), sign_pair(x.y), sign_pair(x.z), sign_pair(x.w)); }
 __device__ __forceinline__ uint4 weight8(const uint4 x) { return make_uint4(weight_pair(x.x), weight_pair(x.y), weight_pair(x.z), weight_pair(x.w)); }
 // Eight rows of a column each: lane (c, h) gets rows row0 + 8 h .. + 7 of column col0 + c of a staged matrix, by two reads that transpose 4 x 4
@@ -118,8 +111,6 @@ __device__ __forceinline__ void tall_product(const AttnGradArgs& a, const HeadVi
                         if (col + e < a.M) d[e >> 1] |= (unsigned)__half_as_ushort(from[e]) << (16 * (e & 1));
                     v = make_uint4(d[0], d[1], d[2], d[3]);
                 }
-                // (entries that do not exist then weigh something, in rows of the output that do not exist either)
-                if constexpr (WEIGHTS) v = weight8(v);
             }
             xreg[p] = v;
         }
@@ -143,8 +134,10 @@ __device__ __forceinline__ void tall_product(const AttnGradArgs& a, const HeadVi
         __syncthreads();
 #pragma unroll
         for (int p = 0; p < XLOADS; p++) {
+            // (weights here and not where they are loaded, which would wait for each load; entries that do not exist weigh something, in rows
+            // of the output that do not exist either or against zeros of Y)
             const int u = tid + 256 * p;
-            *reinterpret_cast<uint4*>(xs + u / XW * XROW + u % XW * 8) = xreg[p];
+            *reinterpret_cast<uint4*>(xs + u / XW * XROW + u % XW * 8) = WEIGHTS ? weight8(xreg[p]) : xreg[p];
         }
 #pragma unroll
         for (int j = 0; j < YLOADS; j++) {
@@ -303,7 +296,10 @@ static int attention_backward(const char* who, const bool context, const void* m
     for (int i = 0; i < 12; i++)
         if (strides[i] % 8) return fail(BGEMM_EALIGN, "%s: strides must be multiples of 8", who);
     const int64_t nb = cdiv(N, 64), mb = cdiv(M, 64);
-    // (enough blocks of grad_P for eight a compute unit)
+    // A strip's columns: more of them read G's rows once, while there are eight blocks a compute unit.  grad_P alone, us with 64 columns, up to 128,
+    // 256 and 512: 192 x 512^2 D = 64 25.5, 22.3, D = 128 48.6, 35.8; 64 x 1024^2 D = 64 33.8, 28.0, 25.0, D = 128 62.7, 45.7, 37.2; 768 x 512^2 D = 64 147,
+    // 132, 112, 107, D = 128 262, 190, 154, 144.  D = 32 hardly cares (64 x 1024^2 22.5, 22.8, 22.9).  From half as many blocks on: D = 128 faster,
+    // 35.5 -> 29.5, but 64 x 1024^2 D = 64 25.8 -> 27.3.
     int64_t chunks = 1;
     while (chunks < 8 && batch * cdiv(N, 128) * cdiv(M, 128 * chunks) >= 2048) chunks *= 2;
     const int64_t strips = cdiv(N, 128) * cdiv(M, 64 * chunks);
