@@ -457,16 +457,16 @@ __global__ __launch_bounds__(KW * 64, FUSEX && KW <= 8 ? 4 : 2) void gemm_skinny
 // ---- split-K kernel that packs more rows than four itself ---------------------------------------
 // 5 to 32 rows (two planes: 16) of no more than a block packs about as quickly as its weights arrive: RT weight row tiles a block, a K-tile a
 // wave, and the waves meet in LDS as above.  A lane turns eight elements of a row into a byte of signs (and one of
-// nonzeros) by gathering the elements' high bytes and a dot product with the bits' weights, 6 vector instructions (12 for the
+// nonzeros) by gathering the elements' high bytes and a dot product with the bits' weights, 6 vector instructions (14 for the
 // nonzeros); the bytes of four rows of four lanes, transposed among those lanes, are a word a lane, which goes to its place in the
 // wave's operand tile in LDS: one write in place of four.  (Whole words a lane need no transposition, but its loads then touch four times
-// the lines: 16 x 4096 ternary rows x 11008 9.3 us for 8.2.)  Rows that do not exist are neither loaded nor cleared: a row of the
+// the lines: a seventh longer for 16 ternary rows.)  Rows that do not exist are neither loaded nor cleared: a row of the
 // operand meets no other, and their outputs are not stored.
-// What bounds it: latency, launch, rows and weights, and from there on the packing, 0.4 to 0.7 us for eight rows of 4096 (ternary 1.8).  Eight
-// waves with two K-tiles each, both requested at once, take 0.3 to 1.5 us more (16 x 4096 x 11008 6.8 / 6.2, 32 x 4096 x 4096 7.4 / 6.4); waves that
+// What bounds it: latency, launch, rows and weights, and from there on the packing, which every block repeats: from a graph, x 4096 x 11008, 8 rows of
+// fp16 5.1 us, ternary 5.4, fp32 6.6; 16 rows 5.8, 6.6, 7.7.  (Ternary 7.7 with nonzeros by a packed minimum, which the compiler takes apart into
+// compares and selects.)  Eight waves with two K-tiles each, both requested at once, take 0.3 to 1.5 us more; waves that
 // walk over further ones of a longer K are as slow as two launches.
 
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 // Sign bits of eight fp16 (element e at bit 14 - e), whose high bytes hold them.
@@ -475,12 +475,11 @@ __device__ __forceinline__ unsigned signs8(const v4i v)
     const unsigned p0 = __builtin_amdgcn_perm(v.y, v.x, 0x07050301u) & 0x80808080u, p1 = __builtin_amdgcn_perm(v.w, v.z, 0x07050301u) & 0x80808080u;
     return __builtin_amdgcn_udot4(p0, 0x10204080u, __builtin_amdgcn_udot4(p1, 0x01020408u, 0u, false), false);
 }
-// Which of eight fp16 are not zero (element e at bit 7 - e).
+// Which of eight fp16 are not zero (element e at bit 14 - e): 0x7fff carries what is not into the sign's place.
 __device__ __forceinline__ unsigned nonzeros8(const v4i v)
 {
-    auto ones = [](const int d) { return __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_bit_cast(u16x2, d & 0x7fff7fff), u16x2{1, 1})); };
-    const unsigned p0 = __builtin_amdgcn_perm(ones(v.y), ones(v.x), 0x06040200u), p1 = __builtin_amdgcn_perm(ones(v.w), ones(v.z), 0x06040200u);
-    return __builtin_amdgcn_udot4(p0, 0x10204080u, __builtin_amdgcn_udot4(p1, 0x01020408u, 0u, false), false);
+    auto carry = [](const int d) { return (int)(((unsigned)d & 0x7fff7fffu) + 0x7fff7fffu); };
+    return signs8(v4i{carry(v.x), carry(v.y), carry(v.z), carry(v.w)});
 }
 
 constexpr int ROWS_KT = 16;            // K-tiles: waves of a block
@@ -565,7 +564,10 @@ __global__ __launch_bounds__(ROWS_KT * 64) void gemm_skinny_rows_kernel(const Ge
                 }
                 const unsigned s = signs8(v);
                 sg |= i == 0 ? s >> 7 : s << (8 * i - 7);
-                if (TWO) nz |= nonzeros8(v) << (8 * i);
+                if (TWO) {
+                    const unsigned n = nonzeros8(v);
+                    nz |= i == 0 ? n >> 7 : n << (8 * i - 7);
+                }
             }
             const int at = (g0 + g) * 32;
             sg = transpose4(sg);
@@ -1149,11 +1151,10 @@ bool gemm_skinny_fusex_shape(int planes, int64_t M, int64_t N)
 }
 
 // Whether a product of 5 to 32 unpacked rows goes to the kernel that packs them itself: rows of whole aligned 16-byte pieces, a K-tile a
-// wave and one round of blocks.  GPU time from a graph, us, two launches / one, N x K x M: fp16 signs 5 x 4096 x 11008 7.2 / 5.1, 32 x 4096 x 11008
-// 8.1 / 7.8, 32 x 4096 x 4096 6.7 / 6.4, 16 x 2048 x 2048 5.9 / 4.1, 32 x 768 x 11008 8.5 / 6.0; ternary 8 x 4096 x 11008 6.8 / 5.8, 16 x 2048 x 16384 6.5 / 5.8, 16 x
-// 3000 x 3000 6.4 / 5.7, 16 x 4096 x 11008 7.3 / 7.7; fp32 8 x 4096 x 11008 7.2 / 6.7, 16 x 4096 x 11008 7.4 / 7.7, 32 x 1024 x 8192 7.0 / 6.0, 32 x 2048 x 2048
-// 6.2 / 6.6 but 24 x 4096 x 4096 6.6 / 7.6.  A call without a graph is the host's time, a launch and an allocation less: 10.2 / 6.4 us a layer, also
-// where the GPU takes some percent longer.  Two rounds of blocks are behind (16 x 2048 x 22016 7.6 / 9.6).
+// wave and one round of blocks.  GPU time from a graph over eight weights, us, two launches / one, N x K x M: fp16 signs 5 x 4096 x 11008 6.9 / 5.0,
+// 32 x 4096 x 11008 7.4 / 7.2, 32 x 4096 x 4096 6.4 / 6.0, 16 x 3000 x 3000 6.6 / 4.4, 32 x 768 x 11008 7.1 / 4.6; ternary 8 x 4096 x 11008 7.0 / 5.4, 16 x 4096 x 11008
+// 7.2 / 6.6, 16 x 3000 x 3000 6.8 / 4.6, 16 x 4096 x 768 6.2 / 5.0; fp32 8 x 4096 x 11008 6.9 / 6.6, 32 x 1024 x 8192 6.1 / 4.5, 32 x 2048 x 2048 5.9 / 5.2 but
+// 24 x 4096 x 4096 6.3 / 7.8.  Two rounds of blocks are behind or not much ahead (32 x 4096 x 22016 8.3 / 11.3, ternary 8 x 4096 x 22016 7.8 / 8.0).
 bool gemm_skinny_rows_shape(int planes, int x_f32, const void* x, int64_t ldx, int64_t M, int64_t N, int64_t K)
 {
     return N >= 5 && N <= (planes == 2 ? 16 : 32) && !(planes == 2 && x_f32) && (!x_f32 || N * K <= 65536) && k_tiles(K) <= ROWS_KT && M <= 16384 && K % 8 == 0 &&
