@@ -62,6 +62,7 @@ SIGNATURES = {
     "bgemm_packed_weight_forward_supported": (_int, [_int, _i64, _i64, _i64]),
     "bgemm_packed_weight_forward": (_int, [_int, _p, _p, _int, _i64, _p, _p, _int, _i64, _i64, _i64, _int, _p, _p, _p, _p, _p]),
     "bgemm_unpacked_workspace_bytes": (_sz, [_int, _p, _int, _i64, _i64, _i64, _i64]),
+    "bgemm_unpacked_workspace_bytes_on": (_sz, [_int, _p, _int, _i64, _i64, _i64, _i64, _p]),
     "bgemm_unpacked_forward": (_int, [_int, _p, _p, _int, _i64, _p, _p, _int, _i64, _i64, _i64, _p, _p, _p, _p, _sz, _p]),
     "bgemm_f16_workspace_bytes": (_sz, [_i64, _i64, _i64, _int]),
     "bgemm_f16_forward": (_int, [_p, _p, _p, _i64, _i64, _i64, _p, _sz, _int, _int, _p]),

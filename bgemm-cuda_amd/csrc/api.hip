@@ -368,11 +368,33 @@ static bool ternary_as_codes(int mode, int out_dtype, int64_t M, int64_t N, int6
            gemm_mfma_kernel_id(1, M, N, k_tiles(K), 2, out_dtype, true) == BGEMM_KERNEL_MFMA_128x256T;
 }
 
+// Bytes for the planes, whatever the route; 0: no shape of ours.
+static size_t unpacked_planes_bytes(int mode, int64_t M, int64_t N, int64_t K, ModeCoef* mc)
+{
+    if (!mode_coef(mode, mc) || M <= 0 || N <= 0 || K <= 0 || K >= (1LL << 24)) return 0;
+    return mc->planes * round256((size_t)bgemm_tiled_words(N, K) * 4);
+}
+
+static bool being_captured(void* stream)
+{
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &s) == hipSuccess) return s == hipStreamCaptureStatusActive;
+    (void)hipGetLastError();         // (the call's launches will say what is wrong with the stream)
+    return false;
+}
+
 extern "C" size_t bgemm_unpacked_workspace_bytes(int mode, const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_t K)
 {
     ModeCoef mc;
-    if (!mode_coef(mode, &mc) || M <= 0 || N <= 0 || K <= 0 || K >= (1LL << 24) || gemm_skinny_rows_shape(mc.planes, x_dtype == BGEMM_SRC_F32, x, ldx, M, N, K)) return 0;
-    return mc.planes * round256((size_t)bgemm_tiled_words(N, K) * 4);
+    const size_t bytes = unpacked_planes_bytes(mode, M, N, K, &mc);
+    return bytes && gemm_skinny_rows_shape(mc.planes, x_dtype == BGEMM_SRC_F32, x, ldx, M, N, K) ? 0 : bytes;
+}
+
+extern "C" size_t bgemm_unpacked_workspace_bytes_on(int mode, const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_t K, void* stream)
+{
+    const size_t bytes = bgemm_unpacked_workspace_bytes(mode, x, x_dtype, ldx, M, N, K);
+    ModeCoef mc;
+    return bytes || !gemm_skinny_rows_behind(x_dtype == BGEMM_SRC_F32, M, N, K) || !being_captured(stream) ? bytes : unpacked_planes_bytes(mode, M, N, K, &mc);
 }
 
 extern "C" int bgemm_unpacked_forward(int mode, const void* W_tiled, const void* x, int x_dtype, int64_t ldx, const void* x_zero_point,
@@ -394,12 +416,13 @@ extern "C" int bgemm_unpacked_forward(int mode, const void* W_tiled, const void*
     if (scaled && (!sw || !sa)) return fail(BGEMM_ENULL, "%s: sw or sa is NULL", who);
     if (((uintptr_t)x & (f32 ? 3 : 1)) || ((uintptr_t)ws & 255) || ((uintptr_t)W_tiled & 15) || ((uintptr_t)out & ((1u << out_elem_shift(out_dtype)) - 1)))
         return fail(BGEMM_EALIGN, "%s: an operand is not aligned", who);
-    if (gemm_skinny_rows_shape(mc.planes, f32, x, ldx, M, N, K)) {
+    const size_t need = unpacked_planes_bytes(mode, M, N, K, &mc);
+    if (gemm_skinny_rows_shape(mc.planes, f32, x, ldx, M, N, K) &&
+        !(ws && ws_bytes >= need && gemm_skinny_rows_behind(f32, M, N, K) && being_captured(stream))) {
         const RawActivations raw = {x, f32, ldx, x_zero_point, true};
         return packed_forward(mode, W_tiled, nullptr, nullptr, out, out_dtype, 1, M, N, K, 0, 0, N * M, 1, BGEMM_VARIANT_AUTO, nullptr, 0, nullptr, 0,
                               scaled ? sw : nullptr, scaled ? sa : nullptr, scaled ? bias : nullptr, nullptr, stream, &raw);
     }
-    const size_t need = bgemm_unpacked_workspace_bytes(mode, x, x_dtype, ldx, M, N, K);
     if (!ws) return fail(BGEMM_ENULL, "%s: null pointer", who);
     if (ws_bytes < need) return fail(BGEMM_EWORKSPACE, "%s: workspace %zu < %zu bytes", who, ws_bytes, need);
     char* const p0 = (char*)ws;

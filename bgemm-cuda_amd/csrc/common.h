@@ -392,6 +392,7 @@ bool gemm_skinny_shape(int planes, int64_t batch, int64_t M, int64_t N, int64_t 
 bool gemm_skinny_fusex_shape(int planes, int64_t M, int64_t N);
 int launch_gemm_skinny(const GemmArgs& a, hipStream_t st, bool fp4);
 bool gemm_skinny_rows_shape(int planes, int x_f32, const void* x, int64_t ldx, int64_t M, int64_t N, int64_t K);      // unpacked rows, more than four
+bool gemm_skinny_rows_behind(int x_f32, int64_t M, int64_t N, int64_t K);      // of those: two launches are quicker on the GPU
 int launch_gemm_skinny_rows(const GemmArgs& a, hipStream_t st);
 // Split-K needs of each family for a shape: bytes of partial-tile scratch, number of counters.
 // (for the split that will actually be used: zero when the shape is not split at all)

@@ -1161,6 +1161,15 @@ bool gemm_skinny_rows_shape(int planes, int x_f32, const void* x, int64_t ldx, i
            (uintptr_t)x % 16 == 0 && ldx * (x_f32 ? 4 : 2) % 16 == 0 && ldx <= (1 << 20);
 }
 
+// Whether the GPU takes longer over that launch than over two: more than eight rows of fp32, whose 16 KB (K = 4096) each block fetches from its L2.
+// Two launches / one from a graph, us: 16 x 4096 x 11008 7.1 / 7.7, 9 x 4096 x 8192 6.2 / 6.5, 18 x 3328 x 8192 + 14 %; but 16 x 3072 x 11008 6.9 / 6.4,
+// 24 x 2560 x 11008 - 2 %, 16 x 4096 x 1024 - 6 %.  Outside a graph the host is slower than both, and one launch is a launch and an allocation
+// less for it (16 x 4096 x 11008 8.6 / 7.6 a call, x 4096 8.5 / 6.6): two are taken where the stream is being captured.
+bool gemm_skinny_rows_behind(int x_f32, int64_t M, int64_t N, int64_t K)
+{
+    return x_f32 && N > 8 && M >= 4096 && (K > 3584 || cdiv(N, 8) * K > 8192);
+}
+
 // Two row tiles a block, which share the packing, where one would be more than a block a compute unit.
 int launch_gemm_skinny_rows(const GemmArgs& a, hipStream_t st)
 {

@@ -113,11 +113,12 @@ bool quiet_call(PyObject* x) { return !c10::GradMode::is_enabled() && plain_gpu(
 void unpacked(const int mode, const Tensor& w, const Rows& x, const Tensor& zp, const Tensor& out, const int kind, const int64_t M, const int64_t N, const int64_t K,
               const Tensor& sw, const Tensor& sa, const Tensor& bias)
 {
-    const size_t bytes = bgemm_unpacked_workspace_bytes(mode, x.t.data_ptr(), src_type(x.t), x.ld, M, N, K);
+    void* const st = stream_of(out);
+    const size_t bytes = bgemm_unpacked_workspace_bytes_on(mode, x.t.data_ptr(), src_type(x.t), x.ld, M, N, K, st);
     Tensor ws;
     if (bytes) ws = at::empty({(int64_t)bytes}, x.t.options().dtype(at::kByte).requires_grad(false));
     check(bgemm_unpacked_forward(mode, w.data_ptr(), x.t.data_ptr(), src_type(x.t), x.ld, data_or_null(zp), out.data_ptr(), kind, M, N, K, data_or_null(sw),
-                                 data_or_null(sa), data_or_null(bias), data_or_null(ws), bytes, stream_of(out)));
+                                 data_or_null(sa), data_or_null(bias), data_or_null(ws), bytes, st));
 }
 
 // linear_infer(module.__dict__, x) -> y

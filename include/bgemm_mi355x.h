@@ -254,8 +254,12 @@ int bgemm_packed_weight_forward(int mode, const void* W_tiled, const void* x, in
 /* Prepacked weights x activations as they are, any number of rows: the pack of the activations (bgemm_pack_sign_centered /
  * bgemm_pack_ternary_f16) and the packed entry point in one call, in whatever form between them suits the size.  out_dtype: BGEMM_OUT_I32,
  * F16 or the scaled kinds (sw, sa; bias optional, as bgemm_packed_forward_scaled).  ws: 256-byte aligned scratch of
- * bgemm_unpacked_workspace_bytes, which need not be initialised (0: a few rows, which one launch packs and multiplies; ws may be NULL). */
+ * bgemm_unpacked_workspace_bytes, which need not be initialised (0: a few rows, which one launch packs and multiplies, and ws may be NULL;
+ * or arguments that the call refuses, as with the other queries).  _bytes_on is the same for a call on that stream: if the stream is being
+ * captured it asks for scratch also for some of those few rows, fp32 ones, which two launches of a graph get through sooner.  Without it
+ * they are one launch there too. */
 size_t bgemm_unpacked_workspace_bytes(int mode, const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_t K);
+size_t bgemm_unpacked_workspace_bytes_on(int mode, const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_t K, void* stream);
 int bgemm_unpacked_forward(int mode, const void* W_tiled, const void* x, int x_dtype, int64_t ldx, const void* x_zero_point,
                            void* out, int out_dtype, int64_t M, int64_t N, int64_t K, const void* sw, const void* sa,
                            const void* bias, void* ws, size_t ws_bytes, void* stream);

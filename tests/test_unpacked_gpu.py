@@ -82,3 +82,29 @@ def test_few_rows_in_one_launch(N, M, K, ld, dtype):
                 got = lk.bgemm_packed_weight_forward(w, x, mode, x_zero_point=zp, scale=scale, **({"out_dtype": out} if out else {}))
                 want = lk.bgemm_packed_forward(w, xp, mode, out or torch.int32, scale=scale)[0]
                 assert got.dtype == want.dtype and torch.equal(got, want), (mode, None if zp is None else zp.item(), out, scale is not None)
+
+
+# fp32 rows whose captured call is two launches, on both sides of that rule: rows, K, rows of eight times K, columns
+@pytest.mark.parametrize("N,M,K,two", [(9, 4096, 3592, True), (9, 4096, 3584, False), (8, 4096, 4096, False), (16, 4095, 4096, False), (16, 16384, 4096, True), (17, 4100, 2736, True),
+                                       (24, 4100, 2728, False), (32, 5000, 2048, False), (25, 5000, 2056, True)])
+def test_rows_captured_are_the_rows_of_a_call(N, M, K, two):
+    g = torch.Generator(device=DEV).manual_seed(N * M + K)
+    L, w, x = _lib.lib(), lk.pack_sign(torch.randn(M, K, generator=g, device=DEV).half()), torch.randn(N, K, generator=g, device=DEV)
+    zp, sw, sa = torch.full((1,), 0.1, device=DEV), torch.randn(M, generator=g, device=DEV), torch.full((1,), 0.3, device=DEV)
+    args = (lk.MODE_XOR, x.data_ptr(), lk.SRC_F32, K, M, N, K)
+    calls = (lambda: lk.bgemm_packed_weight_forward(w, x, lk.MODE_XOR, x_zero_point=zp, scale=(sw, sa, sw)), lambda: lk.bgemm_packed_weight_forward(w, x, lk.MODE_AND))
+    bare = torch.empty(N, M, dtype=torch.int32, device=DEV)
+    [f() for f in calls]
+    assert L.bgemm_unpacked_workspace_bytes(*args) == 0 and L.bgemm_unpacked_workspace_bytes_on(*args, lk._stream()) == 0
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        bytes_on = L.bgemm_unpacked_workspace_bytes_on(*args, lk._stream())
+        got = [f() for f in calls]
+        # (no scratch: one launch there too)
+        _lib.check(L.bgemm_unpacked_forward(lk.MODE_AND, w.data.data_ptr(), x.data_ptr(), lk.SRC_F32, K, None, bare.data_ptr(), lk.OUT_I32, M, N, K, None, None, None, None, 0, lk._stream()))
+    assert bool(bytes_on) == two
+    for _ in range(3):
+        x.copy_(torch.randn(N, K, generator=g, device=DEV))
+        want = [f() for f in calls]
+        graph.replay()
+        assert all(torch.equal(a, b) for a, b in zip([*got, bare], [*want, want[1]]))
