@@ -251,6 +251,7 @@ static int packed_forward(int mode, const void* W_tiled, const void* X_tiled, co
             a.ws_cnt = (uint32_t*)counters;
         }
     }
+    if (codes && (v == BGEMM_VARIANT_VALU || skinny)) return fail(BGEMM_EINVAL, "bgemm_packed_forward: codes are for the signed ternary tile");
     if (v == BGEMM_VARIANT_VALU) return launch_gemm_valu(a, (hipStream_t)stream);
     if (skinny) return launch_gemm_skinny(a, (hipStream_t)stream, fp4);
     return launch_gemm_mfma(a, (hipStream_t)stream, fp4);
@@ -362,10 +363,11 @@ extern "C" int bgemm_packed_weight_forward(int mode, const void* W_tiled, const 
 // few instructions more (tiles x K-tiles; us a call, planes / codes, N x K x M): 11008: 2048 x 4096 x 11008 int32 52.8 / 50.0, fp16 scaled 47.3 / 46.0,
 // 2048 x 11008 x 4096 48.0 / 46.9; 12288: 1500 x 8192 x 8192 54.7 / 52.6; 8192: 2048 x 4096 x 8192 40.0 / 37.5; but 2752: 400 x 4096 x 11008
 // 19.1 / 19.3, 1376: 2048 x 512 x 11008 21.6 / 21.9; 1088: 1024 x 2048 x 4352 15.1 / 15.1.
+// (the packed entry point itself is asked which kernel it will run)
 static bool ternary_as_codes(int mode, int out_dtype, int64_t M, int64_t N, int64_t K)
 {
-    return mode == BGEMM_MODE_BWTA && cdiv(N, 128) * cdiv(M, 256) * k_tiles(K) >= 4096 && pick_variant(mode, 1, M, N, K) == BGEMM_VARIANT_MFMA_F4 && !gemm_skinny_shape(2, 1, M, N, K) &&
-           gemm_mfma_kernel_id(1, M, N, k_tiles(K), 2, out_dtype, true) == BGEMM_KERNEL_MFMA_128x256T;
+    return mode == BGEMM_MODE_BWTA && cdiv(N, 128) * cdiv(M, 256) * k_tiles(K) >= 4096 &&
+           bgemm_packed_kernel_id(mode, out_dtype, 1, M, N, K, 8, BGEMM_VARIANT_AUTO) == BGEMM_KERNEL_MFMA_128x256T;
 }
 
 // Bytes for the planes, whatever the route; 0: no shape of ours.

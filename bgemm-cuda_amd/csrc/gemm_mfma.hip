@@ -993,6 +993,8 @@ static int launch_eng(const GemmArgs& a, hipStream_t st)
 
 int launch_gemm_mfma(const GemmArgs& a, hipStream_t st, bool fp4)
 {
+    if (a.codes && (!fp4 || (a.force >= 0 ? a.force : gemm_mfma_kernel_id(a.batch, a.M, a.N, a.KT, a.mc.planes, a.out_kind, fp4)) != BGEMM_KERNEL_MFMA_128x256T))
+        return fail(BGEMM_EINVAL, "gemm_mfma: codes are for the signed ternary tile");
     return fp4 ? launch_eng<EngF4>(a, st) : launch_eng<EngI8>(a, st);
 }
 

@@ -46,6 +46,23 @@ def test_ternary_rows_as_codes_are_the_two_planes(N, M, K, dtype):
     assert torch.equal(lk.bgemm_packed_weight_forward(ones, wide[:, 3:], lk.MODE_BWTA), -K * wide[:, :1].int().expand(N, M))
 
 
+# Which form the activations take, read from the scratch: codes from 4096 tiles x K-tiles on where the signed tile runs, planes elsewhere
+@pytest.mark.parametrize("N,M,K,codes", [(2048, 4096, 4096, True), (2048, 4096, 3840, False), (1025, 5000, 8000, True), (2048, 16000, 1792, True), (2048, 512, 65536, False), (128, 4096, 65536, False),
+                                         (64, 131072, 2048, False), (129, 8200, 16384, False), (512, 11008, 8192, True)])
+def test_the_form_of_ternary_rows(N, M, K, codes):
+    L, g = _lib.lib(), torch.Generator(device=DEV).manual_seed(N + M + K)
+    signed = L.bgemm_packed_kernel_id(lk.MODE_BWTA, lk.OUT_I32, 1, M, N, K, 8, lk.VARIANT_AUTO) == lk._b.KERNEL_MFMA_128x256T
+    assert codes == (signed and -(-N // 128) * -(-M // 256) * -(-K // 256) >= 4096)
+    w, x = lk.pack_sign(torch.randn(M, K, generator=g, device=DEV).half()), tern(g, N, K, torch.half, False)
+    out, ws = torch.empty(N, M, dtype=torch.int32, device=DEV), torch.empty(L.bgemm_unpacked_workspace_bytes(lk.MODE_BWTA, x.data_ptr(), lk.SRC_F16, K, M, N, K), dtype=torch.uint8, device=DEV)
+    _lib.check(L.bgemm_unpacked_forward(lk.MODE_BWTA, w.data.data_ptr(), x.data_ptr(), lk.SRC_F16, K, None, out.data_ptr(), lk.OUT_I32, M, N, K, None, None, None, ws.data_ptr(), ws.numel(), lk._stream()))
+    planes = lk.pack_ternary(x)
+    words = planes.data.numel()
+    first = ws.view(torch.int32)[:words].view_as(planes.data)
+    assert torch.equal(first, planes.data) != codes
+    assert torch.equal(out, lk.bgemm_packed_forward(w, planes, lk.MODE_BWTA, torch.int32)[0])
+
+
 def test_sign_rows_and_refusals():
     g = torch.Generator(device=DEV).manual_seed(3)
     w, x = lk.pack_sign(torch.randn(4100, 700, generator=g, device=DEV).half()), torch.randn(1030, 700, generator=g, device=DEV)
