@@ -19,6 +19,9 @@ namespace bgemm_native {
 
 using at::Tensor;
 
+// The module's functions as _lib.py knows them (NATIVE_VERSION there): another number when one is added or called another way.
+constexpr long NATIVE_VERSION = 1;
+
 // Turns a negative status into the exception _lib.check() raises.
 inline void check(const int rc)
 {

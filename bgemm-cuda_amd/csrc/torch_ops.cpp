@@ -482,7 +482,7 @@ PyMODINIT_FUNC PyInit__bgemm_native(void)
     module_def.m_methods = all_methods();
     PyObject* const module = PyModule_Create(&module_def);
     // what it was built for: an older one lacks functions that the Python side calls
-    if (module && PyModule_AddIntConstant(module, "abi_version", BGEMM_ABI_VERSION) != 0) {
+    if (module && (PyModule_AddIntConstant(module, "abi_version", BGEMM_ABI_VERSION) != 0 || PyModule_AddIntConstant(module, "native_version", NATIVE_VERSION) != 0)) {
         Py_DECREF(module);
         return nullptr;
     }

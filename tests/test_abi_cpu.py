@@ -407,15 +407,24 @@ def test_a_library_of_another_version_says_so(tmp_path, monkeypatch):
     monkeypatch.setattr(_lib, "SO_PATH", str(so))
     with pytest.raises(ImportError, match="rebuild it"):
         _lib.lib()
+    # of this version, from before an entry point was added
+    src.write_text("int bgemm_abi_version(void) { return %d; }\n" % _lib.ABI_VERSION)
+    subprocess.check_call([gcc, "-shared", "-fPIC", str(src), "-o", str(tmp_path / "older.so")])
+    monkeypatch.setattr(_lib, "SO_PATH", str(tmp_path / "older.so"))
+    with pytest.raises(ImportError, match="rebuild it"):
+        _lib.lib()
 
 
 def test_a_native_host_side_of_another_version_says_so(tmp_path, monkeypatch):
-    """One from before it stated its version, and one of the version before this."""
+    """One from before it stated its version, one of the version before this, and two of this that lack functions added since: one from before
+    it counted them, and one of another count."""
     gcc = shutil.which("gcc")
     if not gcc:
         pytest.skip("no gcc")
     state = 'PyObject* m = PyModule_Create(&def); PyModule_AddIntConstant(m, "abi_version", %d); return m;' % (_lib.ABI_VERSION - 1)
-    for i, body in enumerate(("return PyModule_Create(&def);", state)):
+    now = state.replace(str(_lib.ABI_VERSION - 1), str(_lib.ABI_VERSION))
+    count = now.replace("return m;", 'PyModule_AddIntConstant(m, "native_version", %d); return m;' % (_lib.NATIVE_VERSION - 1))
+    for i, body in enumerate(("return PyModule_Create(&def);", state, now, count)):
         src, so = tmp_path / ("old%d.c" % i), tmp_path / ("old%d.so" % i)
         src.write_text('#include <Python.h>\nstatic struct PyModuleDef def = {PyModuleDef_HEAD_INIT, "_bgemm_native", 0, -1, 0};\n'
                        'PyMODINIT_FUNC PyInit__bgemm_native(void) { %s }\n' % body)
@@ -426,7 +435,7 @@ def test_a_native_host_side_of_another_version_says_so(tmp_path, monkeypatch):
             _lib.native()
     monkeypatch.undo()
     monkeypatch.setattr(_lib, "_native", None)
-    assert _lib.native().abi_version == _lib.ABI_VERSION
+    assert _lib.native().abi_version == _lib.ABI_VERSION and _lib.native().native_version == _lib.NATIVE_VERSION
 
 
 def test_a_native_host_side_that_does_not_load_says_so_on_every_call(tmp_path, monkeypatch):
