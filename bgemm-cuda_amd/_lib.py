@@ -17,7 +17,7 @@ MODE_AND, MODE_XOR, MODE_ATTN, MODE_BWTA, MODE_ATTN_X = 0, 1, 2, 3, 4
 OUT_I32, OUT_F16, OUT_F32_SCALED, OUT_F16_SCALED, OUT_BITS_F32, OUT_BITS_F16 = 0, 1, 2, 3, 4, 5
 SRC_F16, SRC_F32, SRC_BITS = 0, 1, 2
 ABI_VERSION = 12
-NATIVE_VERSION = 1     # of the native part's functions (torch_common.h): another when one is added or called another way
+NATIVE_VERSION = 2     # of the native part's functions (torch_common.h): another when one is added or called another way
 LAYOUT_VERSION = 6     # of the tiled operand layout, written into packed files; changes only when the layout does
 STATIC_SCRATCH_BYTES = 32 << 20      # BGEMM_STATIC_SCRATCH_BYTES
 VARIANT_AUTO, VARIANT_VALU, VARIANT_MFMA, VARIANT_MFMA_F4 = 0, 1, 2, 3

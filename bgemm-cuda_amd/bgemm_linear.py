@@ -76,20 +76,22 @@ def _batched_packed(x_rows, right, mode):
 
 
 # The longest rows the one-launch gradients take, timed up to 4096 against the separate operations (us a backward pass, D = 32 .. 128,
-# 1 to 64 matrices).  The context's kernel is ahead everywhere (16 x 4096^2, D = 128: 1577 -> 744).  The scores' reads an [N][M] matrix
-# twice, which is ahead while the caches hold one (16 x 3072^2, D = 64: 153 -> 146) and not when each reading comes from memory
-# (16 x 4096^2: 217 -> 260).
+# 1 to 192 matrices).  The context's kernel is ahead everywhere (16 x 4096^2, D = 128: 1582 -> 328).  The scores' walks along a row in one chain,
+# where the library splits it: from a graph 12 x 64 x 2560, D = 128, 36 -> 44, 1 x 100 x 3072 20 -> 48, 1 x
+# 3072^2, D = 32, 33 -> 34; and it reads an [N][M] matrix twice, which is level where each reading comes from memory (16 x 4096^2, D = 64, 214 -> 209).  Up to
+# 2048 rows it is ahead (1 x 2048^2, D = 32 .. 128, 21 to 40 -> 17 to 33), and so it is beyond them for many square matrices (4 x 3072^2, D = 64, 73 -> 45),
+# which this line leaves to the library.
 SCORES_GRAD_ROWS, CONTEXT_GRAD_ROWS = 2048, 4096
-SCORES_GRAD_PRODUCT = 6 << 30          # multiplications above D = 64: see _scores_grad_ahead
+SCORES_GRAD_NARROW, SCORES_GRAD_PRODUCT = 96, 6 << 30          # columns, and multiplications a product above those: see _scores_grad_ahead
 
 
 def _scores_grad_ahead(batch, N, M, D):
-    """Whether the scores' one-launch gradients are worth taking at a size their kernel supports.  Its time is that of fetching
-    fragments from LDS, which grows with D while the library products it stands for hardly do.  Above D = 64 the two meet at 6 to
-    8 * 2^30 multiplications a product (D = 96: 64 x 1024^2 = 6 * 2^30 104 -> 88 us, 64 x 1536^2 183 -> 194, 64 x 2048^2 288 -> 324;
-    D = 128: 16 x 1536^2 = 4.5 * 2^30 103 -> 72, 64 x 1024^2 = 8 * 2^30 102 -> 115, 16 x 2048^2 101 -> 115, 64 x 2048^2 306 -> 416); up to
-    64 the kernel is ahead at every such size (D = 64: 64 x 1024^2 104 -> 75, 64 x 1536^2 158 -> 145, 64 x 2048^2 265 -> 253)."""
-    return max(N, M) <= SCORES_GRAD_ROWS and (D <= 64 or batch * N * M * D < SCORES_GRAD_PRODUCT)
+    """Whether the scores' one-launch gradients are worth taking at a size their kernel supports.  Its time grows with D (signs, LDS
+    and products of a step), while that of the library products it stands for hardly does.  At D = 128 the two meet at 6 to
+    8 * 2^30 multiplications a product (192 x 512^2 = 6 * 2^30 87 -> 69 us, 16 x 1536^2 = 4.5 * 2^30 56 -> 46, but 64 x 1024^2 = 8 * 2^30 70 -> 81,
+    16 x 2048^2 60 -> 80, 64 x 2048^2 301 -> 317); up to 96 the kernel is ahead at every such size (D = 96: 64 x 1024^2 73 -> 59, from a graph
+    66 -> 66, 64 x 1536^2 187 -> 140, 64 x 2048^2 300 -> 240; D = 64: 64 x 1024^2 58 -> 46, 64 x 2048^2 264 -> 197)."""
+    return max(N, M) <= SCORES_GRAD_ROWS and (D <= SCORES_GRAD_NARROW or batch * N * M * D < SCORES_GRAD_PRODUCT)
 
 
 def _any_tangent(*tensors):
@@ -146,7 +148,7 @@ class bgemm_matmul(torch.autograd.Function):
             native = _lib.native_or_none()
             if native is not None:
                 mode = lowbit_kernel.MODE_AND if len(args) == 3 and args[2] == 'and' else lowbit_kernel.MODE_XOR
-                out = native.product_train(args[0], args[1], mode, SCORES_GRAD_ROWS, SCORES_GRAD_PRODUCT)
+                out = native.product_train(args[0], args[1], mode, SCORES_GRAD_ROWS, SCORES_GRAD_NARROW, SCORES_GRAD_PRODUCT)
                 if out is not None:
                     return out
         return super().apply(*args, **kwargs)
@@ -184,7 +186,7 @@ class bgemm_attn_matmul(torch.autograd.Function):
                 and lowbit_kernel.context_backward is _CONTEXT_BACKWARD):
             native = _lib.native_or_none()
             if native is not None:
-                out = native.product_train(args[0], args[1], lowbit_kernel.MODE_ATTN_X, CONTEXT_GRAD_ROWS, 1 << 62)
+                out = native.product_train(args[0], args[1], lowbit_kernel.MODE_ATTN_X, CONTEXT_GRAD_ROWS, 0, 1 << 62)
                 if out is not None:
                     return out
         return super().apply(*args, **kwargs)

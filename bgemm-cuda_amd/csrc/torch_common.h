@@ -20,7 +20,7 @@ namespace bgemm_native {
 using at::Tensor;
 
 // The module's functions as _lib.py knows them (NATIVE_VERSION there): another number when one is added or called another way.
-constexpr long NATIVE_VERSION = 1;
+constexpr long NATIVE_VERSION = 2;
 
 // Turns a negative status into the exception _lib.check() raises.
 inline void check(const int rc)
@@ -81,10 +81,10 @@ inline Rows rows_2d(const Tensor& t)
 
 // x [.., N, K] @ right [.., K, M] of binarised operands, one launch over the batch -> fp16 [.., N, M]; undefined: a form it does not take.
 Tensor batched_product_of(const Tensor& x, const Tensor& right, int mode);
-// The gradients of such a product by their one-launch kernel (bgemm_linear._one_launch_grads, and `most` multiplications a product above 64
-// columns); false: a form it does not take.
-bool attention_grads(bool context, const Tensor& m, const Tensor& a, const Tensor& b, bool need0, bool need1, int64_t longest, int64_t most, Tensor& g0,
-                     Tensor& g1);
+// The gradients of such a product by their one-launch kernel (bgemm_linear._one_launch_grads and, above `narrow` columns, fewer than `most`
+// multiplications a product: _scores_grad_ahead); false: a form it does not take.
+bool attention_grads(bool context, const Tensor& m, const Tensor& a, const Tensor& b, bool need0, bool need1, int64_t longest, int64_t narrow, int64_t most,
+                     Tensor& g0, Tensor& g1);
 
 // Functions of the inference and attention part, for the module's table.
 extern PyMethodDef infer_methods[];

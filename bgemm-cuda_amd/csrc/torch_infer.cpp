@@ -586,10 +586,10 @@ void launch_grads(const bool context, const Tensor& m0, const Tensor& a, const T
 }  // namespace
 
 bool attention_grads(const bool context, const Tensor& m, const Tensor& a, const Tensor& b, const bool need0, const bool need1, const int64_t longest,
-                     const int64_t most, Tensor& g0, Tensor& g1)
+                     const int64_t narrow, const int64_t most, Tensor& g0, Tensor& g1)
 {
     if (!is_memory(m) || !is_memory(a) || !is_memory(b) || !grads_match(m, a, b) || !grads_in_one(a, b, longest)) return false;
-    if (a.size(-1) > 64 && a.numel() * b.size(-2) >= most) return false;
+    if (a.size(-1) > narrow && a.numel() * b.size(-2) >= most) return false;
     launch_grads(context, m, a, b, need0, need1, g0, g1);
     return true;
 }

@@ -372,7 +372,7 @@ PyObject* elastic_train(PyObject*, PyObject* const* args, const Py_ssize_t n)
 // of 64, half of that waiting for the interpreter's lock on the engine's thread.
 struct ProductNode : public torch::autograd::Node {
     bool context;
-    int64_t longest, most;
+    int64_t longest, narrow, most;
     SavedVariable x_, right_;
 
     std::string name() const override { return context ? "BinaryContextBackward" : "BinaryScoresBackward"; }
@@ -395,8 +395,8 @@ struct ProductNode : public torch::autograd::Node {
         const Tensor& g = grads[0];
         if (!LayerNode::by_operations(g) && g.scalar_type() == at::kHalf && !has_tangent(x) && !has_tangent(right)) {
             Tensor g0, g1;
-            const bool done = context ? attention_grads(true, x, g, right, need0, need1, longest, most, g0, g1)
-                                      : attention_grads(false, g, x, right.transpose(-1, -2), need0, need1, longest, most, g0, g1);
+            const bool done = context ? attention_grads(true, x, g, right, need0, need1, longest, narrow, most, g0, g1)
+                                      : attention_grads(false, g, x, right.transpose(-1, -2), need0, need1, longest, narrow, most, g0, g1);
             if (done) return {g0, !context && g1.defined() ? g1.transpose(-1, -2) : g1};
         }
         pybind11::gil_scoped_acquire gil;
@@ -421,15 +421,15 @@ struct ProductNode : public torch::autograd::Node {
     }
 };
 
-// product_train(x [.., N, K], right [.., K, M], mode, longest, most) -> fp16 [.., N, M], or None where the Function has to run
+// product_train(x [.., N, K], right [.., K, M], mode, longest, narrow, most) -> fp16 [.., N, M], or None where the Function has to run
 PyObject* product_train(PyObject*, PyObject* const* args, const Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    TORCH_CHECK_TYPE(n == 5, "product_train takes 5 arguments");
+    TORCH_CHECK_TYPE(n == 6, "product_train takes 6 arguments");
     if (!c10::GradMode::is_enabled() || !plain_call(args, 2)) Py_RETURN_NONE;
     const Tensor &x = tensor_at(args[0]), &right = tensor_at(args[1]);
     const int mode = (int)PyLong_AsLong(args[2]);
-    const int64_t longest = PyLong_AsLongLong(args[3]), most = PyLong_AsLongLong(args[4]);
+    const int64_t longest = PyLong_AsLongLong(args[3]), narrow = PyLong_AsLongLong(args[4]), most = PyLong_AsLongLong(args[5]);
     if (PyErr_Occurred()) throw python_error();
     if (!x.requires_grad() && !right.requires_grad()) Py_RETURN_NONE;
     for (const Tensor* t : {&x, &right})
@@ -444,7 +444,7 @@ PyObject* product_train(PyObject*, PyObject* const* args, const Py_ssize_t n)
         if (out.defined()) {
             auto node = std::shared_ptr<ProductNode>(new ProductNode(), torch::autograd::deleteNode);
             node->context = mode == BGEMM_MODE_ATTN_X;
-            node->longest = longest; node->most = most;
+            node->longest = longest; node->narrow = narrow; node->most = most;
             node->x_ = SavedVariable(x, false);
             node->right_ = SavedVariable(right, false);
             node->set_next_edges(torch::autograd::collect_next_edges(x, right));

@@ -24,7 +24,9 @@ def bound(terms):
                                            (1, 5, 130, 200, 64), (4, 12, 512, 512, 64),
                                            # both sides of the dispatch's limits on the rows
                                            (1, 1, 2048, 100, 32), (1, 1, 2049, 100, 32), (1, 1, 90, 2049, 64), (1, 1, 4096, 100, 32),
-                                           (1, 1, 4097, 100, 32)])
+                                           (1, 1, 4097, 100, 32),
+                                           # and of the one on the products, which is for heads of more than 96 columns
+                                           (48, 1, 1024, 1024, 128), (47, 1, 1024, 1024, 128), (64, 1, 1024, 1024, 96)])
 def test_gradients(B, H, N, M, d, monkeypatch):
     g = torch.Generator(device=DEV).manual_seed(N * 131 + M)
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).half()
