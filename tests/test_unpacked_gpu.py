@@ -93,6 +93,10 @@ def test_few_rows_in_one_launch(N, M, K, ld, dtype):
         ternary = mode == lk.MODE_BWTA
         x = (torch.randint(-1, 2, (N, ld), generator=g, device=DEV) if ternary else torch.randn(N, ld, generator=g, device=DEV)).to(dtype)
         x = torch.where(torch.rand(N, ld, generator=g, device=DEV) < 0.3, special[torch.randint(0, 9, (N, ld), generator=g, device=DEV)], x)[:, :K]
+        f32 = dtype == torch.float32
+        one = (5 <= N <= (16 if ternary else 32) and K <= 4096 and K % 8 == 0 and ld * (4 if f32 else 2) % 16 == 0 and M <= 16384
+               and not (f32 and (ternary or N * K > 65536)))
+        assert one == (_lib.lib().bgemm_unpacked_workspace_bytes(mode, x.data_ptr(), lk.SRC_F32 if f32 else lk.SRC_F16, ld, M, N, K) == 0)
         for zp in (None,) if ternary else (None, special[8:], special[2:3]):
             xp = lk.pack_ternary(x) if ternary else lk.pack_sign(x, zero_point=zp)
             for out, scale in ((torch.int32, None), (torch.half, None), (None, (sw, sa, sw)), (None, (sw, sa, None))):
