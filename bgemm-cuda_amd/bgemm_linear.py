@@ -132,19 +132,14 @@ def _context_grads(need, attn, value, grad_out):
     return (g @ v.transpose(-1, -2)) / 2, a01.transpose(-1, -2) @ g
 
 
-_SCORES_BACKWARD, _CONTEXT_BACKWARD = lowbit_kernel.scores_backward, lowbit_kernel.context_backward
-
-
 class bgemm_matmul(torch.autograd.Function):
     """matA [.., N, K] @ matB [K, M] with both operands binarised by sign (bgemm_linear.py:9-42).
     A matB with leading dimensions ([B, H, K, M], as K^T in attention) is a batched matmul."""
 
     @classmethod
     def apply(cls, *args, **kwargs):
-        # Recorded products of fp16 batches are one native node; everything else is this Function, also where a program has put
-        # something else in the place of the gradients' launch, which the Function calls by its name.
-        if (cls is bgemm_matmul and not kwargs and 2 <= len(args) <= 3 and torch.is_grad_enabled()
-                and lowbit_kernel.scores_backward is _SCORES_BACKWARD):
+        # Recorded products of fp16 batches are one native node; everything else is this Function.
+        if cls is bgemm_matmul and not kwargs and 2 <= len(args) <= 3 and torch.is_grad_enabled():
             native = _lib.native_or_none()
             if native is not None:
                 mode = lowbit_kernel.MODE_AND if len(args) == 3 and args[2] == 'and' else lowbit_kernel.MODE_XOR
@@ -182,8 +177,7 @@ class bgemm_attn_matmul(torch.autograd.Function):
 
     @classmethod
     def apply(cls, *args, **kwargs):
-        if (cls is bgemm_attn_matmul and not kwargs and 2 <= len(args) <= 3 and torch.is_grad_enabled()
-                and lowbit_kernel.context_backward is _CONTEXT_BACKWARD):
+        if cls is bgemm_attn_matmul and not kwargs and 2 <= len(args) <= 3 and torch.is_grad_enabled():
             native = _lib.native_or_none()
             if native is not None:
                 out = native.product_train(args[0], args[1], lowbit_kernel.MODE_ATTN_X, CONTEXT_GRAD_ROWS, 0, 1 << 62)
