@@ -20,7 +20,8 @@
 // start tile by tile, operands of +-1 on both sides (11 vector instructions a word of keys instead of 5), and every wave waiting for
 // each word that a block prepares; the last also where there are few waves: 4 x 512 tokens 36 -> 16.4, 8 x 256 20 -> 10.2.  With a whole
 // group's sums on their way (210 registers, two waves a SIMD) 36.9.  A head's blocks are on one XCD: 30.9 -> 30.1, and what the launch behind it
-// takes 17.3 -> 16.2 and 13.6 -> 12.3 (bits of neighbouring heads written into one cache).
+// takes 13.6 -> 12.3 (bits of neighbouring heads written into one cache): the whole block 58.6 -> 57.0 from a graph, also where the kernel alone is
+// not ahead (4 x 512 tokens 18.2 -> 18.6, the block 33.6 -> 33.1; 8 x 256 12.5 and 12.5, 27.7 -> 26.8; 1 x 1024, 16 heads, 29.2 -> 29.6, 45.9 -> 45.6).
 #include "common.h"
 #include "attention_bits.h"
 #include <math.h>
@@ -53,7 +54,8 @@ __global__ __launch_bounds__(512) void attention_kernel(const AttnArgs a)
     uint32_t* const kb = reinterpret_cast<uint32_t*>(tbl + D + 2);                           // [W][S64]
     uint32_t* const vt = kb + W * S64;                                                       // [2 groups][D]: words of 32 keys
 
-    const int id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), bh = id / a.qblocks, qb = id % a.qblocks, b = bh / a.heads, head = bh % a.heads;
+    const unsigned id = xcd_contiguous_id(blockIdx.x, gridDim.x);
+    const int bh = id / a.qblocks, qb = id % a.qblocks, b = bh / a.heads, head = bh % a.heads;
     const int64_t row0 = (int64_t)b * S;
     auto word = [&](const uint32_t* p, const int row, const int w) { return p[tiled_word_offset(row0 + row, head * W + w, a.KT)]; };
 

@@ -259,7 +259,8 @@ template <int DT>
 __global__ __launch_bounds__(256) void scores_grad_kernel(const AttnGradArgs a)
 {
     __shared__ __align__(16) unsigned char smem[ag_lds<DT>()];
-    const int id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), z = id / a.per_batch, t = id % a.per_batch;
+    const unsigned id = xcd_contiguous_id(blockIdx.x, gridDim.x);
+    const int z = id / a.per_batch, t = id % a.per_batch;
     if (t < a.first) tall_product<DT, false, false>(a, a.b, a.ga, z, t * 64, smem);
     else tall_product<DT, true, false>(a, a.a, a.gb, z, (t - a.first) * 64, smem);
 }
@@ -271,10 +272,11 @@ __global__ __launch_bounds__(256) void context_grad_kernel(const AttnGradArgs a)
     // (the longer blocks first)
     const int tall = a.batch * a.first;
     if ((int)blockIdx.x < tall) {
-        const int id = (int)xcd_contiguous_id(blockIdx.x, tall);
+        const unsigned id = xcd_contiguous_id(blockIdx.x, tall);
         return tall_product<DT, true, true>(a, a.a, a.gb, id / a.first, id % a.first * 64, smem);
     }
-    const int id = (int)xcd_contiguous_id(blockIdx.x - tall, gridDim.x - tall), strips = a.per_batch - a.first, u = id % strips;
+    const unsigned id = xcd_contiguous_id(blockIdx.x - tall, gridDim.x - tall), strips = a.per_batch - a.first;
+    const int u = id % strips;
     const int mb = (a.M + 64 * a.chunks - 1) / (64 * a.chunks);
     probs_strip<DT>(a, id / strips, u / mb * 128, u % mb * 64 * a.chunks, smem);
 }

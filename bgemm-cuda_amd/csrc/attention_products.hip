@@ -20,6 +20,7 @@ struct AttnProductArgs {
     AttnView a, b;                    // scores: A, B.  context: P, V
     __half* out;                      // [batch][N][M] or [batch][N][D], dense
     int N, M, inner, nblocks, mblocks, both_negative, past;
+    int one_xcd;                      // scores: a matrix's blocks on one XCD
 };
 
 constexpr int AP_COLS = 256;      // of a block of the scores
@@ -59,8 +60,8 @@ __global__ __launch_bounds__(WAVES * 64) void scores_kernel(const AttnProductArg
     __shared__ uint32_t qb[W * AP_ROWS], kb[W * AP_COLS];
     __shared__ __align__(16) unsigned char stages[WAVES][32 * ATTN_STAGE];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, c = lane & 31;
-    // (a matrix's blocks on one XCD, which reads its operands once: 48 of 512 x 512, D = 64, 8.1 -> 7.4 us under the profiler, the context 13.0 -> 11.9)
-    const int per = a.nblocks * a.mblocks, id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), z = id / per, t = id % per;
+    const unsigned id = a.one_xcd ? xcd_contiguous_id(blockIdx.x, gridDim.x) : blockIdx.x, per = a.nblocks * a.mblocks;
+    const int z = id / per, t = id % per;
     const int n0 = t / a.mblocks * AP_ROWS, m0 = t % a.mblocks * AP_COLS;
     {
         RowBits<W, AP_COLS, THREADS> kr;
@@ -162,6 +163,7 @@ __global__ __launch_bounds__(512, W == 4 ? 2 : 4) void context_kernel(const Attn
     uint32_t* const vb = reinterpret_cast<uint32_t*>(smem);      // [W][S64]: words of a row of V
     uint32_t* const vt = vb + W * S64;                           // [2 groups][D]: words of 32 rows
     unsigned char* const stage = reinterpret_cast<unsigned char*>(vt + W * S64) + wave * 256;
+    // (a matrix's blocks on one XCD: 48 x 512^2, D = 64, 10.7 -> 9.8 us from a graph, 192 x 512^2 28.5 -> 24.9, few matrices level)
     const int id = (int)xcd_contiguous_id(blockIdx.x, gridDim.x), z = id / a.nblocks, q0 = id % a.nblocks * CTX_ROWS + (wave & 3) * 32;
     const int first = groups * part / parts, end = q0 < a.N ? groups * (part + 1) / parts : first;
     const __half* v = view_at(a.b, z, a.inner);
@@ -323,6 +325,11 @@ extern "C" int bgemm_scores_forward(int mode, const void* a, const void* b, cons
     g.nblocks = (int)cdiv(N, waves * 32); g.mblocks = (int)cdiv(M, AP_COLS);
     g.both_negative = mode == BGEMM_MODE_AND;
     g.past = M % 32 == 0 && ((uintptr_t)out & 63) == 0;
+    // Blocks of a matrix go to one XCD, which reads its operands once, where an L2 does not hold the operands of all matrices anyway, and where
+    // lines that two blocks share would be written by two XCDs.  From a graph, us, round robin / one XCD: 192 x 512^2 D = 64 23.4 / 20.1, 64 x 1024^2
+    // 30.7 / 25.9, 128 x 512^2 D = 128 20.6 / 16.8, 96 x 512^2 D = 32 (6 MB of operands) 11.4 / 10.6, 16 x 1000^2 13.3 / 11.9; but 32 x 1024^2 D = 32 (4 MB)
+    // 13.8 / 15.0, 16 x 1024^2 7.9 / 8.5, and 64 x 1024^2 26.8 / 27.6.  Short rows: 192 x 256^2 D = 32 6.9 / 7.7, 400 x 256^2 D = 128 15.5 / 17.3, 48 x 384 x 400 D = 64 8.1 / 8.4.
+    g.one_xcd = M >= 500 && (M % 64 != 0 || (batch * (N + M) * D * 2 >= 6 << 20 && (D > 32 || M <= 512)));
     const int64_t blocks = batch * g.nblocks * g.mblocks;
     if (blocks > 0x7fffffffLL) return fail(BGEMM_EINVAL, "%s: too many blocks", who);
     const dim3 grid((unsigned)blocks), block(waves * 64);
