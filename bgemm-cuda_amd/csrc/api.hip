@@ -360,9 +360,10 @@ extern "C" int bgemm_packed_weight_forward(int mode, const void* W_tiled, const 
 // ---- prepacked weights x activations as they are, any number of rows -------------------------------------------------------------
 // Workspace layout: [plane] [second plane], each rounded to 256 bytes.
 // A ternary operand goes as codes to the tile that multiplies signed operands, where there is enough of that loop to make up for the pack's
-// few instructions more (tiles x K-tiles; us a call, planes / codes, N x K x M): 11008: 2048 x 4096 x 11008 int32 52.8 / 50.0, fp16 scaled 47.3 / 46.0,
-// 2048 x 11008 x 4096 48.0 / 46.9; 12288: 1500 x 8192 x 8192 54.7 / 52.6; 8192: 2048 x 4096 x 8192 40.0 / 37.5; but 2752: 400 x 4096 x 11008
-// 19.1 / 19.3, 1376: 2048 x 512 x 11008 21.6 / 21.9; 1088: 1024 x 2048 x 4352 15.1 / 15.1.
+// few instructions more (tiles x K-tiles; us from a graph, planes / codes, N x K x M, int32): 11008: 2048 x 4096 x 11008 53.5 / 50.6; 10368: 3000 x 9000 x
+// 3000 63.6 / 60.5; 8192: 4096^3 41.8 / 40.6; 6400: 2048 x 5120 x 5120 40.4 / 38.0; 5504: 1024 x 4096 x 11008 32.8 / 30.7, 2048 x 2048 x 11008 34.6 / 33.8,
+// 4096 x 1024 x 11008 42.1 / 42.4; 4096: 2048 x 4096 x 4096 25.8 / 25.6, 4096 x 2048 x 4096 28.4 / 27.8, 8192 x 1024 x 4096 35.4 / 36.0.  A call, below the line:
+// 2752: 400 x 4096 x 11008 19.1 / 19.3; 1376: 2048 x 512 x 11008 21.6 / 21.9; 1088: 1024 x 2048 x 4352 15.1 / 15.1.
 // (the packed entry point itself is asked which kernel it will run)
 static bool ternary_as_codes(int mode, int out_dtype, int64_t M, int64_t N, int64_t K)
 {

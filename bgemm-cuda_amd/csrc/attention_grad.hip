@@ -16,7 +16,7 @@
 // 24), and grad_P leaves from registers, 128 bytes of a row a half-wave.  A block's steps are a chain: loads, signs or weights, LDS, products.  So
 // signs are seven instructions a word (is_signed; with packed minima, which the compiler takes apart into compares and selects, twice as
 // many: 4 x 2048^2, D = 64, scores 34.9 for 29.3), and weights are formed on the way into LDS, not where they are loaded (V's gradient alone
-// 45.9 for 32.5).  Not ahead: stretches of 128 rows, two of them in flight, eight waves a block with stretches of their own and no barrier
+// 45.9 for 32.5).  Waves still wait for 43 (scores) and 48 % of their cycles, vector units are busy for 23 and 21 %, the matrix cores 6.  Not ahead: stretches of 128 rows, two of them in flight, eight waves a block with stretches of their own and no barrier
 // before the sums meet.
 #include "common.h"
 #include <type_traits>
@@ -265,6 +265,9 @@ __global__ __launch_bounds__(256) void scores_grad_kernel(const AttnGradArgs a)
     else tall_product<DT, true, false>(a, a.a, a.gb, z, (t - a.first) * 64, smem);
 }
 
+// Both halves share the registers of the larger, the strips: 4, 3, 3 and 2 waves a SIMD at D = 32 .. 128, where P's half by itself has one or two more.
+// Both gradients take the same time either way; V's alone would gain where the chip is full (64 x 1024^2 D = 64 31.6 -> 26.4 us, 768 x 512^2 D = 128
+// 173 -> 155) and nothing where it is not (48 x 512^2 8.8 -> 8.5).
 template <int DT>
 __global__ __launch_bounds__(256) void context_grad_kernel(const AttnGradArgs a)
 {

@@ -760,11 +760,12 @@ def bgemm_packed_weight_forward(w, x, mode=MODE_XOR, out_dtype=torch.int32, scal
                                 variant=VARIANT_AUTO):
     """Prepacked weights ``w`` (M rows) x activations ``x`` as they are, fp16 or fp32 ``[N,K]`` -> ``[N,M]``.
 
-    For the few rows of a decode step (N <= 4; up to 32, ternary 16, where K is at most 4096 and rows are aligned) this is ONE
-    launch: the kernel forms the
-    activation bits itself (``MODE_BWTA``: the ternary planes of sign(x); the other modes: sign bits of ``x``
-    or, with ``x_zero_point``, of ``(x - x_zero_point).to(torch.half)``).  Larger batches go through the pack
-    kernel and the packed entry point: same results either way.  ``scale`` as in bgemm_packed_forward."""
+    For the few rows of a decode step (N <= 4) this is ONE launch: the kernel forms the activation bits itself (``MODE_BWTA``: the
+    ternary planes of sign(x); the other modes: sign bits of ``x`` or, with ``x_zero_point``, of ``(x - x_zero_point).to(torch.half)``).
+    Larger batches go through the native host part to ``bgemm_unpacked_forward``, which packs up to 32 rows (ternary 16) in
+    the launch that multiplies them where K is at most 4096 and rows are aligned, and writes many ternary rows as codes; without that
+    part, or where something has to see the steps, they are a pack and the packed entry point.  Same results every way.  ``scale`` as in
+    bgemm_packed_forward."""
     if variant == VARIANT_AUTO and type(w) is PackedBits and w.data2 is None and w.batch == 1:
         native = _b.native_or_none()
         if native is not None:
