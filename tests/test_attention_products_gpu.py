@@ -103,7 +103,9 @@ def test_the_contexts_kernel_at_its_limits(B, H, N, M, D):
 
 # blocks of eight waves (256 rows, from 192 of them on) at every D that has them, and of four; whole and ragged column blocks
 @pytest.mark.parametrize("D", [32, 64, 96, 128])
-@pytest.mark.parametrize("B, H, N, M", [(16, 12, 256, 64), (16, 12, 200, 64), (8, 12, 250, 300), (8, 12, 511, 31), (2, 3, 256, 300)])
+@pytest.mark.parametrize("B, H, N, M", [(16, 12, 256, 64), (16, 12, 200, 64), (8, 12, 250, 300), (8, 12, 511, 31), (2, 3, 256, 300),
+                                        # a matrix's blocks on one XCD: broken rows (and 499, which are not), many operands, also of D = 32 up to 512 columns
+                                        (3, 3, 130, 501), (3, 3, 130, 499), (11, 9, 520, 512), (11, 9, 520, 576)])
 def test_the_scores_kernel_in_blocks_of_four_and_eight_waves(B, H, N, M, D):
     g = torch.Generator(device=DEV).manual_seed(N + M + D)
     q, k = operand(g, (B, H, N, D), "heads"), operand(g, (B, H, M, D), "odd")

@@ -9,8 +9,8 @@ F32, F16, BITS_F32 = _lib.OUT_F32_SCALED, _lib.OUT_F16_SCALED, _lib.OUT_BITS_F32
 
 @pytest.mark.parametrize("batch, N, M, D, ahead", [
     (1, 1, 1, 32, True), (64, 2048, 2048, 64, True), (1, 2049, 8, 32, False), (1, 8, 2049, 32, False), (1, 2048, 2048, 128, True),
-    # measured on both sides of the limit on D > 64
-    (16, 1536, 1536, 128, True), (64, 1024, 1024, 128, False), (16, 2048, 2048, 128, False), (64, 1536, 1536, 96, False),
+    # measured on both sides of the limit on D > 96, which D = 96 does not know
+    (16, 1536, 1536, 128, True), (64, 1024, 1024, 128, False), (16, 2048, 2048, 128, False), (64, 1536, 1536, 96, True), (64, 1536, 1536, 128, False),
     (11, 2048, 2048, 128, True), (12, 2048, 2048, 128, False), (12, 2047, 2048, 128, True)])
 def test_scores_gradients_go_where_they_are_ahead(batch, N, M, D, ahead):
     assert bl._scores_grad_ahead(batch, N, M, D) is ahead
